@@ -201,6 +201,26 @@ int wkv6_shift_mix_x_backward(void *stream, int dtype, int64_t B, int64_t T, int
                               const void *x, const float *mix_x, const void *gp, const void *gxx, const void *gxm,
                               void *gx, float *gmix_x);
 
+/* The same with the products in between, i.e. the whole of x -> (xr, xk, xv, xw, xg) and its gradients:
+ *   wkv6_shift_mix_forward:  h = tanh(x_mix A^T) and the five outputs.  a (5R,C): the five mixers' dense_a
+ *       weights as (out, in), stacked; a and w2t are both bf16 or both fp32 (weight_dtype) and enter the
+ *       products as bf16.  `weights` (wkv6_shift_mix_weights_bytes) receives the forms the kernels read;
+ *       it and h are what the backward needs besides x.
+ *   wkv6_shift_mix_backward: gx (B,T,C), ga (5R,C) and gw2t (5,C,R) in weight_dtype, gbias (5,C) and gmix_x (C)
+ *       fp32.  `workspace`: wkv6_shift_mix_backward_workspace_bytes(...) bytes, contents meaningless before
+ *       and after. */
+size_t wkv6_shift_mix_weights_bytes(int64_t C, int64_t R);
+int wkv6_shift_mix_forward(void *stream, int dtype, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R,
+                           const void *x, const float *mix_x, const void *a, const void *w2t, const float *bias,
+                           void *weights, size_t weights_bytes, void *h,
+                           void *xr, void *xk, void *xv, void *xw, void *xg);
+size_t wkv6_shift_mix_backward_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t C, int64_t R);
+int wkv6_shift_mix_backward(void *stream, int dtype, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R,
+                            const void *x, const float *mix_x, const float *bias, const void *weights, const void *h,
+                            const void *gxr, const void *gxk, const void *gxv, const void *gxw, const void *gxg,
+                            void *gx, float *gmix_x, void *ga, void *gw2t, float *gbias,
+                            void *workspace, size_t workspace_bytes);
+
 /* Backward of the stateless forward: gr,gk,gv,gw (B,T,C) and gu (B,C), all in the output type.
  * Replaces backward_{bf16,fp16,fp32}(B,T,C,H,r,k,v,w,u,gy,gr,gk,gv,gw,gu),
  * rwkv_kernel/torch_kernel/wkv6_op.cpp:33-41 (kernel_backward_101/102/103/201,

@@ -300,6 +300,44 @@ int wkv6_shift_mix_x_backward(void *stream, int dtype, int64_t B, int64_t T, int
     return finish(wkv6::shift_mix_x_backward((hipStream_t)stream, B, T, C, x, mix_x, gp, gxx, gxm, gx, gmix_x));
 }
 
+size_t wkv6_shift_mix_weights_bytes(int64_t C, int64_t R) {
+    return wkv6::shift_mix_supported(C, R) ? wkv6::shift_mix_weights_bytes(C, R) : 0;
+}
+
+size_t wkv6_shift_mix_backward_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t C, int64_t R) {
+    return check_mix(dtype, B, T, C, R) == WKV6_OK ? wkv6::shift_mix_backward_workspace_bytes(B, T, C, R) : 0;
+}
+
+int wkv6_shift_mix_forward(void *stream, int dtype, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R,
+                           const void *x, const float *mix_x, const void *a, const void *w2t, const float *bias,
+                           void *weights, size_t weights_bytes, void *h, void *xr, void *xk, void *xv, void *xw, void *xg) {
+    const int rc = check_mix(dtype, B, T, C, R);
+    if (rc != WKV6_OK) return rc;
+    if (weight_dtype != WKV6_BF16 && weight_dtype != WKV6_F32) return WKV6_ERR_ARG;
+    const void *const all[] = {x, mix_x, a, w2t, bias, h, xr, xk, xv, xw, xg};
+    for (const void *p : all)
+        if (!p || !aligned16(p)) return WKV6_ERR_ARG;
+    if (!weights || !aligned16(weights) || weights_bytes < wkv6::shift_mix_weights_bytes(C, R)) return WKV6_ERR_WORKSPACE;
+    void *const out[5] = {xr, xk, xv, xw, xg};
+    return finish(wkv6::shift_mix_forward((hipStream_t)stream, weight_dtype, B, T, C, R, x, mix_x, a, w2t, bias, weights, h, out));
+}
+
+int wkv6_shift_mix_backward(void *stream, int dtype, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R,
+                            const void *x, const float *mix_x, const float *bias, const void *weights, const void *h,
+                            const void *gxr, const void *gxk, const void *gxv, const void *gxw, const void *gxg,
+                            void *gx, float *gmix_x, void *ga, void *gw2t, float *gbias, void *workspace, size_t workspace_bytes) {
+    const int rc = check_mix(dtype, B, T, C, R);
+    if (rc != WKV6_OK) return rc;
+    if (weight_dtype != WKV6_BF16 && weight_dtype != WKV6_F32) return WKV6_ERR_ARG;
+    const void *const all[] = {x, mix_x, bias, weights, h, gxr, gxk, gxv, gxw, gxg, gx, gmix_x, ga, gw2t, gbias};
+    for (const void *p : all)
+        if (!p || !aligned16(p)) return WKV6_ERR_ARG;
+    if (!workspace || !aligned16(workspace) || workspace_bytes < wkv6::shift_mix_backward_workspace_bytes(B, T, C, R)) return WKV6_ERR_WORKSPACE;
+    const void *const gout[5] = {gxr, gxk, gxv, gxw, gxg};
+    return finish(wkv6::shift_mix_backward((hipStream_t)stream, weight_dtype, B, T, C, R, x, mix_x, bias, weights, h, gout,
+                                           gx, gmix_x, ga, gw2t, gbias, workspace));
+}
+
 // Size of the part of the saved block that the kernels of one pass use (chunk states, arrival
 // counters; sized so that the guarded per-timestep pass of the backward can use the same buffer).
 static size_t saved_base_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {

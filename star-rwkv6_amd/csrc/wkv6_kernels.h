@@ -198,6 +198,16 @@ hipError_t shift_mix_five_backward(hipStream_t st, int64_t B, int64_t T, int64_t
 hipError_t shift_mix_x_backward(hipStream_t st, int64_t B, int64_t T, int64_t C, const void *x, const float *mix_x,
                                 const void *gp, const void *gxx, const void *gxm, void *gx, float *gmix_x);
 
+// the whole input side with its products (wkv6_mix_train.hip); a (5R,C), w2t (5,C,R) and their gradients in weight_dtype
+// (kBF16 or kF32); `weights` receives the forms the kernels read and is handed to the backward with h
+size_t shift_mix_weights_bytes(int64_t C, int64_t R);
+hipError_t shift_mix_forward(hipStream_t st, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R, const void *x, const float *mix_x,
+                             const void *a, const void *w2t, const float *bias, void *weights, void *h, void *const out[5]);
+size_t shift_mix_backward_workspace_bytes(int64_t B, int64_t T, int64_t C, int64_t R);
+hipError_t shift_mix_backward(hipStream_t st, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R, const void *x, const float *mix_x,
+                              const float *bias, const void *weights, const void *h, const void *const gout[5],
+                              void *gx, float *gmix_x, void *ga, void *gw2t, float *gbias, void *workspace);
+
 size_t chunk_backward_workspace_bytes(int64_t B, int64_t T, int64_t H);
 // bytes of a forward -> backward hand-over buffer: the workspace plus one arrival counter per head
 // (zeroed by the saving forward, used by the backward's fused batch sum of gu)

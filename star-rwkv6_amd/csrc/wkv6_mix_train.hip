@@ -1,0 +1,826 @@
+// The whole input side of the time-mix layer with gradients (rwkv6_model.py:134-146; notation of wkv6_mix.hip):
+//
+//   h      = tanh(x_mix A^T)                         x_mix = x + xx mix_x, A the five stacked (R, C) first weights
+//   x_s    = x + xx (h_s W_s^T + bias_s)             (shift_mix_five of wkv6_mix.hip)
+// backward, from the gradients g_s of the five outputs, gcoef_s = g_s xx:
+//   gh_s   = gcoef_s W_s                             summed over channels
+//   gpre   = gh (1 - h^2),  gxm = gpre A             gradients of x_mix A^T and of x_mix
+//   gW_s   = gcoef_s^T h_s,  gbias_s = sum gcoef_s,  gA = gpre^T x_mix,  gmix = sum gxm xx      summed over tokens
+//   gx[t]  = sum_s g_s - gxx + gxm (1 - mix_x) + z[t+1],   gxx = sum_s g_s coef_s,  z = gxx + gxm mix_x
+//
+// All of it is bound by the traffic of the (B,T,C) tensors, so none of the products that appear between them is ever
+// written: x_mix, the five coefficients and the five gcoef live in registers (and, where a product sums over tokens, in
+// a wave's own LDS tile).  A sum over channels and a sum over tokens of the same gcoef cannot both be finished by one
+// workgroup, so the gradients g_s are read twice: mix_reduce_kernel<grad> takes whole rows of a few tokens (gpre
+// complete, nothing to combine between workgroups), mix_grads_kernel takes 64 channels of many tokens (the weight
+// gradients stay in accumulators, one partial per workgroup).
+// B8 T1024 C2048 R32, forward and backward through the torch flavour: 250 us; as four elementwise kernels around six
+// library products (gcoef written and read twice, x_mix written and read) 572 us, of which 235 us the skinny products.
+#include "wkv6_common.h"
+#include "wkv6_kernels.h"
+#include "wkv6_mfma.h"
+
+namespace wkv6 {
+
+constexpr int kMix = 5;          // mixers
+constexpr int kFragElems = 512;  // one operand fragment of a 16x16x32 MFMA: 64 lanes x 8 elements
+
+typedef Raw8<bf16_t> Row8;
+// eight elements at a uniform base and a 32-bit byte offset per lane (the scalar-base addressing form)
+__device__ __forceinline__ void load_row8(Row8 &r, const bf16_t *base, uint32_t byteoff) {
+    r.a = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(base) + byteoff);
+}
+
+// ---- DPP moves inside a row of 16 lanes (lane l16 = token): the previous / the next token's value -----------------
+__device__ __forceinline__ uint32_t prev_lane(uint32_t first, uint32_t x) {   // lane 0 keeps `first`
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)x, 0x111, 0xF, 0xF, false);   // row_shr:1
+}
+__device__ __forceinline__ float next_lane(float last, float x) {             // lane 15 keeps `last`
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(last), __float_as_int(x), 0x101, 0xF, 0xF, false));   // row_shl:1
+}
+__device__ __forceinline__ uint32_t last_to_first(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x121, 0xF, 0xF, false); }   // row_ror:1
+__device__ __forceinline__ float first_to_last(float x) {                                                                                     // row_ror:15
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x12F, 0xF, 0xF, false));
+}
+__device__ __forceinline__ Row8 prev_rows(const Row8 &first, const Row8 &x) {
+    Row8 p;
+    p.a.x = prev_lane(first.a.x, x.a.x); p.a.y = prev_lane(first.a.y, x.a.y);
+    p.a.z = prev_lane(first.a.z, x.a.z); p.a.w = prev_lane(first.a.w, x.a.w);
+    return p;
+}
+__device__ __forceinline__ Row8 last_row_first(const Row8 &x) {
+    Row8 p;
+    p.a.x = last_to_first(x.a.x); p.a.y = last_to_first(x.a.y); p.a.z = last_to_first(x.a.z); p.a.w = last_to_first(x.a.w);
+    return p;
+}
+// the values are final here: nothing of their computation moves past this point
+__device__ __forceinline__ void pin8(float (&v)[8]) {
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+}
+__device__ __forceinline__ bf16x8 pack_operand(const float (&v)[8]) {
+    return make_bf16x8(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+}
+
+// ------------------------------------------------------------------------------------------
+// The weights in the forms the kernels read, once per call: two MB of traffic, bound by its launch.
+//   a_frag  [C/32][5R/16][64 lanes][8]      A as operand fragments with the k-slots along 32 channels
+//   wt_frag [C/32][5][R/16][64 lanes][8]    W_s transposed, the same
+//   a_t     (C, 5R)                         A transposed
+//   w       (5, C, R)                       W in bf16
+// One workgroup per 32 channels and matrix (blockIdx.y).
+// ------------------------------------------------------------------------------------------
+template <typename Tw>
+__global__ __launch_bounds__(256) void mix_weights_kernel(int C, int R, const Tw *__restrict__ a, const Tw *__restrict__ w2t,
+        bf16_t *__restrict__ a_frag, bf16_t *__restrict__ wt_frag, bf16_t *__restrict__ a_t, bf16_t *__restrict__ w)
+{
+    __shared__ bf16_t tile[5 * 64][40];   // [stacked row (s, r)][channel of the 32]
+    const int c0 = (int)blockIdx.x * 32, rows = kMix * R;
+    const bool is_a = blockIdx.y == 0;
+    if (is_a) {
+        for (int i = threadIdx.x; i < rows * 8; i += 256) {
+            float v[4];
+            load4(a + (size_t)(i >> 3) * C + c0 + 4 * (i & 7), v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tile[i >> 3][4 * (i & 7) + e] = (bf16_t)v[e];
+        }
+    } else {
+        const int per = R / 4;   // 4-element pieces of a row of W
+        for (int i = threadIdx.x; i < kMix * 32 * per; i += 256) {
+            const int r = (i % per) * 4, c = (i / per) % 32, s = i / (per * 32);
+            float v[4];
+            load4(w2t + ((size_t)s * C + c0 + c) * R + r, v);
+            store4(w + ((size_t)s * C + c0 + c) * R + r, v[0], v[1], v[2], v[3]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tile[s * R + r + e][c] = (bf16_t)v[e];
+        }
+    }
+    __syncthreads();
+    bf16_t *frag = (is_a ? a_frag : wt_frag) + (size_t)blockIdx.x * rows * 32;
+    for (int i = threadIdx.x; i < rows * 4; i += 256) {   // fragment i / 64, lane i % 64
+        const int l = i & 63;
+        *reinterpret_cast<uint4 *>(frag + (size_t)i * 8) = *reinterpret_cast<const uint4 *>(&tile[(i >> 6) * 16 + (l & 15)][8 * (l >> 4)]);
+    }
+    if (is_a)
+        for (int i = threadIdx.x; i < 32 * (rows / 8); i += 256) {
+            const int c = i / (rows / 8), r = (i % (rows / 8)) * 8;
+            uint16_t v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = __builtin_bit_cast(uint16_t, tile[r + e][c]);
+            *reinterpret_cast<uint4 *>(a_t + (size_t)(c0 + c) * rows + r) =
+                make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
+        }
+}
+
+// ------------------------------------------------------------------------------------------
+// Sums over channels:  forward  h = tanh(x_mix A^T);  kGrad  gpre = (gcoef_s W_s)_s (1 - h^2).
+// One workgroup takes all channels of 32 tokens (16 at R = 64: the accumulators), so nothing is left to combine; its
+// eight waves take 32-channel chunks in turn and add up through LDS at the end.  The weights' fragments come from L2 once
+// per workgroup.  A chunk's x and g are fetched while the chunk before it is worked on.
+// ------------------------------------------------------------------------------------------
+constexpr int kReduceWaves = 8;
+template <int R> struct MixReduce {
+    static constexpr int kBlocks = R == 32 ? 2 : 1;          // 16-token blocks per workgroup
+    static constexpr int kTiles = kMix * R / 16;             // 16-row tiles of the stacked rank
+    static constexpr int kRound = kTiles * kBlocks / 2;      // accumulator tiles combined per round
+    static constexpr int kLds = kReduceWaves * kRound * 64 * 16;
+};
+
+template <int R, bool kGrad>
+__global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n_tok, int T, int C,
+        const bf16_t *__restrict__ x, const float *__restrict__ mix_x, const bf16_t *__restrict__ frags,
+        const bf16_t *__restrict__ g0, const bf16_t *__restrict__ g1, const bf16_t *__restrict__ g2, const bf16_t *__restrict__ g3,
+        const bf16_t *__restrict__ g4, const bf16_t *__restrict__ h, bf16_t *__restrict__ out)
+{
+    typedef MixReduce<R> M;
+    constexpr int NB = M::kBlocks, NT = M::kTiles, RT = R / 16;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tok0 = (int64_t)blockIdx.x * (16 * NB);
+    const bf16_t *const gs[kMix] = {g0, g1, g2, g3, g4};
+    const int64_t base = tok0 * C;
+    const int left = (int)(n_tok - 1 - tok0 < 16 * NB ? n_tok - 1 - tok0 : 16 * NB);   // (rows past the end: the last one once more, not stored)
+    uint32_t row[NB];
+    bool first[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int t = min(16 * b + l16, left);
+        row[b] = ((uint32_t)t * (uint32_t)C + 8 * g) * 2u;
+        first[b] = (tok0 + t) % T == 0;
+    }
+    const bool before = l16 == 0 && tok0 % T != 0;
+    // one chunk's operands; each is fetched anew for the wave's next chunk as soon as the current one is done with it
+    Row8 xr[NB], xp, gr[kGrad ? kMix : 1][NB];
+    Raw8<float> mix;
+    bf16x8 wf[NT];
+    auto fetch_x = [&](int c) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_row8(xr[b], x + base + c, row[b]);
+        if (before) load_row8(xp, x + base - C + c, row[0]);
+        if (!kGrad) mix.load(mix_x + c + 8 * g);
+    };
+    auto fetch_g = [&](int s, int c) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_row8(gr[kGrad ? s : 0][b], gs[s] + base + c, row[b]);
+    };
+    auto fetch_w = [&](int i, int c) {
+        wf[i] = *reinterpret_cast<const bf16x8 *>(reinterpret_cast<const char *>(frags + ((size_t)(c >> 5) * NT + i) * kFragElems) + (uint32_t)lane * 16u);
+    };
+    f32x4 acc[NT][NB];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[i][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int nchunk = C / 32;
+    if (wave < nchunk) {
+        xp.zero();
+        fetch_x(32 * wave);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) fetch_w(i, 32 * wave);
+        if (kGrad) {
+#pragma unroll
+            for (int s = 0; s < kMix; ++s) fetch_g(s, 32 * wave);
+        }
+    }
+    for (int ch = wave; ch < nchunk; ch += kReduceWaves) {
+        const int next = 32 * (ch + kReduceWaves < nchunk ? ch + kReduceWaves : ch);   // (the last one once more: no branch around the loads)
+        Row8 carry = xp;
+        float mx[8], xx[NB][8];
+        bf16x8 xmix[NB] = {};
+        if (!kGrad) mix.to_float(mx);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            float xv[8];
+            xr[b].to_float(xv);
+            prev_rows(carry, xr[b]).to_float(xx[b]);
+            carry = last_row_first(xr[b]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xx[b][e] = (first[b] ? 0.f : xx[b][e]) - xv[e];
+            if (!kGrad) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xv[e] = fmaf(xx[b][e], mx[e], xv[e]);
+                xmix[b] = pack_operand(xv);
+            } else {
+                pin8(xx[b]);
+            }
+        }
+        fetch_x(next);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < kMix; ++s) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                bf16x8 o = xmix[b];
+                if (kGrad) {
+                    float gv[8];
+                    gr[kGrad ? s : 0][b].to_float(gv);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) gv[e] *= xx[b][e];
+                    o = pack_operand(gv);
+                }
+#pragma unroll
+                for (int i = s * RT; i < (s + 1) * RT; ++i) acc[i][b] = mfma32(wf[i], o, acc[i][b]);
+            }
+            if (kGrad) fetch_g(s, next);
+#pragma unroll
+            for (int i = s * RT; i < (s + 1) * RT; ++i) fetch_w(i, next);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // add up over the waves, two rounds of kRound tiles; thread (tile, lane) then holds four neighbouring rows of one token
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem);
+#pragma unroll
+    for (int rd = 0; rd < 2; ++rd) {
+        if (rd) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < M::kRound; ++i) {
+            const int tile = rd * M::kRound + i;
+            red[(wave * M::kRound + i) * 64 + lane] = acc[tile / NB][tile % NB];
+        }
+        __syncthreads();
+        for (int j = threadIdx.x; j < M::kRound * 64; j += kReduceWaves * 64) {
+            f32x4 s = red[j];
+#pragma unroll
+            for (int q = 1; q < kReduceWaves; ++q) s += red[q * M::kRound * 64 + j];
+            const int tile = rd * M::kRound + (j >> 6), l = j & 63;
+            const int64_t t = tok0 + 16 * (tile % NB) + (l & 15);
+            if (t >= n_tok) continue;
+            const size_t o = (size_t)t * (kMix * R) + 16 * (tile / NB) + 4 * (l >> 4);
+            if (kGrad) {
+                float hv[4];
+                load4(h + o, hv);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] *= fmaf(-hv[e], hv[e], 1.f);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[e] = tanhf(s[e]);
+            }
+            store4(out + o, s[0], s[1], s[2], s[3]);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// Everything else of the backward: gx, and the sums over tokens.
+//
+// Workgroup: 64 channels, two token ranges side by side; wave (half, range): 32 channels of one range, which it walks in
+// steps of 32 tokens (the k-slots of one MFMA).  A lane holds 8 neighbouring channels of a token (16-byte accesses), the
+// order in which coef and gxm come out of their MFMAs when W's and A's rows are assigned as in wkv6_mix.hip; the
+// neighbouring tokens are neighbouring lanes (DPP), across steps they are carried in registers.  The operands of the
+// sums over tokens (gcoef, x_mix transposed) go through a tile of the wave's own in LDS and the transposing read.
+// One wave per SIMD: the two sets of accumulators are 160 registers, and a step's loads are issued a step ahead,
+// each into the registers the current step has just finished with.
+//
+// kGx: gx (and gmix).  kAcc: the weight gradients for 32 columns r of the rank, from r0 on.  R = 32 does both in one
+// launch; R = 64 takes one launch for gx and one for each half of the rank (the accumulators of 64 columns are more
+// than the registers hold).
+// ------------------------------------------------------------------------------------------
+constexpr int kGradThreads = 256, kGradTok = 32;
+template <int R, bool kGx, bool kAcc> struct MixGrads {
+    static constexpr int kCols = kMix * (kGx ? R : 32);      // columns of h and gpre the launch reads
+    static constexpr int kPitch = kCols + 8;                 // elements per token row of their tiles: 8 rows on 8 different bank groups
+    static constexpr int kStagePitch = 40;
+    static constexpr bool kLdsA = R == 32;                   // A's fragments in LDS, too (R = 64: they do not fit, from L2)
+    static constexpr int kW = 0;                                                 // [5][R/32][4][64][8]
+    static constexpr int kA = kW + (kGx ? kMix * R * 64 * 2 : 0);                // [5R/32][4][64][8]
+    static constexpr int kBias = kA + (kGx && kLdsA ? kMix * R * 64 * 2 : 0);    // [5][64] fp32
+    static constexpr int kMixX = kBias + kMix * 64 * 4;                          // [64] fp32
+    static constexpr int kH = kMixX + 64 * 4;                                    // [2 ranges][32][kPitch]
+    static constexpr int kG = kH + 2 * kGradTok * kPitch * 2;
+    static constexpr int kStage = kG + 2 * kGradTok * kPitch * 2;                // [4 waves][32][kStagePitch]
+    static constexpr int kBytes0 = kStage + 4 * kGradTok * kStagePitch * 2;
+    static constexpr int kFold = kAcc ? 2 * 40 * 64 * 16 : 0;                    // the ranges' accumulators are added up here at the end
+    static constexpr int kBytes = kBytes0 > kFold ? kBytes0 : kFold;
+    static_assert(kBytes <= 160 * 1024, "LDS of mix_grads_kernel");
+};
+
+struct MixGradArgs {
+    int64_t n_tok;
+    int T, C, nruns, steps;      // a range is steps * 32 tokens, a run two ranges, ranges in token order
+    int r0;                      // kAcc: first column of the rank
+    const bf16_t *x, *h, *gpre, *w, *a_t, *g[kMix];
+    const float *bias, *mix_x;
+    bf16_t *gx;
+    float *edge_first, *edge_last;   // (ranges, C): z of a range's first token; gx of its last token without the next token's z
+    float *part_w, *part_a;          // [nruns][C/64][2 halves][20 tiles][64 lanes][4] accumulator tiles
+    float *part_bias, *part_mix;     // (ranges, 5, C), (ranges, C)
+};
+
+template <int R, bool kGx, bool kAcc>
+__global__ __launch_bounds__(kGradThreads) void mix_grads_kernel(MixGradArgs p)
+{
+    typedef MixGrads<R, kGx, kAcc> L;
+    constexpr int KW = R / 32, KA = kMix * R / 32, kCols = L::kCols, kPitch = L::kPitch;
+    constexpr int kPieces = kCols / 32;                        // 16-byte pieces of a range's h (gpre) tile per thread
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave & 1, rg = wave >> 1;
+    const int C = p.C, T = p.T;
+    const int run = (int)blockIdx.x % p.nruns, cg = (int)blockIdx.x / p.nruns;
+    const int range = run * 2 + rg;
+    const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
+    const int c0 = cg * 64 + half * 32, cl = c0 + 8 * g;
+    bf16_t *wf = reinterpret_cast<bf16_t *>(smem + L::kW), *af = reinterpret_cast<bf16_t *>(smem + L::kA);
+    float *bias_l = reinterpret_cast<float *>(smem + L::kBias), *mix_l = reinterpret_cast<float *>(smem + L::kMixX);
+    bf16_t *ht = reinterpret_cast<bf16_t *>(smem + L::kH) + rg * kGradTok * kPitch;
+    bf16_t *gt = reinterpret_cast<bf16_t *>(smem + L::kG) + rg * kGradTok * kPitch;
+    bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + wave * kGradTok * L::kStagePitch;
+
+    // operand row l16 of tile (half, m) <-> this channel of the workgroup's 64
+    auto frag_channel = [&](int ct, int l) { return 32 * (ct >> 1) + 8 * (l >> 2) + 4 * (ct & 1) + (l & 3); };
+    if (kGx) {
+        for (int i = threadIdx.x; i < kMix * KW * 4 * 64; i += kGradThreads) {
+            const int l = i & 63, ct = (i >> 6) & 3, kk = (i >> 8) % KW, s = (i >> 8) / KW;
+            *reinterpret_cast<uint4 *>(wf + (size_t)i * 8) =
+                *reinterpret_cast<const uint4 *>(p.w + ((size_t)s * C + cg * 64 + frag_channel(ct, l & 15)) * R + 32 * kk + 8 * (l >> 4));
+        }
+        if (L::kLdsA)
+            for (int i = threadIdx.x; i < KA * 4 * 64; i += kGradThreads) {
+                const int l = i & 63, ct = (i >> 6) & 3, kk = i >> 8;
+                *reinterpret_cast<uint4 *>(af + (size_t)i * 8) =
+                    *reinterpret_cast<const uint4 *>(p.a_t + (size_t)(cg * 64 + frag_channel(ct, l & 15)) * (kMix * R) + 32 * kk + 8 * (l >> 4));
+            }
+        for (int i = threadIdx.x; i < kMix * 64; i += kGradThreads) bias_l[i] = p.bias[(size_t)(i >> 6) * C + cg * 64 + (i & 63)];
+    }
+    if (threadIdx.x < 64) mix_l[threadIdx.x] = p.mix_x[cg * 64 + threadIdx.x];
+
+    // ---- loads of a step ------------------------------------------------------------------
+    Row8 xr[2], gr[kMix][2], xfirst;
+    u32x4 hp[kPieces], gp[kPieces];
+    // (tokens past the end: the last token once more, with xx and the staged x_mix zero, so that it adds nothing)
+    int64_t step_base = 0;
+    uint32_t off[2];
+    auto aim = [&](int step) {
+        const int64_t t0 = min(first_tok + step * kGradTok, p.n_tok - 1), rest = p.n_tok - 1 - t0;
+        const int left = rest < kGradTok ? (int)rest : kGradTok;
+        step_base = t0 * C + c0;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) off[b] = ((uint32_t)min(16 * b + l16, left) * (uint32_t)C + 8 * g) * 2u;
+    };
+    auto fetch_x = [&]() {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) load_row8(xr[b], p.x + step_base, off[b]);
+    };
+    auto fetch_g = [&](int s) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) load_row8(gr[s][b], p.g[s] + step_base, off[b]);
+    };
+    // the range's h and gpre rows: four threads per token, 32 columns at a time
+    const int tile_row = (threadIdx.x & 127) >> 2, tile_col = (threadIdx.x & 3) * 8;
+    auto fetch_tiles = [&](int step) {
+        const int64_t t0 = min(first_tok + step * kGradTok, p.n_tok - 1), rest = p.n_tok - 1 - t0;
+        const uint32_t o = (uint32_t)(min(tile_row, (int)(rest < kGradTok ? rest : kGradTok)) * (kMix * R) + tile_col + (kGx ? 0 : p.r0)) * 2u;
+        const char *hb = reinterpret_cast<const char *>(p.h + t0 * (kMix * R)), *gb = reinterpret_cast<const char *>(p.gpre + t0 * (kMix * R));
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) {
+            hp[j] = *reinterpret_cast<const u32x4 *>(hb + o + j * (kGx ? 64 : 2 * R));
+            gp[j] = *reinterpret_cast<const u32x4 *>(gb + o + j * (kGx ? 64 : 2 * R));
+        }
+    };
+    f32x4 acc_w[kAcc ? kMix : 1][2][2], acc_a[kAcc ? 2 * kMix : 1][2];   // [s][rank tile][channel tile], [stacked rank tile][channel tile]
+    float sum_b[kAcc ? kMix : 1][2];
+    if (kAcc) {
+#pragma unroll
+        for (int s = 0; s < kMix; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    acc_w[s][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                    acc_a[2 * s + i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                }
+                sum_b[s][i] = 0.f;
+            }
+    }
+    float gmix[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float pend[8];                                    // gx of the step's last token, waiting for the next token's z
+    bool pend_valid = false, pend_last = false;
+    int pos[2];                                       // the lane's tokens' positions in their sequences
+#pragma unroll
+    for (int b = 0; b < 2; ++b) pos[b] = (int)((first_tok + 16 * b + l16) % T);
+    const int pos_step = kGradTok % T;
+    xfirst.zero();
+    if (l16 == 0 && first_tok < p.n_tok && first_tok % T != 0) xfirst.load(p.x + (size_t)(first_tok - 1) * C + cl);
+    fetch_tiles(0);
+    aim(0);
+    fetch_x();
+#pragma unroll
+    for (int s = 0; s < kMix; ++s) fetch_g(s);
+
+    // operand fragment with the k-slots along the step's 32 tokens: column n0 + l16 of a tile of pitch `pitch`, slots
+    // 4g + e and 16 + 4g + e
+    auto frag_tokens = [&](const bf16_t *tile, int pitch, int n0) {
+        const bf16_t *q = tile + (4 * g + (l16 >> 2)) * pitch + n0 + 4 * (l16 & 3);
+        typedef s16x4 __attribute__((address_space(3))) *lds4;
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)q));
+        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(q + 16 * pitch)));
+        return make_bf16x8(lo[0], lo[1], hi[0], hi[1]);
+    };
+    auto stage_rows = [&](int b, bf16x8 v) { *reinterpret_cast<bf16x8 *>(stage + (16 * b + l16) * L::kStagePitch + 8 * g) = v; };
+
+    for (int step = 0; step < p.steps; ++step) {
+        __syncthreads();   // the step before has read its h and gpre tiles
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) {
+            *reinterpret_cast<u32x4 *>(ht + tile_row * kPitch + tile_col + 32 * j) = hp[j];
+            *reinterpret_cast<u32x4 *>(gt + tile_row * kPitch + tile_col + 32 * j) = gp[j];
+        }
+        const int next = min(step + 1, p.steps - 1);   // (the last step fetches itself once more: no branch, and its lines are at hand)
+        fetch_tiles(next);
+        __syncthreads();
+        const int64_t cur_base = step_base, step_tok = first_tok + step * kGradTok;
+        const uint32_t cur_off[2] = {off[0], off[1]};
+        bool valid[2], last[2];
+        float xx[2][8], mx[8];
+        {
+            const float4 m0 = *reinterpret_cast<const float4 *>(mix_l + 32 * half + 8 * g), m1 = *reinterpret_cast<const float4 *>(mix_l + 32 * half + 8 * g + 4);
+            mx[0] = m0.x; mx[1] = m0.y; mx[2] = m0.z; mx[3] = m0.w; mx[4] = m1.x; mx[5] = m1.y; mx[6] = m1.z; mx[7] = m1.w;
+        }
+        bf16x8 xmix[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            valid[b] = step_tok + 16 * b + l16 < p.n_tok;
+            const bool first = pos[b] == 0;
+            last[b] = pos[b] == T - 1;
+            pos[b] += pos_step;
+            if (pos[b] >= T) pos[b] -= T;
+            float xv[8];
+            xr[b].to_float(xv);
+            prev_rows(xfirst, xr[b]).to_float(xx[b]);
+            xfirst = last_row_first(xr[b]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xx[b][e] = valid[b] ? (first ? 0.f : xx[b][e]) - xv[e] : 0.f;
+            if (kAcc) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xv[e] = valid[b] ? fmaf(xx[b][e], mx[e], xv[e]) : 0.f;
+                stage_rows(b, pack_operand(xv));
+            }
+        }
+        aim(next);
+        fetch_x();
+        __builtin_amdgcn_sched_barrier(0);
+        if (kAcc) {   // gA
+            const bf16x8 xt[2] = {frag_tokens(stage, L::kStagePitch, 0), frag_tokens(stage, L::kStagePitch, 16)};
+#pragma unroll
+            for (int i = 0; i < 2 * kMix; ++i) {
+                const bf16x8 gq = frag_tokens(gt, kPitch, kGx ? (i >> 1) * R + 16 * (i & 1) : 16 * i);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc_a[kAcc ? i : 0][j] = mfma32(xt[j], gq, acc_a[kAcc ? i : 0][j]);
+                if (i & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float gsum[2][8], gxx[2][8];
+        if (kGx) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { gsum[b][e] = 0.f; gxx[b][e] = 0.f; }
+        }
+#pragma unroll
+        for (int s = 0; s < kMix; ++s) {
+            f32x4 cf[2][2];
+            if (kGx) {
+                bf16x8 wfr[2][KW];
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const float4 bb = *reinterpret_cast<const float4 *>(bias_l + 64 * s + 32 * half + 8 * g + 4 * m);
+                    cf[0][m] = cf[1][m] = (f32x4){bb.x, bb.y, bb.z, bb.w};
+#pragma unroll
+                    for (int kk = 0; kk < KW; ++kk)
+                        wfr[m][kk] = *reinterpret_cast<const bf16x8 *>(wf + (size_t)(((s * KW + kk) * 4 + 2 * half + m) * 64 + lane) * 8);
+                }
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int kk = 0; kk < KW; ++kk) {
+                        const bf16x8 hr = *reinterpret_cast<const bf16x8 *>(ht + (16 * b + l16) * kPitch + s * R + 32 * kk + 8 * g);
+#pragma unroll
+                        for (int m = 0; m < 2; ++m) cf[b][m] = mfma32(wfr[m][kk], hr, cf[b][m]);
+                    }
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float gv[8];
+                gr[s][b].to_float(gv);
+                if (kGx) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        gsum[b][e] += gv[e];
+                        gxx[b][e] = fmaf(gv[e], cf[b][e >> 2][e & 3], gxx[b][e]);
+                    }
+                    pin8(gsum[b]);   // (or the sums sink to their use behind the branches below, with every g still in registers)
+                    pin8(gxx[b]);
+                }
+                if (kAcc) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) gv[e] *= xx[b][e];
+                    stage_rows(b, pack_operand(gv));
+                }
+            }
+            fetch_g(s);
+            if (kAcc) {
+                const bf16x8 gc[2] = {frag_tokens(stage, L::kStagePitch, 0), frag_tokens(stage, L::kStagePitch, 16)};
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    float f[8];
+                    unpack8(gc[j], f);
+                    sum_b[kAcc ? s : 0][j] += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const bf16x8 hq = frag_tokens(ht, kPitch, (kGx ? s * R : s * 32) + 16 * i);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc_w[kAcc ? s : 0][i][j] = mfma32(hq, gc[j], acc_w[kAcc ? s : 0][i][j]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kGx) {
+            f32x4 xm[2][2];   // gxm, the same lane order as coef
+#pragma unroll
+            for (int b = 0; b < 2; ++b) xm[b][0] = xm[b][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < KA; ++kk) {
+                bf16x8 afr[2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    afr[m] = L::kLdsA ? *reinterpret_cast<const bf16x8 *>(af + (size_t)((kk * 4 + 2 * half + m) * 64 + lane) * 8)
+                                      : *reinterpret_cast<const bf16x8 *>(p.a_t + (size_t)(cg * 64 + frag_channel(2 * half + m, l16)) * (kMix * R) + 32 * kk + 8 * g);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const bf16x8 gq = *reinterpret_cast<const bf16x8 *>(gt + (16 * b + l16) * kPitch + 32 * kk + 8 * g);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) xm[b][m] = mfma32(afr[m], gq, xm[b][m]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            float o[2][8];
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float m = xm[b][e >> 2][e & 3];
+                    gmix[e] = fmaf(m, xx[b][e], gmix[e]);
+                    o[b][e] = gsum[b][e] - gxx[b][e] + m * (1.f - mx[e]);
+                    gxx[b][e] = fmaf(m, mx[e], gxx[b][e]);             // z
+                }
+            pin8(o[0]); pin8(o[1]); pin8(gmix);
+            __builtin_amdgcn_sched_barrier(0);
+            if (step == 0 && l16 == 0) {
+                float *q = p.edge_first + (size_t)range * C + cl;
+                *reinterpret_cast<float4 *>(q) = make_float4(gxx[0][0], gxx[0][1], gxx[0][2], gxx[0][3]);
+                *reinterpret_cast<float4 *>(q + 4) = make_float4(gxx[0][4], gxx[0][5], gxx[0][6], gxx[0][7]);
+            }
+            float z0[8];   // lane 15: z of this step's first token
+#pragma unroll
+            for (int e = 0; e < 8; ++e) z0[e] = first_to_last(gxx[0][e]);
+            auto put = [&](int64_t base, uint32_t o, const float (&v)[8]) {
+                *reinterpret_cast<bf16x8 *>(reinterpret_cast<char *>(p.gx + base) + o) = pack_operand(v);
+            };
+            if (step > 0 && pend_valid && l16 == 15) {
+                if (!pend_last) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) pend[e] += z0[e];
+                }
+                put((step_tok - 1) * C + c0, 16u * g, pend);
+            }
+            float zn[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) zn[e] = next_lane(first_to_last(gxx[1][e]), gxx[0][e]);
+            if (!last[0]) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[0][e] += zn[e];
+            }
+            if (valid[0]) put(cur_base, cur_off[0], o[0]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) pend[e] = o[1][e];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) zn[e] = next_lane(0.f, gxx[1][e]);
+            if (!last[1]) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[1][e] += zn[e];
+            }
+            if (valid[1] && l16 < 15) put(cur_base, cur_off[1], o[1]);
+            pend_valid = valid[1]; pend_last = last[1];
+        }
+    }
+    if (kGx) {
+        if (pend_valid && l16 == 15) {   // the range's last token: complete if a sequence ends with it
+            if (pend_last) *reinterpret_cast<bf16x8 *>(p.gx + (first_tok + (int64_t)p.steps * kGradTok - 1) * C + cl) = pack_operand(pend);
+            else {
+                float *q = p.edge_last + (size_t)range * C + cl;
+                *reinterpret_cast<float4 *>(q) = make_float4(pend[0], pend[1], pend[2], pend[3]);
+                *reinterpret_cast<float4 *>(q + 4) = make_float4(pend[4], pend[5], pend[6], pend[7]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int m = 8; m >= 1; m >>= 1) gmix[e] += __shfl_xor(gmix[e], m);
+        if (l16 == 0) {
+            float *q = p.part_mix + (size_t)range * C + cl;
+            *reinterpret_cast<float4 *>(q) = make_float4(gmix[0], gmix[1], gmix[2], gmix[3]);
+            *reinterpret_cast<float4 *>(q + 4) = make_float4(gmix[4], gmix[5], gmix[6], gmix[7]);
+        }
+    }
+    if (kAcc) {
+#pragma unroll
+        for (int s = 0; s < kMix; ++s)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float v = sum_rows(sum_b[kAcc ? s : 0][j]);
+                if (p.r0 == 0 && g == 0) p.part_bias[((size_t)range * kMix + s) * C + c0 + 16 * j + l16] = v;
+            }
+        // the second range's accumulators through LDS to the first's wave, then one partial per workgroup
+        f32x4 *fold = reinterpret_cast<f32x4 *>(smem) + half * 40 * 64;
+        __syncthreads();
+        if (rg == 1) {
+#pragma unroll
+            for (int i = 0; i < 20; ++i) {
+                fold[i * 64 + lane] = acc_w[kAcc ? i >> 2 : 0][(i >> 1) & 1][i & 1];
+                fold[(20 + i) * 64 + lane] = acc_a[kAcc ? i >> 1 : 0][i & 1];
+            }
+        }
+        __syncthreads();
+        if (rg == 0) {
+            const size_t base = ((size_t)(run * (C / 64) + cg) * 2 + half) * 20 * 64 + lane;
+            f32x4 *pw = reinterpret_cast<f32x4 *>(p.part_w) + base, *pa = reinterpret_cast<f32x4 *>(p.part_a) + base;
+#pragma unroll
+            for (int i = 0; i < 20; ++i) {
+                pw[i * 64] = acc_w[kAcc ? i >> 2 : 0][(i >> 1) & 1][i & 1] + fold[i * 64 + lane];
+                pa[i * 64] = acc_a[kAcc ? i >> 1 : 0][i & 1] + fold[(20 + i) * 64 + lane];
+            }
+        }
+    }
+}
+
+// Sums of the workgroups' partials -> gradients of the weights, and gx of the tokens at the ends of the ranges.
+// blockIdx.y: 0 gW, 1 gA (columns r0..r0+31 of the rank), 2 gbias and gmix, 3 the ranges' ends.
+template <typename Tw>
+__global__ __launch_bounds__(256) void mix_finish_kernel(MixGradArgs p, int R, Tw *__restrict__ gw, Tw *__restrict__ ga,
+                                                         float *__restrict__ gbias, float *__restrict__ gmix)
+{
+    const int C = p.C, nranges = 2 * p.nruns;
+    const int i = (int)blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.y < 2) {
+        const int per_run = (C / 64) * 2 * 20 * 64;
+        if (i >= per_run) return;
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(blockIdx.y == 0 ? p.part_w : p.part_a) + i;
+        f32x4 s = src[0];
+        for (int q = 1; q < p.nruns; ++q) s += src[(size_t)q * per_run];
+        const int lane = i & 63, l16 = lane & 15, g = lane >> 4, tile = (i >> 6) % 20, c0 = (i / (64 * 20)) * 32;
+        if (blockIdx.y == 0) {   // tile (s, rank tile, channel tile): rows = rank, columns = channels
+            const int r = p.r0 + 16 * ((tile >> 1) & 1) + 4 * g, c = c0 + 16 * (tile & 1) + l16;
+            store4(gw + ((size_t)(tile >> 2) * C + c) * R + r, s[0], s[1], s[2], s[3]);
+        } else {                 // tile (s, rank tile, channel tile): rows = channels, columns = rank
+            const int r = (tile >> 2) * R + p.r0 + 16 * ((tile >> 1) & 1) + l16, c = c0 + 16 * (tile & 1) + 4 * g;
+            store4(ga + (size_t)r * C + c, s[0], s[1], s[2], s[3]);
+        }
+    } else if (blockIdx.y == 2) {
+        if (i >= (kMix + 1) * C) return;
+        const bool is_mix = i >= kMix * C;
+        float s = 0.f;
+        for (int q = 0; q < nranges; ++q) s += is_mix ? p.part_mix[(size_t)q * C + i - kMix * C] : p.part_bias[(size_t)q * kMix * C + i];
+        if (is_mix) gmix[i - kMix * C] = s; else gbias[i] = s;
+    } else {
+        const int per = C / 4;
+        for (int j = i; j < (nranges - 1) * per; j += (int)gridDim.x * 256) {
+            const int e = j / per, c = (j % per) * 4;
+            const int64_t t = (int64_t)(e + 1) * p.steps * kGradTok - 1;
+            if (t >= p.n_tok || t % p.T == p.T - 1) continue;
+            const float4 a = *reinterpret_cast<const float4 *>(p.edge_last + (size_t)e * C + c);
+            const float4 z = *reinterpret_cast<const float4 *>(p.edge_first + (size_t)(e + 1) * C + c);
+            store4(p.gx + (size_t)t * C + c, a.x + z.x, a.y + z.y, a.z + z.z, a.w + z.w);
+        }
+    }
+}
+
+// ---- host side ----------------------------------------------------------------------------
+static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+size_t shift_mix_weights_bytes(int64_t C, int64_t R) { return 4 * align256((size_t)(kMix * R * C) * sizeof(bf16_t)); }
+
+struct MixWeightForms {
+    bf16_t *a_frag, *wt_frag, *a_t, *w;
+    MixWeightForms(void *block, int64_t C, int64_t R) {
+        char *b = reinterpret_cast<char *>(block);
+        const size_t n = align256((size_t)(kMix * R * C) * sizeof(bf16_t));
+        a_frag = (bf16_t *)b; wt_frag = (bf16_t *)(b + n); a_t = (bf16_t *)(b + 2 * n); w = (bf16_t *)(b + 3 * n);
+    }
+};
+
+template <int R, bool kGrad>
+static hipError_t launch_reduce(hipStream_t st, int64_t n, int64_t T, int64_t C, const void *x, const float *mix_x, const bf16_t *frags,
+                                const void *const g[5], const void *h, void *out) {
+    constexpr auto kern = mix_reduce_kernel<R, kGrad>;
+    hipError_t e = allow_dynamic_lds<kern>(MixReduce<R>::kLds);
+    if (e != hipSuccess) return e;
+    auto gp = [&](int i) { return g ? (const bf16_t *)g[i] : nullptr; };
+    const int64_t per = 16 * MixReduce<R>::kBlocks;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + per - 1) / per)), dim3(kReduceWaves * 64), MixReduce<R>::kLds, st, n, (int)T, (int)C,
+                       (const bf16_t *)x, mix_x, frags, gp(0), gp(1), gp(2), gp(3), gp(4), (const bf16_t *)h, (bf16_t *)out);
+    return hipGetLastError();
+}
+
+hipError_t shift_mix_forward(hipStream_t st, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R, const void *x, const float *mix_x,
+                             const void *a, const void *w2t, const float *bias, void *weights, void *h, void *const out[5]) {
+    const MixWeightForms w(weights, C, R);
+    const dim3 grid((unsigned)(C / 32), 2);
+    if (weight_dtype == kF32)
+        hipLaunchKernelGGL(mix_weights_kernel<float>, grid, dim3(256), 0, st, (int)C, (int)R, (const float *)a, (const float *)w2t, w.a_frag, w.wt_frag, w.a_t, w.w);
+    else
+        hipLaunchKernelGGL(mix_weights_kernel<bf16_t>, grid, dim3(256), 0, st, (int)C, (int)R, (const bf16_t *)a, (const bf16_t *)w2t, w.a_frag, w.wt_frag, w.a_t, w.w);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    e = R == 32 ? launch_reduce<32, false>(st, B * T, T, C, x, mix_x, w.a_frag, nullptr, nullptr, h)
+                : launch_reduce<64, false>(st, B * T, T, C, x, mix_x, w.a_frag, nullptr, nullptr, h);
+    if (e != hipSuccess) return e;
+    return shift_mix_five(st, B, T, C, R, x, h, w.w, bias, out);
+}
+
+// how the tokens are cut for mix_grads_kernel: runs of two ranges each, enough workgroups for the chip and no more (a
+// partial of every weight gradient per run)
+struct MixCut {
+    int nruns, steps;
+    MixCut(int64_t n, int64_t C) {
+        const int64_t groups = C / 64, want = (compute_units() + groups - 1) / groups;      // runs that fill the chip once
+        const int64_t most = (n + 2 * kGradTok - 1) / (2 * kGradTok);                       // runs of one step per range
+        const int64_t runs = want < most ? want : most;
+        steps = (int)((n + runs * 2 * kGradTok - 1) / (runs * 2 * kGradTok));
+        nruns = (int)((n + (int64_t)steps * 2 * kGradTok - 1) / ((int64_t)steps * 2 * kGradTok));
+    }
+};
+
+struct MixWorkspace {
+    size_t gpre, part_w, part_a, part_bias, part_mix, edge_first, edge_last, bytes;
+    MixWorkspace(int64_t n, int64_t C, int64_t R, const MixCut &cut) {
+        size_t o = 0;
+        auto take = [&](size_t b) { const size_t at = o; o += align256(b); return at; };
+        gpre = take((size_t)(n * kMix * R) * 2);
+        part_w = take((size_t)cut.nruns * kMix * 32 * C * 4);
+        part_a = take((size_t)cut.nruns * kMix * 32 * C * 4);
+        part_bias = take((size_t)2 * cut.nruns * kMix * C * 4);
+        part_mix = take((size_t)2 * cut.nruns * C * 4);
+        edge_first = take((size_t)2 * cut.nruns * C * 4);
+        edge_last = take((size_t)2 * cut.nruns * C * 4);
+        bytes = o;
+    }
+};
+
+size_t shift_mix_backward_workspace_bytes(int64_t B, int64_t T, int64_t C, int64_t R) {
+    return MixWorkspace(B * T, C, R, MixCut(B * T, C)).bytes;
+}
+
+template <int R, bool kGx, bool kAcc>
+static hipError_t launch_grads(hipStream_t st, const MixGradArgs &p) {
+    constexpr auto kern = mix_grads_kernel<R, kGx, kAcc>;
+    constexpr int lds = MixGrads<R, kGx, kAcc>::kBytes;
+    hipError_t e = allow_dynamic_lds<kern>(lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(p.nruns * (p.C / 64))), dim3(kGradThreads), lds, st, p);
+    return hipGetLastError();
+}
+
+hipError_t shift_mix_backward(hipStream_t st, int weight_dtype, int64_t B, int64_t T, int64_t C, int64_t R, const void *x, const float *mix_x,
+                              const float *bias, const void *weights, const void *h, const void *const gout[5],
+                              void *gx, float *gmix_x, void *ga, void *gw2t, float *gbias, void *workspace) {
+    const MixWeightForms w(const_cast<void *>(weights), C, R);
+    const int64_t n = B * T;
+    const MixCut cut(n, C);
+    const MixWorkspace ws(n, C, R, cut);
+    char *base = reinterpret_cast<char *>(workspace);
+    void *gpre = base + ws.gpre;
+    hipError_t e = R == 32 ? launch_reduce<32, true>(st, n, T, C, x, mix_x, w.wt_frag, gout, h, gpre)
+                           : launch_reduce<64, true>(st, n, T, C, x, mix_x, w.wt_frag, gout, h, gpre);
+    if (e != hipSuccess) return e;
+    MixGradArgs p = {};
+    p.n_tok = n; p.T = (int)T; p.C = (int)C; p.nruns = cut.nruns; p.steps = cut.steps;
+    p.x = (const bf16_t *)x; p.h = (const bf16_t *)h; p.gpre = (const bf16_t *)gpre; p.w = w.w; p.a_t = w.a_t;
+    for (int s = 0; s < kMix; ++s) p.g[s] = (const bf16_t *)gout[s];
+    p.bias = bias; p.mix_x = mix_x; p.gx = (bf16_t *)gx;
+    p.edge_first = (float *)(base + ws.edge_first); p.edge_last = (float *)(base + ws.edge_last);
+    p.part_w = (float *)(base + ws.part_w); p.part_a = (float *)(base + ws.part_a);
+    p.part_bias = (float *)(base + ws.part_bias); p.part_mix = (float *)(base + ws.part_mix);
+    auto finish = [&](unsigned rows) {
+        // (blockIdx.y counts from 0; with rows = 2 only the weights' sums)
+        const dim3 grid((unsigned)(((C / 64) * 2 * 20 * 64 + 255) / 256), rows);
+        if (weight_dtype == kF32)
+            hipLaunchKernelGGL(mix_finish_kernel<float>, grid, dim3(256), 0, st, p, (int)R, (float *)gw2t, (float *)ga, gbias, gmix_x);
+        else
+            hipLaunchKernelGGL(mix_finish_kernel<bf16_t>, grid, dim3(256), 0, st, p, (int)R, (bf16_t *)gw2t, (bf16_t *)ga, gbias, gmix_x);
+        return hipGetLastError();
+    };
+    if (R == 32) {
+        e = launch_grads<32, true, true>(st, p);
+        return e != hipSuccess ? e : finish(4);
+    }
+    e = launch_grads<64, true, false>(st, p);
+    for (p.r0 = 0; e == hipSuccess && p.r0 < 64; p.r0 += 32) {
+        e = launch_grads<64, false, true>(st, p);
+        if (e == hipSuccess) e = finish(p.r0 == 0 ? 4 : 2);
+    }
+    return e;
+}
+
+}  // namespace wkv6

@@ -34,6 +34,10 @@ SIGNATURES = {
     "wkv6_shift_mix_five": (_int, [_p, _int] + [_i64] * 4 + [_p] * 9),
     "wkv6_shift_mix_five_backward": (_int, [_p, _int] + [_i64] * 4 + [_p] * 10 + [_i64, _p, _p]),
     "wkv6_shift_mix_x_backward": (_int, [_p, _int] + [_i64] * 3 + [_p] * 7),
+    "wkv6_shift_mix_weights_bytes": (_sz, [_i64] * 2),
+    "wkv6_shift_mix_forward": (_int, [_p, _int, _int] + [_i64] * 4 + [_p] * 6 + [_sz] + [_p] * 6),
+    "wkv6_shift_mix_backward_workspace_bytes": (_sz, [_int] + [_i64] * 4),
+    "wkv6_shift_mix_backward": (_int, [_p, _int, _int] + [_i64] * 4 + [_p] * 16 + [_sz]),
     "wkv6_backward": (_int, [_p, _int] + [_i64] * 4 + [_p] * 11 + [_p, _sz]),
     "wkv6_backward_workspace_bytes": (_sz, [_int] + [_i64] * 4),
     "wkv6_backward_static": (_int, [_p, _int] + [_i64] * 4 + [_p] * 11),

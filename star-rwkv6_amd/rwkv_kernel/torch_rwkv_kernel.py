@@ -231,11 +231,8 @@ class _WKV6GnGate(torch.autograd.Function):
 
 
 class _ShiftMix(torch.autograd.Function):
-    """The layer's input side (rwkv6_model.py:134-146) with gradients, bf16: x -> (xr, xk, xv, xw, xg).
-    Token shift and x_mix in one kernel (wkv6_shift_mix_x), the GEMM against the stacked first mixer
-    weights and its tanh in torch, then one kernel that expands the rank-R coefficients on the matrix
-    cores and writes the five outputs (wkv6_shift_mix_five).  Backward: wkv6_shift_mix_five_backward,
-    the reductions over channels and over tokens as batched GEMMs, wkv6_shift_mix_x_backward."""
+    """The layer's input side (rwkv6_model.py:134-146) with gradients, bf16: x -> (xr, xk, xv, xw, xg), all of it
+    in the library's kernels (wkv6_shift_mix_forward / wkv6_shift_mix_backward)."""
 
     @staticmethod
     def forward(ctx, x, mix_x, a, w2t, bias):
@@ -244,18 +241,19 @@ class _ShiftMix(torch.autograd.Function):
             B, T, C = x.shape
             R = w2t.shape[2]
             code = _DTYPE_CODE[x.dtype]
-            mx = mix_x.detach().to(torch.float32).contiguous()
-            a16 = a.detach().to(x.dtype).contiguous()
-            w16 = w2t.detach().to(x.dtype).contiguous()
-            b32 = bias.detach().to(torch.float32).contiguous()
-            x_mix = torch.empty_like(x)
+            mx = mix_x.to(torch.float32).contiguous()
+            b32 = bias.to(torch.float32).contiguous()
+            wdt = a.dtype if a.dtype == w2t.dtype and a.dtype in (torch.bfloat16, torch.float32) else torch.float32
+            aw, ww = a.to(wdt).contiguous(), w2t.to(wdt).contiguous()
+            nw = lib.wkv6_shift_mix_weights_bytes(C, R)
             outs = _staggered(5, (B, T, C), x.dtype, x.device, first=1)
-            with torch.cuda.device(x.device):
-                _native.check(lib.wkv6_shift_mix_x(_stream(), code, B, T, C, _ptr(x), _ptr(mx), _ptr(x_mix)))
-                h = torch.tanh(x_mix.view(B * T, C) @ a16.t())            # (B*T, 5R)
-                _native.check(lib.wkv6_shift_mix_five(_stream(), code, B, T, C, R, _ptr(x), _ptr(h), _ptr(w16), _ptr(b32),
-                                                      *[_ptr(o) for o in outs]))
-            ctx.save_for_backward(x, x_mix, h, mx, a16, w16, b32)
+            # (not out of the outputs' block: a caller may change an output in place)
+            h, weights = _carve(x.device, [((B, T, 5 * R), x.dtype, 6), ((nw,), torch.uint8, 0)])
+            with _on_device(x.device):
+                _native.check(lib.wkv6_shift_mix_forward(_stream(), code, _DTYPE_CODE[wdt], B, T, C, R, _ptr(x), _ptr(mx), _ptr(aw),
+                                                         _ptr(ww), _ptr(b32), _ptr(weights), nw, _ptr(h), *[_ptr(o) for o in outs]))
+            ctx.save_for_backward(x, h, weights, mx, b32)
+            ctx.weight_dtype = wdt
             ctx.param_dtypes = (mix_x.dtype, a.dtype, w2t.dtype, bias.dtype)
             return tuple(outs)
 
@@ -263,33 +261,20 @@ class _ShiftMix(torch.autograd.Function):
     def backward(ctx, *gouts):
         lib = _native.load()
         with torch.no_grad():
-            x, x_mix, h, mx, a16, w16, b32 = ctx.saved_tensors
+            x, h, weights, mx, b32 = ctx.saved_tensors
             B, T, C = x.shape
-            n, R = B * T, w16.shape[2]
-            code = _DTYPE_CODE[x.dtype]
+            R = h.shape[2] // 5
+            code, wdt = _DTYPE_CODE[x.dtype], ctx.weight_dtype
             gouts = [torch.zeros_like(x) if g is None else g.to(x.dtype).contiguous() for g in gouts]
-            # the five planes of gcoef 256 bytes further apart than they are long (see _staggered)
-            plane = n * C + _STAGGER // 2
-            gcoef = torch.empty(5 * plane, device=x.device, dtype=x.dtype).as_strided((5, n, C), (plane, C, 1))
-            gp, gxx, gx = _staggered(3, (B, T, C), x.dtype, x.device, first=1)
-            gmx = torch.empty(C, device=x.device, dtype=torch.float32)
-            with torch.cuda.device(x.device):
-                _native.check(lib.wkv6_shift_mix_five_backward(
-                    _stream(), code, B, T, C, R, _ptr(x), _ptr(h), _ptr(w16), _ptr(b32), *[_ptr(g) for g in gouts],
-                    _ptr(gcoef), plane, _ptr(gp), _ptr(gxx)))
-                gh = torch.bmm(gcoef, w16)                                   # (5, n, R): summed over channels
-                # sums over tokens: gcoef^T h for the weights and, through eight more columns of which
-                # the first holds ones, gcoef^T 1 for the biases -- one pass over gcoef for both
-                h3 = torch.zeros((5, n, R + 8), device=x.device, dtype=x.dtype)
-                h3[:, :, :R] = h.view(n, 5, R).permute(1, 0, 2)
-                h3[:, :, R] = 1
-                gwb = torch.bmm(gcoef.transpose(1, 2), h3)                   # (5, C, R + 8)
-                gw2t, gbias = gwb[:, :, :R], gwb[:, :, R]
-                gpre = (gh.permute(1, 0, 2).reshape(n, 5 * R).float() * (1.0 - h.float() ** 2)).to(x.dtype)
-                ga = gpre.t() @ x_mix.view(n, C)                             # (5R, C)
-                gxm = (gpre @ a16).view(B, T, C)
-                _native.check(lib.wkv6_shift_mix_x_backward(_stream(), code, B, T, C, _ptr(x), _ptr(mx), _ptr(gp), _ptr(gxx),
-                                                            _ptr(gxm), _ptr(gx), _ptr(gmx)))
+            f32 = torch.float32
+            gx, ga, gw2t, gbias, gmx = _carve(x.device, [((B, T, C), x.dtype, 6), ((5 * R, C), wdt, 0), ((5, C, R), wdt, 0),
+                                                         ((5, C), f32, 0), ((C,), f32, 0)])
+            n = lib.wkv6_shift_mix_backward_workspace_bytes(code, B, T, C, R)
+            ws = torch.empty(n, device=x.device, dtype=torch.uint8)
+            with _on_device(x.device):
+                _native.check(lib.wkv6_shift_mix_backward(
+                    _stream(), code, _DTYPE_CODE[wdt], B, T, C, R, _ptr(x), _ptr(mx), _ptr(b32), _ptr(weights), _ptr(h),
+                    *[_ptr(g) for g in gouts], _ptr(gx), _ptr(gmx), _ptr(ga), _ptr(gw2t), _ptr(gbias), _ptr(ws), n))
             dm, da, dw, db = ctx.param_dtypes
             return gx, gmx.to(dm), ga.to(da), gw2t.to(dw), gbias.to(db)
 

@@ -338,3 +338,40 @@ def test_fixed_mix_on_its_own(B, T, C):
     check_close("x_mix", out, want.detach().numpy(), BF16)
     check_close("gx", x.grad, xr.grad.numpy(), BF16, is_grad=True)
     check_close("gmix", mix.grad.double().cpu().numpy(), mr.grad.numpy(), torch.float32, is_grad=True)
+
+
+@pytest.mark.parametrize("B,T,C,R,wdt", [
+    (1, 33, 64, 32, torch.float32),       # one token more than a step of the token sums, one workgroup of channels
+    (70, 1, 64, 64, torch.bfloat16),      # every token is both ends of its sequence
+    (3, 700, 64, 32, torch.float32),      # as many token runs as steps: a range boundary every 32 tokens
+    (1, 5000, 1024, 32, torch.bfloat16),  # several steps per range, the last range short
+    (5, 999, 1088, 64, torch.float32),    # ... both halves of the rank, sequence ends inside steps and between ranges
+])
+def test_layer_forward_and_backward_edges(oracle, B, T, C, R, wdt):
+    """op.shift_mix where its token ranges, steps and channel groups end, against float64 on the same rounded
+    inputs.  The weights' gradients are fp32 sums of products of bf16-rounded operands, the tensors' gradients
+    bf16: 1e-2 in the l2 norm as everywhere for 16-bit tensors, three times that element-wise."""
+    import rwkv_kernel
+    op = rwkv_kernel.RWKVKernelOperator(64, 8192)
+    print("shift_mix edges B=%d T=%d C=%d R=%d" % (B, T, C, R), flush=True)
+    dev, ref = _inputs(B, T, C, R, 7 * T + R)
+    dev["a"], dev["w2t"] = dev["a"].to(wdt), dev["w2t"].to(wdt)
+    g = torch.Generator().manual_seed(T + 3)
+    gouts = [torch.randn(B, T, C, generator=g).to(BF16).cuda() for _ in range(5)]
+    leaves = {k: v.clone().requires_grad_(True) for k, v in dev.items()}
+    outs = op.shift_mix(leaves["x"], leaves["mix_x"], leaves["a"], leaves["w2t"], leaves["bias"])
+    torch.autograd.backward(outs, gouts)
+    torch.cuda.synchronize()
+    t = {k: torch.tensor(v, requires_grad=True) for k, v in ref.items()}
+    x = t["x"]
+    xx = torch.cat([torch.zeros(B, 1, C, dtype=torch.float64), x[:, :-1]], 1) - x
+    hh = torch.tanh((x + xx * t["mix_x"]) @ t["a"].T).view(B, T, 5, R)
+    want = [x + xx * (hh[:, :, s] @ t["w2t"][s].T + t["bias"][s]) for s in range(5)]
+    for s in range(5):
+        check_close("x_s%d" % s, outs[s], want[s].detach().numpy(), BF16)
+    torch.autograd.backward(want, [go.double().cpu() for go in gouts])
+    for k in ("x", "mix_x", "a", "w2t", "bias"):
+        assert leaves[k].grad.dtype == dev[k].dtype
+        got, ref_g = to_np(leaves[k].grad), t[k].grad.numpy()
+        e1, e2 = rel_inf(got, ref_g), rel_l2(got, ref_g)
+        assert e2 <= 1e-2 and e1 <= 3e-2, (k, e1, e2)
