@@ -20,6 +20,8 @@
 #include "wkv6_kernels.h"
 #include "wkv6_mfma.h"
 
+#include <type_traits>
+
 namespace wkv6 {
 
 constexpr int kMix = 5;          // mixers
@@ -31,6 +33,11 @@ __device__ __forceinline__ void load_row8(Row8 &r, const bf16_t *base, uint32_t 
     r.a = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(base) + byteoff);
 }
 
+// a value that is the same in every lane, pinned to scalar registers (the compiler keeps some in vector registers)
+__device__ __forceinline__ int64_t uniform64(int64_t x) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)x >> 32));
+    return (int64_t)((uint64_t)hi << 32 | lo);
+}
 // ---- DPP moves inside a row of 16 lanes (lane l16 = token): the previous / the next token's value -----------------
 __device__ __forceinline__ uint32_t prev_lane(uint32_t first, uint32_t x) {   // lane 0 keeps `first`
     return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)x, 0x111, 0xF, 0xF, false);   // row_shr:1
@@ -69,23 +76,28 @@ __device__ __forceinline__ bf16x8 pack_operand(const float (&v)[8]) {
 //   w       (5, C, R)                       W in bf16
 // One workgroup per 32 channels and matrix (blockIdx.y).
 // ------------------------------------------------------------------------------------------
-template <typename Tw>
-__global__ __launch_bounds__(256) void mix_weights_kernel(int C, int R, const Tw *__restrict__ a, const Tw *__restrict__ w2t,
+template <typename Tw, int R>
+__global__ __launch_bounds__(256) void mix_weights_kernel(int C, const Tw *__restrict__ a, const Tw *__restrict__ w2t,
         bf16_t *__restrict__ a_frag, bf16_t *__restrict__ wt_frag, bf16_t *__restrict__ a_t, bf16_t *__restrict__ w)
 {
-    __shared__ bf16_t tile[5 * 64][40];   // [stacked row (s, r)][channel of the 32]
-    const int c0 = (int)blockIdx.x * 32, rows = kMix * R;
+    constexpr int rows = kMix * R;
+    __shared__ bf16_t tile[rows][40];   // [stacked row (s, r)][channel of the 32]
+    const int c0 = (int)blockIdx.x * 32;
     const bool is_a = blockIdx.y == 0;
     if (is_a) {
-        for (int i = threadIdx.x; i < rows * 8; i += 256) {
+#pragma unroll
+        for (int j = 0; j < rows * 8 / 256; ++j) {
+            const int i = j * 256 + threadIdx.x;
             float v[4];
             load4(a + (size_t)(i >> 3) * C + c0 + 4 * (i & 7), v);
 #pragma unroll
             for (int e = 0; e < 4; ++e) tile[i >> 3][4 * (i & 7) + e] = (bf16_t)v[e];
         }
     } else {
-        const int per = R / 4;   // 4-element pieces of a row of W
-        for (int i = threadIdx.x; i < kMix * 32 * per; i += 256) {
+        constexpr int per = R / 4;   // 4-element pieces of a row of W
+#pragma unroll
+        for (int j = 0; j < kMix * 32 * per / 256; ++j) {
+            const int i = j * 256 + threadIdx.x;
             const int r = (i % per) * 4, c = (i / per) % 32, s = i / (per * 32);
             float v[4];
             load4(w2t + ((size_t)s * C + c0 + c) * R + r, v);
@@ -109,6 +121,15 @@ __global__ __launch_bounds__(256) void mix_weights_kernel(int C, int R, const Tw
             *reinterpret_cast<uint4 *>(a_t + (size_t)(c0 + c) * rows + r) =
                 make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
         }
+}
+
+// tanh to well under half a unit of bf16 (2^-9): 1 - 2 / (e^{2x} + 1), and where that difference cancels the series
+// x (1 - x^2/3 + 2 x^4/15), whose next term is 17 x^6/315 < 3e-5 below |x| = 1/4.
+__device__ __forceinline__ float tanh_bf16(float x) {
+    const float x2 = x * x;
+    const float small = x * fmaf(x2, fmaf(x2, 2.f / 15.f, -1.f / 3.f), 1.f);
+    const float big = 1.f - 2.f * __builtin_amdgcn_rcpf(exp2_fast(x * (2.f * kLog2e)) + 1.f);
+    return x2 < 0.0625f ? small : big;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -171,19 +192,26 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
     for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[i][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const int nchunk = C / 32;
-    if (wave < nchunk) {
+    // Every workgroup starts at another place of its rows: in step from the first channel on, all of them would be at
+    // the same 512 bytes of every 4 KiB row at any time, i.e. at two of the 16 memory channels those rows cover.
+    const int nchunk = C / 32, nturn = (nchunk + kReduceWaves - 1) / kReduceWaves;
+    const int n_my = nchunk % kReduceWaves == 0 || wave < nchunk % kReduceWaves ? nturn : nturn - 1;   // the wave's chunks
+    auto my_chunk = [&](int i) {
+        return (i + (int)(blockIdx.x % n_my)) % n_my * kReduceWaves + wave;
+    };
+    if (n_my > 0) {
+        const int c = 32 * my_chunk(0);
         xp.zero();
-        fetch_x(32 * wave);
+        fetch_x(c);
 #pragma unroll
-        for (int i = 0; i < NT; ++i) fetch_w(i, 32 * wave);
+        for (int i = 0; i < NT; ++i) fetch_w(i, c);
         if (kGrad) {
 #pragma unroll
-            for (int s = 0; s < kMix; ++s) fetch_g(s, 32 * wave);
+            for (int s = 0; s < kMix; ++s) fetch_g(s, c);
         }
     }
-    for (int ch = wave; ch < nchunk; ch += kReduceWaves) {
-        const int next = 32 * (ch + kReduceWaves < nchunk ? ch + kReduceWaves : ch);   // (the last one once more: no branch around the loads)
+    for (int turn = 0; turn < n_my; ++turn) {
+        const int next = 32 * my_chunk(min(turn + 1, n_my - 1));   // (the last one once more: no branch around the loads)
         Row8 carry = xp;
         float mx[8], xx[NB][8];
         bf16x8 xmix[NB] = {};
@@ -219,11 +247,11 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
                     o = pack_operand(gv);
                 }
 #pragma unroll
-                for (int i = s * RT; i < (s + 1) * RT; ++i) acc[i][b] = mfma32(wf[i], o, acc[i][b]);
+                for (int q = s * RT; q < (s + 1) * RT; ++q) acc[q][b] = mfma32(wf[q], o, acc[q][b]);
             }
             if (kGrad) fetch_g(s, next);
 #pragma unroll
-            for (int i = s * RT; i < (s + 1) * RT; ++i) fetch_w(i, next);
+            for (int q = s * RT; q < (s + 1) * RT; ++q) fetch_w(q, next);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -253,7 +281,7 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
                 for (int e = 0; e < 4; ++e) s[e] *= fmaf(-hv[e], hv[e], 1.f);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[e] = tanhf(s[e]);
+                for (int e = 0; e < 4; ++e) s[e] = tanh_bf16(s[e]);
             }
             store4(out + o, s[0], s[1], s[2], s[3]);
         }
@@ -263,33 +291,35 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
 // ------------------------------------------------------------------------------------------
 // Everything else of the backward: gx, and the sums over tokens.
 //
-// Workgroup: 64 channels, two token ranges side by side; wave (half, range): 32 channels of one range, which it walks in
-// steps of 32 tokens (the k-slots of one MFMA).  A lane holds 8 neighbouring channels of a token (16-byte accesses), the
-// order in which coef and gxm come out of their MFMAs when W's and A's rows are assigned as in wkv6_mix.hip; the
-// neighbouring tokens are neighbouring lanes (DPP), across steps they are carried in registers.  The operands of the
-// sums over tokens (gcoef, x_mix transposed) go through a tile of the wave's own in LDS and the transposing read.
-// One wave per SIMD: the two sets of accumulators are 160 registers, and a step's loads are issued a step ahead,
-// each into the registers the current step has just finished with.
-//
-// kGx: gx (and gmix).  kAcc: the weight gradients for 32 columns r of the rank, from r0 on.  R = 32 does both in one
-// launch; R = 64 takes one launch for gx and one for each half of the rank (the accumulators of 64 columns are more
-// than the registers hold).
+// Workgroup: 64 channels, two token ranges side by side, each walked in steps of 32 tokens (the k-slots of one MFMA).
+// A lane holds 8 neighbouring channels of a token (16-byte accesses), the order in which coef and gxm come out of their
+// MFMAs when W's and A's rows are assigned as in wkv6_mix.hip; the neighbouring tokens are neighbouring lanes (DPP),
+// across steps they are carried in registers.  Three waves take the same 32 channels of a range, one of each role on
+// every SIMD:
+//   gx waves:  coef, gxx, gxm and from them gx and gmix;
+//   W waves:   gcoef, transposed through a tile of their own in LDS (the transposing read), for gW and gbias;
+//   A waves:   x_mix, the same way, for gA; they also bring the h and gpre rows that all roles read from LDS.
+// (The roles read the same x and g: the later reads find the lines in L1 or L2.  One wave doing everything had a SIMD to
+// itself for its 440 registers and every LDS and MFMA latency in the open.)
+// R = 64: a second launch without gx waves (kGx false) does the other half of the rank's columns.
 // ------------------------------------------------------------------------------------------
-constexpr int kGradThreads = 256, kGradTok = 32;
-template <int R, bool kGx, bool kAcc> struct MixGrads {
+constexpr int kGradTok = 32;
+template <int R, bool kGx> struct MixGrads {
+    static constexpr int kThreads = kGx ? 768 : 512;
     static constexpr int kCols = kMix * (kGx ? R : 32);      // columns of h and gpre the launch reads
     static constexpr int kPitch = kCols + 8;                 // elements per token row of their tiles: 8 rows on 8 different bank groups
+    static constexpr int kBufs = kCols == 160 ? 2 : 1;       // (two of 320 columns do not fit: filled between two barriers instead)
     static constexpr int kStagePitch = 40;
-    static constexpr bool kLdsA = R == 32;                   // A's fragments in LDS, too (R = 64: they do not fit, from L2)
+    static constexpr bool kLdsA = R == 32;                   // A's fragments in LDS, too (R = 64: from L2)
+    static constexpr int kTile = kGradTok * kPitch * 2;      // bytes of one range's rows
     static constexpr int kW = 0;                                                 // [5][R/32][4][64][8]
     static constexpr int kA = kW + (kGx ? kMix * R * 64 * 2 : 0);                // [5R/32][4][64][8]
     static constexpr int kBias = kA + (kGx && kLdsA ? kMix * R * 64 * 2 : 0);    // [5][64] fp32
     static constexpr int kMixX = kBias + kMix * 64 * 4;                          // [64] fp32
-    static constexpr int kH = kMixX + 64 * 4;                                    // [2 ranges][32][kPitch]
-    static constexpr int kG = kH + 2 * kGradTok * kPitch * 2;
-    static constexpr int kStage = kG + 2 * kGradTok * kPitch * 2;                // [4 waves][32][kStagePitch]
-    static constexpr int kBytes0 = kStage + 4 * kGradTok * kStagePitch * 2;
-    static constexpr int kFold = kAcc ? 2 * 40 * 64 * 16 : 0;                    // the ranges' accumulators are added up here at the end
+    static constexpr int kTiles = kMixX + 64 * 4;                                // [kBufs][2 ranges][h, gpre][32][kPitch]
+    static constexpr int kStage = kTiles + kBufs * 4 * kTile;                    // [8 waves][32][kStagePitch]
+    static constexpr int kBytes0 = kStage + 8 * kGradTok * kStagePitch * 2;
+    static constexpr int kFold = 2 * 40 * 64 * 16;                               // the ranges' accumulators are added up here at the end
     static constexpr int kBytes = kBytes0 > kFold ? kBytes0 : kFold;
     static_assert(kBytes <= 160 * 1024, "LDS of mix_grads_kernel");
 };
@@ -297,7 +327,7 @@ template <int R, bool kGx, bool kAcc> struct MixGrads {
 struct MixGradArgs {
     int64_t n_tok;
     int T, C, nruns, steps;      // a range is steps * 32 tokens, a run two ranges, ranges in token order
-    int r0;                      // kAcc: first column of the rank
+    int r0;                      // first column of the rank for the W and A waves
     const bf16_t *x, *h, *gpre, *w, *a_t, *g[kMix];
     const float *bias, *mix_x;
     bf16_t *gx;
@@ -306,352 +336,439 @@ struct MixGradArgs {
     float *part_bias, *part_mix;     // (ranges, 5, C), (ranges, C)
 };
 
-template <int R, bool kGx, bool kAcc>
-__global__ __launch_bounds__(kGradThreads) void mix_grads_kernel(MixGradArgs p)
-{
-    typedef MixGrads<R, kGx, kAcc> L;
-    constexpr int KW = R / 32, KA = kMix * R / 32, kCols = L::kCols, kPitch = L::kPitch;
-    constexpr int kPieces = kCols / 32;                        // 16-byte pieces of a range's h (gpre) tile per thread
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave & 1, rg = wave >> 1;
-    const int C = p.C, T = p.T;
-    const int run = (int)blockIdx.x % p.nruns, cg = (int)blockIdx.x / p.nruns;
-    const int range = run * 2 + rg;
-    const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
-    const int c0 = cg * 64 + half * 32, cl = c0 + 8 * g;
-    bf16_t *wf = reinterpret_cast<bf16_t *>(smem + L::kW), *af = reinterpret_cast<bf16_t *>(smem + L::kA);
-    float *bias_l = reinterpret_cast<float *>(smem + L::kBias), *mix_l = reinterpret_cast<float *>(smem + L::kMixX);
-    bf16_t *ht = reinterpret_cast<bf16_t *>(smem + L::kH) + rg * kGradTok * kPitch;
-    bf16_t *gt = reinterpret_cast<bf16_t *>(smem + L::kG) + rg * kGradTok * kPitch;
-    bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + wave * kGradTok * L::kStagePitch;
+// What a wave walks: its range's tokens, its 32 channels, and the step's x and g, each fetched again for the next step as
+// soon as the current one is done with it (the last step fetches itself once more: no branch, and its lines are at hand).
+// Tokens past the end read the last token's rows; their x and previous-token values are taken as zero.
+struct MixWalk {
+    const MixGradArgs &p;
+    const int l16, g, c0;
+    const int64_t first_tok;
+    int64_t base;                // element offset of the step last aimed at
+    uint32_t off[2];             // the lane's byte offset in its two 16-token blocks
+    int pos[2], pos_step;        // the lane's tokens' positions in their sequences
+    int64_t left;                // tokens from the current step's first to the end
+    Row8 xr[2], gr[kMix][2], before;   // before: in lane 0, the row of the token before the step
+    bool valid[2], last[2];      // of the current step's tokens: not past the end, the last of a sequence
 
-    // operand row l16 of tile (half, m) <-> this channel of the workgroup's 64
-    auto frag_channel = [&](int ct, int l) { return 32 * (ct >> 1) + 8 * (l >> 2) + 4 * (ct & 1) + (l & 3); };
-    if (kGx) {
-        for (int i = threadIdx.x; i < kMix * KW * 4 * 64; i += kGradThreads) {
-            const int l = i & 63, ct = (i >> 6) & 3, kk = (i >> 8) % KW, s = (i >> 8) / KW;
-            *reinterpret_cast<uint4 *>(wf + (size_t)i * 8) =
-                *reinterpret_cast<const uint4 *>(p.w + ((size_t)s * C + cg * 64 + frag_channel(ct, l & 15)) * R + 32 * kk + 8 * (l >> 4));
-        }
-        if (L::kLdsA)
-            for (int i = threadIdx.x; i < KA * 4 * 64; i += kGradThreads) {
-                const int l = i & 63, ct = (i >> 6) & 3, kk = i >> 8;
-                *reinterpret_cast<uint4 *>(af + (size_t)i * 8) =
-                    *reinterpret_cast<const uint4 *>(p.a_t + (size_t)(cg * 64 + frag_channel(ct, l & 15)) * (kMix * R) + 32 * kk + 8 * (l >> 4));
-            }
-        for (int i = threadIdx.x; i < kMix * 64; i += kGradThreads) bias_l[i] = p.bias[(size_t)(i >> 6) * C + cg * 64 + (i & 63)];
+    __device__ __forceinline__ MixWalk(const MixGradArgs &a, int range, int chan, int lane)
+        : p(a), l16(lane & 15), g(lane >> 4), c0(chan), first_tok((int64_t)range * a.steps * kGradTok) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) pos[b] = (int)((first_tok + 16 * b + l16) % p.T);
+        pos_step = kGradTok % p.T;
+        left = p.n_tok - first_tok;
+        before.zero();
+        if (l16 == 0 && left > 0 && pos[0] != 0) before.load(p.x + (first_tok - 1) * p.C + c0 + 8 * g);
+        aim(0);
+        fetch_x();
     }
-    if (threadIdx.x < 64) mix_l[threadIdx.x] = p.mix_x[cg * 64 + threadIdx.x];
-
-    // ---- loads of a step ------------------------------------------------------------------
-    Row8 xr[2], gr[kMix][2], xfirst;
-    u32x4 hp[kPieces], gp[kPieces];
-    // (tokens past the end: the last token once more, with xx and the staged x_mix zero, so that it adds nothing)
-    int64_t step_base = 0;
-    uint32_t off[2];
-    auto aim = [&](int step) {
+    __device__ __forceinline__ void aim(int step) {
         const int64_t t0 = min(first_tok + step * kGradTok, p.n_tok - 1), rest = p.n_tok - 1 - t0;
-        const int left = rest < kGradTok ? (int)rest : kGradTok;
-        step_base = t0 * C + c0;
+        const int most = rest < kGradTok ? (int)rest : kGradTok;
+        base = uniform64(t0 * p.C + c0);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) off[b] = ((uint32_t)min(16 * b + l16, left) * (uint32_t)C + 8 * g) * 2u;
-    };
-    auto fetch_x = [&]() {
-#pragma unroll
-        for (int b = 0; b < 2; ++b) load_row8(xr[b], p.x + step_base, off[b]);
-    };
-    auto fetch_g = [&](int s) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b) load_row8(gr[s][b], p.g[s] + step_base, off[b]);
-    };
-    // the range's h and gpre rows: four threads per token, 32 columns at a time
-    const int tile_row = (threadIdx.x & 127) >> 2, tile_col = (threadIdx.x & 3) * 8;
-    auto fetch_tiles = [&](int step) {
-        const int64_t t0 = min(first_tok + step * kGradTok, p.n_tok - 1), rest = p.n_tok - 1 - t0;
-        const uint32_t o = (uint32_t)(min(tile_row, (int)(rest < kGradTok ? rest : kGradTok)) * (kMix * R) + tile_col + (kGx ? 0 : p.r0)) * 2u;
-        const char *hb = reinterpret_cast<const char *>(p.h + t0 * (kMix * R)), *gb = reinterpret_cast<const char *>(p.gpre + t0 * (kMix * R));
-#pragma unroll
-        for (int j = 0; j < kPieces; ++j) {
-            hp[j] = *reinterpret_cast<const u32x4 *>(hb + o + j * (kGx ? 64 : 2 * R));
-            gp[j] = *reinterpret_cast<const u32x4 *>(gb + o + j * (kGx ? 64 : 2 * R));
-        }
-    };
-    f32x4 acc_w[kAcc ? kMix : 1][2][2], acc_a[kAcc ? 2 * kMix : 1][2];   // [s][rank tile][channel tile], [stacked rank tile][channel tile]
-    float sum_b[kAcc ? kMix : 1][2];
-    if (kAcc) {
-#pragma unroll
-        for (int s = 0; s < kMix; ++s)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    acc_w[s][i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                    acc_a[2 * s + i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                }
-                sum_b[s][i] = 0.f;
-            }
+        for (int b = 0; b < 2; ++b) off[b] = ((uint32_t)min(16 * b + l16, most) * (uint32_t)p.C + 8 * g) * 2u;
     }
-    float gmix[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float pend[8];                                    // gx of the step's last token, waiting for the next token's z
-    bool pend_valid = false, pend_last = false;
-    int pos[2];                                       // the lane's tokens' positions in their sequences
+    __device__ __forceinline__ void fetch_x() {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) pos[b] = (int)((first_tok + 16 * b + l16) % T);
-    const int pos_step = kGradTok % T;
-    xfirst.zero();
-    if (l16 == 0 && first_tok < p.n_tok && first_tok % T != 0) xfirst.load(p.x + (size_t)(first_tok - 1) * C + cl);
-    fetch_tiles(0);
-    aim(0);
-    fetch_x();
+        for (int b = 0; b < 2; ++b) load_row8(xr[b], p.x + base, off[b]);
+    }
+    __device__ __forceinline__ void fetch_g(int s) {
 #pragma unroll
-    for (int s = 0; s < kMix; ++s) fetch_g(s);
-
-    // operand fragment with the k-slots along the step's 32 tokens: column n0 + l16 of a tile of pitch `pitch`, slots
-    // 4g + e and 16 + 4g + e
-    auto frag_tokens = [&](const bf16_t *tile, int pitch, int n0) {
-        const bf16_t *q = tile + (4 * g + (l16 >> 2)) * pitch + n0 + 4 * (l16 & 3);
-        typedef s16x4 __attribute__((address_space(3))) *lds4;
-        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)q));
-        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(q + 16 * pitch)));
-        return make_bf16x8(lo[0], lo[1], hi[0], hi[1]);
-    };
-    auto stage_rows = [&](int b, bf16x8 v) { *reinterpret_cast<bf16x8 *>(stage + (16 * b + l16) * L::kStagePitch + 8 * g) = v; };
-
-    for (int step = 0; step < p.steps; ++step) {
-        __syncthreads();   // the step before has read its h and gpre tiles
-#pragma unroll
-        for (int j = 0; j < kPieces; ++j) {
-            *reinterpret_cast<u32x4 *>(ht + tile_row * kPitch + tile_col + 32 * j) = hp[j];
-            *reinterpret_cast<u32x4 *>(gt + tile_row * kPitch + tile_col + 32 * j) = gp[j];
-        }
-        const int next = min(step + 1, p.steps - 1);   // (the last step fetches itself once more: no branch, and its lines are at hand)
-        fetch_tiles(next);
-        __syncthreads();
-        const int64_t cur_base = step_base, step_tok = first_tok + step * kGradTok;
-        const uint32_t cur_off[2] = {off[0], off[1]};
-        bool valid[2], last[2];
-        float xx[2][8], mx[8];
-        {
-            const float4 m0 = *reinterpret_cast<const float4 *>(mix_l + 32 * half + 8 * g), m1 = *reinterpret_cast<const float4 *>(mix_l + 32 * half + 8 * g + 4);
-            mx[0] = m0.x; mx[1] = m0.y; mx[2] = m0.z; mx[3] = m0.w; mx[4] = m1.x; mx[5] = m1.y; mx[6] = m1.z; mx[7] = m1.w;
-        }
-        bf16x8 xmix[2];
+        for (int b = 0; b < 2; ++b) load_row8(gr[s][b], p.g[s] + base, off[b]);
+    }
+    // x and xx of the step's tokens; moves on to the next step's positions
+    __device__ __forceinline__ void x_and_xx(float (&xv)[2][8], float (&xx)[2][8]) {
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            valid[b] = step_tok + 16 * b + l16 < p.n_tok;
-            const bool first = pos[b] == 0;
-            last[b] = pos[b] == T - 1;
+            valid[b] = 16 * b + l16 < left;
+            last[b] = pos[b] == p.T - 1;
+            Row8 prev = prev_rows(before, xr[b]), cur = xr[b];
+            before = last_row_first(xr[b]);
+            const bool use_prev = valid[b] && pos[b] != 0;
+            prev.a.x = use_prev ? prev.a.x : 0; prev.a.y = use_prev ? prev.a.y : 0; prev.a.z = use_prev ? prev.a.z : 0; prev.a.w = use_prev ? prev.a.w : 0;
+            cur.a.x = valid[b] ? cur.a.x : 0; cur.a.y = valid[b] ? cur.a.y : 0; cur.a.z = valid[b] ? cur.a.z : 0; cur.a.w = valid[b] ? cur.a.w : 0;
+            cur.to_float(xv[b]);
+            prev.to_float(xx[b]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xx[b][e] -= xv[b][e];
             pos[b] += pos_step;
-            if (pos[b] >= T) pos[b] -= T;
-            float xv[8];
-            xr[b].to_float(xv);
-            prev_rows(xfirst, xr[b]).to_float(xx[b]);
-            xfirst = last_row_first(xr[b]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) xx[b][e] = valid[b] ? (first ? 0.f : xx[b][e]) - xv[e] : 0.f;
-            if (kAcc) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) xv[e] = valid[b] ? fmaf(xx[b][e], mx[e], xv[e]) : 0.f;
-                stage_rows(b, pack_operand(xv));
-            }
+            if (pos[b] >= p.T) pos[b] -= p.T;
         }
-        aim(next);
-        fetch_x();
-        __builtin_amdgcn_sched_barrier(0);
-        if (kAcc) {   // gA
-            const bf16x8 xt[2] = {frag_tokens(stage, L::kStagePitch, 0), frag_tokens(stage, L::kStagePitch, 16)};
+        left -= kGradTok;
+    }
+};
+
+__device__ __forceinline__ void load8(const float *p, float (&v)[8]) {
+    const f32x4 a = *reinterpret_cast<const f32x4 *>(p), b = *reinterpret_cast<const f32x4 *>(p + 4);
 #pragma unroll
-            for (int i = 0; i < 2 * kMix; ++i) {
-                const bf16x8 gq = frag_tokens(gt, kPitch, kGx ? (i >> 1) * R + 16 * (i & 1) : 16 * i);
+    for (int e = 0; e < 4; ++e) { v[e] = a[e]; v[4 + e] = b[e]; }
+}
+__device__ __forceinline__ void store8(float *p, const float (&v)[8]) {
+    *reinterpret_cast<f32x4 *>(p) = (f32x4){v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f32x4 *>(p + 4) = (f32x4){v[4], v[5], v[6], v[7]};
+}
+
+// Rows of h or gpre for a range's tile: 128 threads, four per token, 32 columns at a time
+template <int R, bool kGx> struct MixTile {
+    static constexpr int kPieces = MixGrads<R, kGx>::kCols / 32;
+    u32x4 v[kPieces];
+    __device__ __forceinline__ void fetch(const MixGradArgs &p, const bf16_t *src, int64_t first_tok, int step, int tid) {
+        const int64_t t0 = uniform64(min(first_tok + step * kGradTok, p.n_tok - 1)), rest = p.n_tok - 1 - t0;
+        const uint32_t o = (uint32_t)(min(tid >> 2, (int)(rest < kGradTok ? rest : kGradTok)) * (kMix * R) + (tid & 3) * 8 + (kGx ? 0 : p.r0)) * 2u;
+        const char *b = reinterpret_cast<const char *>(src + t0 * (kMix * R));
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc_a[kAcc ? i : 0][j] = mfma32(xt[j], gq, acc_a[kAcc ? i : 0][j]);
-                if (i & 1) __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int j = 0; j < kPieces; ++j) v[j] = *reinterpret_cast<const u32x4 *>(b + o + j * (kGx ? 64 : 2 * R));
+    }
+    __device__ __forceinline__ void put(bf16_t *tile, int tid) const {
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            *reinterpret_cast<u32x4 *>(tile + (tid >> 2) * MixGrads<R, kGx>::kPitch + (tid & 3) * 8 + 32 * j) = v[j];
+    }
+};
+// where a range's h (which = 0) or gpre (1) rows of a step are
+template <int R, bool kGx> __device__ __forceinline__ bf16_t *mix_tile(unsigned char *smem, int step, int rg, int which) {
+    typedef MixGrads<R, kGx> L;
+    return reinterpret_cast<bf16_t *>(smem + L::kTiles + (((L::kBufs == 2 ? step & 1 : 0) * 2 + rg) * 2 + which) * L::kTile);
+}
+// the barriers at the head of a step: its rows are in LDS behind them
+template <int R, bool kGx> __device__ __forceinline__ void mix_step_begins() {
+    __syncthreads();
+    if (MixGrads<R, kGx>::kBufs == 1) __syncthreads();   // (the A waves fill the only buffer in between)
+}
+// operand fragment with the k-slots along a step's 32 tokens: column n0 + l16 of a tile.  A lane group's four slots are
+// tokens two apart: with 20 banks from row to row, their four 32-byte pieces then lie on all 32 different banks.
+__device__ __forceinline__ bf16x8 mix_frag_tokens(const bf16_t *tile, int pitch, int n0, int l16, int g) {
+    const bf16_t *q = tile + (8 * (g >> 1) + (g & 1) + 2 * (l16 >> 2)) * pitch + n0 + 4 * (l16 & 3);
+    typedef s16x4 __attribute__((address_space(3))) *lds4;
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)q));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(q + 16 * pitch)));
+    return make_bf16x8(lo[0], lo[1], hi[0], hi[1]);
+}
+
+// operand row l of tile ct <-> this channel of the workgroup's 64
+__device__ __forceinline__ int mix_frag_channel(int ct, int l) { return 32 * (ct >> 1) + 8 * (l >> 2) + 4 * (ct & 1) + (l & 3); }
+
+template <int R>
+__device__ __forceinline__ void mix_gx_wave(const MixGradArgs &p, unsigned char *smem, int range, int rg, int cg, int half, int lane)
+{
+    typedef MixGrads<R, true> L;
+    constexpr int KW = R / 32, KA = kMix * R / 32, kPitch = L::kPitch;
+    const int l16 = lane & 15, g = lane >> 4, C = p.C;
+    const bf16_t *wf = reinterpret_cast<const bf16_t *>(smem + L::kW), *af = reinterpret_cast<const bf16_t *>(smem + L::kA);
+    const float *bias_l = reinterpret_cast<const float *>(smem + L::kBias) + 32 * half + 8 * g;
+    const float *mix_l = reinterpret_cast<const float *>(smem + L::kMixX) + 32 * half + 8 * g;
+    const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
+    MixWalk wk(p, range, cg * 64 + half * 32, lane);
+#pragma unroll
+    for (int s = 0; s < kMix; ++s) wk.fetch_g(s);
+    float gmix[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float pend[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // gx of the step's last token, waiting for the next token's z
+    bool pend_valid = false, pend_last = false;
+    auto put = [&](int64_t base, uint32_t o, const float (&v)[8]) {
+        *reinterpret_cast<bf16x8 *>(reinterpret_cast<char *>(p.gx + base) + o) = pack_operand(v);
+    };
+    for (int step = 0; step < p.steps; ++step) {
+        mix_step_begins<R, true>();
+        const bf16_t *ht = mix_tile<R, true>(smem, step, rg, 0), *gt = mix_tile<R, true>(smem, step, rg, 1);
+        const int next = min(step + 1, p.steps - 1);
+        const int64_t cur_base = wk.base, step_tok = first_tok + step * kGradTok;
+        const uint32_t cur_off[2] = {wk.off[0], wk.off[1]};
+        float xx[2][8], gsum[2][8], gxx[2][8];
+        {
+            float xv[2][8];
+            wk.x_and_xx(xv, xx);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        float gsum[2][8], gxx[2][8];
-        if (kGx) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { gsum[b][e] = 0.f; gxx[b][e] = 0.f; }
-        }
+        wk.aim(next);
+        wk.fetch_x();
 #pragma unroll
         for (int s = 0; s < kMix; ++s) {
             f32x4 cf[2][2];
-            if (kGx) {
-                bf16x8 wfr[2][KW];
+            bf16x8 wfr[2][KW];
 #pragma unroll
-                for (int m = 0; m < 2; ++m) {
-                    const float4 bb = *reinterpret_cast<const float4 *>(bias_l + 64 * s + 32 * half + 8 * g + 4 * m);
-                    cf[0][m] = cf[1][m] = (f32x4){bb.x, bb.y, bb.z, bb.w};
+            for (int m = 0; m < 2; ++m) {
+                cf[0][m] = cf[1][m] = *reinterpret_cast<const f32x4 *>(bias_l + 64 * s + 4 * m);
 #pragma unroll
-                    for (int kk = 0; kk < KW; ++kk)
-                        wfr[m][kk] = *reinterpret_cast<const bf16x8 *>(wf + (size_t)(((s * KW + kk) * 4 + 2 * half + m) * 64 + lane) * 8);
-                }
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int kk = 0; kk < KW; ++kk) {
-                        const bf16x8 hr = *reinterpret_cast<const bf16x8 *>(ht + (16 * b + l16) * kPitch + s * R + 32 * kk + 8 * g);
-#pragma unroll
-                        for (int m = 0; m < 2; ++m) cf[b][m] = mfma32(wfr[m][kk], hr, cf[b][m]);
-                    }
+                for (int kk = 0; kk < KW; ++kk)
+                    wfr[m][kk] = *reinterpret_cast<const bf16x8 *>(wf + (size_t)(((s * KW + kk) * 4 + 2 * half + m) * 64 + lane) * 8);
             }
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                float gv[8];
-                gr[s][b].to_float(gv);
-                if (kGx) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        gsum[b][e] += gv[e];
-                        gxx[b][e] = fmaf(gv[e], cf[b][e >> 2][e & 3], gxx[b][e]);
-                    }
-                    pin8(gsum[b]);   // (or the sums sink to their use behind the branches below, with every g still in registers)
-                    pin8(gxx[b]);
-                }
-                if (kAcc) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) gv[e] *= xx[b][e];
-                    stage_rows(b, pack_operand(gv));
-                }
-            }
-            fetch_g(s);
-            if (kAcc) {
-                const bf16x8 gc[2] = {frag_tokens(stage, L::kStagePitch, 0), frag_tokens(stage, L::kStagePitch, 16)};
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    float f[8];
-                    unpack8(gc[j], f);
-                    sum_b[kAcc ? s : 0][j] += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
-                }
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const bf16x8 hq = frag_tokens(ht, kPitch, (kGx ? s * R : s * 32) + 16 * i);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) acc_w[kAcc ? s : 0][i][j] = mfma32(hq, gc[j], acc_w[kAcc ? s : 0][i][j]);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (kGx) {
-            f32x4 xm[2][2];   // gxm, the same lane order as coef
-#pragma unroll
-            for (int b = 0; b < 2; ++b) xm[b][0] = xm[b][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kk = 0; kk < KA; ++kk) {
-                bf16x8 afr[2];
-#pragma unroll
-                for (int m = 0; m < 2; ++m)
-                    afr[m] = L::kLdsA ? *reinterpret_cast<const bf16x8 *>(af + (size_t)((kk * 4 + 2 * half + m) * 64 + lane) * 8)
-                                      : *reinterpret_cast<const bf16x8 *>(p.a_t + (size_t)(cg * 64 + frag_channel(2 * half + m, l16)) * (kMix * R) + 32 * kk + 8 * g);
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const bf16x8 gq = *reinterpret_cast<const bf16x8 *>(gt + (16 * b + l16) * kPitch + 32 * kk + 8 * g);
-#pragma unroll
-                    for (int m = 0; m < 2; ++m) xm[b][m] = mfma32(afr[m], gq, xm[b][m]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            float o[2][8];
 #pragma unroll
             for (int b = 0; b < 2; ++b)
 #pragma unroll
+                for (int kk = 0; kk < KW; ++kk) {
+                    const bf16x8 hr = *reinterpret_cast<const bf16x8 *>(ht + (16 * b + l16) * kPitch + s * R + 32 * kk + 8 * g);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) cf[b][m] = mfma32(wfr[m][kk], hr, cf[b][m]);
+                }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float gv[8];
+                wk.gr[s][b].to_float(gv);
+#pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float m = xm[b][e >> 2][e & 3];
-                    gmix[e] = fmaf(m, xx[b][e], gmix[e]);
-                    o[b][e] = gsum[b][e] - gxx[b][e] + m * (1.f - mx[e]);
-                    gxx[b][e] = fmaf(m, mx[e], gxx[b][e]);             // z
+                    gsum[b][e] = s == 0 ? gv[e] : gsum[b][e] + gv[e];
+                    gxx[b][e] = s == 0 ? gv[e] * cf[b][e >> 2][e & 3] : fmaf(gv[e], cf[b][e >> 2][e & 3], gxx[b][e]);
                 }
-            pin8(o[0]); pin8(o[1]); pin8(gmix);
-            __builtin_amdgcn_sched_barrier(0);
-            if (step == 0 && l16 == 0) {
-                float *q = p.edge_first + (size_t)range * C + cl;
-                *reinterpret_cast<float4 *>(q) = make_float4(gxx[0][0], gxx[0][1], gxx[0][2], gxx[0][3]);
-                *reinterpret_cast<float4 *>(q + 4) = make_float4(gxx[0][4], gxx[0][5], gxx[0][6], gxx[0][7]);
+                pin8(gsum[b]);   // (or the sums sink to their use behind the branches below, with every g still in registers)
+                pin8(gxx[b]);
             }
-            float z0[8];   // lane 15: z of this step's first token
-#pragma unroll
-            for (int e = 0; e < 8; ++e) z0[e] = first_to_last(gxx[0][e]);
-            auto put = [&](int64_t base, uint32_t o, const float (&v)[8]) {
-                *reinterpret_cast<bf16x8 *>(reinterpret_cast<char *>(p.gx + base) + o) = pack_operand(v);
-            };
-            if (step > 0 && pend_valid && l16 == 15) {
-                if (!pend_last) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) pend[e] += z0[e];
-                }
-                put((step_tok - 1) * C + c0, 16u * g, pend);
-            }
-            float zn[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) zn[e] = next_lane(first_to_last(gxx[1][e]), gxx[0][e]);
-            if (!last[0]) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[0][e] += zn[e];
-            }
-            if (valid[0]) put(cur_base, cur_off[0], o[0]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pend[e] = o[1][e];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) zn[e] = next_lane(0.f, gxx[1][e]);
-            if (!last[1]) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[1][e] += zn[e];
-            }
-            if (valid[1] && l16 < 15) put(cur_base, cur_off[1], o[1]);
-            pend_valid = valid[1]; pend_last = last[1];
+            wk.fetch_g(s);
+            if (s & 1) __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 xm[2][2];   // gxm, the same lane order as coef
+#pragma unroll
+        for (int b = 0; b < 2; ++b) xm[b][0] = xm[b][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < KA; ++kk) {
+            bf16x8 afr[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                afr[m] = L::kLdsA ? *reinterpret_cast<const bf16x8 *>(af + (size_t)((kk * 4 + 2 * half + m) * 64 + lane) * 8)
+                                  : *reinterpret_cast<const bf16x8 *>(p.a_t + (size_t)(cg * 64 + mix_frag_channel(2 * half + m, l16)) * (kMix * R) + 32 * kk + 8 * g);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const bf16x8 gq = *reinterpret_cast<const bf16x8 *>(gt + (16 * b + l16) * kPitch + 32 * kk + 8 * g);
+#pragma unroll
+                for (int m = 0; m < 2; ++m) xm[b][m] = mfma32(afr[m], gq, xm[b][m]);
+            }
+            if (kk & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        float o[2][8], mx[8];
+        load8(mix_l, mx);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float m = xm[b][e >> 2][e & 3];
+                gmix[e] = fmaf(m, xx[b][e], gmix[e]);
+                gxx[b][e] = fmaf(m, mx[e], gxx[b][e]);             // z
+                o[b][e] = (gsum[b][e] + m) - gxx[b][e];
+            }
+        pin8(o[0]); pin8(o[1]); pin8(gmix);
+        __builtin_amdgcn_sched_barrier(0);
+        if (step == 0 && l16 == 0) store8(p.edge_first + (size_t)range * C + wk.c0 + 8 * g, gxx[0]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {                  // lane 15: z of this step's first token
+            const float z = first_to_last(gxx[0][e]);  // (with all lanes: a lane that is switched off is not read)
+            pend[e] += pend_last ? 0.f : z;
+        }
+        if (step > 0 && pend_valid && l16 == 15) {
+            put((step_tok - 1) * C + wk.c0, 16u * g, pend);
+        }
+        float zn[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) zn[e] = next_lane(first_to_last(gxx[1][e]), gxx[0][e]);
+        if (!wk.last[0]) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[0][e] += zn[e];
+        }
+        if (wk.valid[0]) put(cur_base, cur_off[0], o[0]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            pend[e] = o[1][e];
+            zn[e] = next_lane(0.f, gxx[1][e]);
+        }
+        if (!wk.last[1]) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[1][e] += zn[e];
+        }
+        if (wk.valid[1] && l16 < 15) put(cur_base, cur_off[1], o[1]);
+        pend_valid = wk.valid[1]; pend_last = wk.last[1];
     }
+    if (pend_valid && l16 == 15) {   // the range's last token: complete if a sequence ends with it
+        if (pend_last) put((first_tok + (int64_t)p.steps * kGradTok - 1) * C + wk.c0, 16u * g, pend);
+        else store8(p.edge_last + (size_t)range * C + wk.c0 + 8 * g, pend);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) gmix[e] += __shfl_xor(gmix[e], m);
+    if (l16 == 0) store8(p.part_mix + (size_t)range * C + wk.c0 + 8 * g, gmix);
+    __syncthreads();   // (the other waves fold their accumulators in two phases)
+    __syncthreads();
+}
+
+// The second range's accumulators through LDS to the first's wave, then one partial per workgroup.
+template <int N>
+__device__ __forceinline__ void mix_fold(const f32x4 (&acc)[N], f32x4 *fold, float *part, size_t tile0, int rg, int lane)
+{
+    __syncthreads();
+    if (rg == 1) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) fold[i * 64 + lane] = acc[i];
+    }
+    __syncthreads();
+    if (rg == 0) {
+        f32x4 *q = reinterpret_cast<f32x4 *>(part) + tile0 * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i * 64] = acc[i] + fold[i * 64 + lane];
+    }
+}
+
+template <int R, bool kGx>
+__device__ __forceinline__ void mix_w_wave(const MixGradArgs &p, unsigned char *smem, int range, int rg, int run, int cg, int half, int lane)
+{
+    typedef MixGrads<R, kGx> L;
+    const int l16 = lane & 15, g = lane >> 4, C = p.C;
+    bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + (2 * rg + half) * kGradTok * L::kStagePitch;
+    const int col0 = kGx ? p.r0 : 0;                          // of a mixer's columns in the tile
+    constexpr int kMixCols = kGx ? R : 32;
+    f32x4 acc[4 * kMix];                                      // (s, rank tile, channel tile): rows = rank, columns = channels
+    f32x4 acc_b[2];                                           // row s: gbias of mixer s
+#pragma unroll
+    for (int i = 0; i < 4 * kMix; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    acc_b[0] = acc_b[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    MixWalk wk(p, range, cg * 64 + half * 32, lane);
+    // g_s is fetched only while g_{s-kAhead} is worked on, for the registers' sake: the gx waves brought its lines to L2
+    constexpr int kAhead = 2;
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) wk.fetch_g(s);
+    for (int step = 0; step < p.steps; ++step) {
+        mix_step_begins<R, kGx>();
+        const bf16_t *ht = mix_tile<R, kGx>(smem, step, rg, 0);
+        float xx[2][8];
+        {
+            float xv[2][8];
+            wk.x_and_xx(xv, xx);
+            pin8(xx[0]); pin8(xx[1]);
+        }
+#pragma unroll
+        for (int s = 0; s < kMix; ++s) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                float gv[8];
+                wk.gr[s][b].to_float(gv);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) gv[e] *= xx[b][e];
+                *reinterpret_cast<bf16x8 *>(stage + (16 * b + l16) * L::kStagePitch + 8 * g) = pack_operand(gv);
+            }
+            if (s + kAhead == kMix) { wk.aim(min(step + 1, p.steps - 1)); wk.fetch_x(); }
+            wk.fetch_g((s + kAhead) % kMix);
+            const bf16x8 gc[2] = {mix_frag_tokens(stage, L::kStagePitch, 0, l16, g), mix_frag_tokens(stage, L::kStagePitch, 16, l16, g)};
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16x8 hq = mix_frag_tokens(ht, L::kPitch, s * kMixCols + col0 + 16 * i, l16, g);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[4 * s + 2 * i + j] = mfma32(hq, gc[j], acc[4 * s + 2 * i + j]);
+            }
+            uint32_t one = l16 == s ? 0x3f803f80u : 0u;         // bf16 ones in row s alone: the mixers' sums share a tile
+            asm volatile("" : "+v"(one));                       // (made where it is used: five operands kept across the loop are 20 registers)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc_b[j] = mfma32(make_bf16x8(one, one, one, one), gc[j], acc_b[j]);
+            if (s & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (p.r0 == 0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (4 * g + e < kMix) p.part_bias[((size_t)range * kMix + 4 * g + e) * C + wk.c0 + 16 * j + l16] = acc_b[j][e];
+    }
+    mix_fold(acc, reinterpret_cast<f32x4 *>(smem) + half * 40 * 64, p.part_w, ((size_t)(run * (C / 64) + cg) * 2 + half) * 20, rg, lane);
+}
+
+template <int R, bool kGx>
+__device__ __forceinline__ void mix_a_wave(const MixGradArgs &p, unsigned char *smem, int range, int rg, int run, int cg, int half, int lane)
+{
+    typedef MixGrads<R, kGx> L;
+    const int l16 = lane & 15, g = lane >> 4, tid = half * 64 + lane, C = p.C;
+    const float *mix_l = reinterpret_cast<const float *>(smem + L::kMixX) + 32 * half + 8 * g;
+    bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + (4 + 2 * rg + half) * kGradTok * L::kStagePitch;
+    const int col0 = kGx ? p.r0 : 0;
+    constexpr int kMixCols = kGx ? R : 32;
+    f32x4 acc[4 * kMix];                                      // (s, rank tile, channel tile): rows = channels, columns = rank
+#pragma unroll
+    for (int i = 0; i < 4 * kMix; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
+    MixTile<R, kGx> tile;
+    auto fill = [&](const bf16_t *src, int from, int step, int which) {
+        tile.fetch(p, src, first_tok, from, tid);
+        tile.put(mix_tile<R, kGx>(smem, step, rg, which), tid);
+    };
+    if (L::kBufs == 2) {
+        fill(p.h, 0, 0, 0);
+        fill(p.gpre, 0, 0, 1);
+    }
+    MixWalk wk(p, range, cg * 64 + half * 32, lane);
+    for (int step = 0; step < p.steps; ++step) {
+        __syncthreads();
+        const int next = min(step + 1, p.steps - 1);
+        if (L::kBufs == 1) {
+            fill(p.h, step, step, 0);
+            fill(p.gpre, step, step, 1);
+            __syncthreads();
+        } else {
+            tile.fetch(p, p.h, first_tok, next, tid);
+        }
+        {
+            float xv[2][8], xx[2][8], mx[8];
+            wk.x_and_xx(xv, xx);
+            wk.aim(next);
+            wk.fetch_x();
+            load8(mix_l, mx);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) xv[b][e] = fmaf(xx[b][e], mx[e], xv[b][e]);
+                *reinterpret_cast<bf16x8 *>(stage + (16 * b + l16) * L::kStagePitch + 8 * g) = pack_operand(xv[b]);
+            }
+        }
+        if (L::kBufs == 2) {
+            tile.put(mix_tile<R, kGx>(smem, step + 1, rg, 0), tid);
+            tile.fetch(p, p.gpre, first_tok, next, tid);
+        }
+        const bf16x8 xt[2] = {mix_frag_tokens(stage, L::kStagePitch, 0, l16, g), mix_frag_tokens(stage, L::kStagePitch, 16, l16, g)};
+        const bf16_t *gt = mix_tile<R, kGx>(smem, step, rg, 1);
+#pragma unroll
+        for (int i = 0; i < 2 * kMix; ++i) {
+            const bf16x8 gq = mix_frag_tokens(gt, L::kPitch, (i >> 1) * kMixCols + col0 + 16 * (i & 1), l16, g);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[2 * i + j] = mfma32(xt[j], gq, acc[2 * i + j]);
+            if (i % 5 == 4) __builtin_amdgcn_sched_barrier(0);
+        }
+        if (L::kBufs == 2) tile.put(mix_tile<R, kGx>(smem, step + 1, rg, 1), tid);
+    }
+    mix_fold(acc, reinterpret_cast<f32x4 *>(smem) + (half * 40 + 20) * 64, p.part_a, ((size_t)(run * (C / 64) + cg) * 2 + half) * 20, rg, lane);
+}
+
+template <int R, bool kGx>
+__global__ __launch_bounds__(kGx ? 768 : 512) void mix_grads_kernel(MixGradArgs p)
+{
+    typedef MixGrads<R, kGx> L;
+    constexpr int KW = R / 32, KA = kMix * R / 32;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = wave & 1, rg = (wave >> 1) & 1;
+    const int run = (int)blockIdx.x % p.nruns, cg = (int)blockIdx.x / p.nruns, range = run * 2 + rg;
+    bf16_t *wf = reinterpret_cast<bf16_t *>(smem + L::kW), *af = reinterpret_cast<bf16_t *>(smem + L::kA);
+    float *bias_l = reinterpret_cast<float *>(smem + L::kBias), *mix_l = reinterpret_cast<float *>(smem + L::kMixX);
     if (kGx) {
-        if (pend_valid && l16 == 15) {   // the range's last token: complete if a sequence ends with it
-            if (pend_last) *reinterpret_cast<bf16x8 *>(p.gx + (first_tok + (int64_t)p.steps * kGradTok - 1) * C + cl) = pack_operand(pend);
-            else {
-                float *q = p.edge_last + (size_t)range * C + cl;
-                *reinterpret_cast<float4 *>(q) = make_float4(pend[0], pend[1], pend[2], pend[3]);
-                *reinterpret_cast<float4 *>(q + 4) = make_float4(pend[4], pend[5], pend[6], pend[7]);
+        for (int i = threadIdx.x; i < kMix * KW * 4 * 64; i += L::kThreads) {
+            const int l = i & 63, ct = (i >> 6) & 3, kk = (i >> 8) % KW, s = (i >> 8) / KW;
+            *reinterpret_cast<uint4 *>(wf + (size_t)i * 8) =
+                *reinterpret_cast<const uint4 *>(p.w + ((size_t)s * p.C + cg * 64 + mix_frag_channel(ct, l & 15)) * R + 32 * kk + 8 * (l >> 4));
+        }
+        if (L::kLdsA)
+            for (int i = threadIdx.x; i < KA * 4 * 64; i += L::kThreads) {
+                const int l = i & 63, ct = (i >> 6) & 3, kk = i >> 8;
+                *reinterpret_cast<uint4 *>(af + (size_t)i * 8) =
+                    *reinterpret_cast<const uint4 *>(p.a_t + (size_t)(cg * 64 + mix_frag_channel(ct, l & 15)) * (kMix * R) + 32 * kk + 8 * (l >> 4));
             }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-#pragma unroll
-            for (int m = 8; m >= 1; m >>= 1) gmix[e] += __shfl_xor(gmix[e], m);
-        if (l16 == 0) {
-            float *q = p.part_mix + (size_t)range * C + cl;
-            *reinterpret_cast<float4 *>(q) = make_float4(gmix[0], gmix[1], gmix[2], gmix[3]);
-            *reinterpret_cast<float4 *>(q + 4) = make_float4(gmix[4], gmix[5], gmix[6], gmix[7]);
-        }
+        for (int i = threadIdx.x; i < kMix * 64; i += L::kThreads) bias_l[i] = p.bias[(size_t)(i >> 6) * p.C + cg * 64 + (i & 63)];
     }
-    if (kAcc) {
-#pragma unroll
-        for (int s = 0; s < kMix; ++s)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float v = sum_rows(sum_b[kAcc ? s : 0][j]);
-                if (p.r0 == 0 && g == 0) p.part_bias[((size_t)range * kMix + s) * C + c0 + 16 * j + l16] = v;
-            }
-        // the second range's accumulators through LDS to the first's wave, then one partial per workgroup
-        f32x4 *fold = reinterpret_cast<f32x4 *>(smem) + half * 40 * 64;
-        __syncthreads();
-        if (rg == 1) {
-#pragma unroll
-            for (int i = 0; i < 20; ++i) {
-                fold[i * 64 + lane] = acc_w[kAcc ? i >> 2 : 0][(i >> 1) & 1][i & 1];
-                fold[(20 + i) * 64 + lane] = acc_a[kAcc ? i >> 1 : 0][i & 1];
-            }
-        }
-        __syncthreads();
-        if (rg == 0) {
-            const size_t base = ((size_t)(run * (C / 64) + cg) * 2 + half) * 20 * 64 + lane;
-            f32x4 *pw = reinterpret_cast<f32x4 *>(p.part_w) + base, *pa = reinterpret_cast<f32x4 *>(p.part_a) + base;
-#pragma unroll
-            for (int i = 0; i < 20; ++i) {
-                pw[i * 64] = acc_w[kAcc ? i >> 2 : 0][(i >> 1) & 1][i & 1] + fold[i * 64 + lane];
-                pa[i * 64] = acc_a[kAcc ? i >> 1 : 0][i & 1] + fold[(20 + i) * 64 + lane];
-            }
-        }
+    if (threadIdx.x < 64) mix_l[threadIdx.x] = p.mix_x[cg * 64 + threadIdx.x];
+    __syncthreads();
+    // (the waves that fetch from memory and fill the tiles go first where a SIMD has a choice)
+    if (wave < 4) {
+        __builtin_amdgcn_s_setprio(3);
+        mix_a_wave<R, kGx>(p, smem, range, rg, run, cg, half, lane);
+    } else if (wave < 8) {
+        mix_w_wave<R, kGx>(p, smem, range, rg, run, cg, half, lane);
+    } else if (kGx) {
+        __builtin_amdgcn_s_setprio(3);
+        mix_gx_wave<R>(p, smem, range, rg, cg, half, lane);
     }
 }
 
@@ -668,6 +785,7 @@ __global__ __launch_bounds__(256) void mix_finish_kernel(MixGradArgs p, int R, T
         if (i >= per_run) return;
         const f32x4 *src = reinterpret_cast<const f32x4 *>(blockIdx.y == 0 ? p.part_w : p.part_a) + i;
         f32x4 s = src[0];
+#pragma unroll 8
         for (int q = 1; q < p.nruns; ++q) s += src[(size_t)q * per_run];
         const int lane = i & 63, l16 = lane & 15, g = lane >> 4, tile = (i >> 6) % 20, c0 = (i / (64 * 20)) * 32;
         if (blockIdx.y == 0) {   // tile (s, rank tile, channel tile): rows = rank, columns = channels
@@ -681,6 +799,7 @@ __global__ __launch_bounds__(256) void mix_finish_kernel(MixGradArgs p, int R, T
         if (i >= (kMix + 1) * C) return;
         const bool is_mix = i >= kMix * C;
         float s = 0.f;
+#pragma unroll 8
         for (int q = 0; q < nranges; ++q) s += is_mix ? p.part_mix[(size_t)q * C + i - kMix * C] : p.part_bias[(size_t)q * kMix * C + i];
         if (is_mix) gmix[i - kMix * C] = s; else gbias[i] = s;
     } else {
@@ -727,10 +846,12 @@ hipError_t shift_mix_forward(hipStream_t st, int weight_dtype, int64_t B, int64_
                              const void *a, const void *w2t, const float *bias, void *weights, void *h, void *const out[5]) {
     const MixWeightForms w(weights, C, R);
     const dim3 grid((unsigned)(C / 32), 2);
-    if (weight_dtype == kF32)
-        hipLaunchKernelGGL(mix_weights_kernel<float>, grid, dim3(256), 0, st, (int)C, (int)R, (const float *)a, (const float *)w2t, w.a_frag, w.wt_frag, w.a_t, w.w);
-    else
-        hipLaunchKernelGGL(mix_weights_kernel<bf16_t>, grid, dim3(256), 0, st, (int)C, (int)R, (const bf16_t *)a, (const bf16_t *)w2t, w.a_frag, w.wt_frag, w.a_t, w.w);
+    auto pack = [&](auto kernel, auto *tag) {
+        typedef std::remove_pointer_t<decltype(tag)> Tw;
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, (int)C, (const Tw *)a, (const Tw *)w2t, w.a_frag, w.wt_frag, w.a_t, w.w);
+    };
+    if (weight_dtype == kF32) R == 32 ? pack(mix_weights_kernel<float, 32>, (float *)nullptr) : pack(mix_weights_kernel<float, 64>, (float *)nullptr);
+    else R == 32 ? pack(mix_weights_kernel<bf16_t, 32>, (bf16_t *)nullptr) : pack(mix_weights_kernel<bf16_t, 64>, (bf16_t *)nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = R == 32 ? launch_reduce<32, false>(st, B * T, T, C, x, mix_x, w.a_frag, nullptr, nullptr, h)
@@ -772,13 +893,13 @@ size_t shift_mix_backward_workspace_bytes(int64_t B, int64_t T, int64_t C, int64
     return MixWorkspace(B * T, C, R, MixCut(B * T, C)).bytes;
 }
 
-template <int R, bool kGx, bool kAcc>
+template <int R, bool kGx>
 static hipError_t launch_grads(hipStream_t st, const MixGradArgs &p) {
-    constexpr auto kern = mix_grads_kernel<R, kGx, kAcc>;
-    constexpr int lds = MixGrads<R, kGx, kAcc>::kBytes;
-    hipError_t e = allow_dynamic_lds<kern>(lds);
+    constexpr auto kern = mix_grads_kernel<R, kGx>;
+    typedef MixGrads<R, kGx> L;
+    hipError_t e = allow_dynamic_lds<kern>(L::kBytes);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(p.nruns * (p.C / 64))), dim3(kGradThreads), lds, st, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(p.nruns * (p.C / 64))), dim3(L::kThreads), L::kBytes, st, p);
     return hipGetLastError();
 }
 
@@ -811,14 +932,12 @@ hipError_t shift_mix_backward(hipStream_t st, int weight_dtype, int64_t B, int64
             hipLaunchKernelGGL(mix_finish_kernel<bf16_t>, grid, dim3(256), 0, st, p, (int)R, (bf16_t *)gw2t, (bf16_t *)ga, gbias, gmix_x);
         return hipGetLastError();
     };
-    if (R == 32) {
-        e = launch_grads<32, true, true>(st, p);
-        return e != hipSuccess ? e : finish(4);
-    }
-    e = launch_grads<64, true, false>(st, p);
-    for (p.r0 = 0; e == hipSuccess && p.r0 < 64; p.r0 += 32) {
-        e = launch_grads<64, false, true>(st, p);
-        if (e == hipSuccess) e = finish(p.r0 == 0 ? 4 : 2);
+    e = R == 32 ? launch_grads<32, true>(st, p) : launch_grads<64, true>(st, p);
+    if (e == hipSuccess) e = finish(4);
+    if (R == 64 && e == hipSuccess) {
+        p.r0 = 32;
+        e = launch_grads<64, false>(st, p);
+        if (e == hipSuccess) e = finish(2);
     }
     return e;
 }
