@@ -14,8 +14,8 @@
 // workgroup, so the gradients g_s are read twice: mix_reduce_kernel<grad> takes whole rows of a few tokens (gpre
 // complete, nothing to combine between workgroups), mix_grads_kernel takes 64 channels of many tokens (the weight
 // gradients stay in accumulators, one partial per workgroup).
-// B8 T1024 C2048 R32, forward and backward through the torch flavour: 250 us; as four elementwise kernels around six
-// library products (gcoef written and read twice, x_mix written and read) 572 us, of which 235 us the skinny products.
+// B8 T1024 C2048 R32, forward and backward: 195 us of kernels; as four elementwise kernels around six library products
+// (gcoef written and read twice, x_mix written and read) 504 us, of which 235 us the skinny products.
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
 #include "wkv6_mfma.h"
@@ -136,7 +136,9 @@ __device__ __forceinline__ float tanh_bf16(float x) {
 // Sums over channels:  forward  h = tanh(x_mix A^T);  kGrad  gpre = (gcoef_s W_s)_s (1 - h^2).
 // One workgroup takes all channels of 32 tokens (16 at R = 64: the accumulators), so nothing is left to combine; its
 // eight waves take 32-channel chunks in turn and add up through LDS at the end.  The weights' fragments come from L2 once
-// per workgroup.  A chunk's x and g are fetched while the chunk before it is worked on.
+// per workgroup (16 tokens per workgroup, i.e. twice that traffic: 30 and 73 us instead of 21 and 50).  A chunk's x and
+// g are fetched while the chunk before it is worked on.  B8 T1024 C2048 R32: 21 us forward, latencies of a launch of one
+// workgroup per compute unit (12 us with nothing fetched in the loop); 50 us backward for 201 MB read.
 // ------------------------------------------------------------------------------------------
 constexpr int kReduceWaves = 8;
 template <int R> struct MixReduce {
@@ -300,7 +302,8 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
 //   W waves:   gcoef, transposed through a tile of their own in LDS (the transposing read), for gW and gbias;
 //   A waves:   x_mix, the same way, for gA; they also bring the h and gpre rows that all roles read from LDS.
 // (The roles read the same x and g: the later reads find the lines in L1 or L2.  One wave doing everything had a SIMD to
-// itself for its 440 registers and every LDS and MFMA latency in the open.)
+// itself for its 440 registers and every LDS and MFMA latency in the open: 84 us at B8 T1024 C2048 R32 against 74 so.  The
+// traffic alone, 256 MB, would take 50 us; the roles alone take 45, 44 and 32 us: vector instructions and LDS on top.)
 // R = 64: a second launch without gx waves (kGx false) does the other half of the rank's columns.
 // ------------------------------------------------------------------------------------------
 constexpr int kGradTok = 32;
