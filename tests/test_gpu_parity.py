@@ -616,6 +616,13 @@ def test_group_norm_gate_backward_kernel(op, B, T, H):
     check_close("goffset", go.cpu().double().numpy().reshape(H, N), ot.grad.numpy(), torch.float32, is_grad=True)
 
 
+# the kernel's waves take 8 heads of up to 4 tokens: one head and one token, a second wave of heads with one and with
+# four of its eight, token counts that end inside a wave's four
+@pytest.mark.parametrize("B,T,H", [(1, 1, 1), (1, 5, 9), (3, 683, 20)])
+def test_group_norm_gate_backward_kernel_edges(op, B, T, H):
+    test_group_norm_gate_backward_kernel(op, B, T, H)
+
+
 # (the last shape: one layer of the training benchmark, B = 8, T = 1024, 32 heads)
 @pytest.mark.parametrize("B,T,H", [(2, 64, 2), (3, 150, 2), (1, 1000, 3), (8, 256, 8), (75, 64, 4), (8, 1024, 32)])
 def test_fused_group_norm_gate_training(op, oracle, B, T, H):
