@@ -1,16 +1,19 @@
-"""Compiles the HIP sources in csrc/ into lib/libwkv6_gfx950.so (gfx950 only).
+"""Compiles the HIP sources in csrc/ into lib/libwkv6_gfx950.so (gfx950 only) and torch's side of the operator,
+csrc/torch_binding.cpp, into lib/_wkv6_torch.so.
 
 Usage: python star-rwkv6_amd/build.py            (hipcc cross-compiles; no GPU needed)
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libwkv6_gfx950.so")
+TORCH_LIB = os.path.join(LIBDIR, "_wkv6_torch.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -50,7 +53,30 @@ def build(verbose=False, extra_flags=()):
     p = subprocess.run(cmd, capture_output=True, text=True)
     if p.returncode != 0:
         raise RuntimeError("link failed:\n" + p.stdout + p.stderr)
+    build_torch_binding(verbose)
     return LIB
+
+
+def build_torch_binding(verbose=False):
+    """Host code only, for the torch that this interpreter has."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-Wall",
+           "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           *[x for d in includes for x in ("-isystem", d)], "-I" + INCLUDE, os.path.join(CSRC, "torch_binding.cpp"), "-o", TORCH_LIB,
+           "-L" + LIBDIR, "-lwkv6_gfx950", "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10",
+           "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    p = subprocess.run(cmd, capture_output=True, text=True)
+    if p.returncode != 0:
+        raise RuntimeError("building the torch binding failed:\n" + p.stdout + p.stderr)
+    if verbose and (p.stdout + p.stderr).strip():
+        print(p.stdout + p.stderr)
+    return TORCH_LIB
 
 
 if __name__ == "__main__":

@@ -1,13 +1,16 @@
-"""ctypes binding of libwkv6_gfx950.so (the C ABI declared in include/wkv6.h).
+"""ctypes binding of libwkv6_gfx950.so (the C ABI declared in include/wkv6.h), and the torch flavour's native module.
 
-The library is built in-tree by star-rwkv6_amd/build.py.  There is no fallback: if it is missing
+Both are built in-tree by star-rwkv6_amd/build.py.  There is no fallback: if it is missing
 or a call fails, an exception is raised.
 """
 import ctypes
+import importlib.util
 import os
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG, "lib", "libwkv6_gfx950.so")
+
+TORCH_PATH = os.path.join(_PKG, "lib", "_wkv6_torch.so")
 
 BF16, F16, F32 = 0, 1, 2
 ALGO_AUTO, ALGO_SCAN, ALGO_CHUNK = 0, 1, 2
@@ -61,6 +64,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_torch = None
 
 
 class WKV6Error(RuntimeError):
@@ -82,6 +86,19 @@ def load():
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+def load_torch():
+    """Returns the torch flavour's native module (csrc/torch_binding.cpp); raises WKV6Error when it has not been built."""
+    global _torch
+    if _torch is None:
+        if not os.path.exists(TORCH_PATH):
+            raise WKV6Error("%s not found: build it with `python star-rwkv6_amd/build.py`" % TORCH_PATH)
+        spec = importlib.util.spec_from_file_location("_wkv6_torch", TORCH_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _torch = module
+    return _torch
 
 
 def check(status):

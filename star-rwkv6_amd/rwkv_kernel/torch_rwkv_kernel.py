@@ -1,8 +1,9 @@
-"""torch flavour of the WKV6 operator: autograd.Function over libwkv6_gfx950.so.
+"""torch flavour of the WKV6 operator: autograd nodes over libwkv6_gfx950.so.
 
 Mirrors rwkv_kernel/torch_rwkv_kernel.py of the reference (constructor, call signature, argument
-checks, 2-tuple return, dtype rules) but binds the library through its C ABI with ctypes instead
-of JIT-building a torch C++ extension, and launches on torch's CURRENT stream.
+checks, 2-tuple return, dtype rules) but launches on torch's CURRENT stream.  Calls in their plain form
+(contiguous tensors of one shape, one initial state per row or none) go straight to csrc/torch_binding.cpp, built
+ahead of time; what that declines is checked, or brought into that form, here.
 
 Where the reference's torch flavour is broken as committed, the behaviour of its working
 flavours is implemented: the default state_map for a single shared state has length batch
@@ -45,238 +46,20 @@ def _staggered(count, shape, dtype, device, first=1):
     return [block[first * _STAGGER + i * step: first * _STAGGER + i * step + n * es].view(dtype).view(shape) for i in range(count)]
 
 
-def _carve(device, specs):
-    """Tensors of different shapes and dtypes out of ONE allocation: specs = [(shape, dtype, slot), ...]; each tensor
-    starts `slot` * 256 bytes past a 4 KiB boundary of the block (see _staggered for why)."""
-    offs, total = [], 0
-    for shape, dtype, slot in specs:
-        n = 1
-        for d in shape:
-            n *= d
-        nb = n * _ELEMENT_SIZE[dtype]
-        offs.append((total + slot * _STAGGER, nb))
-        total += (slot * _STAGGER + nb + 4095) // 4096 * 4096
-    block = torch.empty(total, dtype=torch.uint8, device=device)
-    return [block[o:o + nb].view(dtype).view(shape) for (o, nb), (shape, dtype, _) in zip(offs, specs)]
-
-
-_ELEMENT_SIZE = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4, torch.uint8: 1}
-_saved_bytes_cache = {}
-
-
-def _saved_bytes(lib, code, algo, B, T, C, H):
-    key = (code, algo, B, T, C, H)
-    n = _saved_bytes_cache.get(key)
-    if n is None:
-        n = _saved_bytes_cache[key] = int(lib.wkv6_saved_bytes(code, algo, B, T, C, H))
-    return n
-
-
-class _on_device:
-    """torch.cuda.device(dev) only where dev is not already the current device (the context manager costs as much
-    host time as a kernel launch)."""
-
-    def __init__(self, dev):
-        self.ctx = None if dev.index is None or dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
-
-    def __enter__(self):
-        if self.ctx is not None:
-            self.ctx.__enter__()
-
-    def __exit__(self, *exc):
-        if self.ctx is not None:
-            self.ctx.__exit__(*exc)
-
-
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-class _WKV6(torch.autograd.Function):
-    """Stateless operator with gradients (rwkv_kernel/torch_rwkv_kernel.py:14-75).
-
-    When a gradient will be needed and the library has something worth keeping for it (the chunked
-    kernels' per-chunk states), the forward runs as wkv6_forward_save and the backward as
-    wkv6_backward_saved; otherwise the plain pair the reference's binding corresponds to."""
+class _WKV6:
+    """Stateless operator with gradients (rwkv_kernel/torch_rwkv_kernel.py:14-75)."""
 
     @staticmethod
-    def forward(ctx, B, T, C, H, r, k, v, w, u, algo):
-        lib = _native.load()
-        with torch.no_grad():
-            assert r.dtype == k.dtype == v.dtype == w.dtype == u.dtype
-            assert r.dtype in _DTYPE_CODE
-            for x in (r, k, v, w, u):
-                assert x.is_contiguous()
-            ctx.dims = (B, T, C, H)
-            ctx.algo = algo
-            code = _DTYPE_CODE[r.dtype]
-            need_grad = any(ctx.needs_input_grad[4:9])
-            nsave = _saved_bytes(lib, code, algo, B, T, C, H) if need_grad else 0
-            saved = None
-            if nsave:
-                y, saved = _carve(r.device, [((B, T, C), _out_dtype(r.dtype), 5), ((nsave,), torch.uint8, 6)])
-            else:
-                (y,) = _staggered(1, (B, T, C), _out_dtype(r.dtype), r.device, first=5)
-            with _on_device(r.device):
-                if nsave:
-                    _native.check(lib.wkv6_forward_save(_stream(), code, algo, B, T, C, H,
-                                                        _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(y),
-                                                        _ptr(saved), nsave))
-                else:
-                    # optional workspace: a long sequence of few (batch, head) pairs runs as time segments
-                    n = lib.wkv6_forward_workspace_bytes(code, algo, B, T, C, H)
-                    ws = torch.empty(int(n), device=r.device, dtype=torch.uint8) if n else None
-                    _native.check(lib.wkv6_forward_ex(_stream(), code, algo, B, T, C, H,
-                                                      _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(y), _ptr(ws), n))
-            ctx.saved_states = saved
-            ctx.save_for_backward(r, k, v, w, u)
-            return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        lib = _native.load()
-        assert gy.is_cuda
-        with torch.no_grad():
-            B, T, C, H = ctx.dims
-            r, k, v, w, u = ctx.saved_tensors
-            odt = _out_dtype(r.dtype)
-            assert gy.dtype in (torch.bfloat16, torch.float32) and gy.dtype == odt
-            gy = gy.contiguous()
-            big = ((B, T, C), odt)
-            gr, gk, gv, gw, gu, gu_sum = _carve(gy.device, [big + (7,), big + (8,), big + (9,), big + (10,),
-                                                            ((B, C), odt, 0), ((C,), odt, 0)])
-            code = _DTYPE_CODE[r.dtype]
-            args = (_ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(gy), _ptr(gr), _ptr(gk), _ptr(gv), _ptr(gw), _ptr(gu))
-            with _on_device(gy.device):
-                saved = ctx.saved_states
-                if saved is not None:
-                    # the batch sum of gu (rwkv_kernel/torch_rwkv_kernel.py:73) comes out of the same launch
-                    ctx.saved_states = None
-                    _native.check(lib.wkv6_backward_saved_sum(_stream(), code, ctx.algo, B, T, C, H, *args, _ptr(gu_sum),
-                                                              _ptr(saved), saved.numel()))
-                    return (None, None, None, None, gr, gk, gv, gw, gu_sum.reshape(u.shape), None)
-                else:
-                    ws_bytes = lib.wkv6_backward_workspace_bytes_ex(code, ctx.algo, B, T, C, H)
-                    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=gy.device) if ws_bytes else None
-                    _native.check(lib.wkv6_backward_ex(_stream(), code, ctx.algo, B, T, C, H, *args, _ptr(ws), ws_bytes))
-            # per-batch partials -> shape of u, rwkv_kernel/torch_rwkv_kernel.py:73
-            gu = torch.sum(gu, 0).reshape(u.shape)
-            return (None, None, None, None, gr, gk, gv, gw, gu, None)
-
-
-class _WKV6GnGate(torch.autograd.Function):
-    """out = (group_norm_head(wkv6(r, k, v, w, u)) * gn_scale + gn_offset) * gate with gradients, bf16,
-    zero initial state: the operator and what the layer does with its output next
-    (rwkv6_model.py:94-99,158-160) in one forward kernel (wkv6_forward_gn_gate_save: y never makes the
-    trip to the norm's own kernels and back), the norm's and the gate's backward in one elementwise
-    kernel (wkv6_gn_gate_backward), then the operator's backward from the saved chunk states."""
-
-    @staticmethod
-    def forward(ctx, B, T, C, H, r, k, v, w, u, gate, gn_scale, gn_offset, eps):
-        lib = _native.load()
-        with torch.no_grad():
-            code = _DTYPE_CODE[r.dtype]
-            sc = gn_scale.detach().to(dtype=torch.float32).contiguous()
-            of = gn_offset.detach().to(dtype=torch.float32).contiguous()
-            out, y = _staggered(2, (B, T, C), r.dtype, r.device, first=5)
-            stats = torch.empty((B, T, H, 2), device=r.device, dtype=torch.float32)
-            with torch.cuda.device(r.device):
-                nsave = lib.wkv6_saved_bytes(code, _native.ALGO_CHUNK, B, T, C, H)
-                (saved,) = _staggered(1, (nsave,), torch.uint8, r.device, first=7)
-                _native.check(lib.wkv6_forward_gn_gate_save(
-                    _stream(), code, B, T, C, H, _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(gate), _ptr(sc), _ptr(of),
-                    float(eps), _ptr(out), _ptr(y), _ptr(stats), _ptr(saved), nsave))
-            ctx.dims = (B, T, C, H)
-            ctx.saved_states = saved
-            ctx.save_for_backward(r, k, v, w, u, gate, sc, of, y, stats)
-            ctx.param_shapes = (gn_scale.shape, gn_offset.shape, gn_scale.dtype, gn_offset.dtype)
-            return out
-
-    @staticmethod
-    def backward(ctx, gout):
-        lib = _native.load()
-        with torch.no_grad():
-            B, T, C, H = ctx.dims
-            r, k, v, w, u, gate, sc, of, y, stats = ctx.saved_tensors
-            saved, ctx.saved_states = ctx.saved_states, None
-            assert gout.dtype == r.dtype
-            gout = gout.contiguous()
-            code = _DTYPE_CODE[r.dtype]
-            gy, ggate = _staggered(2, (B, T, C), r.dtype, r.device, first=5)
-            gr, gk, gv, gw = _staggered(4, (B, T, C), r.dtype, r.device, first=7)
-            gsc = torch.empty(C, device=r.device, dtype=torch.float32)
-            gof = torch.empty(C, device=r.device, dtype=torch.float32)
-            gu = torch.empty((B, C), device=r.device, dtype=r.dtype)
-            gu_sum = torch.empty(C, device=r.device, dtype=r.dtype)
-            with torch.cuda.device(r.device):
-                _native.check(lib.wkv6_gn_gate_backward(_stream(), code, B, T, C, H, _ptr(gout), _ptr(y), _ptr(stats), _ptr(gate),
-                                                        _ptr(sc), _ptr(of), _ptr(gy), _ptr(ggate), _ptr(gsc), _ptr(gof)))
-                if saved is not None:
-                    _native.check(lib.wkv6_backward_saved_sum(_stream(), code, _native.ALGO_CHUNK, B, T, C, H,
-                                                              _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(gy),
-                                                              _ptr(gr), _ptr(gk), _ptr(gv), _ptr(gw), _ptr(gu), _ptr(gu_sum),
-                                                              _ptr(saved), saved.numel()))
-                else:
-                    # a second backward over the same graph (retain_graph): the saved block went with the
-                    # first one (its counters are used up); the plain backward rebuilds the states itself
-                    ws_bytes = lib.wkv6_backward_workspace_bytes_ex(code, _native.ALGO_CHUNK, B, T, C, H)
-                    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=r.device) if ws_bytes else None
-                    _native.check(lib.wkv6_backward_ex(_stream(), code, _native.ALGO_CHUNK, B, T, C, H,
-                                                       _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(gy),
-                                                       _ptr(gr), _ptr(gk), _ptr(gv), _ptr(gw), _ptr(gu), _ptr(ws), ws_bytes))
-                    gu_sum = torch.sum(gu, 0)
-            s_shape, o_shape, s_dt, o_dt = ctx.param_shapes
-            return (None, None, None, None, gr, gk, gv, gw, gu_sum.reshape(u.shape), ggate,
-                    gsc.reshape(s_shape).to(s_dt), gof.reshape(o_shape).to(o_dt), None)
-
-
-class _ShiftMix(torch.autograd.Function):
-    """The layer's input side (rwkv6_model.py:134-146) with gradients, bf16: x -> (xr, xk, xv, xw, xg), all of it
-    in the library's kernels (wkv6_shift_mix_forward / wkv6_shift_mix_backward)."""
-
-    @staticmethod
-    def forward(ctx, x, mix_x, a, w2t, bias):
-        lib = _native.load()
-        with torch.no_grad():
-            B, T, C = x.shape
-            R = w2t.shape[2]
-            code = _DTYPE_CODE[x.dtype]
-            mx = mix_x.to(torch.float32).contiguous()
-            b32 = bias.to(torch.float32).contiguous()
-            wdt = a.dtype if a.dtype == w2t.dtype and a.dtype in (torch.bfloat16, torch.float32) else torch.float32
-            aw, ww = a.to(wdt).contiguous(), w2t.to(wdt).contiguous()
-            nw = lib.wkv6_shift_mix_weights_bytes(C, R)
-            outs = _staggered(5, (B, T, C), x.dtype, x.device, first=1)
-            # (not out of the outputs' block: a caller may change an output in place)
-            h, weights = _carve(x.device, [((B, T, 5 * R), x.dtype, 6), ((nw,), torch.uint8, 0)])
-            with _on_device(x.device):
-                _native.check(lib.wkv6_shift_mix_forward(_stream(), code, _DTYPE_CODE[wdt], B, T, C, R, _ptr(x), _ptr(mx), _ptr(aw),
-                                                         _ptr(ww), _ptr(b32), _ptr(weights), nw, _ptr(h), *[_ptr(o) for o in outs]))
-            ctx.save_for_backward(x, h, weights, mx, b32)
-            ctx.weight_dtype = wdt
-            ctx.param_dtypes = (mix_x.dtype, a.dtype, w2t.dtype, bias.dtype)
-            return tuple(outs)
-
-    @staticmethod
-    def backward(ctx, *gouts):
-        lib = _native.load()
-        with torch.no_grad():
-            x, h, weights, mx, b32 = ctx.saved_tensors
-            B, T, C = x.shape
-            R = h.shape[2] // 5
-            code, wdt = _DTYPE_CODE[x.dtype], ctx.weight_dtype
-            gouts = [torch.zeros_like(x) if g is None else g.to(x.dtype).contiguous() for g in gouts]
-            f32 = torch.float32
-            gx, ga, gw2t, gbias, gmx = _carve(x.device, [((B, T, C), x.dtype, 6), ((5 * R, C), wdt, 0), ((5, C, R), wdt, 0),
-                                                         ((5, C), f32, 0), ((C,), f32, 0)])
-            n = lib.wkv6_shift_mix_backward_workspace_bytes(code, B, T, C, R)
-            ws = torch.empty(n, device=x.device, dtype=torch.uint8)
-            with _on_device(x.device):
-                _native.check(lib.wkv6_shift_mix_backward(
-                    _stream(), code, _DTYPE_CODE[wdt], B, T, C, R, _ptr(x), _ptr(mx), _ptr(b32), _ptr(weights), _ptr(h),
-                    *[_ptr(g) for g in gouts], _ptr(gx), _ptr(gmx), _ptr(ga), _ptr(gw2t), _ptr(gbias), _ptr(ws), n))
-            dm, da, dw, db = ctx.param_dtypes
-            return gx, gmx.to(dm), ga.to(da), gw2t.to(dw), gbias.to(db)
+    def apply(B, T, C, H, r, k, v, w, u, algo):
+        assert r.dtype == k.dtype == v.dtype == w.dtype == u.dtype
+        assert r.dtype in _DTYPE_CODE
+        for x in (r, k, v, w, u):
+            assert x.is_contiguous()
+        return _native.load_torch().wkv6(r, k, v, w, u, H, algo)
 
 
 class _ShiftMixX(torch.autograd.Function):
@@ -313,25 +96,11 @@ class _ShiftMixX(torch.autograd.Function):
 
 def _forward_with_state(B, T, C, H, state_map, r, k, v, w, u, init_state, algo=_native.ALGO_AUTO, state_dtype=None):
     """Stateful forward, no gradient (rwkv_kernel/torch_rwkv_kernel.py:76-95)."""
-    lib = _native.load()
-    with torch.no_grad():
-        # state_map None with an init_state means the identity map (row b starts from init_state[b])
-        assert init_state is not None or state_map is None, "state_map needs init_state"
-        assert state_map is None or state_map.dtype == torch.int64
-        odt = _out_dtype(r.dtype)
-        sdt = init_state.dtype if init_state is not None else (state_dtype or odt)
-        N = C // H
-        (y,) = _staggered(1, (B, T, C), odt, r.device, first=5)
-        ys = torch.empty((B, H, N, N), device=r.device, dtype=sdt)
-        with torch.cuda.device(r.device):
-            # optional workspace: lets a long sequence of few (batch, head) pairs run as time segments
-            n = lib.wkv6_forward_workspace_bytes(_DTYPE_CODE[r.dtype], algo, B, T, C, H)
-            ws = torch.empty(int(n), device=r.device, dtype=torch.uint8) if n else None
-            _native.check(lib.wkv6_forward_with_state_ex(
-                _stream(), _DTYPE_CODE[r.dtype], _DTYPE_CODE[sdt], algo, B, T, C, H,
-                int(init_state is not None), _ptr(state_map),
-                _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(init_state), _ptr(y), _ptr(ys), _ptr(ws), n))
-    return y, ys
+    # state_map None with an init_state means the identity map (row b starts from init_state[b])
+    assert init_state is not None or state_map is None, "state_map needs init_state"
+    assert state_map is None or state_map.dtype == torch.int64
+    sdt = init_state.dtype if init_state is not None else (state_dtype or _out_dtype(r.dtype))
+    return _native.load_torch().forward_with_state(H, state_map, r, k, v, w, u, init_state, algo, _DTYPE_CODE[sdt])
 
 
 class _WKV6State(torch.autograd.Function):
@@ -384,6 +153,7 @@ def _backward_with_state(B, T, C, H, r, k, v, w, u, s0, gy, gsT, algo, want_gs0)
 class RWKVKernelOperator:
     def __init__(self, head_size, max_sequence_length):
         lib = _native.load()
+        self._torch = _native.load_torch()
         assert isinstance(head_size, int) and isinstance(max_sequence_length, int)
         assert head_size > 0 and max_sequence_length > 0
         assert head_size % 4 == 0, "head_size must be a multiple of 4"
@@ -456,6 +226,10 @@ class RWKVKernelOperator:
         return init_state.contiguous(), state_map
 
     def __call__(self, r, k, v, w, u, return_state=False, init_state=None, state_map=None):
+        if state_map is None:
+            res = self._torch.try_call(self.head_size, self.algo, r, k, v, w, u, return_state, init_state)
+            if res is not None:
+                return res
         B, T, C, H, N, u, init_state, state_map = self._check(r, k, v, w, u, init_state, state_map)
         if return_state:
             init_state, state_map = self._resolve_state(B, r, init_state, state_map)
@@ -499,7 +273,7 @@ class RWKVKernelOperator:
         R = w2t.shape[2]
         assert a.shape == (5 * R, C) and w2t.shape == (5, C, R) and bias.shape == (5, C)
         assert self.shift_mix_supported(x, R), "shift_mix takes bf16 tensors on the GPU with rank 32 or 64"
-        return _ShiftMix.apply(x, mix_x.reshape(C), a, w2t, bias)
+        return self._torch.shift_mix(x, mix_x.reshape(C), a, w2t, bias)
 
     def forward_gn_gate(self, r, k, v, w, u, gate, gn_scale, gn_offset, epsilon=64e-5,
                         return_state=False, init_state=None, state_map=None):
@@ -510,6 +284,10 @@ class RWKVKernelOperator:
         never written and the stateful arguments work as in ``__call__``.  With gradients enabled and
         required (training; no state arguments) the call is differentiable in r, k, v, w, u, gate,
         gn_scale and gn_offset.  Not part of the reference's operator."""
+        if state_map is None:
+            res = self._torch.try_gn_gate(self.head_size, r, k, v, w, u, gate, gn_scale, gn_offset, epsilon, return_state, init_state)
+            if res is not None:
+                return res
         B, T, C, H, N, u, init_state, state_map = self._check(r, k, v, w, u, init_state, state_map)
         assert r.dtype == torch.bfloat16, "the fused output stage takes bf16 tensors"
         assert gate.shape == r.shape and gate.dtype == r.dtype and gate.device == r.device
@@ -521,7 +299,7 @@ class RWKVKernelOperator:
                 assert x.is_contiguous()
             lib = _native.load()
             if lib.wkv6_forward_gn_gate_save_supported(_DTYPE_CODE[r.dtype], B, T, C, H):
-                return _WKV6GnGate.apply(B, T, C, H, r, k, v, w, u, gate, gn_scale.to(r.device), gn_offset.to(r.device), epsilon), None
+                return self._torch.wkv6_gn_gate(r, k, v, w, u, gate, gn_scale.to(r.device), gn_offset.to(r.device), H, epsilon), None
             # (a shape the fused training kernels do not take, e.g. a sequence too long for the chunk form: unfused calls)
             y, _ = self(r, k, v, w, u)
             z = torch.nn.functional.layer_norm(y.float().view(B, T, H, N), (N,), eps=epsilon).view(B, T, C)
@@ -530,20 +308,4 @@ class RWKVKernelOperator:
         init_state, state_map = self._resolve_state(B, r, init_state, state_map)
         for x in (r, k, v, w, u, gate):
             assert x.is_contiguous()
-        lib = _native.load()
-        with torch.no_grad():
-            sc = gn_scale.detach().to(device=r.device, dtype=torch.float32).contiguous()
-            of = gn_offset.detach().to(device=r.device, dtype=torch.float32).contiguous()
-            sdt = init_state.dtype if init_state is not None else torch.float32
-            out = torch.empty_like(r)
-            ys = torch.empty((B, H, N, N), device=r.device, dtype=sdt) if return_state else None
-            with torch.cuda.device(r.device):
-                # optional workspace: a long sequence of few (batch, head) pairs runs as time segments
-                n = lib.wkv6_forward_workspace_bytes(_DTYPE_CODE[r.dtype], _native.ALGO_CHUNK, B, T, C, H)
-                ws = torch.empty(int(n), device=r.device, dtype=torch.uint8) if n else None
-                _native.check(lib.wkv6_forward_gn_gate_ex(
-                    _stream(), _DTYPE_CODE[r.dtype], _DTYPE_CODE[sdt], B, T, C, H,
-                    int(init_state is not None), _ptr(state_map),
-                    _ptr(r), _ptr(k), _ptr(v), _ptr(w), _ptr(u), _ptr(init_state), _ptr(gate), _ptr(sc), _ptr(of),
-                    float(epsilon), _ptr(out), _ptr(ys), _ptr(ws), n))
-        return out, ys
+        return self._torch.forward_gn_gate(H, state_map, r, k, v, w, u, init_state, gate, gn_scale, gn_offset, epsilon, bool(return_state))
