@@ -90,6 +90,21 @@ __device__ __forceinline__ float sum_rows4(float x) {
     s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
+// running sums over the 16 lanes of a row: lane n gets x_n + .. + x_15
+__device__ __forceinline__ float row_sum_down(float x) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x101, 0xF, 0xF, true));   // row_shl:1
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x102, 0xF, 0xF, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x104, 0xF, 0xF, true));
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x108, 0xF, 0xF, true));
+    return x;
+}
+// x of the row's next lane (0 behind lane 15) ; of its lane 0
+__device__ __forceinline__ float next_in_row(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x101, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float first_of_row(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150, 0xF, 0xF, false));   // row_newbcast:0
+}
 // sum over the 16 lanes of a row, in every lane of it
 __device__ __forceinline__ float row_sum16(float x) {
     x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]

@@ -21,7 +21,7 @@
 //                   update of G^T, the tiles of B; S_0^T comes straight from the saved states
 // Both G and G^T are kept so that neither K' G nor v G^T needs a sum across waves.  Two workgroup barriers per chunk:
 //   phase 1  tiles of A and B -> LDS ; K' G ; gy S_0^T ; v G^T
-//   phase 2  the three products with A and B ; gradients out (16 lanes x 4 bytes per row piece) ; G, G^T updates
+//   phase 2  the three products with A and B ; gradients out (lane = token, 16 bytes each) ; G, G^T updates
 #include "wkv6_chunk32.h"
 #include "wkv6_kernels.h"
 #include "wkv6_scan_body.h"
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         const int q = wave, n = lane & 15, g = lane >> 4, col = 16 * q + n;
         Tout *gv = reinterpret_cast<Tout *>(a.gv);
         const f32x4 zero = (f32x4){0.f, 0.f, 0.f, 0.f};
-        const int lane_off = 4 * g * (int)C + col;
+        const int lane_off = n * (int)C + 16 * q + 4 * g;   // outputs: token n of a half chunk, four channels
         f32x4 G[4];   // G[ib][e] = G[16ib+4g+e][col]
 #pragma unroll
         for (int i = 0; i < 4; ++i) G[i] = zero;
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                 for (int ib = 0; ib < 4; ++ib) {
                     const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.K[buf][16 * sb + n][16 * ib + 4 * g]) *
                                      *reinterpret_cast<const f32x4 *>(&L.F3[buf][16 * sb + n][16 * ib + 4 * g]);
-                    gvt[sb] = mfma16(fk, G[ib], gvt[sb]);
+                    gvt[sb] = mfma16(G[ib], fk, gvt[sb]);   // transposed: lane (n, g) gets token n, channels 4g ..
                 }
             __syncthreads();
             // ---- phase 2: gv += A^T gy, out ; G <- e^{c_32} o G + R'^T gy ----
@@ -231,16 +231,14 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     f32x4 fat;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) fat[e] = L.A[16 * tb + 4 * g + e][16 * sb + n];
-                    gvt[sb] = mfma16(fat, gyb[tb], gvt[sb]);
+                    gvt[sb] = mfma16(gyb[tb], fat, gvt[sb]);
                 }
             {
                 Tout *const out = gv + base + (int64_t)c * kC32 * C;   // (uniform; the lane's part of the address is lane_off)
-                const int left = T - c * kC32 - 4 * g;                 // rows of the lane's four-row groups that exist
+                const int left = T - c * kC32 - n;                     // (token 16 x + n exists: 16 x < left)
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (full || 16 * x + e < left) store1(out + (16 * x + e) * C + lane_off, gvt[x][e]);
+                    if (full || 16 * x < left) store4(out + 16 * x * C + lane_off, gvt[x][0], gvt[x][1], gvt[x][2], gvt[x][3]);
             }
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) {
@@ -267,11 +265,12 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         const int q = wave - 4, n = lane & 15, g = lane >> 4, col = 16 * q + n;
         Tout *gr = reinterpret_cast<Tout *>(a.gr), *gk = reinterpret_cast<Tout *>(a.gk), *gw = reinterpret_cast<Tout *>(a.gw);
         const f32x4 zero = (f32x4){0.f, 0.f, 0.f, 0.f};
-        const int lane_off = 4 * g * (int)C + col;
+        const int ch = 16 * q + 4 * g;                // outputs: token n of a half chunk, channels ch .. ch+3
+        const int lane_off = n * (int)C + ch;
         f32x4 Gt[4], St[4];   // Gt[jb][e] = G[col][16jb+4g+e] ; St likewise of S_0
 #pragma unroll
         for (int i = 0; i < 4; ++i) Gt[i] = zero;
-        float E = 0.f, gu_acc = 0.f;
+        f32x4 E = zero, gu_acc = zero;   // of channels ch .. ch+3 (E the same in every lane of a row)
         if (a.gsT) {   // G_T^T, and the anchor of the decay gradient's sums: E_T = sum_j S_T o G_T over the row
             const float *pg = a.gsT + (int64_t)pair * (kN * kN) + col * kN + 4 * g;
             const float *ps = a.sT + (int64_t)pair * (kN * kN) + col * kN + 4 * g;
@@ -282,9 +281,12 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                 const f32x4 sv = *reinterpret_cast<const f32x4 *>(ps + 16 * jb);
                 part += (sv[0] * Gt[jb][0] + sv[1] * Gt[jb][1]) + (sv[2] * Gt[jb][2] + sv[3] * Gt[jb][3]);
             }
-            E = sum_rows4(part);
+            part = sum_rows4(part);   // row `col`; lane n of every row of lanes
+#pragma unroll
+            for (int e = 0; e < 4; ++e) E[e] = __shfl(part, 4 * g + e);
         }
-        const float u_lane = load1(u + h * kN + col);
+        float fu[4];
+        load4(u + h * kN + ch, fu);
         // S_0^T from the forward's fragment order: S[i][j] sits in tile (j / 16, i / 16) at lane (j % 16) + 16 ((i % 16) / 4), element i % 4
         auto load_state = [&](int c) {
             const float *p0 = ck + (int64_t)c * (kN * kN) + (q * 64 + 4 * g + 16 * (n >> 2)) * 4 + (n & 3);
@@ -324,34 +326,32 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                 for (int jb = 0; jb < 4; ++jb) {
                     const f32x4 fg = *reinterpret_cast<const f32x4 *>(&L.GY[buf][16 * x + n][16 * jb + 4 * g]);
                     const f32x4 fv = *reinterpret_cast<const f32x4 *>(&L.V[buf][16 * x + n][16 * jb + 4 * g]);
-                    Z[x] = mfma16(fg, St[jb], Z[x]);
-                    W[x] = mfma16(fv, Gt[jb], W[x]);
+                    Z[x] = mfma16(St[jb], fg, Z[x]);   // transposed: lane (n, g) gets token n, channels ch ..
+                    W[x] = mfma16(Gt[jb], fv, W[x]);
                 }
-            const float e_all = L.e_all[buf][col], e_mid = L.e_mid[buf][col], e_rest = L.e_rest[buf][col];
-            const float inv0 = L.inv0[buf][col], inv1 = L.inv1[buf][col];
+            const float e_all = L.e_all[buf][col], inv0 = L.inv0[buf][col], inv1 = L.inv1[buf][col];
             // the products with B come scaled from the middle of the chunk: bring these to that scale, all back at the end
+            const f32x4 e_mid = *reinterpret_cast<const f32x4 *>(&L.e_mid[buf][ch]), e_rest = *reinterpret_cast<const f32x4 *>(&L.e_rest[buf][ch]);
 #pragma unroll
             for (int x = 0; x < 2; ++x) { Z[x] *= e_mid; W[x] *= e_rest; }
             if (c > 0) load_state(c - 1);
             __syncthreads();
             // ---- phase 2 ----
-            f32x4 rc[2], kc[2], rp[2], kp[2];   // element e: token 16x + 4g + e, channel col
+            f32x4 rp[2], kp[2];   // R', K'; element e: token 16x + 4g + e, channel col
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int t = 16 * x + 4 * g + e;
-                    rc[x][e] = L.R[buf][t][col];
-                    kc[x][e] = L.K[buf][t][col];
-                    rp[x][e] = rc[x][e] * L.F1[buf][t][col];
-                    kp[x][e] = kc[x][e] * L.F3[buf][t][col];
+                    rp[x][e] = L.R[buf][t][col] * L.F1[buf][t][col];
+                    kp[x][e] = L.K[buf][t][col] * L.F3[buf][t][col];
                 }
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
                 for (int sb = 0; sb <= tb; ++sb) {
                     const f32x4 fb = *reinterpret_cast<const f32x4 *>(&L.Bm[16 * tb + n][16 * sb + 4 * g]);
-                    Z[tb] = mfma16(fb, kp[sb] * inv1, Z[tb]);
+                    Z[tb] = mfma16(kp[sb] * inv1, fb, Z[tb]);
                 }
 #pragma unroll
             for (int sb = 0; sb < 2; ++sb)
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     f32x4 fbt;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) fbt[e] = L.Bm[16 * tb + 4 * g + e][16 * sb + n];
-                    W[sb] = mfma16(fbt, rp[tb] * inv0, W[sb]);
+                    W[sb] = mfma16(rp[tb] * inv0, fbt, W[sb]);
                 }
             // G^T <- e^{c_32} o G^T + gy^T R' (before the outputs: they need no matrix unit)
 #pragma unroll
@@ -374,62 +374,56 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     Gt[jb] = mfma16(fga, rp[tb], Gt[jb]);
                 }
             }
-            // gradients out
-            float zt[2][4], kgk[2][4];
+            // gradients out, lane = token 16x + n, four channels: whole 16-byte pieces of the operand tiles and of the
+            // gradients (with lane = channel a wave sent twelve times the store instructions, four bytes a lane)
+            f32x4 zt[2], kgk[2];
+            const f32x4 row0 = *reinterpret_cast<const f32x4 *>(&L.inv0[buf][ch]), row1 = *reinterpret_cast<const f32x4 *>(&L.inv1[buf][ch]);
             const int64_t out0 = base + (int64_t)c * kC32 * C;   // (uniform; the lane's part of the address is lane_off)
-            const int left = T - c * kC32 - 4 * g;               // rows of the lane's four-row groups that exist
+            const int left = T - c * kC32 - n;                   // (token 16 x + n exists: 16 x < left)
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
-                const f32x4 vg = *reinterpret_cast<const f32x4 *>(&L.vgy[16 * x + 4 * g]);
-                Z[x] *= inv0;
-                W[x] *= inv1;
+                const int t = 16 * x + n;
+                const f32x4 rt = *reinterpret_cast<const f32x4 *>(&L.R[buf][t][ch]), kt = *reinterpret_cast<const f32x4 *>(&L.K[buf][t][ch]);
+                const f32x4 f1 = *reinterpret_cast<const f32x4 *>(&L.F1[buf][t][ch]), f3 = *reinterpret_cast<const f32x4 *>(&L.F3[buf][t][ch]);
+                const float vg = L.vgy[t];
+                Z[x] *= row0;
+                W[x] *= row1;
+                f32x4 o_r, o_k;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int tl = 16 * x + 4 * g + e;
-                    const float f1 = L.F1[buf][tl][col], f3 = L.F3[buf][tl][col];
-                    const float o_r = fmaf(f1, Z[x][e], u_lane * kc[x][e] * vg[e]);
-                    const float o_k = fmaf(f3, W[x][e], u_lane * rc[x][e] * vg[e]);
-                    kgk[x][e] = kp[x][e] * W[x][e];
-                    zt[x][e] = fmaf(rp[x][e], Z[x][e], -kgk[x][e]);
-                    gu_acc = fmaf(rc[x][e] * kc[x][e], vg[e], gu_acc);
-                    if (full || 16 * x + e < left) {
-                        store1(gr + out0 + (16 * x + e) * C + lane_off, o_r);
-                        store1(gk + out0 + (16 * x + e) * C + lane_off, o_k);
-                    }
+                    o_r[e] = fmaf(f1[e], Z[x][e], fu[e] * kt[e] * vg);
+                    o_k[e] = fmaf(f3[e], W[x][e], fu[e] * rt[e] * vg);
+                    kgk[x][e] = kt[e] * f3[e] * W[x][e];
+                    zt[x][e] = fmaf(rt[e] * f1[e], Z[x][e], -kgk[x][e]);
+                    gu_acc[e] = fmaf(rt[e] * kt[e], vg, gu_acc[e]);
+                }
+                if (full || 16 * x < left) {
+                    store4(gr + out0 + 16 * x * C + lane_off, o_r[0], o_r[1], o_r[2], o_r[3]);
+                    store4(gk + out0 + 16 * x * C + lane_off, o_k[0], o_k[1], o_k[2], o_k[3]);
                 }
             }
-            {   // E_{t+1} = E at the chunk's end + what the later tokens of the chunk add
-                float tot[2], other[2][4], later[2];
+            // E_{t+1} = E at the chunk's end + what the later tokens of the chunk add
 #pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    tot[x] = (zt[x][0] + zt[x][1]) + (zt[x][2] + zt[x][3]);
-                    rows4(tot[x], other[x]);
-                    later[x] = (g < 1 ? other[x][1] : 0.f) + (g < 2 ? other[x][2] : 0.f) + (g < 3 ? other[x][3] : 0.f);
+            for (int x = 1; x >= 0; --x) {
+                const f32x4 d = *reinterpret_cast<const f32x4 *>(&L.D[buf][16 * x + n][ch]);
+                f32x4 o_w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float from_here = row_sum_down(zt[x][e]);
+                    o_w[e] = (E[e] + next_in_row(from_here) - kgk[x][e]) * d[e];
+                    E[e] += first_of_row(from_here);
                 }
-                const float all1 = (other[1][0] + other[1][1]) + (other[1][2] + other[1][3]);
-                const float all0 = (other[0][0] + other[0][1]) + (other[0][2] + other[0][3]);
-                later[0] += all1;
-#pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    float run = E + later[x];
-#pragma unroll
-                    for (int e = 3; e >= 0; --e) {
-                        const int tl = 16 * x + 4 * g + e;
-                        float o_w = (run - kgk[x][e]) * L.D[buf][tl][col];
-                        // (a zero initial state: the first decay reaches no output, its gradient is zero and not
-                        // what rounding leaves of two equal sums)
-                        if (x == 0 && e == 0 && a.s0 == nullptr && c == 0 && g == 0) o_w = 0.f;
-                        if (full || 16 * x + e < left) store1(gw + out0 + (16 * x + e) * C + lane_off, o_w);
-                        run += zt[x][e];
-                    }
-                }
-                E += all0 + all1;
+                // (a zero initial state: the first decay reaches no output, its gradient is zero and not
+                // what rounding leaves of two equal sums)
+                if (x == 0 && a.s0 == nullptr && c == 0 && n == 0) o_w = zero;
+                if (full || 16 * x < left) store4(gw + out0 + 16 * x * C + lane_off, o_w[0], o_w[1], o_w[2], o_w[3]);
             }
             __syncthreads();
         }
-        // gu: the four row groups of the wave hold the tokens 4g .. 4g+3 (mod 16) of every chunk
-        gu_acc = sum_rows4(gu_acc);
-        if (g == 0) store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + col, gu_acc);
+        // gu: the lanes of a row hold the tokens n (mod 16) of every chunk
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gu_acc[e] = row_sum16(gu_acc[e]);
+        if (n < 4) store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + ch + n, n == 0 ? gu_acc[0] : n == 1 ? gu_acc[1] : n == 2 ? gu_acc[2] : gu_acc[3]);
     }
     __syncthreads();
     // a pair whose decay left the reach: once more, one timestep at a time (the pair's slice of the saved
