@@ -17,11 +17,13 @@
 //   loading waves   tiles r, k, e^{c_t}, e^{c_32-c_{t+1}}, v, gy, d of the next chunk -> LDS (loads issued one phase
 //                   ahead of their use: the kernel is bound by arithmetic, not by memory)
 //   value waves     wave q owns value columns 16q.. of G: gv = K' G + A^T gy, the update of G, the tiles of A
-//   key waves       wave q owns key rows 16q.. of G^T and of every per-channel output: Z, W, gr, gk, gw, gu, the
-//                   update of G^T, the tiles of B; S_0^T comes straight from the saved states
-// Both G and G^T are kept so that neither K' G nor v G^T needs a sum across waves.  Two workgroup barriers per chunk:
-//   phase 1  tiles of A and B -> LDS ; K' G ; gy S_0^T ; v G^T
-//   phase 2  the three products with A and B ; gradients out (lane = token, 16 bytes each) ; G, G^T updates
+//   key waves       wave q owns key rows 16q.. of every per-channel output: Z, W, gr, gk, gw, gu, the tiles of B; S_0^T
+//                   comes straight from the saved states, G^T from the value waves through LDS (a copy kept up to date by
+//                   the key waves themselves cost a seventh of all matrix instructions)
+// Two workgroup barriers per chunk, the matrix instructions shared out evenly between the two phases (24 and 25 products
+// over 16 indices per SIMD):
+//   phase 1  tiles of A and B -> LDS ; K' G ; v G^T
+//   phase 2  gy S_0^T ; the three products with A and B ; gradients out (lane = token, 16 bytes each) ; G update -> LDS
 #include "wkv6_chunk32.h"
 #include "wkv6_kernels.h"
 #include "wkv6_scan_body.h"
@@ -34,6 +36,7 @@ struct C32BwdLds {
     float R[2][kC32][kLd], K[2][kC32][kLd], F1[2][kC32][kLd], F3[2][kC32][kLd];   // r, k, e^{c_t}, e^{c_32 - c_{t+1}}
     float V[2][kC32][kLd], GY[2][kC32][kLd], D[2][kC32][kLd];                     // v, gy, log decay
     float A[kC32][kLa], Bm[kC32][kLa];
+    float G[kN][kLd];                                                             // dL/dS at the chunk's end, [value][key]
     float e_all[2][kN], e_mid[2][kN], e_rest[2][kN], inv0[2][kN], inv1[2][kN];    // e^{c_32}, e^{m}, e^{c_32-m}, e^{-m}, e^{m-c_32}
     float ruk[2][4][kC32];
     float vgy[kC32];
@@ -181,6 +184,11 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) G[ib][e] = p[(16 * ib + 4 * g + e) * kN];
         }
+        auto publish = [&]() {
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) *reinterpret_cast<f32x4 *>(&L.G[col][16 * ib + 4 * g]) = G[ib];
+        };
+        publish();
         __syncthreads();
         for (int s = 0; s < nchunk; ++s) {
             const int c = nchunk - 1 - s, buf = s & 1;
@@ -251,6 +259,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     G[ib] = mfma16(fra, gyb[tb], G[ib]);
                 }
             }
+            publish();
             __syncthreads();
         }
         if (a.gs0) {   // what is left after the first chunk is dL/dS_0
@@ -267,19 +276,16 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         const f32x4 zero = (f32x4){0.f, 0.f, 0.f, 0.f};
         const int ch = 16 * q + 4 * g;                // outputs: token n of a half chunk, channels ch .. ch+3
         const int lane_off = n * (int)C + ch;
-        f32x4 Gt[4], St[4];   // Gt[jb][e] = G[col][16jb+4g+e] ; St likewise of S_0
-#pragma unroll
-        for (int i = 0; i < 4; ++i) Gt[i] = zero;
+        f32x4 St[4];   // St[jb][e] = S_0[col][16jb+4g+e]
         f32x4 E = zero, gu_acc = zero;   // of channels ch .. ch+3 (E the same in every lane of a row)
-        if (a.gsT) {   // G_T^T, and the anchor of the decay gradient's sums: E_T = sum_j S_T o G_T over the row
+        if (a.gsT) {   // the anchor of the decay gradient's sums: E_T = sum_j S_T o G_T over the row
             const float *pg = a.gsT + (int64_t)pair * (kN * kN) + col * kN + 4 * g;
             const float *ps = a.sT + (int64_t)pair * (kN * kN) + col * kN + 4 * g;
             float part = 0.f;
 #pragma unroll
             for (int jb = 0; jb < 4; ++jb) {
-                Gt[jb] = *reinterpret_cast<const f32x4 *>(pg + 16 * jb);
-                const f32x4 sv = *reinterpret_cast<const f32x4 *>(ps + 16 * jb);
-                part += (sv[0] * Gt[jb][0] + sv[1] * Gt[jb][1]) + (sv[2] * Gt[jb][2] + sv[3] * Gt[jb][3]);
+                const f32x4 gv = *reinterpret_cast<const f32x4 *>(pg + 16 * jb), sv = *reinterpret_cast<const f32x4 *>(ps + 16 * jb);
+                part += (sv[0] * gv[0] + sv[1] * gv[1]) + (sv[2] * gv[2] + sv[3] * gv[3]);
             }
             part = sum_rows4(part);   // row `col`; lane n of every row of lanes
 #pragma unroll
@@ -300,7 +306,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         for (int s = 0; s < nchunk; ++s) {
             const int c = nchunk - 1 - s, buf = s & 1;
             const bool full = (c + 1) * kC32 <= T;
-            // ---- phase 1: a tile of B (wave 0: (0,0), 1: (1,1), 3: (1,0)), gy S_0^T, v G^T ----
+            // ---- phase 1: a tile of B (wave 0: (0,0), 1: (1,1), 3: (1,0)), v G^T ----
             if (q != 2) {
                 const int tb = q == 0 ? 0 : 1, sb = q == 1 ? 1 : 0;
                 f32x4 bt = zero;
@@ -321,22 +327,33 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
             }
             f32x4 Z[2] = {zero, zero}, W[2] = {zero, zero};
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
+            for (int jb = 0; jb < 4; ++jb) {
+                f32x4 gt;   // G[col][16jb+4g+e]
 #pragma unroll
-                for (int jb = 0; jb < 4; ++jb) {
-                    const f32x4 fg = *reinterpret_cast<const f32x4 *>(&L.GY[buf][16 * x + n][16 * jb + 4 * g]);
+                for (int e = 0; e < 4; ++e) gt[e] = L.G[16 * jb + 4 * g + e][col];
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
                     const f32x4 fv = *reinterpret_cast<const f32x4 *>(&L.V[buf][16 * x + n][16 * jb + 4 * g]);
-                    Z[x] = mfma16(St[jb], fg, Z[x]);   // transposed: lane (n, g) gets token n, channels ch ..
-                    W[x] = mfma16(Gt[jb], fv, W[x]);
+                    W[x] = mfma16(gt, fv, W[x]);   // transposed: lane (n, g) gets token n, channels ch ..
                 }
-            const float e_all = L.e_all[buf][col], inv0 = L.inv0[buf][col], inv1 = L.inv1[buf][col];
+            }
+            const float inv0 = L.inv0[buf][col], inv1 = L.inv1[buf][col];
             // the products with B come scaled from the middle of the chunk: bring these to that scale, all back at the end
             const f32x4 e_mid = *reinterpret_cast<const f32x4 *>(&L.e_mid[buf][ch]), e_rest = *reinterpret_cast<const f32x4 *>(&L.e_rest[buf][ch]);
 #pragma unroll
-            for (int x = 0; x < 2; ++x) { Z[x] *= e_mid; W[x] *= e_rest; }
-            if (c > 0) load_state(c - 1);
+            for (int x = 0; x < 2; ++x) W[x] *= e_rest;
             __syncthreads();
-            // ---- phase 2 ----
+            // ---- phase 2: gy S_0^T, the products with B, the gradients ----
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+#pragma unroll
+                for (int jb = 0; jb < 4; ++jb) {
+                    const f32x4 fg = *reinterpret_cast<const f32x4 *>(&L.GY[buf][16 * x + n][16 * jb + 4 * g]);
+                    Z[x] = mfma16(St[jb], fg, Z[x]);
+                }
+                Z[x] *= e_mid;
+            }
+            if (c > 0) load_state(c - 1);
             f32x4 rp[2], kp[2];   // R', K'; element e: token 16x + 4g + e, channel col
 #pragma unroll
             for (int x = 0; x < 2; ++x)
@@ -362,18 +379,6 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     for (int e = 0; e < 4; ++e) fbt[e] = L.Bm[16 * tb + 4 * g + e][16 * sb + n];
                     W[sb] = mfma16(rp[tb] * inv0, fbt, W[sb]);
                 }
-            // G^T <- e^{c_32} o G^T + gy^T R' (before the outputs: they need no matrix unit)
-#pragma unroll
-            for (int jb = 0; jb < 4; ++jb) {
-                Gt[jb] *= e_all;
-#pragma unroll
-                for (int tb = 0; tb < 2; ++tb) {
-                    f32x4 fga;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) fga[e] = L.GY[buf][16 * tb + 4 * g + e][16 * jb + n];
-                    Gt[jb] = mfma16(fga, rp[tb], Gt[jb]);
-                }
-            }
             // gradients out, lane = token 16x + n, four channels: whole 16-byte pieces of the operand tiles and of the
             // gradients (with lane = channel a wave sent twelve times the store instructions, four bytes a lane)
             f32x4 zt[2], kgk[2];
