@@ -14,8 +14,8 @@
 //
 // One workgroup of twelve waves per (batch, head) pair, three roles of four waves (one wave of each role per SIMD,
 // so that one role's waits are another's issue slots):
-//   loading waves   tiles r, k, e^{c_t}, e^{c_32-c_{t+1}}, v, gy, d of the next chunk -> LDS (loads issued one phase
-//                   ahead of their use: the kernel is bound by arithmetic, not by memory)
+//   loading waves   tiles R', K', v, gy of the next chunk and r, k, e^{c_t}, e^{c_32-c_{t+1}}, d of the chunk in hand
+//                   -> LDS (loads issued a step and a half ahead of their use)
 //   value waves     wave q owns value columns 16q.. of G: gv = K' G + A^T gy, the update of G, the tiles of A
 //   key waves       wave q owns key rows 16q.. of every per-channel output: Z, W, gr, gk, gw, gu, the tiles of B; S_0^T
 //                   comes straight from the saved states, G^T from the value waves through LDS (a copy kept up to date by
@@ -33,8 +33,9 @@
 namespace wkv6 {
 
 struct C32BwdLds {
-    float R[2][kC32][kLd], K[2][kC32][kLd], F1[2][kC32][kLd], F3[2][kC32][kLd];   // r, k, e^{c_t}, e^{c_32 - c_{t+1}}
-    float V[2][kC32][kLd], GY[2][kC32][kLd], D[2][kC32][kLd];                     // v, gy, log decay
+    float Rp[2][kC32][kLd], Kp[2][kC32][kLd], V[2][kC32][kLd], GY[2][kC32][kLd];   // R', K', v, gy of the chunk in hand and the next
+    // what only the key waves' second phase reads: one copy, written in the first phase of the same step
+    float R[kC32][kLd], K[kC32][kLd], F1[kC32][kLd], F3[kC32][kLd], D[kC32][kLd];   // r, k, e^{c_t}, e^{c_32 - c_{t+1}}, log decay
     float A[kC32][kLa], Bm[kC32][kLa];
     float G[kN][kLd];                                                             // dL/dS at the chunk's end, [value][key]
     float e_all[2][kN], e_mid[2][kN], e_rest[2][kN], inv0[2][kN], inv1[2][kN];    // e^{c_32}, e^{m}, e^{c_32-m}, e^{-m}, e^{m-c_32}
@@ -83,88 +84,98 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         const int p = wave - 8, t16 = lane & 15, ch = 16 * p + 4 * (lane >> 4);
         float fu[4];
         load4(u + h * kN + ch, fu);
-        float nr[2][4], nk[2][4], nv[2][4], nw[2][4], ng[2][4];   // the group's chunk as loaded (r, k, v, gy stay until handed on)
-        auto fetch = [&](int s) {
+        struct Set { Raw4<Tin> r[2], k[2], v[2], w[2]; Raw4<Tout> g[2]; };   // a chunk as loaded
+        Set set0, set1;
+        auto fetch = [&](Set &n, int s) {
+            if (s >= nchunk) return;
             const int c = nchunk - 1 - s;
             const int64_t row0 = base + (int64_t)c * kC32 * C;   // (uniform)
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
                 const int o = min(16 * x + t16, T - 1 - c * kC32) * (int)C + ch;   // rows past the end read the last one
-                load4(r + row0 + o, nr[x]); load4(k + row0 + o, nk[x]); load4(v + row0 + o, nv[x]); load4(w + row0 + o, nw[x]);
-                load4(gy + row0 + o, ng[x]);
+                n.r[x].load(r + row0 + o); n.k[x].load(k + row0 + o); n.v[x].load(v + row0 + o); n.w[x].load(w + row0 + o);
+                n.g[x].load(gy + row0 + o);
             }
         };
-        float f1[2][4], f3[2][4], dd[2][4], e_all[4], e_mid[4], e_rest[4], inv0[4], inv1[4], part[2];
+        float f1[2][4], f3[2][4], dd[2][4];
         bool wild = false;
-        // two channels of the lane's four at a time (a barrier in between)
-        auto form = [&](auto half, int s) {
-            constexpr int E0 = 2 * decltype(half)::value;
-            const int c = nchunk - 1 - s;
+        auto as4 = [](const float (&f)[4]) { return (f32x4){f[0], f[1], f[2], f[3]}; };
+        // operands of step s -> LDS, the scale factors stay in registers for rows()
+        auto form = [&](const Set &n, int s) {
+            if (s >= nchunk) return;
+            const int c = nchunk - 1 - s, buf = s & 1;
             const bool valid[2] = {c * kC32 + t16 < T, c * kC32 + 16 + t16 < T};
             C32Scale sc;
             sc.wild = false;
-            c32_scale<E0, E0 + 2>(nw, valid, sc, dd);
+            float fw[2][4];
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) fw[x][e] = n.w[x].at(e);
+            c32_scale<0, 4>(fw, valid, sc, dd);
             wild |= sc.wild;
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
-                float acc = E0 == 0 ? 0.f : part[x];
+                const int t = 16 * x + t16;
+                float acc = 0.f;
+                f32x4 rp, kp, fv, fg;
 #pragma unroll
-                for (int e = E0; e < E0 + 2; ++e) {
-                    if (!valid[x]) { nr[x][e] = 0.f; nk[x][e] = 0.f; nv[x][e] = 0.f; ng[x][e] = 0.f; }
+                for (int e = 0; e < 4; ++e) {
+                    const float fr = valid[x] ? n.r[x].at(e) : 0.f, fk = valid[x] ? n.k[x].at(e) : 0.f;
+                    fv[e] = valid[x] ? n.v[x].at(e) : 0.f;
+                    fg[e] = valid[x] ? n.g[x].at(e) : 0.f;
                     f1[x][e] = sc.rp[x][e];
                     f3[x][e] = sc.kp[x][e];
-                    e_all[e] = sc.all[e]; e_mid[e] = sc.mid[e]; e_rest[e] = sc.rest[e]; inv0[e] = sc.inv0[e]; inv1[e] = sc.inv1[e];
-                    acc = fmaf(nr[x][e] * nk[x][e], fu[e], acc);
+                    rp[e] = fr * f1[x][e];
+                    kp[e] = fk * f3[x][e];
+                    acc = fmaf(fr * fk, fu[e], acc);
                 }
-                part[x] = E0 == 0 ? acc : sum_rows4(acc);
+                acc = sum_rows4(acc);
+                *reinterpret_cast<f32x4 *>(&L.Rp[buf][t][ch]) = rp;
+                *reinterpret_cast<f32x4 *>(&L.Kp[buf][t][ch]) = kp;
+                *reinterpret_cast<f32x4 *>(&L.V[buf][t][ch]) = fv;
+                *reinterpret_cast<f32x4 *>(&L.GY[buf][t][ch]) = fg;
+                if (lane < 16) L.ruk[buf][p][t] = acc;
+            }
+            if (t16 == 0) {
+                *reinterpret_cast<f32x4 *>(&L.e_all[buf][ch]) = as4(sc.all);
+                *reinterpret_cast<f32x4 *>(&L.e_mid[buf][ch]) = as4(sc.mid);
+                *reinterpret_cast<f32x4 *>(&L.e_rest[buf][ch]) = as4(sc.rest);
+                *reinterpret_cast<f32x4 *>(&L.inv0[buf][ch]) = as4(sc.inv0);
+                *reinterpret_cast<f32x4 *>(&L.inv1[buf][ch]) = as4(sc.inv1);
             }
         };
-        auto as4 = [](const float (&f)[4]) { return (f32x4){f[0], f[1], f[2], f[3]}; };
-        auto publish = [&](int s) {
-            const int buf = s & 1;
+        auto rows = [&](const Set &n, int s) {
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
                 const int t = 16 * x + t16;
-                *reinterpret_cast<f32x4 *>(&L.R[buf][t][ch]) = as4(nr[x]);
-                *reinterpret_cast<f32x4 *>(&L.K[buf][t][ch]) = as4(nk[x]);
-                *reinterpret_cast<f32x4 *>(&L.F1[buf][t][ch]) = as4(f1[x]);
-                *reinterpret_cast<f32x4 *>(&L.F3[buf][t][ch]) = as4(f3[x]);
-                *reinterpret_cast<f32x4 *>(&L.V[buf][t][ch]) = as4(nv[x]);
-                *reinterpret_cast<f32x4 *>(&L.GY[buf][t][ch]) = as4(ng[x]);
-                *reinterpret_cast<f32x4 *>(&L.D[buf][t][ch]) = as4(dd[x]);
-                if (lane < 16) L.ruk[buf][p][t] = part[x];
-            }
-            if (t16 == 0) {
-                *reinterpret_cast<f32x4 *>(&L.e_all[buf][ch]) = as4(e_all);
-                *reinterpret_cast<f32x4 *>(&L.e_mid[buf][ch]) = as4(e_mid);
-                *reinterpret_cast<f32x4 *>(&L.e_rest[buf][ch]) = as4(e_rest);
-                *reinterpret_cast<f32x4 *>(&L.inv0[buf][ch]) = as4(inv0);
-                *reinterpret_cast<f32x4 *>(&L.inv1[buf][ch]) = as4(inv1);
+                const bool valid = (nchunk - 1 - s) * kC32 + t < T;
+                f32x4 fr, fk;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { fr[e] = valid ? n.r[x].at(e) : 0.f; fk[e] = valid ? n.k[x].at(e) : 0.f; }
+                *reinterpret_cast<f32x4 *>(&L.R[t][ch]) = fr;
+                *reinterpret_cast<f32x4 *>(&L.K[t][ch]) = fk;
+                *reinterpret_cast<f32x4 *>(&L.F1[t][ch]) = as4(f1[x]);
+                *reinterpret_cast<f32x4 *>(&L.F3[t][ch]) = as4(f3[x]);
+                *reinterpret_cast<f32x4 *>(&L.D[t][ch]) = as4(dd[x]);
             }
         };
-        const std::integral_constant<int, 0> h0;
-        const std::integral_constant<int, 1> h1;
-        // While step s is computed: the tiles of step s + 1 go to LDS and the loads of step s + 2 are issued
-        // (phase 1), the scale factors of step s + 2 are formed (phase 2).
-        fetch(0);
-        form(h0, 0);
-        form(h1, 0);
-        publish(0);
-        if (nchunk > 1) {
-            fetch(1);
-            form(h0, 1);
-            form(h1, 1);
-        }
+        // Phase 1 of step s: the rows of step s to LDS, the loads of step s + 2 issued into the registers that this frees.
+        // Phase 2: the operands of step s + 1 formed and published (their loads are a step and a half old).
+        auto step = [&](Set &now, Set &next, int s) {
+            rows(now, s);
+            fetch(now, s + 2);
+            __syncthreads();
+            form(next, s + 1);
+            __syncthreads();
+        };
+        fetch(set0, 0);
+        fetch(set1, 1);
+        form(set0, 0);
         __syncthreads();
-        for (int s = 0; s < nchunk; ++s) {
-            if (s + 1 < nchunk) publish(s + 1);
-            if (s + 2 < nchunk) fetch(s + 2);
-            __syncthreads();
-            if (s + 2 < nchunk) {
-                form(h0, s + 2);
-                form(h1, s + 2);
-            }
-            __syncthreads();
+        for (int s = 0; s < nchunk; s += 2) {
+            step(set0, set1, s);
+            if (s + 1 < nchunk) step(set1, set0, s + 1);
         }
         const bool any = __any(wild);
         if (lane == 0) L.wild[p] = any;
@@ -200,11 +211,9 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
                 for (int ib = 0; ib < 4; ++ib) {
                     const int i0 = 16 * ib + 4 * g;
-                    const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.K[buf][16 * sb + n][i0]) *
-                                     *reinterpret_cast<const f32x4 *>(&L.F3[buf][16 * sb + n][i0]) *
+                    const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.Kp[buf][16 * sb + n][i0]) *
                                      *reinterpret_cast<const f32x4 *>(&L.inv1[buf][i0]);
-                    const f32x4 fr = *reinterpret_cast<const f32x4 *>(&L.R[buf][16 * tb + n][i0]) *
-                                     *reinterpret_cast<const f32x4 *>(&L.F1[buf][16 * tb + n][i0]) *
+                    const f32x4 fr = *reinterpret_cast<const f32x4 *>(&L.Rp[buf][16 * tb + n][i0]) *
                                      *reinterpret_cast<const f32x4 *>(&L.inv0[buf][i0]);
                     at = mfma16(fk, fr, at);
                 }
@@ -221,8 +230,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
             for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
                 for (int ib = 0; ib < 4; ++ib) {
-                    const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.K[buf][16 * sb + n][16 * ib + 4 * g]) *
-                                     *reinterpret_cast<const f32x4 *>(&L.F3[buf][16 * sb + n][16 * ib + 4 * g]);
+                    const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.Kp[buf][16 * sb + n][16 * ib + 4 * g]);
                     gvt[sb] = mfma16(G[ib], fk, gvt[sb]);   // transposed: lane (n, g) gets token n, channels 4g ..
                 }
             __syncthreads();
@@ -255,7 +263,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                 for (int tb = 0; tb < 2; ++tb) {
                     f32x4 fra;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) fra[e] = L.R[buf][16 * tb + 4 * g + e][16 * ib + n] * L.F1[buf][16 * tb + 4 * g + e][16 * ib + n];
+                    for (int e = 0; e < 4; ++e) fra[e] = L.Rp[buf][16 * tb + 4 * g + e][16 * ib + n];
                     G[ib] = mfma16(fra, gyb[tb], G[ib]);
                 }
             }
@@ -360,8 +368,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int t = 16 * x + 4 * g + e;
-                    rp[x][e] = L.R[buf][t][col] * L.F1[buf][t][col];
-                    kp[x][e] = L.K[buf][t][col] * L.F3[buf][t][col];
+                    rp[x][e] = L.Rp[buf][t][col];
+                    kp[x][e] = L.Kp[buf][t][col];
                 }
 #pragma unroll
             for (int tb = 0; tb < 2; ++tb)
@@ -388,8 +396,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
                 const int t = 16 * x + n;
-                const f32x4 rt = *reinterpret_cast<const f32x4 *>(&L.R[buf][t][ch]), kt = *reinterpret_cast<const f32x4 *>(&L.K[buf][t][ch]);
-                const f32x4 f1 = *reinterpret_cast<const f32x4 *>(&L.F1[buf][t][ch]), f3 = *reinterpret_cast<const f32x4 *>(&L.F3[buf][t][ch]);
+                const f32x4 rt = *reinterpret_cast<const f32x4 *>(&L.R[t][ch]), kt = *reinterpret_cast<const f32x4 *>(&L.K[t][ch]);
+                const f32x4 f1 = *reinterpret_cast<const f32x4 *>(&L.F1[t][ch]), f3 = *reinterpret_cast<const f32x4 *>(&L.F3[t][ch]);
                 const float vg = L.vgy[t];
                 Z[x] *= row0;
                 W[x] *= row1;
@@ -410,7 +418,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
             // E_{t+1} = E at the chunk's end + what the later tokens of the chunk add
 #pragma unroll
             for (int x = 1; x >= 0; --x) {
-                const f32x4 d = *reinterpret_cast<const f32x4 *>(&L.D[buf][16 * x + n][ch]);
+                const f32x4 d = *reinterpret_cast<const f32x4 *>(&L.D[16 * x + n][ch]);
                 f32x4 o_w;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
