@@ -110,8 +110,7 @@ int wkv6_forward_with_state_ex(void *stream, int dtype, int state_dtype, int alg
  * non-zero -- a long bf16 sequence with so few (batch, head) pairs that most of the chip would idle --
  * passing that many bytes lets the forward run as time segments side by side (same results to
  * rounding); without it the call works as always.  Batches need T to divide into equal segments
- * of whole 64-token chunks; a single sequence (B = 1) may have any length if its final state is
- * fp32 or not asked for. */
+ * of whole 64-token chunks; a single sequence (B = 1) may have any length. */
 size_t wkv6_forward_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);
 
 /* Forward (inference) with the layer's output stage fused in; y itself is not written:
@@ -274,8 +273,8 @@ size_t wkv6_backward_workspace_bytes_ex(int dtype, int algo, int64_t B, int64_t 
  * skips its own forward state sweep.  `saved` is caller-owned device memory of wkv6_saved_bytes()
  * bytes (0 = this path saves nothing; pass NULL), must be left untouched between the two calls,
  * and serves the backward as its workspace too.  A long sequence (T >= 1024) of so few (batch, head)
- * pairs that they fill at most half of the compute units runs as 2, 4, 8 or 16 time segments side by
- * side in both calls (same results to rounding); wkv6_saved_bytes() includes what that keeps.
+ * pairs that they fill at most half of the compute units runs as 2 to 16 time segments side by side in
+ * both calls, whatever its length (same results to rounding); wkv6_saved_bytes() includes what that keeps.
  * No counterpart in the reference, whose backward
  * recomputes everything from the inputs (rwkv_kernel/torch_rwkv_kernel.py:33 saves only r,k,v,w,u). */
 size_t wkv6_saved_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);

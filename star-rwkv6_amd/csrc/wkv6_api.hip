@@ -141,10 +141,7 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
         return finish(wkv6::scan_forward(st, dtype, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys));
     if (!saved && workspace && aligned16(workspace)) {
         const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H);
-        // (tokens left over behind the equal segments are run from an fp32 state: possible when the
-        // final state is fp32 or not wanted)
-        const bool remainder_ok = wkv6::chunk_forward_segments_remainder(B, T, H) == 0 || state_dtype == WKV6_F32 || !ys;
-        if (need > 0 && workspace_bytes >= need && remainder_ok)
+        if (need > 0 && workspace_bytes >= need)
             return finish(wkv6::chunk_forward_segments_run(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, workspace));
     }
     return finish(wkv6::chunk_forward(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, saved));
@@ -189,8 +186,7 @@ int wkv6_forward_gn_gate_ex(void *stream, int dtype, int state_dtype,
                                                gate, gn_scale, gn_offset, gn_eps, out, ys));
     if (workspace && aligned16(workspace)) {   // optional: few pairs, long sequence -> time segments side by side
         const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H);
-        const bool remainder_ok = wkv6::chunk_forward_segments_remainder(B, T, H) == 0 || state_dtype == WKV6_F32 || !ys;
-        if (need > 0 && workspace_bytes >= need && remainder_ok)
+        if (need > 0 && workspace_bytes >= need)
             return finish(wkv6::chunk_forward_segments_run((hipStream_t)stream, state_dtype, B, T, H, r, k, v, w, u,
                                                            has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
                                                            out, ys, workspace, gate, gn_scale, gn_offset, gn_eps));
@@ -222,7 +218,7 @@ int wkv6_forward_gn_gate_save(void *stream, int dtype, int64_t B, int64_t T, int
     if (!saved || saved_bytes < need || !aligned16(saved)) return WKV6_ERR_WORKSPACE;
     const int P = train_segments(dtype, WKV6_ALGO_CHUNK, B, T, C, H);
     if (P > 1) {   // few pairs, long sequence: time segments side by side, the output stage in their second pass
-        char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H);
+        char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_forward_fused_save_segments((hipStream_t)stream, B, T, H, r, k, v, w, u, gate, gn_scale, gn_offset,
                                                               gn_eps, out, y, stats, saved, extra));
     }
@@ -345,7 +341,7 @@ static size_t saved_base_bytes(int dtype, int algo, int64_t B, int64_t T, int64_
     return ((ws > sv ? ws : sv) + 255) & ~(size_t)255;
 }
 // Segments the training pair of this shape runs in (1: one piece).  A (B,T,C) tensor cut into P
-// segments is handled as a (B*P, T/P, C) tensor, so the base part is sized for that shape.
+// segments is handled as a (B*P, L, C) tensor, so the base part is sized for that shape.
 static int train_segments(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
     const bool chunk = (algo == WKV6_ALGO_CHUNK && chunk_possible(dtype, T, C)) ||
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
@@ -371,7 +367,7 @@ size_t wkv6_saved_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, in
     if (!chunk) return 0;
     const int P = train_segments(dtype, algo, B, T, C, H);
     if (P > 1)
-        return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H) + wkv6::train_segments_layout(B, T, H, nullptr).bytes;
+        return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H) + wkv6::train_segments_layout(B, T, H, nullptr).bytes;
     const size_t ws = wkv6_backward_workspace_bytes_ex(dtype, algo, B, T, C, H), sv = wkv6::chunk_saved_bytes(B, T, H);
     return ws > sv ? ws : sv;
 }
@@ -395,7 +391,7 @@ int wkv6_forward_save(void *stream, int dtype, int algo, int64_t B, int64_t T, i
         const int P = train_segments(dtype, algo, B, T, C, H);
         if (!r || !k || !v || !w || !u || !y) return WKV6_ERR_ARG;
         if (!aligned16(r) || !aligned16(k) || !aligned16(v) || !aligned16(w) || !aligned16(y)) return WKV6_ERR_ARG;
-        char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H);
+        char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_forward_save_segments((hipStream_t)stream, B, T, H, r, k, v, w, u, y, saved, extra));
     }
     return forward_impl(stream, dtype, out_type(dtype), algo, B, T, C, H, 0, nullptr, r, k, v, w, u, nullptr, y, nullptr,
@@ -424,11 +420,11 @@ int wkv6_forward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64
 }
 
 // Workspace of a backward without saved states that runs in time segments (0: it does not): the
-// saved-states block of the (B*P, T/P, C) shape, then the segments' states.
+// saved-states block of the (B*P, L, C) shape, then the segments' states.
 static size_t segments_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
     const int P = train_segments(dtype, algo, B, T, C, H);
     if (P <= 1) return 0;
-    return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H) + wkv6::train_segments_layout(B, T, H, nullptr).bytes;
+    return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H) + wkv6::train_segments_layout(B, T, H, nullptr).bytes;
 }
 
 size_t wkv6_backward_workspace_bytes_ex(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
@@ -464,7 +460,7 @@ static int backward_segments_impl(void *stream, int dtype, int algo, int64_t B, 
         !aligned16(gk) || !aligned16(gv) || !aligned16(gw)) return WKV6_ERR_ARG;
     if (!saved || saved_bytes < wkv6_saved_bytes(dtype, algo, B, T, C, H) || !aligned16(saved)) return WKV6_ERR_WORKSPACE;
     const int P = train_segments(dtype, algo, B, T, C, H);
-    char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H);
+    char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
     return finish(wkv6::chunk_backward_saved_segments((hipStream_t)stream, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, gu_sum,
                                                       saved, extra));
 }
@@ -508,7 +504,7 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
     }
     if (!states_ready && train_segments(dtype, algo, B, T, C, H) > 1) {
         const int P = train_segments(dtype, algo, B, T, C, H);
-        char *extra = reinterpret_cast<char *>(workspace) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H);
+        char *extra = reinterpret_cast<char *>(workspace) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_backward_state_segments(st, B, T, H, r, k, v, w, u, nullptr, gy, nullptr, gr, gk, gv, gw, gu, nullptr,
                                                           workspace, extra));
     }
@@ -621,7 +617,7 @@ int wkv6_backward_with_state(void *stream, int dtype, int algo, int64_t B, int64
         return finish(wkv6::scan_backward_state(st, dtype, B, T, H, r, k, v, w, u, s0, gy, gsT, gr, gk, gv, gw, gu, gs0, workspace));
     const int P = train_segments(dtype, algo, B, T, C, H);
     if (P > 1) {
-        char *extra = reinterpret_cast<char *>(workspace) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, T / P, C, H);
+        char *extra = reinterpret_cast<char *>(workspace) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_backward_state_segments(st, B, T, H, r, k, v, w, u, s0, gy, gsT, gr, gk, gv, gw, gu, gs0,
                                                           workspace, extra));
     }

@@ -56,6 +56,8 @@ static_assert(BlockBwdLds::kBytes <= 160 * 1024, "LDS block of the block-form ba
 struct BlockBwdArgs {
     int T, H, B;
     int bstep;        // batch rows between two pairs of a workgroup (B: one pair per workgroup)
+    int slice;        // chunks of a pair's slice of `ckpt` (those of the longest row)
+    RowCut cut;       // rows that are time segments (!kMulti and kRagged)
     const bf16_t *r, *k, *v, *w, *u, *gy;
     bf16_t *gr, *gk, *gv, *gw, *gu;
     bf16_t *gu_sum;   // null, or C elements: receives the sum of gu over the batch
@@ -482,7 +484,7 @@ __device__ __forceinline__ void block_bwd_producer(const BlockBwdArgs &a, unsign
     // first element of the workgroup's pair number `slot` in a (B,T,C) tensor; its saved states
     auto pair_base = [&](int slot) { return (int64_t)(b0 + slot * a.bstep) * T * C + (int64_t)h * kN; };
     auto pair_states = [&](int slot) {
-        return reinterpret_cast<const bf16_t *>(a.ckpt + (int64_t)((b0 + slot * a.bstep) * H + h) * nchunk * (kN * kN));
+        return reinterpret_cast<const bf16_t *>(a.ckpt + (int64_t)((b0 + slot * a.bstep) * H + h) * a.slice * (kN * kN));
     };
     const int lrow = lane >> 3;
     const uint32_t lpiece = (uint32_t)(((lane & 7) ^ lrow) << 4);
@@ -608,13 +610,19 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
     const int pair0 = (int)blockIdx.x;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (kRagged && !kMulti && a.cut.segments) {
+        const RowView rv = row_view(a.cut, pair0 / a.H, a.T);
+        const int64_t n = rv.shift * a.H * kN;
+        a.T = rv.tokens;
+        move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.gy, n);
+        move_rows(a.gr, n); move_rows(a.gk, n); move_rows(a.gv, n); move_rows(a.gw, n);
+    }
     if (wave < 4) block_bwd_producer<kMulti, kRagged>(a, smem, s_wild, pair0, wave, lane);
     else if (wave < 8) block_bwd_xw<0, kMulti, kRagged>(a, smem, s_wild, pair0, wave - 4, lane);
     else block_bwd_xw<1, kMulti, kRagged>(a, smem, s_wild, pair0, wave - 8, lane);
     const int b0 = pair0 / a.H, h = pair0 - b0 * a.H;
     const int npw = kMulti ? (a.B - b0 + a.bstep - 1) / a.bstep : 1;
-    const int nchunk = (a.T + kBlockTokens - 1) / kBlockTokens;
-    const int64_t slice = (int64_t)nchunk * (kN * kN), C = (int64_t)a.H * kN;
+    const int64_t slice = (int64_t)a.slice * (kN * kN), C = (int64_t)a.H * kN;
     const int tid = threadIdx.x;
     __threadfence_block();
     __syncthreads();
@@ -684,9 +692,11 @@ bool block_backward_applies(int64_t B, int64_t T, int64_t H) { return block_forw
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
-                          const float *s0, const float *gsT, float *gs0)
+                          const float *s0, const float *gsT, float *gs0, RowCut cut)
 {
     BlockBwdArgs a = {};
+    a.cut = cut;
+    a.slice = (int)((T + kBlockTokens - 1) / kBlockTokens);
     a.T = (int)T; a.H = (int)H; a.B = (int)B;
     const int64_t grid = block_grid(B, H);
     a.bstep = B * H <= grid ? (int)B : (int)(grid / H);
@@ -697,7 +707,8 @@ hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
     a.s0 = s0; a.gsT = gsT; a.gs0 = gs0;
     a.ckpt = (float *)workspace;
     a.arrivals = reinterpret_cast<int *>(reinterpret_cast<char *>(workspace) + chunk_backward_workspace_bytes(B, T, H));
-    const bool multi = B * H > grid, ragged = (T % kBlockTokens) != 0;
+    const bool multi = B * H > grid, ragged = (T % kBlockTokens) != 0 || cut.segments;
+    if (cut.segments && multi) return hipErrorInvalidValue;
     auto launch = [&](auto multi_tag, auto ragged_tag) -> hipError_t {
         constexpr auto kern = block_bwd_kernel<decltype(multi_tag)::value, decltype(ragged_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockBwdLds::kBytes);

@@ -54,6 +54,8 @@ static_assert(BlockFwdLdsT<false>::kBytes <= 160 * 1024 && BlockFwdLdsT<true>::k
 struct BlockFwdArgs {
     int T, H, B;
     int bstep;               // batch rows between two pairs of a workgroup (B: one pair per workgroup)
+    int slice;               // chunks of a pair's slice of `ckpt` (those of the longest row)
+    RowCut cut;              // rows that are time segments (one pair per workgroup and kRagged)
     const bf16_t *r, *k, *v, *w, *u;
     const void *s0;          // initial state (B or n_state, H, 64, 64) [key][value] in Ts, or null
     const int64_t *map;      // batch row -> state row, or null
@@ -243,7 +245,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
 #pragma unroll
         for (int i = 0; i < 8; ++i) { gsc[i] = sp[i]; gof[i] = op_[i]; }
     }
-    char *ckb = kSave ? reinterpret_cast<char *>(a.ckpt + (int64_t)(b0 * H + h) * nchunk * (kN * kN)) : nullptr;
+    char *ckb = kSave ? reinterpret_cast<char *>(a.ckpt + (int64_t)(b0 * H + h) * a.slice * (kN * kN)) : nullptr;
     // Vector-memory operations this wave has issued so far, and the count right after the r, k, w loads
     // of visit j went out: a wave's operations complete in program order, so "the loads of visit j have
     // landed" is "at most (issued - mark of j) operations are still in flight".
@@ -336,7 +338,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
             co.c = 0; ++co.slot;
             yb = (kFuse ? a.out : a.y) + pair_base(co.slot);
             if (kFuse && y2b) y2b = a.y + pair_base(co.slot);
-            if (kSave) ckb = reinterpret_cast<char *>(a.ckpt + (int64_t)((b0 + co.slot * a.bstep) * H + h) * nchunk * (kN * kN));
+            if (kSave) ckb = reinterpret_cast<char *>(a.ckpt + (int64_t)((b0 + co.slot * a.bstep) * H + h) * a.slice * (kN * kN));
         }
     };
     float u4[4];
@@ -422,6 +424,13 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pair0 = (int)blockIdx.x;
+    if (kRagged && a.cut.segments) {
+        const RowView rv = row_view(a.cut, pair0 / a.H, a.T);
+        const int64_t n = rv.shift * a.H * kN;
+        a.T = rv.tokens;
+        move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.y, n);
+        if (kFuse) { move_rows(a.gate, n); move_rows(a.out, n); move_rows(a.stats, rv.shift * a.H * 2); }
+    }
     if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
     else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse>(a, smem, pair0, wave - 4, lane);
     else block_fwd_producer<kSave, kRagged, kFuse, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
@@ -465,12 +474,15 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H) {
 static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                        const void *r, const void *k, const void *v, const void *w, const void *u,
                                        const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
-                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats)
+                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats, RowCut cut)
 {
     BlockFwdArgs a = {};
+    a.cut = cut;
+    a.slice = (int)((T + kBlockTokens - 1) / kBlockTokens);
     a.T = (int)T; a.H = (int)H; a.B = (int)B;
     const int64_t grid = block_grid(B, H);
     a.bstep = B * H <= grid ? (int)B : (int)(grid / H);
+    if (cut.segments && B * H > grid) return hipErrorInvalidValue;
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
@@ -484,7 +496,7 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
         return hipGetLastError();
     };
     auto launch_ts = [&](auto ts_tag, auto save_tag, auto fuse_tag) -> hipError_t {
-        return (T % kBlockTokens) != 0 ? launch(ts_tag, save_tag, std::true_type{}, fuse_tag) : launch(ts_tag, save_tag, std::false_type{}, fuse_tag);
+        return (T % kBlockTokens) != 0 || cut.segments ? launch(ts_tag, save_tag, std::true_type{}, fuse_tag) : launch(ts_tag, save_tag, std::false_type{}, fuse_tag);
     };
     const bool save = saved_states != nullptr;
     if (gate != nullptr) {
@@ -498,19 +510,19 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
 
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters)
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters,
-                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr);
+                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, cut);
 }
 
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                               void *out, void *y, float *stats, void *sT, void *saved_states)
+                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, saved_states != nullptr,
-                                gate, gn_scale, gn_offset, gn_eps, out, stats);
+                                gate, gn_scale, gn_offset, gn_eps, out, stats, cut);
 }
 
 }  // namespace wkv6

@@ -64,6 +64,8 @@ static_assert(BwdLds::kBytes <= 160 * 1024, "LDS block of the backward kernel");
 
 struct BwdArgs {
     int T, H;
+    int slice;        // chunks of a pair's slice of `ckpt` (those of the longest row)
+    RowCut cut;       // rows that are time segments (kRagged)
     const bf16_t *r, *k, *v, *w, *u, *gy;   // 16-bit elements: bf16, or fp16 with v and gy bf16 copies (see OutOf)
     const void *v_orig, *gy_orig;           // v and gy as the caller holds them (read by the exact per-timestep pass)
     bf16_t *gr, *gk, *gv, *gw, *gu;         // elements of the output type (bf16, or fp32 for fp16 tensors)
@@ -422,7 +424,7 @@ __device__ __forceinline__ void bwd_producer(const BwdArgs &a, unsigned char *sm
     // the rows of the pair
     const int64_t base0 = (int64_t)b0 * T * C + (int64_t)h * kN;
     const bf16_t *rb = a.r + base0, *kb_ = a.k + base0, *vb = a.v + base0, *wb = a.w + base0, *gb = a.gy + base0;   // loads
-    const bf16_t *ckb = reinterpret_cast<const bf16_t *>(a.ckpt + (int64_t)(b0 * H + h) * nchunk * (kN * kN));      // state loads
+    const bf16_t *ckb = reinterpret_cast<const bf16_t *>(a.ckpt + (int64_t)(b0 * H + h) * a.slice * (kN * kN));      // state loads
     Tout *gvb = reinterpret_cast<Tout *>(a.gv) + base0;                                                            // gv role
     // this lane's part of an 8-row block load: row (lane >> 3), 16-byte piece swizzled with the row
     const int lrow = lane >> 3;
@@ -604,6 +606,15 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int role = wave >> 2, q = wave & 3;
     typedef typename OutOf<Tin>::type Tout;
+    if (kRagged && a.cut.segments) {
+        const RowView rv = row_view(a.cut, pair0 / a.H, a.T);
+        const int64_t n = rv.shift * a.H * kN;
+        a.T = rv.tokens;
+        move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.gy, n);
+        a.v_orig = reinterpret_cast<const Tin *>(a.v_orig) + n; a.gy_orig = reinterpret_cast<const Tout *>(a.gy_orig) + n;
+        auto out_rows = [&](bf16_t *&p) { p = reinterpret_cast<bf16_t *>(reinterpret_cast<Tout *>(p) + n); };
+        out_rows(a.gr); out_rows(a.gk); out_rows(a.gv); out_rows(a.gw);
+    }
     if (role == 0) bwd_producer<Tin, kRagged>(a, smem, s_wild, pair0, q, lane);
     else if (role == 1) bwd_consumer<Tin, kRagged, 0>(a, smem, s_wild, pair0, q, lane);
     else bwd_consumer<Tin, kRagged, 1>(a, smem, s_wild, pair0, q, lane);
@@ -611,8 +622,7 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
     // pair's own slice of the state workspace (nchunk x 64 x 64 floats = T' x 64) holds P
     if (s_wild[0]) {
         const int b = pair0 / a.H, h = pair0 % a.H;
-        const int nchunk = (a.T + CL - 1) / CL;
-        float *ck = a.ckpt + (int64_t)(b * a.H + h) * nchunk * (kN * kN);
+        float *ck = a.ckpt + (int64_t)(b * a.H + h) * a.slice * (kN * kN);
         const int64_t so = (int64_t)(b * a.H + h) * (kN * kN);
         const float *s0p = a.s0 ? a.s0 + so : nullptr, *gsTp = a.gsT ? a.gsT + so : nullptr;
         const bool states = a.s0 || a.gsT || a.gs0;
@@ -635,8 +645,7 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
     if (a.gu_sum != nullptr) {
         __shared__ int s_last;
         const int h = pair0 % a.H;
-        const int nchunk = (a.T + CL - 1) / CL;
-        const int64_t slice = (int64_t)nchunk * (kN * kN), C = (int64_t)a.H * kN;
+        const int64_t slice = (int64_t)a.slice * (kN * kN), C = (int64_t)a.H * kN;
         const int nparts = a.B;   // what adds up to the head's sum: one partial per batch row
         __threadfence_block();   // this workgroup's gu rows (consumer group 0 or the second pass) are written
         __syncthreads();
@@ -688,12 +697,14 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, bool states_ready,
                           void *gu_sum, const float *s0, const float *gsT, float *gs0,
-                          int in_dtype, const void *v_orig, const void *gy_orig)
+                          int in_dtype, const void *v_orig, const void *gy_orig, RowCut cut)
 {
     const size_t lds = BwdLds::kBytes;
     BwdArgs a;
     a.v_orig = v_orig ? v_orig : v; a.gy_orig = gy_orig ? gy_orig : gy;
     a.s0 = s0; a.gsT = gsT; a.gs0 = gs0;
+    a.cut = cut;
+    a.slice = (int)((T + CL - 1) / CL);
     a.T = (int)T; a.H = (int)H;
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w;
     a.u = (const bf16_t *)u; a.gy = (const bf16_t *)gy;
@@ -715,16 +726,16 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
         if (in_dtype == kF16) return states_ready && v_orig && gy_orig ? launch_in(f16_t{}, ragged_tag) : hipErrorInvalidValue;
         return launch_in(bf16_t{}, ragged_tag);
     };
-    const bool ragged = (T % CL) != 0;   // the last chunk has tokens past the end
+    const bool ragged = (T % CL) != 0 || cut.segments;   // the last chunk has tokens past the end
     // (gradients through the state: the block form takes them with one pair per workgroup)
     const bool block_form = in_dtype == kBF16 && block_backward_applies(B, T, H) && ((!s0 && !gsT && !gs0) || B * H <= block_grid(B, H));
     if (!states_ready) {
         // No states from a saving forward: the forward kernel's state-only pass (no y) leaves them in
         // the workspace first.
-        hipError_t e = chunk_forward(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, nullptr, nullptr, workspace, nullptr, false, false);
+        hipError_t e = chunk_forward(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, nullptr, nullptr, workspace, nullptr, false, false, cut);
         if (e != hipSuccess) return e;
     }
-    if (block_form) return block_backward(st, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, a.gu_sum, s0, gsT, gs0);
+    if (block_form) return block_backward(st, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, a.gu_sum, s0, gsT, gs0, cut);
     return ragged ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
@@ -749,17 +760,17 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
                                          void *saved, void *extra)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
-    const int64_t L = T / s.P, rows = B * s.P;
+    const int64_t L = s.L, rows = B * s.P;
     // (1) What each segment alone sends back into its incoming state: G_0 = sum_t (prod_{s<t} d_s) r_t^T gy_t.
     // That is the state the FORWARD recurrence builds from zero over the segment read back to front
     // with r in the place of k and gy in the place of v, so the forward kernel's state-only pass does it.
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true);
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     // (2) chained backwards in time: the gradient arriving at the end of every segment
     if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates)) != hipSuccess) return e;
     // (3) every segment again, between its true incoming state and its true arriving gradient
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, gu_sum,
-                       s.states, s.gstates, nullptr);
+                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
     if (e != hipSuccess) return e;
     const int C = (int)(H * kN);
     hipLaunchKernelGGL(segments_finish_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
@@ -777,17 +788,17 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
                                          void *saved, void *extra)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
-    const int64_t L = T / s.P, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum);
+    const int64_t L = s.L, rows = B * s.P;
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_forward(st, s.P, B, H, s.dsum, s.states, s0)) != hipSuccess) return e;
-    e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, nullptr, nullptr, saved, nullptr, false, false);
+    e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, nullptr, nullptr, saved, nullptr, false, false, s.cut);
     if (e != hipSuccess) return e;
-    e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true);
+    e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates, gsT, gs0)) != hipSuccess) return e;
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, nullptr,
-                       s.states, s.gstates, nullptr);
+                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
     if (e != hipSuccess) return e;
     const int C = (int)(H * kN);
     // (the decay gradient at an end of the sequence is zero by definition only where no state / no gradient comes in)

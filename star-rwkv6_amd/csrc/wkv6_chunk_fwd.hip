@@ -70,7 +70,9 @@ struct FwdArgs {
     int T, H;
     int nitems;      // B * H (batch, head) pairs; with kMulti a workgroup takes every gridDim.x-th of them
     int split;       // 1, 2 or 4 workgroups per pair, each with the consumer waves of 4 / split column slices
-    int reverse;     // 1: the time axis is read back to front (row T-1-t in the place of row t); T a multiple of 64
+    int reverse;     // 1: the time axis is read back to front (row T-1-t in the place of row t)
+    int slice;       // chunks of a pair's slice of `ckpt` (those of the longest row)
+    RowCut cut;      // rows that are time segments (one pair per workgroup and kRagged)
     float *dsum;     // null, or [4 tiles][pairs][64]: per pair, log2(e) * sum of exp(w) over the tokens of tile p of every chunk
     const bf16_t *r, *k, *v, *w, *u;   // 16-bit elements: bf16, or fp16 with v a bf16 copy (see OutOf)
     const void *v_orig;                // v as the caller holds it (the exact per-timestep pass reads this one)
@@ -140,7 +142,7 @@ __device__ __forceinline__ void fwd_consumer(const FwdArgs &a, const unsigned ch
                 // eight contiguous bytes there, so a chunk takes four stores per lane.  They are issued behind
                 // the barrier (the state registers do not change before the end of tile 0) and queue while
                 // the other waves already work on the chunk.
-                char *dst = reinterpret_cast<char *>(a.ckpt + (int64_t)bh * nchunk * (kN * kN)) + (int64_t)c * (kN * kN * 2) + (16 * q + l16) * (kN * 2) + 8 * g;
+                char *dst = reinterpret_cast<char *>(a.ckpt + (int64_t)bh * a.slice * (kN * kN)) + (int64_t)c * (kN * kN * 2) + (16 * q + l16) * (kN * 2) + 8 * g;
 #pragma unroll
                 for (int m = 0; m < 4; ++m)
                     *reinterpret_cast<uint2 *>(dst + 32 * m) = make_uint2(pack_bf16x2(S[m][0], S[m][1]), pack_bf16x2(S[m][2], S[m][3]));
@@ -283,7 +285,7 @@ __device__ __forceinline__ void fwd_producer(const FwdArgs &a, unsigned char *sm
         if (kFuse) gb = a.gate + base;
     };
     point_loads();
-    // Rows past the end of the sequence are fetched from row T-1 (valid memory); the operand
+    // Rows past the end of the sequence are fetched from its last row (valid memory); the operand
     // preparation turns them into r = k = 0, w = -inf (decay 1), and the v rows only ever meet zero
     // operands.  Each wave loads what it reads itself, so its own vmcnt covers its inputs; v is
     // picked up by the consumers a barrier later.
@@ -296,7 +298,7 @@ __device__ __forceinline__ void fwd_producer(const FwdArgs &a, unsigned char *sm
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
             const int t = tb + 8 * blk + lrow;
-            const uint32_t o = (uint32_t)(kRagged ? min(t, T - 1) : a.reverse ? T - 1 - t : t) * rowbytes + lpiece;
+            const uint32_t o = (uint32_t)(a.reverse ? (kRagged ? max(T - 1 - t, 0) : T - 1 - t) : kRagged ? min(t, T - 1) : t) * rowbytes + lpiece;
             load_rows8_to_lds(wb, o, rkw + 2 * kTileBytes + 8 * blk * kTileRow);
             if (!kNoR) load_rows8_to_lds(rb, o, rkw + 8 * blk * kTileRow);
             load_rows8_to_lds(kb_, o, rkw + kTileBytes + 8 * blk * kTileRow);
@@ -523,6 +525,15 @@ __global__ __launch_bounds__(kFwdThreads) void chunk_fwd_kernel(FwdArgs a)
     const int split = kMulti || kFuse ? 1 : a.split;
     const int bh0 = (int)blockIdx.x / split, part = (int)blockIdx.x - bh0 * split;
     const int nq = 4 / split;   // consumer waves per group
+    if (kRagged && !kMulti && a.cut.segments) {
+        const RowView rv = row_view(a.cut, bh0 / a.H, a.T);
+        const int64_t n = rv.shift * a.H * kN;
+        a.T = rv.tokens;
+        move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n);
+        a.v_orig = reinterpret_cast<const Tin *>(a.v_orig) + n;
+        if (a.y) a.y = reinterpret_cast<bf16_t *>(reinterpret_cast<typename OutOf<Tin>::type *>(a.y) + n);
+        if (kFuse) { move_rows(a.gate, n); move_rows(a.out, n); move_rows(a.stats, rv.shift * a.H * 2); }
+    }
     if (wave < 4) {
         fwd_producer<Tin, kSave, kRagged, kMulti, kFuse, kNoR>(a, smem, s_wild, bh0, part, wave, lane);
     } else {
@@ -608,21 +619,23 @@ static unsigned forward_grid(int64_t pairs, bool *multi, int *split) {
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *dsum, bool reverse,
-                         bool counters)
+                         bool counters, RowCut cut)
 {
     if (y != nullptr && dsum == nullptr && !reverse && block_forward_applies(B, T, H))
-        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters);
+        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters, cut);
     FwdArgs a = {};
     a.dsum = dsum;
-    a.reverse = reverse && (T % CL) == 0;
-    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H);
+    a.reverse = reverse;
+    a.cut = cut;
+    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.v_orig = v;
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     bool multi;
     const unsigned grid = forward_grid(B * H, &multi, &a.split);
-    const bool save = saved_states != nullptr, ragged = (T % CL) != 0;
+    if (cut.segments && multi) return hipErrorInvalidValue;
+    const bool save = saved_states != nullptr, ragged = (T % CL) != 0 || cut.segments;
     return state_dtype == kF32 ? launch_fwd<float>(st, a, save, ragged, multi, grid)
                                : launch_fwd<bf16_t>(st, a, save, ragged, multi, grid);
 }
@@ -655,7 +668,7 @@ hipError_t chunk_forward_save_f16(hipStream_t st, int64_t B, int64_t T, int64_t 
                                   void *y, void *saved_states)
 {
     FwdArgs a = {};
-    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H);
+    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v_bf16; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.v_orig = v;
     a.y = (bf16_t *)y; a.ckpt = (float *)saved_states;
@@ -669,12 +682,12 @@ hipError_t chunk_forward_save_f16(hipStream_t st, int64_t B, int64_t T, int64_t 
 hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale,
-                               const float *gn_offset, float gn_eps, void *out, void *sT)
+                               const float *gn_offset, float gn_eps, void *out, void *sT, RowCut cut)
 {
     if (block_forward_applies(B, T, H))
-        return block_forward_fused(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, gate, gn_scale, gn_offset, gn_eps, out, nullptr, nullptr, sT, nullptr);
+        return block_forward_fused(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, gate, gn_scale, gn_offset, gn_eps, out, nullptr, nullptr, sT, nullptr, cut);
     FwdArgs a = {};
-    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H);
+    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.s0 = s0; a.map = map; a.sT = sT;
     a.v_orig = v;
@@ -682,7 +695,9 @@ hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64
     bool multi;
     const unsigned grid = forward_grid(B * H, &multi, &a.split);
     a.split = 1;   // the output stage needs a chunk's whole rows in one workgroup
-    const bool ragged = (T % CL) != 0;
+    a.cut = cut;
+    if (cut.segments && multi) return hipErrorInvalidValue;
+    const bool ragged = (T % CL) != 0 || cut.segments;
     return state_dtype == kF32 ? launch_fwd_fused<float>(st, a, ragged, multi, grid)
                                : launch_fwd_fused<bf16_t>(st, a, ragged, multi, grid);
 }
@@ -693,13 +708,13 @@ hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64
 static hipError_t fused_save_from(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                   const void *r, const void *k, const void *v, const void *w, const void *u, const float *s0,
                                   const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                  void *out, void *y, float *stats, void *saved_states)
+                                  void *out, void *y, float *stats, void *saved_states, RowCut cut = RowCut())
 {
     if (block_forward_applies(B, T, H))
-        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states);
+        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states, cut);
     FwdArgs a = {};
     a.s0 = s0;
-    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H);
+    a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.v_orig = v;
     a.gate = (const bf16_t *)gate; a.gn_scale = gn_scale; a.gn_offset = gn_offset; a.gn_eps = gn_eps; a.out = (bf16_t *)out;
@@ -708,7 +723,9 @@ static hipError_t fused_save_from(hipStream_t st, int64_t B, int64_t T, int64_t 
     bool multi;
     const unsigned grid = forward_grid(B * H, &multi, &a.split);
     a.split = 1;
-    return (T % CL) != 0 ? launch_fwd<bf16_t, float, true, true, true>(st, a, multi, grid)
+    a.cut = cut;
+    if (cut.segments && multi) return hipErrorInvalidValue;
+    return (T % CL) != 0 || cut.segments ? launch_fwd<bf16_t, float, true, true, true>(st, a, multi, grid)
                          : launch_fwd<bf16_t, float, true, false, true>(st, a, multi, grid);
 }
 hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -726,33 +743,34 @@ hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_
 // pair walks its sequence alone.  The map from a segment's incoming state to its outgoing state is
 // affine, S_out = D o S_in + U with D[j] = exp(-sum_t exp(w_t[j])) over the segment and U the state
 // the segment builds from zero, so: (A) every segment runs from a zero state (all segments at once;
-// a (B,T,C) tensor cut into P equal segments IS a (B*P, T/P, C) tensor; no y in this pass) and leaves
+// a (B,T,C) tensor cut into P equal segments IS a (B*P, T/P, C) tensor, and RowCut stands for other lengths; no y in this pass) and leaves
 // U and, from the producer waves, the exponent of D; (B) a tiny kernel chains the P affine maps per pair,
 // leaving each segment's true incoming state where its U was (and the final state); (C) every
 // segment runs again from its true state and writes y.  Twice the forward work on P times the
 // workgroups.
 // ------------------------------------------------------------------------------------------
+constexpr int kMostSegments = 16;
 // kReverse: the same chain walked from the last segment to the first, which is what the reverse
 // state of the backward pass obeys (the gradient arriving at the end of segment p is what segment
 // p + 1 sends into its incoming state: its own contribution plus D_{p+1} times what arrives at its end).
-template <typename Ts, bool kReverse, int P>
-__global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
-                                                            const float *__restrict__ dsum, float *__restrict__ states, Ts *__restrict__ sT,
-                                                            float *__restrict__ sT32)   // the final state: as Ts and / or as fp32 (either may be null)
+template <typename Ts, bool kReverse, int kMost>
+__global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
+                                                            const float *__restrict__ dsum, float *__restrict__ states, Ts *__restrict__ sT)   // sT: the final state, or null
 {
     // Thread: four value columns i0..i0+3 of one key row j of one (batch, head): 1024 threads per pair,
     // gridDim.x * 256 = B * H * 1024.  states[(b*P + seg), h] holds U on entry and the segment's
-    // incoming state on exit.  All P loads are issued before the chain is walked (their addresses do
+    // incoming state on exit (P <= kMost segments).  All P loads are issued before the chain is walked (their addresses do
     // not depend on it): the kernel takes about two memory round trips instead of 2 P.
     const int e = blockIdx.x * 256 + threadIdx.x;
     const int i0 = (e & 15) * 4, j = (e >> 4) & 63, bh = e >> 10;
     const int b = bh / H, h = bh - b * H;
     const int64_t np = (int64_t)(gridDim.x >> 2) * P;   // pairs of all segments
     auto pair_of_step = [&](int n) { return ((int64_t)b * P + (kReverse ? P - 1 - n : n)) * H + h; };   // step n of the walk
-    float4 x[P];
-    float d[P];
+    float4 x[kMost];
+    float d[kMost];
 #pragma unroll
-    for (int n = 0; n < P; ++n) {
+    for (int n = 0; n < kMost; ++n) {
+        if (n >= P) break;
         const int64_t vp = pair_of_step(n);
         x[n] = *reinterpret_cast<const float4 *>(states + (vp * kN + j) * kN + i0);
         d[n] = (dsum[vp * kN + j] + dsum[(np + vp) * kN + j]) + (dsum[(2 * np + vp) * kN + j] + dsum[(3 * np + vp) * kN + j]);
@@ -763,65 +781,77 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__r
         load4(s0 + ((row * H + h) * kN + j) * kN + i0, S);
     }
 #pragma unroll
-    for (int n = 0; n < P; ++n) {
+    for (int n = 0; n < kMost; ++n) {
+        if (n >= P) break;
         const float dd = exp2_fast(-d[n]);
         *reinterpret_cast<float4 *>(states + (pair_of_step(n) * kN + j) * kN + i0) = make_float4(S[0], S[1], S[2], S[3]);
         S[0] = fmaf(S[0], dd, x[n].x); S[1] = fmaf(S[1], dd, x[n].y); S[2] = fmaf(S[2], dd, x[n].z); S[3] = fmaf(S[3], dd, x[n].w);
     }
     if (sT) store4(sT + (((int64_t)b * H + h) * kN + j) * kN + i0, S[0], S[1], S[2], S[3]);
-    if (sT32) store4(sT32 + (((int64_t)b * H + h) * kN + j) * kN + i0, S[0], S[1], S[2], S[3]);
 }
 template <typename Ts, bool kReverse>
 static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, const Ts *s0, const int64_t *map,
-                               const float *dsum, float *states, Ts *sT, float *sT32 = nullptr)
+                               const float *dsum, float *states, Ts *sT)
 {
     const dim3 grid((unsigned)(B * H * 4)), block(256);
-    switch (P) {
-    case 2: hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, 2>), grid, block, 0, st, (int)H, s0, map, dsum, states, sT, sT32); break;
-    case 4: hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, 4>), grid, block, 0, st, (int)H, s0, map, dsum, states, sT, sT32); break;
-    case 8: hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, 8>), grid, block, 0, st, (int)H, s0, map, dsum, states, sT, sT32); break;
-    case 16: hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, 16>), grid, block, 0, st, (int)H, s0, map, dsum, states, sT, sT32); break;
-    default: return hipErrorInvalidValue;
-    }
+    if (P < 2 || P > kMostSegments) return hipErrorInvalidValue;
+    auto run = [&](auto most) {
+        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, decltype(most)::value>), grid, block, 0, st, (int)H, P, s0, map, dsum, states, sT);
+    };
+    if (P <= 4) run(std::integral_constant<int, 4>{});
+    else if (P <= 8) run(std::integral_constant<int, 8>{});
+    else run(std::integral_constant<int, kMostSegments>{});
     return hipGetLastError();
 }
 
-// Number of segments for this shape (1 = not worth it / not possible) and their length: the pairs
-// times the segments should still fit the chip once, a segment is a whole number of chunks and at
-// least four of them.  A single sequence need not divide evenly: what is left over behind the P
-// segments (less than P chunks) follows as an ordinary pass from the state the segments end in.
-// (With B > 1 the first P * L tokens of every batch row are not one contiguous (B*P, L, C) tensor.)
+// Segments of a sequence of T tokens when `pairs` (batch, head) pairs share the chip: as many as still fit it once, each a
+// whole number of chunks and at least `least` of them; the last one ends with the sequence.  (Segments that had to
+// divide the sequence left training at all other lengths to one workgroup per pair; a prompt's tokens behind its equal
+// segments took a pass of their own.  Forward and backward at H32: B1 T8191 771 -> 193 us, B1 T2049 211 -> 93, B4 T4001
+// 427 -> 338; H8 B1 T5003 475 -> 110; prompts of H32: T1337 38 -> 24.5 us, T1024 37 -> 23 (six segments of three chunks
+// instead of four of four), T3000 with the output stage 57 -> 37.)
+static int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
+    const int64_t chunks = (T + CL - 1) / CL, fit = compute_units() / pairs;
+    const int64_t most = fit < kMostSegments ? fit : kMostSegments;
+    if (most < 2) return 1;
+    int64_t n = (chunks + most - 1) / most;
+    if (n < least) n = least;
+    *L = n * CL;
+    return (int)((chunks + n - 1) / n);
+}
+static RowCut cut_of(int P, int64_t L, int64_t T) {
+    RowCut c;
+    if (P * L != T) { c.segments = P; c.total = T; }
+    return c;
+}
+
 static int forward_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
-    const int64_t pairs = B * H, cus = compute_units();
     // (two passes over T / P tokens and two more launches against one pass over T: nothing to gain
     // below four segments or on short sequences)
     if (T < 1024) return 1;
-    for (int P = 16; P >= 4; P >>= 1) {
-        const int64_t l = T / P / CL * CL;
-        if (pairs * P > cus || l < 4 * CL) continue;
-        if (P * l != T && B != 1) continue;
-        *L = l;
-        return P;
+    if (B == 1) {
+        const int P = plan_segments(H, T, 3, L);
+        return P >= 4 ? P : 1;
     }
+    // (the interface promises segments to batches whose length divides evenly, and no workspace to others)
+    for (int P = kMostSegments; P >= 4; P >>= 1)
+        if (B * H * P <= compute_units() && T % (P * CL) == 0 && T / P >= 4 * CL) {
+            *L = T / P;
+            return P;
+        }
     return 1;
 }
 int chunk_forward_segments(int64_t B, int64_t T, int64_t H) {
     int64_t L;
     return forward_segments_plan(B, T, H, &L);
 }
-int64_t chunk_forward_segments_remainder(int64_t B, int64_t T, int64_t H) {
-    int64_t L = 0;
-    const int P = forward_segments_plan(B, T, H, &L);
-    return P <= 1 ? 0 : T - P * L;
-}
 size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H) {
     const int P = chunk_forward_segments(B, T, H);
-    // per segment and pair a state and the decay exponents; per pair the state the segments end in
-    return P <= 1 ? 0 : ((size_t)(B * P * H) * (kN * kN + 4 * kN) + (size_t)(B * H) * kN * kN) * sizeof(float);
+    // per segment and pair a state and the decay exponents
+    return P <= 1 ? 0 : (size_t)(B * P * H) * (kN * kN + 4 * kN) * sizeof(float);
 }
 
-// A remainder needs fp32 states at the boundary or no final state (see the API layer's check).
-// With `gate` the passes that produce output run the fused output stage (y = out then).
+// With `gate` the second pass runs the fused output stage (y = out then).
 hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                       const void *r, const void *k, const void *v, const void *w, const void *u,
                                       const void *s0, const int64_t *map, void *y, void *sT, void *workspace,
@@ -829,23 +859,16 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
 {
     int64_t L = 0;
     const int P = forward_segments_plan(B, T, H, &L);
-    const int64_t rows = B * P, rem = T - P * L;
-    float *states = (float *)workspace, *dsum = states + rows * H * kN * kN, *mid = dsum + rows * H * 4 * kN;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, dsum);
+    const int64_t rows = B * P;
+    const RowCut cut = cut_of(P, L, T);
+    float *states = (float *)workspace, *dsum = states + rows * H * kN * kN;
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, dsum, false, true, cut);
     if (e != hipSuccess) return e;
-    void *end_state = rem ? nullptr : sT;   // with a remainder the segments end in `mid`
-    e = state_dtype == kF32 ? launch_chain<float, false>(st, P, B, H, (const float *)s0, map, dsum, states, (float *)end_state, rem ? mid : nullptr)
-                            : launch_chain<bf16_t, false>(st, P, B, H, (const bf16_t *)s0, map, dsum, states, (bf16_t *)end_state, rem ? mid : nullptr);
+    e = state_dtype == kF32 ? launch_chain<float, false>(st, P, B, H, (const float *)s0, map, dsum, states, (float *)sT)
+                            : launch_chain<bf16_t, false>(st, P, B, H, (const bf16_t *)s0, map, dsum, states, (bf16_t *)sT);
     if (e != hipSuccess) return e;
-    e = gate ? chunk_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr)
-             : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, y, nullptr, nullptr);
-    if (e != hipSuccess || rem == 0) return e;
-    const int64_t off = P * L * H * kN;   // (B == 1) elements in front of the remainder
-    auto at = [&](const void *p) { return (const void *)((const bf16_t *)p + off); };
-    if (gate)
-        return chunk_forward_fused(st, kF32, B, rem, H, at(r), at(k), at(v), at(w), u, mid, nullptr, at(gate), gn_scale, gn_offset, gn_eps,
-                                   (bf16_t *)y + off, sT);
-    return chunk_forward(st, kF32, B, rem, H, at(r), at(k), at(v), at(w), u, mid, nullptr, (bf16_t *)y + off, sT, nullptr);
+    return gate ? chunk_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr, cut)
+                : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, y, nullptr, nullptr, nullptr, false, true, cut);
 }
 
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
@@ -861,18 +884,22 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 // keeps every segment's incoming state and decay exponents for the backward, whose reverse state
 // is chained the same way (see chunk_backward_saved_segments).
 // ------------------------------------------------------------------------------------------
-int chunk_train_segments(int64_t B, int64_t T, int64_t H) {
-    const int64_t pairs = B * H, cus = compute_units();
+static int train_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
     // (two state-only passes at 0.7 of a forward each on top of the forward and the backward: 1.5
     // times the work on P times the workgroups, and three small kernels)
     if (T < 1024) return 1;
-    for (int P = 16; P >= 2; P >>= 1)
-        if (pairs * P <= cus && T % (P * CL) == 0 && T / P >= 4 * CL && (T >= 2048 || P >= 4)) return P;
-    return 1;
+    const int P = plan_segments(B * H, T, 4, L);
+    return T >= 2048 || P >= 4 ? P : 1;
+}
+int chunk_train_segments(int64_t B, int64_t T, int64_t H) {
+    int64_t L;
+    return train_segments_plan(B, T, H, &L);
 }
 TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra) {
     TrainSegments s;
-    s.P = chunk_train_segments(B, T, H);
+    s.L = T;
+    s.P = train_segments_plan(B, T, H, &s.L);
+    s.cut = cut_of(s.P, s.L, T);
     const size_t pairs = (size_t)(B * s.P * H);
     s.states = reinterpret_cast<float *>(extra);
     s.dsum = s.states + pairs * kN * kN;
@@ -887,26 +914,26 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
                                        void *y, void *saved, void *extra)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
-    const int64_t L = T / s.P, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum);
+    const int64_t L = s.L, rows = B * s.P;
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = launch_chain<float, false>(st, s.P, B, H, nullptr, nullptr, s.dsum, s.states, nullptr)) != hipSuccess) return e;
-    return chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, y, nullptr, saved);
+    return chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, y, nullptr, saved, nullptr, false, true, s.cut);
 }
 
 // The same with the fused output stage in the second pass.  out, y, gate and the statistics are indexed by
-// token, and the tokens of the (B*P, T/P) rows are those of the (B, T) rows in the same order.
+// token, and the tokens of the B*P rows are those of the (B, T) rows in the same order.
 hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                              const void *r, const void *k, const void *v, const void *w, const void *u,
                                              const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
                                              void *out, void *y, float *stats, void *saved, void *extra)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
-    const int64_t L = T / s.P, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum);
+    const int64_t L = s.L, rows = B * s.P;
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = launch_chain<float, false>(st, s.P, B, H, nullptr, nullptr, s.dsum, s.states, nullptr)) != hipSuccess) return e;
-    return fused_save_from(st, rows, L, H, r, k, v, w, u, s.states, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved);
+    return fused_save_from(st, rows, L, H, r, k, v, w, u, s.states, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, s.cut);
 }
 
 }  // namespace wkv6

@@ -63,13 +63,38 @@ hipError_t scan_backward_state(hipStream_t st, int dtype, int64_t B, int64_t T, 
                                const float *s0, const void *gy, const float *gsT,
                                void *gr, void *gk, void *gv, void *gw, void *gu, float *gs0, void *workspace);
 
+// Time segments as rows of a (B * segments, L, C) view.  Segments that do not divide the sequence evenly start at
+// (row / segments) * total + (row % segments) * L and the last one of a sequence ends with it: `total` tokens,
+// `segments` per sequence.  Zero segments: the rows are sequences of their own (or the segments divide evenly, which
+// is the same thing).
+struct RowCut {
+    int segments = 0;
+    int64_t total = 0;
+};
+// What a workgroup of one row makes of it at its start: its own number of tokens and the tokens its pointers move by, so that
+// everything behind addresses row `row` of `tokens` tokens as ever (all of the workgroup's pairs lie in this row).
+struct RowView {
+    int tokens;
+    int64_t shift;
+};
+__device__ __forceinline__ RowView row_view(const RowCut &cut, int row, int L) {
+    const int b = row / cut.segments, s = row - b * cut.segments;
+    const int64_t first = (int64_t)s * L, left = cut.total - first;
+    const int tokens = left < L ? (int)left : L;
+    return {tokens, b * cut.total + first - (int64_t)row * tokens};
+}
+template <typename P> __device__ __forceinline__ void move_rows(P *&p, int64_t elements) {
+    if (p) p += elements;
+}
+
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states,
                          float *dsum = nullptr,    // dsum: see chunk_forward_segments_run
-                         bool reverse = false,     // the time axis read back to front (T a multiple of 64, no y)
-                         bool counters = true);    // saved_states ends with the per-head counters of the fused gu sum (zeroed here)
+                         bool reverse = false,     // the time axis read back to front (no y)
+                         bool counters = true,     // saved_states ends with the per-head counters of the fused gu sum (zeroed here)
+                         RowCut cut = RowCut());
 
 // --- block form (wkv6_block_fwd.hip, wkv6_block_bwd.hip): a 64-token chunk as one block of the
 // recurrence; bf16 tensors, T a multiple of 64, between half a pair and one pair per compute unit.
@@ -79,20 +104,20 @@ int64_t block_grid(int64_t B, int64_t H);
 bool block_forward_applies(int64_t B, int64_t T, int64_t H);
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters);
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut = RowCut());
 
 // the block-form forward with the layer's output stage fused in (see chunk_forward_fused / chunk_forward_fused_save):
 // y and stats may be null (inference), saved_states null without a backward to follow
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                               void *out, void *y, float *stats, void *sT, void *saved_states);
+                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut = RowCut());
 bool block_backward_applies(int64_t B, int64_t T, int64_t H);
 // workspace: the chunk-start states as a forward pass leaves them, followed by the per-head counters; gu_sum may be null
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
-                          const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr);
+                          const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr, RowCut cut = RowCut());
 
 // --- full-precision chunk form (wkv6_chunk32_fwd.hip, wkv6_chunk32_bwd.hip): fp32 and fp16 tensors on the
 // fp32 matrix instructions, chunks of 32 tokens, fp32 states; any T (the last chunk may be short).
@@ -123,7 +148,6 @@ hipError_t chunk_forward_save_f16(hipStream_t st, int64_t B, int64_t T, int64_t 
 // Few pairs, long sequence: the forward as P time segments side by side (two passes joined by the
 // affine map of a segment's state).  chunk_forward_segments = P for the shape (1 = does not apply).
 int chunk_forward_segments(int64_t B, int64_t T, int64_t H);
-int64_t chunk_forward_segments_remainder(int64_t B, int64_t T, int64_t H);   // tokens behind the P equal segments (single sequence only)
 size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H);
 hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                       const void *r, const void *k, const void *v, const void *w, const void *u,
@@ -136,6 +160,8 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
 // exponents; the backward chains its reverse state through the same affine maps (two passes each).
 struct TrainSegments {
     int P;              // segments per sequence (1: does not apply)
+    int64_t L;          // tokens of a segment (the last one of a sequence may be shorter)
+    RowCut cut;         // how the kernels find them
     float *states;      // [B*P][H][64][64] state entering each segment
     float *dsum;        // decay exponents of each segment (as chunk_forward leaves them)
     float *gstates;     // [B*P][H][64][64] gradient arriving at the end of each segment
@@ -167,7 +193,7 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
 hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale,
-                               const float *gn_offset, float gn_eps, void *out, void *sT);
+                               const float *gn_offset, float gn_eps, void *out, void *sT, RowCut cut = RowCut());
 
 // The same for training: also writes y (bf16), the norm's statistics (B,T,H,2: mean, rstd) and the chunk states
 hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -218,7 +244,7 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, bool states_ready,
                           void *gu_sum, const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr,
-                          int in_dtype = kBF16, const void *v_orig = nullptr, const void *gy_orig = nullptr);
+                          int in_dtype = kBF16, const void *v_orig = nullptr, const void *gy_orig = nullptr, RowCut cut = RowCut());
 // s0 / gsT / gs0: gradients through the state, as in scan_backward_state (with states_ready = false)
 // in_dtype kF16 (needs states_ready): r, k, w, u fp16, v and gy their bf16 copies, v_orig / gy_orig the
 // caller's fp16 v and fp32 gy, gradients fp32

@@ -832,6 +832,47 @@ def test_training_pair_in_time_segments(op, oracle, B, T, H, P):
     assert float(gw[:, 0].abs().max()) == 0.0 and float(gw[:, -1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("B,T,H,P", [(1, 1025, 2, 5), (2, 1279, 3, 5), (1, 2049, 40, 6), (3, 2111, 3, 9), (1, 4095, 32, 8), (5, 2050, 13, 3)])
+def test_training_pair_in_time_segments_of_any_length(op, oracle, B, T, H, P):
+    """Lengths the segments do not divide: the last segment of every sequence is shorter (of one token, of a whole
+    number of chunks less one token, ...), in the tile form and (a full chip) the block form."""
+    from rwkv_kernel import _native
+
+    lib = _native.load()
+    states = B * P * H * 2 * 64 * 64 * 4
+    assert lib.wkv6_saved_bytes(_native.BF16, CHUNK, B, T, H * 64, H) >= B * H * ((T + 63) // 64) * 64 * 64 * 4 + states
+    _, grads = _case(op, oracle, B, T, H, 190 + H, torch.bfloat16, CHUNK)
+    gw = grads[3]
+    assert float(gw[:, 0].abs().max()) == 0.0 and float(gw[:, -1].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("B,T,H,wild", [(1, 2049, 2, True), (2, 1500, 3, False), (1, 2100, 32, False), (2, 1999, 20, True)])
+def test_segments_of_any_length_through_the_other_calls(op, oracle, B, T, H, wild):
+    _state_grad_case(op, oracle, B, T, H, 290 + H, torch.bfloat16, CHUNK, wild=wild)
+    _fused_training_case(op, oracle, B, T, H, 390 + H, wild=wild)
+
+
+@pytest.mark.parametrize("T,H,sdt", [(1025, 3, torch.bfloat16), (1337, 32, torch.float32), (1535, 20, torch.float32), (1601, 50, torch.float32)])
+def test_prompt_in_time_segments_of_any_length(op, oracle, T, H, sdt):
+    N = 64
+    ins = oracle.make_inputs(1, T, H, N, 61, with_state=True)
+    ins[3][0, T - 9:T - 1, 20:40] = 6.0        # the short last segment's first head is redone exactly
+    dev, ref = cast_inputs(ins[:5], torch.bfloat16)
+    s_dev, s_ref = cast_inputs([ins[6][:1]], sdt)
+    g = torch.Generator().manual_seed(5)
+    gate_dev, gate_ref = cast_inputs([torch.randn(1, T, H * N, generator=g)], torch.bfloat16)
+    scale, offset = torch.rand(H, N, generator=g) + 0.5, torch.randn(H, N, generator=g) * 0.3
+    op.algo = CHUNK
+    y, sT = op(*dev, return_state=True, init_state=s_dev[0])
+    out, oT = op.forward_gn_gate(*dev, gate_dev[0], scale.cuda(), offset.cuda(), return_state=True, init_state=s_dev[0])
+    torch.cuda.synchronize()
+    y_ref, sT_ref = oracle.forward_c(*ref, N, s_ref[0])
+    check_close("y", y, y_ref, torch.bfloat16)
+    check_close("sT", sT, sT_ref, torch.bfloat16)
+    check_close("sT fused", oT, sT_ref, torch.bfloat16)
+    check_close("out", out, oracle.group_norm_gate_np(y_ref, gate_ref[0], scale.numpy(), offset.numpy(), N), torch.bfloat16)
+
+
 def test_training_pair_in_time_segments_with_fallback_segments(op, oracle):
     # segments whose decay the tile scaling cannot represent are redone by the exact per-timestep
     # code in every pass (forward passes, both backward passes); decay exactly 0 and exactly 1
