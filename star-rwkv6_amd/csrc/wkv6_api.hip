@@ -198,6 +198,7 @@ int wkv6_forward_gn_gate_ex(void *stream, int dtype, int state_dtype,
 
 static int train_segments(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);
 static size_t saved_base_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);
+static int train_segments32(int dtype, int algo, int64_t B, int64_t T, int64_t H);
 
 int wkv6_forward_gn_gate_save_supported(int dtype, int64_t B, int64_t T, int64_t C, int64_t H) {
     return check_shape(dtype, B, T, C, H) == WKV6_OK && dtype == WKV6_BF16 && chunk_possible(dtype, T, C);
@@ -348,6 +349,12 @@ static int train_segments(int dtype, int algo, int64_t B, int64_t T, int64_t C, 
     return chunk ? wkv6::chunk_train_segments(B, T, H) : 1;
 }
 
+// ... of fp32 and fp16 tensors on the full-precision chunk form
+static int train_segments32(int dtype, int algo, int64_t B, int64_t T, int64_t H) {
+    int64_t L;
+    return train_chunk32(dtype, algo, B, T, H) ? wkv6::chunk32_train_segments(B, T, H, &L) : 1;
+}
+
 // fp16 training pair: the bf16 copies of v and gy sit behind the base part of the saved block
 static size_t f16_stage_offset(int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
     const size_t ws = wkv6::scan_backward_workspace_bytes(B, T, C), cw = wkv6::chunk_backward_workspace_bytes(B, T, H),
@@ -359,6 +366,7 @@ static size_t f16_stage_offset(int algo, int64_t B, int64_t T, int64_t C, int64_
 
 size_t wkv6_saved_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
     if (check_shape(dtype, B, T, C, H) != WKV6_OK) return 0;
+    if (train_segments32(dtype, algo, B, T, H) > 1) return wkv6::chunk32_segments_layout(B, T, H, nullptr).bytes;
     if (train_chunk32(dtype, algo, B, T, H)) return wkv6_backward_workspace_bytes_ex(dtype, algo, B, T, C, H);
     if (dtype == WKV6_F16)
         return train_chunk(dtype, algo, T, C) ? f16_stage_offset(algo, B, T, C, H) + 2 * (size_t)(B * T * C) * 2 : 0;
@@ -385,6 +393,12 @@ int wkv6_forward_save(void *stream, int dtype, int algo, int64_t B, int64_t T, i
         hipError_t e = wkv6::convert_to_bf16((hipStream_t)stream, wkv6::kF16, v, v_bf16, B * T * C);
         if (e != hipSuccess) return finish(e);
         return finish(wkv6::chunk_forward_save_f16((hipStream_t)stream, B, T, H, r, k, v, v_bf16, w, u, y, saved));
+    }
+    if (need > 0 && train_segments32(dtype, algo, B, T, H) > 1) {
+        if (!r || !k || !v || !w || !u || !y) return WKV6_ERR_ARG;
+        if (algo < WKV6_ALGO_AUTO || algo > WKV6_ALGO_CHUNK) return WKV6_ERR_ARG;
+        if (!aligned16(r) || !aligned16(k) || !aligned16(v) || !aligned16(w) || !aligned16(y)) return WKV6_ERR_ARG;
+        return finish(wkv6::chunk32_forward_save_segments((hipStream_t)stream, dtype, B, T, H, r, k, v, w, u, y, saved));
     }
     if (need > 0 && train_segments(dtype, algo, B, T, C, H) > 1) {
         // few pairs, long sequence: time segments side by side
@@ -490,7 +504,12 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
             rc = finish(wkv6::chunk32_forward(st, dtype, WKV6_F32, B, T, H, r, k, v, w, u, nullptr, nullptr, nullptr, nullptr, workspace));
             if (rc != WKV6_OK) return rc;
         }
-        rc = finish(wkv6::chunk32_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+        if (states_ready && train_segments32(dtype, algo, B, T, H) > 1) {
+            if (workspace_bytes < wkv6_saved_bytes(dtype, algo, B, T, C, H)) return WKV6_ERR_WORKSPACE;
+            rc = finish(wkv6::chunk32_backward_saved_segments(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+        } else {
+            rc = finish(wkv6::chunk32_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+        }
         if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
         return rc;
     }

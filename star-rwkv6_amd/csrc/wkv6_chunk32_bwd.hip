@@ -59,16 +59,30 @@ struct C32BwdArgs {
     // the final state, the final state itself (read where gsT is given: E_T = sum_j S_T o gsT), dL/dS_0 (out)
     const float *s0, *gsT, *sT;
     float *gs0;
+    int slice;      // chunks of a pair's slice of `saved` (those of the longest row)
+    RowCut cut;     // rows that are time segments
 };
 
-template <typename Tin, typename Tout>
-__global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
+// kOnlyG: only the reverse state is wanted (gs0): the value waves update it, everything else is left out.  (A pair that is
+// redone per timestep writes its gradients too, for the pass behind this one to write again.)
+template <typename Tin, typename Tout, bool kOnlyG>
+__global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char c32_smem[];
     C32BwdLds &L = reinterpret_cast<C32BwdSmem *>(c32_smem)->chunk;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int T = a.T, H = a.H;
-    const int pair = blockIdx.x, b = pair / H, h = pair - b * H;
+    const int H = a.H, pair = blockIdx.x, b = pair / H, h = pair - b * H;
+    if (a.cut.segments) {
+        const RowView rv = row_view(a.cut, b, a.T);
+        const int64_t m = rv.shift * H * kN;
+        a.T = rv.tokens;
+        a.r = reinterpret_cast<const Tin *>(a.r) + m; a.k = reinterpret_cast<const Tin *>(a.k) + m;
+        a.v = reinterpret_cast<const Tin *>(a.v) + m; a.w = reinterpret_cast<const Tin *>(a.w) + m;
+        a.gy = reinterpret_cast<const Tout *>(a.gy) + m;
+        a.gr = reinterpret_cast<Tout *>(a.gr) + m; a.gk = reinterpret_cast<Tout *>(a.gk) + m;
+        a.gv = reinterpret_cast<Tout *>(a.gv) + m; a.gw = reinterpret_cast<Tout *>(a.gw) + m;
+    }
+    const int T = a.T;
     const int64_t C = (int64_t)H * kN;
     const int64_t base = (int64_t)b * T * C + (int64_t)h * kN;
     const int nchunk = (T + kC32 - 1) / kC32;
@@ -76,7 +90,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
     const Tin *v = reinterpret_cast<const Tin *>(a.v), *w = reinterpret_cast<const Tin *>(a.w);
     const Tin *u = reinterpret_cast<const Tin *>(a.u);
     const Tout *gy = reinterpret_cast<const Tout *>(a.gy);
-    float *const ck = a.saved + (int64_t)pair * nchunk * (kN * kN);
+    float *const ck = a.saved + (int64_t)pair * a.slice * (kN * kN);
     // step s handles chunk nchunk - 1 - s
 
     if (wave >= 8) {
@@ -93,7 +107,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
             for (int x = 0; x < 2; ++x) {
                 const int o = min(16 * x + t16, T - 1 - c * kC32) * (int)C + ch;   // rows past the end read the last one
-                n.r[x].load(r + row0 + o); n.k[x].load(k + row0 + o); n.v[x].load(v + row0 + o); n.w[x].load(w + row0 + o);
+                n.r[x].load(r + row0 + o); n.w[x].load(w + row0 + o);
+                if (!kOnlyG) { n.k[x].load(k + row0 + o); n.v[x].load(v + row0 + o); }
                 n.g[x].load(gy + row0 + o);
             }
         };
@@ -121,8 +136,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                 f32x4 rp, kp, fv, fg;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float fr = valid[x] ? n.r[x].at(e) : 0.f, fk = valid[x] ? n.k[x].at(e) : 0.f;
-                    fv[e] = valid[x] ? n.v[x].at(e) : 0.f;
+                    const float fr = valid[x] ? n.r[x].at(e) : 0.f, fk = !kOnlyG && valid[x] ? n.k[x].at(e) : 0.f;
+                    fv[e] = !kOnlyG && valid[x] ? n.v[x].at(e) : 0.f;
                     fg[e] = valid[x] ? n.g[x].at(e) : 0.f;
                     f1[x][e] = sc.rp[x][e];
                     f3[x][e] = sc.kp[x][e];
@@ -130,8 +145,12 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     kp[e] = fk * f3[x][e];
                     acc = fmaf(fr * fk, fu[e], acc);
                 }
-                acc = sum_rows4(acc);
                 *reinterpret_cast<f32x4 *>(&L.Rp[buf][t][ch]) = rp;
+                if (kOnlyG) {
+                    *reinterpret_cast<f32x4 *>(&L.GY[buf][t][ch]) = fg;
+                    continue;
+                }
+                acc = sum_rows4(acc);
                 *reinterpret_cast<f32x4 *>(&L.Kp[buf][t][ch]) = kp;
                 *reinterpret_cast<f32x4 *>(&L.V[buf][t][ch]) = fv;
                 *reinterpret_cast<f32x4 *>(&L.GY[buf][t][ch]) = fg;
@@ -163,7 +182,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
         // Phase 1 of step s: the rows of step s to LDS, the loads of step s + 2 issued into the registers that this frees.
         // Phase 2: the operands of step s + 1 formed and published (their loads are a step and a half old).
         auto step = [&](Set &now, Set &next, int s) {
-            rows(now, s);
+            if (!kOnlyG) rows(now, s);
             fetch(now, s + 2);
             __syncthreads();
             form(next, s + 1);
@@ -205,7 +224,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
             const int c = nchunk - 1 - s, buf = s & 1;
             const bool full = (c + 1) * kC32 <= T;
             // ---- phase 1: a tile of A (wave 0: (0,0), 1: (1,1), 2: (1,0)), K' G ----
-            if (q < 3) {
+            if (!kOnlyG && q < 3) {
                 const int tb = q == 0 ? 0 : 1, sb = q == 1 ? 1 : 0;
                 f32x4 at = zero;
 #pragma unroll
@@ -227,7 +246,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
             }
             f32x4 gvt[2] = {zero, zero};
 #pragma unroll
-            for (int sb = 0; sb < 2; ++sb)
+            for (int sb = 0; !kOnlyG && sb < 2; ++sb)
 #pragma unroll
                 for (int ib = 0; ib < 4; ++ib) {
                     const f32x4 fk = *reinterpret_cast<const f32x4 *>(&L.Kp[buf][16 * sb + n][16 * ib + 4 * g]);
@@ -241,7 +260,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) gyb[x][e] = L.GY[buf][16 * x + 4 * g + e][col];
 #pragma unroll
-            for (int sb = 0; sb < 2; ++sb)
+            for (int sb = 0; !kOnlyG && sb < 2; ++sb)
 #pragma unroll
                 for (int tb = sb; tb < 2; ++tb) {
                     f32x4 fat;
@@ -249,7 +268,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     for (int e = 0; e < 4; ++e) fat[e] = L.A[16 * tb + 4 * g + e][16 * sb + n];
                     gvt[sb] = mfma16(gyb[tb], fat, gvt[sb]);
                 }
-            {
+            if (!kOnlyG) {
                 Tout *const out = gv + base + (int64_t)c * kC32 * C;   // (uniform; the lane's part of the address is lane_off)
                 const int left = T - c * kC32 - n;                     // (token 16 x + n exists: 16 x < left)
 #pragma unroll
@@ -267,7 +286,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
                     G[ib] = mfma16(fra, gyb[tb], G[ib]);
                 }
             }
-            publish();
+            if (!kOnlyG) publish();
             __syncthreads();
         }
         if (a.gs0) {   // what is left after the first chunk is dL/dS_0
@@ -277,6 +296,9 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) p[(16 * ib + 4 * g + e) * kN] = G[ib][e];
         }
+    } else if (kOnlyG) {
+        __syncthreads();   // (the barriers of the others)
+        for (int s = 0; s < nchunk; ++s) { __syncthreads(); __syncthreads(); }
     } else {
         // ---------------- key waves ----------------
         const int q = wave - 4, n = lane & 15, g = lane >> 4, col = 16 * q + n;
@@ -459,29 +481,49 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(const C32BwdArgs a)
     }
 }
 
-template <typename Tin, typename Tout>
+template <typename Tin, typename Tout, bool kOnlyG = false>
 static hipError_t launch(hipStream_t st, int64_t B, const C32BwdArgs &a) {
     constexpr int lds = (int)sizeof(C32BwdSmem);
-    const hipError_t e = allow_dynamic_lds<chunk32_bwd_kernel<Tin, Tout>>(lds);
+    const hipError_t e = allow_dynamic_lds<chunk32_bwd_kernel<Tin, Tout, kOnlyG>>(lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((chunk32_bwd_kernel<Tin, Tout>), dim3((unsigned)(B * a.H)), dim3(768), lds, st, a);
+    hipLaunchKernelGGL((chunk32_bwd_kernel<Tin, Tout, kOnlyG>), dim3((unsigned)(B * a.H)), dim3(768), lds, st, a);
     return hipGetLastError();
 }
 
 hipError_t chunk32_backward(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
                             const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                             void *gr, void *gk, void *gv, void *gw, void *gu, void *saved_states,
-                            const float *s0, const float *gsT, const float *sT, float *gs0)
+                            const float *s0, const float *gsT, const float *sT, float *gs0, RowCut cut, bool only_gs0)
 {
     if (gsT != nullptr && sT == nullptr) return hipErrorInvalidValue;   // (the anchor of the decay gradient needs S_T)
     C32BwdArgs a;
+    a.cut = cut; a.slice = (int)((T + kC32 - 1) / kC32);
     a.s0 = s0; a.gsT = gsT; a.sT = sT; a.gs0 = gs0;
     a.T = (int)T; a.H = (int)H;
     a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.gy = gy;
     a.gr = gr; a.gk = gk; a.gv = gv; a.gw = gw; a.gu = gu;
     a.saved = reinterpret_cast<float *>(saved_states);
+    if (only_gs0) return dtype == kF32 ? launch<float, float, true>(st, B, a) : launch<f16_t, float, true>(st, B, a);
     if (dtype == kF32) return launch<float, float>(st, B, a);
     return launch<f16_t, float>(st, B, a);
+}
+
+hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+                                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
+                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *saved)
+{
+    const C32Segments s = chunk32_segments_layout(B, T, H, saved);
+    const int64_t rows = B * s.P;
+    // what each segment alone sends back into its incoming state; the chain backwards in time; every segment between its
+    // true incoming state and its true arriving gradient
+    hipError_t e = chunk32_backward(st, dtype, rows, s.L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, s.chunks,
+                                    s.states, nullptr, nullptr, s.gstates, s.cut, true);
+    if (e != hipSuccess) return e;
+    if ((e = segment_chain_factors(st, s.P, B, H, s.decay, s.gstates, true)) != hipSuccess) return e;
+    e = chunk32_backward(st, dtype, rows, s.L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, s.chunks,
+                         s.states, s.gstates, s.ends, nullptr, s.cut);
+    if (e != hipSuccess) return e;
+    return segments_finish<float>(st, s.P, B, T, H, s.gu_rows, (float *)gu, (float *)gw, true, true);
 }
 
 }  // namespace wkv6

@@ -47,17 +47,28 @@ struct C32FwdArgs {
     const int64_t *map;
     void *y, *sT;
     float *saved;   // [pair][chunk][4096] chunk-start states in fragment order (null: not kept)
+    int slice;      // chunks of a pair's slice of `saved` (those of the longest row)
+    RowCut cut;     // rows that are time segments
+    float *decay;   // null, or (states only) [2][pair][64]: the decay of the whole row, as the product of the two loading groups' chunks
 };
 
 // kOut = false: only the states (chunk states and / or the final one): no y, no R-side operands
 template <typename Tin, typename Tout, typename Ts, int kGroups, bool kOut>
-__global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(const C32FwdArgs a)
+__global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32FwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char c32_smem[];
     C32FwdLds &L = reinterpret_cast<C32FwdSmem *>(c32_smem)->chunk;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int T = a.T, H = a.H;
-    const int pair = blockIdx.x, b = pair / H, h = pair - b * H;
+    const int H = a.H, pair = blockIdx.x, b = pair / H, h = pair - b * H;
+    if (a.cut.segments) {
+        const RowView rv = row_view(a.cut, b, a.T);
+        const int64_t m = rv.shift * H * kN;
+        a.T = rv.tokens;
+        a.r = reinterpret_cast<const Tin *>(a.r) + m; a.k = reinterpret_cast<const Tin *>(a.k) + m;
+        a.v = reinterpret_cast<const Tin *>(a.v) + m; a.w = reinterpret_cast<const Tin *>(a.w) + m;
+        if (a.y) a.y = reinterpret_cast<Tout *>(a.y) + m;
+    }
+    const int T = a.T;
     const int64_t C = (int64_t)H * kN;
     const int64_t base = (int64_t)b * T * C + (int64_t)h * kN;
     const int nchunk = (T + kC32 - 1) / kC32;
@@ -83,6 +94,7 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(const 
         // the chunk whose operands are formed: two channels of the lane's four at a time (a barrier in between)
         float op_r[2][4], op_k[2][4], op_v[2][4], hm_r[2][4], hm_k[2][4], e_all[4], part[2];
         bool wild = false;
+        float decay[4] = {1.f, 1.f, 1.f, 1.f};   // of the group's chunks
         auto form = [&](auto half, int c) {
             constexpr int E0 = 2 * decltype(half)::value;
             const bool valid[2] = {c * kC32 + t16 < T, c * kC32 + 16 + t16 < T};
@@ -109,6 +121,7 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(const 
                     }
                     op_v[x][e] = valid[x] ? nv[x].at(e) : 0.f;
                     e_all[e] = sc.all[e];
+                    if (!kOut && x == 0) decay[e] *= sc.all[e];
                     s = fmaf(fr * fk, fu[e], s);
                 }
                 if (kOut) part[x] = E0 == 0 ? s : sum_rows4(s);
@@ -182,6 +195,8 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(const 
         }
         const bool any = __any(wild);
         if (lane == 0) L.wild[wave - 4] = any;
+        if (!kOut && a.decay && t16 == 0)
+            *reinterpret_cast<f32x4 *>(a.decay + ((int64_t)grp * gridDim.x + pair) * kN + ch) = (f32x4){decay[0], decay[1], decay[2], decay[3]};
     } else {
         // ---------------- computing waves ----------------
         const int q = wave, n = lane & 15, g = lane >> 4;
@@ -210,7 +225,7 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(const 
                 if (t < T) store4(y + base + (int64_t)t * C + ch, o[0], o[1], o[2], o[3]);
             }
         };
-        float *saved = a.saved ? a.saved + (int64_t)pair * nchunk * (kN * kN) + (q * 4) * 256 + lane * 4 : nullptr;
+        float *saved = a.saved ? a.saved + (int64_t)pair * a.slice * (kN * kN) + (q * 4) * 256 + lane * 4 : nullptr;
         __syncthreads();
         for (int c = 0; c < nchunk; ++c) {
             const int buf = c & 1;
@@ -318,16 +333,58 @@ static hipError_t launch(hipStream_t st, int64_t B, const C32FwdArgs &a) {
 
 hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B, int64_t T, int64_t H,
                            const void *r, const void *k, const void *v, const void *w, const void *u,
-                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states)
+                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, RowCut cut)
 {
     (void)state_dtype;   // fp32 and fp16 tensors keep fp32 states
     C32FwdArgs a;
+    a.cut = cut; a.decay = decay; a.slice = (int)((T + kC32 - 1) / kC32);
     a.T = (int)T; a.H = (int)H;
     a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.s0 = s0; a.map = map; a.y = y; a.sT = sT;
     a.saved = reinterpret_cast<float *>(saved_states);
     if (y == nullptr)
         return dtype == kF32 ? launch<float, float, float, false>(st, B, a) : launch<f16_t, float, float, false>(st, B, a);
     return dtype == kF32 ? launch<float, float, float, true>(st, B, a) : launch<f16_t, float, float, true>(st, B, a);
+}
+
+// ------------------------------------------------------------------------------------------
+// The training pair of a long sequence of few pairs in time segments, as in the bf16 forms (wkv6_chunk_fwd.hip): a
+// states-only pass over all segments at once, the chain, and the saving forward from every segment's true state.  The
+// decay of a segment is carried as the product of its chunks' e^{c_32} themselves, not as an exponent.
+// Without segments a pair's chunks follow each other in one workgroup whatever else is idle.  Forward and backward, before and
+// now: fp32 B1 T8191 H32 2317 -> 449 us, B2 T2048 H16 580 -> 129, B1 T1031 H64 307 -> 144, B2 T1024 H64 (128 pairs, not
+// taken by the rule: two segments only from 2048 tokens on) 310 -> 269 from the kernels alone; fp16 B1 T5003 H8 1420 -> 181, B4
+// T2100 H32 704 -> 520.
+// ------------------------------------------------------------------------------------------
+int chunk32_train_segments(int64_t B, int64_t T, int64_t H, int64_t *L) {
+    if (T < 1024) return 1;
+    const int P = plan_segments(B * H, T, 4, L);
+    return T >= 2048 || P >= 4 ? P : 1;
+}
+C32Segments chunk32_segments_layout(int64_t B, int64_t T, int64_t H, void *saved) {
+    C32Segments s;
+    s.L = T;
+    s.P = chunk32_train_segments(B, T, H, &s.L);
+    s.cut = cut_of(s.P, s.L, T);
+    const size_t pairs = (size_t)(B * s.P * H);
+    s.chunks = reinterpret_cast<float *>(saved);
+    s.states = s.chunks + chunk32_saved_bytes(B * s.P, s.L, H) / sizeof(float);
+    s.ends = s.states + pairs * kN * kN;
+    s.gstates = s.ends + pairs * kN * kN;
+    s.decay = s.gstates + pairs * kN * kN;
+    s.gu_rows = s.decay + 2 * pairs * kN;
+    s.bytes = reinterpret_cast<char *>(s.gu_rows + pairs * kN) - reinterpret_cast<char *>(s.chunks);
+    return s;
+}
+hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+                                         const void *r, const void *k, const void *v, const void *w, const void *u,
+                                         void *y, void *saved)
+{
+    const C32Segments s = chunk32_segments_layout(B, T, H, saved);
+    const int64_t rows = B * s.P;
+    hipError_t e = chunk32_forward(st, dtype, kF32, rows, s.L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, s.cut);
+    if (e != hipSuccess) return e;
+    if ((e = segment_chain_factors(st, s.P, B, H, s.decay, s.states, false)) != hipSuccess) return e;
+    return chunk32_forward(st, dtype, kF32, rows, s.L, H, r, k, v, w, u, s.states, nullptr, y, s.ends, s.chunks, nullptr, s.cut);
 }
 
 }  // namespace wkv6

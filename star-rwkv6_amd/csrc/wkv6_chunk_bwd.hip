@@ -742,8 +742,9 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
 // Training pair in time segments, last step: gu of a batch row = sum over its segments; the decay
 // gradient at the first and the last token of a sequence is zero by definition
 // (rwkv_kernels.cu:381,406), where the kernels, given explicit states, leave rounding residue.
-__global__ void segments_finish_kernel(int P, int64_t T, int C, const bf16_t *__restrict__ gu_rows,
-                                       bf16_t *__restrict__ gu, bf16_t *__restrict__ gw, bool zero_first, bool zero_last)
+template <typename E>
+__global__ void segments_finish_kernel(int P, int64_t T, int C, const E *__restrict__ gu_rows,
+                                       E *__restrict__ gu, E *__restrict__ gw, bool zero_first, bool zero_last)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
     if (c >= C) return;
@@ -753,6 +754,16 @@ __global__ void segments_finish_kernel(int P, int64_t T, int C, const bf16_t *__
     if (zero_first) store1(gw + (int64_t)b * T * C + c, 0.f);
     if (zero_last) store1(gw + ((int64_t)b * T + T - 1) * C + c, 0.f);
 }
+
+template <typename E>
+hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const E *gu_rows, E *gu, E *gw, bool zero_first, bool zero_last)
+{
+    const int C = (int)(H * kN);
+    hipLaunchKernelGGL(segments_finish_kernel<E>, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
+                       P, T, C, gu_rows, gu, gw, zero_first, zero_last);
+    return hipGetLastError();
+}
+template hipError_t segments_finish<float>(hipStream_t, int, int64_t, int64_t, int64_t, const float *, float *, float *, bool, bool);
 
 hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                          const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
@@ -772,10 +783,7 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, gu_sum,
                        s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
     if (e != hipSuccess) return e;
-    const int C = (int)(H * kN);
-    hipLaunchKernelGGL(segments_finish_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
-                       s.P, T, C, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, true, true);
-    return hipGetLastError();
+    return segments_finish(st, s.P, B, T, H, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, true, true);
 }
 
 // The same with an initial state, a gradient arriving at the final state and dL/dS_0 wanted
@@ -800,11 +808,8 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, nullptr,
                        s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
     if (e != hipSuccess) return e;
-    const int C = (int)(H * kN);
     // (the decay gradient at an end of the sequence is zero by definition only where no state / no gradient comes in)
-    hipLaunchKernelGGL(segments_finish_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
-                       s.P, T, C, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, s0 == nullptr, gsT == nullptr);
-    return hipGetLastError();
+    return segments_finish(st, s.P, B, T, H, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, s0 == nullptr, gsT == nullptr);
 }
 
 }  // namespace wkv6

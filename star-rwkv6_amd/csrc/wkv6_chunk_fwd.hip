@@ -753,7 +753,8 @@ constexpr int kMostSegments = 16;
 // kReverse: the same chain walked from the last segment to the first, which is what the reverse
 // state of the backward pass obeys (the gradient arriving at the end of segment p is what segment
 // p + 1 sends into its incoming state: its own contribution plus D_{p+1} times what arrives at its end).
-template <typename Ts, bool kReverse, int kMost>
+// kFactors: dsum holds two factors of each segment's decay, [2][pairs][64], instead of its exponent's four parts.
+template <typename Ts, bool kReverse, int kMost, bool kFactors>
 __global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
                                                             const float *__restrict__ dsum, float *__restrict__ states, Ts *__restrict__ sT)   // sT: the final state, or null
 {
@@ -773,7 +774,8 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const 
         if (n >= P) break;
         const int64_t vp = pair_of_step(n);
         x[n] = *reinterpret_cast<const float4 *>(states + (vp * kN + j) * kN + i0);
-        d[n] = (dsum[vp * kN + j] + dsum[(np + vp) * kN + j]) + (dsum[(2 * np + vp) * kN + j] + dsum[(3 * np + vp) * kN + j]);
+        if (kFactors) d[n] = dsum[vp * kN + j] * dsum[(np + vp) * kN + j];
+        else d[n] = (dsum[vp * kN + j] + dsum[(np + vp) * kN + j]) + (dsum[(2 * np + vp) * kN + j] + dsum[(3 * np + vp) * kN + j]);
     }
     float S[4] = {0.f, 0.f, 0.f, 0.f};
     if (s0) {
@@ -783,20 +785,20 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const 
 #pragma unroll
     for (int n = 0; n < kMost; ++n) {
         if (n >= P) break;
-        const float dd = exp2_fast(-d[n]);
+        const float dd = kFactors ? d[n] : exp2_fast(-d[n]);
         *reinterpret_cast<float4 *>(states + (pair_of_step(n) * kN + j) * kN + i0) = make_float4(S[0], S[1], S[2], S[3]);
         S[0] = fmaf(S[0], dd, x[n].x); S[1] = fmaf(S[1], dd, x[n].y); S[2] = fmaf(S[2], dd, x[n].z); S[3] = fmaf(S[3], dd, x[n].w);
     }
     if (sT) store4(sT + (((int64_t)b * H + h) * kN + j) * kN + i0, S[0], S[1], S[2], S[3]);
 }
-template <typename Ts, bool kReverse>
+template <typename Ts, bool kReverse, bool kFactors = false>
 static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, const Ts *s0, const int64_t *map,
                                const float *dsum, float *states, Ts *sT)
 {
     const dim3 grid((unsigned)(B * H * 4)), block(256);
     if (P < 2 || P > kMostSegments) return hipErrorInvalidValue;
     auto run = [&](auto most) {
-        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, decltype(most)::value>), grid, block, 0, st, (int)H, P, s0, map, dsum, states, sT);
+        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, decltype(most)::value, kFactors>), grid, block, 0, st, (int)H, P, s0, map, dsum, states, sT);
     };
     if (P <= 4) run(std::integral_constant<int, 4>{});
     else if (P <= 8) run(std::integral_constant<int, 8>{});
@@ -810,7 +812,7 @@ static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, cons
 // segments took a pass of their own.  Forward and backward at H32: B1 T8191 771 -> 193 us, B1 T2049 211 -> 93, B4 T4001
 // 427 -> 338; H8 B1 T5003 475 -> 110; prompts of H32: T1337 38 -> 24.5 us, T1024 37 -> 23 (six segments of three chunks
 // instead of four of four), T3000 with the output stage 57 -> 37.)
-static int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
+int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
     const int64_t chunks = (T + CL - 1) / CL, fit = compute_units() / pairs;
     const int64_t most = fit < kMostSegments ? fit : kMostSegments;
     if (most < 2) return 1;
@@ -819,7 +821,7 @@ static int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
     *L = n * CL;
     return (int)((chunks + n - 1) / n);
 }
-static RowCut cut_of(int P, int64_t L, int64_t T) {
+RowCut cut_of(int P, int64_t L, int64_t T) {
     RowCut c;
     if (P * L != T) { c.segments = P; c.total = T; }
     return c;
@@ -874,6 +876,10 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
                                  const float *arriving, float *leaving) {
     return launch_chain<float, true>(st, P, B, H, arriving, nullptr, dsum, states, leaving);
+}
+hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse) {
+    return reverse ? launch_chain<float, true, true>(st, P, B, H, nullptr, nullptr, decay, states, nullptr)
+                   : launch_chain<float, false, true>(st, P, B, H, nullptr, nullptr, decay, states, nullptr);
 }
 hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states, const float *s0) {
     return launch_chain<float, false>(st, P, B, H, s0, nullptr, dsum, states, nullptr);

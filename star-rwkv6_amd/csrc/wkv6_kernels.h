@@ -126,7 +126,9 @@ size_t chunk32_saved_bytes(int64_t B, int64_t T, int64_t H);   // one fp32 state
 // saved_states (may be null): receives the chunk-start states for chunk32_backward; y may be null then
 hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B, int64_t T, int64_t H,
                            const void *r, const void *k, const void *v, const void *w, const void *u,
-                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states);
+                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states,
+                           float *decay = nullptr,   // [2][pair][64]: two factors of each row's decay
+                           RowCut cut = RowCut());
 
 // saved_states: what chunk32_forward left (the pair's slice also serves the per-timestep pass of a pair
 // whose decay left the chunk form's reach); gu (B, C)
@@ -135,7 +137,28 @@ hipError_t chunk32_backward(hipStream_t st, int dtype, int64_t B, int64_t T, int
                             void *gr, void *gk, void *gv, void *gw, void *gu, void *saved_states,
                             // gradients through the state ((B,H,64,64) fp32 [key][value]; sT = the forward's final state,
                             // needed with gsT); the saved states come from a forward that started from s0
-                            const float *s0 = nullptr, const float *gsT = nullptr, const float *sT = nullptr, float *gs0 = nullptr);
+                            const float *s0 = nullptr, const float *gsT = nullptr, const float *sT = nullptr, float *gs0 = nullptr,
+                            RowCut cut = RowCut(), bool only_gs0 = false);   // only_gs0: nothing but gs0 is wanted
+
+// The training pair in time segments; what the forward leaves for the backward in `saved` (the first part as chunk32_forward).
+struct C32Segments {
+    int P;             // segments per sequence (1: does not apply)
+    int64_t L;         // tokens of a segment (the last one of a sequence may be shorter)
+    RowCut cut;
+    float *chunks;     // chunk states of the segments
+    float *states, *ends, *gstates;   // [B*P][H][64][64]: state entering and leaving each segment, gradient arriving at its end
+    float *decay;      // [2][B*P][H][64]
+    float *gu_rows;    // [B*P][C]
+    size_t bytes;
+};
+int chunk32_train_segments(int64_t B, int64_t T, int64_t H, int64_t *L);
+C32Segments chunk32_segments_layout(int64_t B, int64_t T, int64_t H, void *saved);
+hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+                                         const void *r, const void *k, const void *v, const void *w, const void *u,
+                                         void *y, void *saved);
+hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+                                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
+                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *saved);
 
 // fp16 tensors on the chunked kernels (training pair only: y and the gradients are fp32).  r, k, w stay
 // fp16 (the kernels unpack them exactly); v and gy are consumed as bf16 MFMA operands, so the caller
@@ -174,6 +197,12 @@ TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra
 // state, from s0 or zero; reverse: the gradient arriving at its end, from `arriving` or zero, and
 // `leaving` receives what leaves the first segment, dL/dS_0).
 hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states, const float *s0);
+// the same with the segments' decays as two factors each, [2][B*P][H][64]
+hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse);
+int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
+RowCut cut_of(int P, int64_t L, int64_t T);
+template <typename T>
+hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T_, int64_t H, const T *gu_rows, T *gu, T *gw, bool zero_first, bool zero_last);
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
 hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,

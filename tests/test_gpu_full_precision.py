@@ -91,6 +91,23 @@ def test_shapes_and_ragged_ends(op, oracle, dt, B, T, H):
     _case(op, oracle, B, T, H, 100 + T, DTYPES[dt])
 
 
+@pytest.mark.parametrize("dt", ["f32", "f16"])
+@pytest.mark.parametrize("B,T,H,P,wild", [(1, 1025, 2, 5, False), (2, 1279, 3, 5, True), (1, 2048, 32, 8, False), (3, 2111, 2, 9, True),
+                                          (5, 2050, 13, 3, False)])
+def test_training_pair_in_time_segments(op, lib, oracle, dt, B, T, H, P, wild):
+    """Few pairs, long sequence: the training pair runs as P segments per sequence, the last one of one token, one less
+    than a chunk, ...; with a pair that is redone per timestep inside a segment."""
+    code = 2 if dt == "f32" else 1
+    chunks = B * H * ((T + 31) // 32) * N * N * 4
+    assert lib.wkv6_saved_bytes(code, AUTO, B, T, H * N, H) >= chunks + B * P * H * 3 * N * N * 4
+
+    def edit(ins):
+        if wild:
+            ins[3][B - 1, T // 2:T // 2 + 20, 5:25] = 6.0
+            ins[3][0, 250:260] = -1e9      # decay 1 across a boundary of segments
+    _case(op, oracle, B, T, H, 700 + T, DTYPES[dt], edit)
+
+
 def test_more_pairs_than_compute_units(op, oracle):
     _case(op, oracle, 40, 96, 8, 7, torch.float32)
 
