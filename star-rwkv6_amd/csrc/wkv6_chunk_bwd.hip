@@ -331,8 +331,11 @@ __device__ __forceinline__ void bwd_consumer(const BwdArgs &a, unsigned char *sm
     if (GRP == 1 && g == 0) gu_lds[col] = gu_acc;
     __threadfence_block();
     __syncthreads();
-    if (GRP == 0 && g == 0 && !*s_wild)     // (the exact second pass writes gu itself)
-        store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + col, gu_acc + gu_lds[col]);
+    if (GRP == 0 && g == 0 && !*s_wild) {   // (the exact second pass writes gu itself)
+        gu_acc += gu_lds[col];
+        gu_lds[col] = gu_acc;               // for the fused batch sum, unrounded
+        store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + col, gu_acc);
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -651,7 +654,9 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
         __syncthreads();
         const int tid = threadIdx.x;
         if (tid < kN) {          // wave 0
-            const float part = load1(reinterpret_cast<const Tout *>(a.gu) + (int64_t)(pair0 / a.H) * C + h * kN + tid);
+            // (not the rounded row, where the chunked code has it: with time segments there are up to 16 rows a sequence)
+            const float part = s_wild[0] ? load1(reinterpret_cast<const Tout *>(a.gu) + (int64_t)(pair0 / a.H) * C + h * kN + tid)
+                                         : reinterpret_cast<const float *>(smem + BwdLds::kGu)[tid];
             __hip_atomic_store(a.ckpt + (int64_t)pair0 * slice + slice / 2 + tid, part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (tid == 0)

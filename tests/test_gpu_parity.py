@@ -873,6 +873,20 @@ def test_prompt_in_time_segments_of_any_length(op, oracle, T, H, sdt):
     check_close("out", out, oracle.group_norm_gate_np(y_ref, gate_ref[0], scale.numpy(), offset.numpy(), N), torch.bfloat16)
 
 
+def test_segments_add_up_the_bonus_gradient_unrounded(op, oracle):
+    # gu of a sequence in segments is rounded to bf16 once: half an ulp (2^-9 relative) of every value, no more but
+    # for the operands' own rounding, whose share falls with the 1031 tokens that are summed
+    B, T, H = 1, 1031, 4
+    ins = oracle.make_inputs(B, T, H, 64, 5)
+    for x in (ins[0], ins[1], ins[2], ins[5]):
+        x.abs_()                              # sums without cancellation: the operands' rounding averages out
+    dev, ref = cast_inputs(ins[:5], torch.bfloat16)
+    gy_dev, gy_ref = cast_inputs(ins[5:6], torch.bfloat16)
+    _, grads = _run_fwd_bwd(op, dev + gy_dev, CHUNK)
+    gu, want = to_np(grads[4]).reshape(H, 64), oracle.backward_c(*ref, gy_ref[0], 64)[4]
+    assert np.abs(gu / want - 1).max() <= 2.0 ** -8 * 1.1
+
+
 def test_training_pair_in_time_segments_with_fallback_segments(op, oracle):
     # segments whose decay the tile scaling cannot represent are redone by the exact per-timestep
     # code in every pass (forward passes, both backward passes); decay exactly 0 and exactly 1
