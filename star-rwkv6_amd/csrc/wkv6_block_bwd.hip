@@ -60,6 +60,7 @@ struct BlockBwdArgs {
     RowCut cut;       // rows that are time segments (!kMulti and kRagged)
     const bf16_t *r, *k, *v, *w, *u, *gy;
     bf16_t *gr, *gk, *gv, *gw, *gu;
+    float *gu_rows;   // null, or (rows, C): takes every row's gu unrounded, in the place of gu (rows that are time segments; !kMulti)
     bf16_t *gu_sum;   // null, or C elements: receives the sum of gu over the batch
     int *arrivals;    // per head: workgroups that have delivered their gu partial (zero on entry)
     float *ckpt;
@@ -124,7 +125,7 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
     float gu_acc[4] = {0.f, 0.f, 0.f, 0.f};
     float pend = 1.f;   // per-column factor the reverse state Gj has still to be multiplied with
     // gu of a pair: both halves leave their part in LDS (rows of the pair's parity); after the next barrier
-    // half 0 adds them, stores the pair's row and adds it, as stored, to the sum over the workgroup's pairs
+    // half 0 adds them, stores the pair's row and adds it, as stored (to bf16; or unrounded), to the sum over the workgroup's pairs
     // (for the fused batch sum; a lane owns its four channels of that row)
     float *gu_lds = reinterpret_cast<float *>(smem + BlockBwdLds::kGu);
     auto deliver_gu = [&](int done) {   // done: number of the pair
@@ -132,7 +133,13 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
             const float *rows = gu_lds + (done & 1) * 2 * kN + 16 * q + 4 * g;
             const float4 x = *reinterpret_cast<const float4 *>(rows), y = *reinterpret_cast<const float4 *>(rows + kN);
             const float t0 = x.x + y.x, t1 = x.y + y.y, t2 = x.z + y.z, t3 = x.w + y.w;
-            store4(a.gu + (int64_t)(b0 + done * a.bstep) * C + h * kN + 16 * q + 4 * g, t0, t1, t2, t3);
+            const int64_t e = (int64_t)(b0 + done * a.bstep) * C + h * kN + 16 * q + 4 * g;
+            if (!kMulti && a.gu_rows) {   // one pair per workgroup: its row is the sum
+                *reinterpret_cast<float4 *>(a.gu_rows + e) = make_float4(t0, t1, t2, t3);
+                *reinterpret_cast<float4 *>(gu_lds + 4 * kN + 16 * q + 4 * g) = make_float4(t0, t1, t2, t3);
+                return;
+            }
+            store4(a.gu + e, t0, t1, t2, t3);
             const uint32_t p01 = pack_bf16x2(t0, t1), p23 = pack_bf16x2(t2, t3);
             float4 *sum = reinterpret_cast<float4 *>(gu_lds + 4 * kN + 16 * q + 4 * g);
             float4 acc = *sum;
@@ -645,7 +652,8 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
         const bool states = s0p || gsTp || gs0p;
         __syncthreads();
         scan_bwd_a_body<bf16_t, bf16_t>(*reinterpret_cast<ScanBwdALds *>(smem), b, h, a.T, a.H, a.r + z, a.k + z, a.v + z, a.w + z, a.u + z, a.gy + z,
-                                        a.gr + z, a.gu + z, ck, kN, s0p, gsTp, states ? s_ft : nullptr);
+                                        a.gr + z, a.gu + z, ck, kN, s0p, gsTp, states ? s_ft : nullptr,
+                                        !kMulti && a.gu_rows ? a.gu_rows + (int64_t)pair0 * kN + z : nullptr);
         __threadfence_block();
         __syncthreads();
         const int z2 = fresh_s(0);
@@ -661,7 +669,10 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
     if (a.gu_sum != nullptr && lane_id < kN) {
         part = s_gu_wg[lane_id];
         for (int slot = 0; slot < npw; ++slot)   // the redone pairs' rows, as the second pass stored them
-            if (s_wild[slot]) part += load1(a.gu + (int64_t)(b0 + slot * a.bstep) * C + h * kN + lane_id);
+            if (s_wild[slot]) {
+                const int64_t e = (int64_t)(b0 + slot * a.bstep) * C + h * kN + lane_id;
+                part += !kMulti && a.gu_rows ? a.gu_rows[e] : load1(a.gu + e);
+            }
     }
     // Fused batch sum of gu: the workgroup that is the last of its head to deliver adds up the partials, one per
     // workgroup of the head.  They travel as written-through (agent scope) stores into the unused second half of
@@ -692,10 +703,10 @@ bool block_backward_applies(int64_t B, int64_t T, int64_t H) { return block_forw
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
-                          const float *s0, const float *gsT, float *gs0, RowCut cut)
+                          const float *s0, const float *gsT, float *gs0, RowCut cut, float *gu_rows)
 {
     BlockBwdArgs a = {};
-    a.cut = cut;
+    a.cut = cut; a.gu_rows = gu_rows;
     a.slice = (int)((T + kBlockTokens - 1) / kBlockTokens);
     a.T = (int)T; a.H = (int)H; a.B = (int)B;
     const int64_t grid = block_grid(B, H);
@@ -708,7 +719,7 @@ hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
     a.ckpt = (float *)workspace;
     a.arrivals = reinterpret_cast<int *>(reinterpret_cast<char *>(workspace) + chunk_backward_workspace_bytes(B, T, H));
     const bool multi = B * H > grid, ragged = (T % kBlockTokens) != 0 || cut.segments;
-    if (cut.segments && multi) return hipErrorInvalidValue;
+    if ((cut.segments || gu_rows) && multi) return hipErrorInvalidValue;
     auto launch = [&](auto multi_tag, auto ragged_tag) -> hipError_t {
         constexpr auto kern = block_bwd_kernel<decltype(multi_tag)::value, decltype(ragged_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockBwdLds::kBytes);

@@ -69,6 +69,7 @@ struct BwdArgs {
     const bf16_t *r, *k, *v, *w, *u, *gy;   // 16-bit elements: bf16, or fp16 with v and gy bf16 copies (see OutOf)
     const void *v_orig, *gy_orig;           // v and gy as the caller holds them (read by the exact per-timestep pass)
     bf16_t *gr, *gk, *gv, *gw, *gu;         // elements of the output type (bf16, or fp32 for fp16 tensors)
+    float *gu_rows;   // null, or (rows, C): takes every row's gu unrounded, in the place of gu (rows that are time segments)
     bf16_t *gu_sum;   // null, or C elements: receives the sum of gu over the batch
     int *arrivals;    // per head: workgroups that have delivered their gu partial (zero on entry)
     int B;
@@ -334,7 +335,9 @@ __device__ __forceinline__ void bwd_consumer(const BwdArgs &a, unsigned char *sm
     if (GRP == 0 && g == 0 && !*s_wild) {   // (the exact second pass writes gu itself)
         gu_acc += gu_lds[col];
         gu_lds[col] = gu_acc;               // for the fused batch sum, unrounded
-        store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + col, gu_acc);
+        const int64_t e = (int64_t)b * C + h * kN + col;
+        if (a.gu_rows) a.gu_rows[e] = gu_acc;
+        else store1(reinterpret_cast<Tout *>(a.gu) + e, gu_acc);
     }
 }
 
@@ -634,7 +637,8 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
         auto out = [](void *p) { return reinterpret_cast<Tout *>(p); };
         const Tout *gyp = reinterpret_cast<const Tout *>(a.gy_orig);
         scan_bwd_a_body<Tin, Tout>(*reinterpret_cast<ScanBwdALds *>(smem), b, h, a.T, a.H, in(a.r), in(a.k), in(a.v_orig), in(a.w), in(a.u), gyp,
-                                   out(a.gr), out(a.gu), ck, kN, s0p, gsTp, states ? s_ft : nullptr);
+                                   out(a.gr), out(a.gu), ck, kN, s0p, gsTp, states ? s_ft : nullptr,
+                                   a.gu_rows ? a.gu_rows + (int64_t)pair0 * kN : nullptr);
         __threadfence_block();
         __syncthreads();
         scan_bwd_b_body<Tin, Tout>(*reinterpret_cast<ScanBwdBLds *>(smem), b, h, a.T, a.H, in(a.r), in(a.k), in(a.v_orig), in(a.w), in(a.u), gyp, ck, kN,
@@ -655,8 +659,9 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
         const int tid = threadIdx.x;
         if (tid < kN) {          // wave 0
             // (not the rounded row, where the chunked code has it: with time segments there are up to 16 rows a sequence)
-            const float part = s_wild[0] ? load1(reinterpret_cast<const Tout *>(a.gu) + (int64_t)(pair0 / a.H) * C + h * kN + tid)
-                                         : reinterpret_cast<const float *>(smem + BwdLds::kGu)[tid];
+            const int64_t e = (int64_t)(pair0 / a.H) * C + h * kN + tid;
+            const float part = !s_wild[0] ? reinterpret_cast<const float *>(smem + BwdLds::kGu)[tid]
+                             : a.gu_rows ? a.gu_rows[e] : load1(reinterpret_cast<const Tout *>(a.gu) + e);
             __hip_atomic_store(a.ckpt + (int64_t)pair0 * slice + slice / 2 + tid, part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (tid == 0)
@@ -702,13 +707,13 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, bool states_ready,
                           void *gu_sum, const float *s0, const float *gsT, float *gs0,
-                          int in_dtype, const void *v_orig, const void *gy_orig, RowCut cut)
+                          int in_dtype, const void *v_orig, const void *gy_orig, RowCut cut, float *gu_rows)
 {
     const size_t lds = BwdLds::kBytes;
     BwdArgs a;
     a.v_orig = v_orig ? v_orig : v; a.gy_orig = gy_orig ? gy_orig : gy;
     a.s0 = s0; a.gsT = gsT; a.gs0 = gs0;
-    a.cut = cut;
+    a.cut = cut; a.gu_rows = gu_rows;
     a.slice = (int)((T + CL - 1) / CL);
     a.T = (int)T; a.H = (int)H;
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w;
@@ -740,28 +745,29 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
         hipError_t e = chunk_forward(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, nullptr, nullptr, workspace, nullptr, false, false, cut);
         if (e != hipSuccess) return e;
     }
-    if (block_form) return block_backward(st, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, a.gu_sum, s0, gsT, gs0, cut);
+    if (block_form) return block_backward(st, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, a.gu_sum, s0, gsT, gs0, cut, gu_rows);
     return ragged ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
-// Training pair in time segments, last step: gu of a batch row = sum over its segments; the decay
+// Training pair in time segments, last step: gu of a batch row = sum over its segments, which come unrounded (up to 16 of
+// them rounded to bf16 first made gu's error 1.05 to 1.17 times that of one piece, T 1100 to 5003); the decay
 // gradient at the first and the last token of a sequence is zero by definition
 // (rwkv_kernels.cu:381,406), where the kernels, given explicit states, leave rounding residue.
 template <typename E>
-__global__ void segments_finish_kernel(int P, int64_t T, int C, const E *__restrict__ gu_rows,
+__global__ void segments_finish_kernel(int P, int64_t T, int C, const float *__restrict__ gu_rows,
                                        E *__restrict__ gu, E *__restrict__ gw, bool zero_first, bool zero_last)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
     if (c >= C) return;
     float acc = 0.f;
-    for (int p = 0; p < P; ++p) acc += load1(gu_rows + ((int64_t)b * P + p) * C + c);
+    for (int p = 0; p < P; ++p) acc += gu_rows[((int64_t)b * P + p) * C + c];
     store1(gu + (int64_t)b * C + c, acc);
     if (zero_first) store1(gw + (int64_t)b * T * C + c, 0.f);
     if (zero_last) store1(gw + ((int64_t)b * T + T - 1) * C + c, 0.f);
 }
 
 template <typename E>
-hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const E *gu_rows, E *gu, E *gw, bool zero_first, bool zero_last)
+hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, E *gu, E *gw, bool zero_first, bool zero_last)
 {
     const int C = (int)(H * kN);
     hipLaunchKernelGGL(segments_finish_kernel<E>, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
@@ -785,10 +791,10 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
     // (2) chained backwards in time: the gradient arriving at the end of every segment
     if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates)) != hipSuccess) return e;
     // (3) every segment again, between its true incoming state and its true arriving gradient
-    e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, gu_sum,
-                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
+    e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, nullptr, saved, true, gu_sum,
+                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut, s.gu_rows);
     if (e != hipSuccess) return e;
-    return segments_finish(st, s.P, B, T, H, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, true, true);
+    return segments_finish(st, s.P, B, T, H, s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, true, true);
 }
 
 // The same with an initial state, a gradient arriving at the final state and dL/dS_0 wanted
@@ -810,11 +816,11 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
     e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates, gsT, gs0)) != hipSuccess) return e;
-    e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, saved, true, nullptr,
-                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut);
+    e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, nullptr, saved, true, nullptr,
+                       s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut, s.gu_rows);
     if (e != hipSuccess) return e;
     // (the decay gradient at an end of the sequence is zero by definition only where no state / no gradient comes in)
-    return segments_finish(st, s.P, B, T, H, (const bf16_t *)s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, s0 == nullptr, gsT == nullptr);
+    return segments_finish(st, s.P, B, T, H, s.gu_rows, (bf16_t *)gu, (bf16_t *)gw, s0 == nullptr, gsT == nullptr);
 }
 
 }  // namespace wkv6

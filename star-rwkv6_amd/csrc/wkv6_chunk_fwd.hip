@@ -911,7 +911,7 @@ TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra
     s.dsum = s.states + pairs * kN * kN;
     s.gstates = s.dsum + pairs * 4 * kN;
     s.gu_rows = s.gstates + pairs * kN * kN;
-    s.bytes = (pairs * (2 * kN * kN + 4 * kN) + (size_t)(B * s.P * H) * kN) * sizeof(float);   // (gu rows: room for fp32)
+    s.bytes = (pairs * (2 * kN * kN + 4 * kN) + pairs * kN) * sizeof(float);
     return s;
 }
 

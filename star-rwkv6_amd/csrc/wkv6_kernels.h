@@ -117,7 +117,8 @@ bool block_backward_applies(int64_t B, int64_t T, int64_t H);
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
-                          const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr, RowCut cut = RowCut());
+                          const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr, RowCut cut = RowCut(),
+                          float *gu_rows = nullptr);   // gu_rows: see chunk_backward; one pair per workgroup
 
 // --- full-precision chunk form (wkv6_chunk32_fwd.hip, wkv6_chunk32_bwd.hip): fp32 and fp16 tensors on the
 // fp32 matrix instructions, chunks of 32 tokens, fp32 states; any T (the last chunk may be short).
@@ -188,7 +189,7 @@ struct TrainSegments {
     float *states;      // [B*P][H][64][64] state entering each segment
     float *dsum;        // decay exponents of each segment (as chunk_forward leaves them)
     float *gstates;     // [B*P][H][64][64] gradient arriving at the end of each segment
-    void *gu_rows;      // [B*P][C] gu of each segment
+    float *gu_rows;     // [B*P][C] gu of each segment
     size_t bytes;       // size of the block
 };
 int chunk_train_segments(int64_t B, int64_t T, int64_t H);
@@ -202,7 +203,7 @@ hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, co
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
 RowCut cut_of(int P, int64_t L, int64_t T);
 template <typename T>
-hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T_, int64_t H, const T *gu_rows, T *gu, T *gw, bool zero_first, bool zero_last);
+hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T_, int64_t H, const float *gu_rows, T *gu, T *gw, bool zero_first, bool zero_last);
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
 hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -273,7 +274,8 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, bool states_ready,
                           void *gu_sum, const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr,
-                          int in_dtype = kBF16, const void *v_orig = nullptr, const void *gy_orig = nullptr, RowCut cut = RowCut());
+                          int in_dtype = kBF16, const void *v_orig = nullptr, const void *gy_orig = nullptr, RowCut cut = RowCut(),
+                          float *gu_rows = nullptr);   // (B, C): takes every row's gu unrounded, in the place of gu
 // s0 / gsT / gs0: gradients through the state, as in scan_backward_state (with states_ready = false)
 // in_dtype kF16 (needs states_ready): r, k, w, u fp16, v and gy their bf16 copies, v_orig / gy_orig the
 // caller's fp16 v and fp32 gy, gradients fp32

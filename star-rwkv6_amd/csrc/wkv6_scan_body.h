@@ -173,7 +173,8 @@ __device__ __forceinline__ void scan_bwd_a_body(ScanBwdALdsT<NW> &L, int b, int 
         const Tin *__restrict__ r, const Tin *__restrict__ k, const Tin *__restrict__ v,
         const Tin *__restrict__ w, const Tin *__restrict__ u, const Tout *__restrict__ gy,
         Tout *__restrict__ gr, Tout *__restrict__ gu, float *__restrict__ wsP, int64_t pstride,
-        const float *__restrict__ s0 = nullptr, const float *__restrict__ gsT = nullptr, float *fT = nullptr)
+        const float *__restrict__ s0 = nullptr, const float *__restrict__ gsT = nullptr, float *fT = nullptr,
+        float *__restrict__ gu_row = nullptr)   // gu_row: takes the pair's 64 values of gu unrounded, in the place of gu
 {
     // State gradients (all three null for the stateless operator): s0 = this pair's initial state
     // [key][value] fp32; gsT = the gradient arriving at its final state; fT[64] receives
@@ -310,7 +311,8 @@ __device__ __forceinline__ void scan_bwd_a_body(ScanBwdALdsT<NW> &L, int b, int 
     __syncthreads();
     if (tid < kN) {
         const float g = s_part[0][0][tid] + s_part[0][1][tid] + s_part[0][2][tid] + s_part[0][3][tid];
-        store1(gu + (int64_t)b * C + h * kN + tid, g);
+        if (gu_row) gu_row[tid] = g;
+        else store1(gu + (int64_t)b * C + h * kN + tid, g);
         if (fT) {
             float f = 0.f;
 #pragma unroll

@@ -887,6 +887,48 @@ def test_segments_add_up_the_bonus_gradient_unrounded(op, oracle):
     assert np.abs(gu / want - 1).max() <= 2.0 ** -8 * 1.1
 
 
+@pytest.mark.parametrize("call", ["pair", "again", "state", "rows"])
+@pytest.mark.parametrize("T,H,wild", [(1031, 4, False), (2049, 3, True), (2049, 40, False)])
+def test_segments_round_the_bonus_gradient_once(op, oracle, T, H, wild, call):
+    """gu of a bf16 sequence in segments (tile form, one redone segment, block form) in the training pair, in a second
+    backward over one graph, with gradients through the state and as the row of the batch: half a unit in the last place
+    from the exact sum, plus what the terms bring along.  A term r k <v,gy> is formed from four bf16 operands (r and k
+    times a scale factor, and the factors), each off by up to 2^-9, by 2^-9 / sqrt 3 in the root mean square: 2.3e-3
+    together.  Over T terms of one sign, products of half normals ((E x^2)^(1/2) / E x <= 1.6), that is 3.6e-3 / sqrt T of
+    the sum and, where a unit is smallest (2^-8 of the value), 0.92 / sqrt T units; five times that is allowed."""
+    from rwkv_kernel import _native
+
+    ins = oracle.make_inputs(1, T, H, 64, 5)
+    for x in (ins[0], ins[1], ins[2], ins[5]):
+        x.abs_()
+    if wild:
+        ins[3][0, T // 3:T // 3 + 20, 5:25] = 6.0
+    dev, ref = cast_inputs(ins[:5], torch.bfloat16)
+    gy_dev, gy_ref = cast_inputs(ins[5:6], torch.bfloat16)
+    op.algo = CHUNK
+    leaves = [x.clone().requires_grad_(True) for x in dev]
+    if call == "rows":
+        lib, C = _native.load(), H * 64
+        buf = torch.empty(lib.wkv6_saved_bytes(_native.BF16, CHUNK, 1, T, C, H), dtype=torch.uint8, device="cuda")
+        y, *outs = (torch.empty_like(dev[0]) for _ in range(5))
+        gu = torch.full((1, C), float("nan"), dtype=torch.bfloat16, device="cuda")
+        st, P = torch.cuda.current_stream().cuda_stream, lambda t: t.data_ptr()
+        _native.check(lib.wkv6_forward_save(st, _native.BF16, CHUNK, 1, T, C, H, *map(P, dev), P(y), P(buf), buf.numel()))
+        _native.check(lib.wkv6_backward_saved(st, _native.BF16, CHUNK, 1, T, C, H, *map(P, dev), P(gy_dev[0]), *map(P, outs), P(gu), P(buf), buf.numel()))
+    elif call == "state":
+        y, _ = op(*leaves, return_state=True)
+        gu = torch.autograd.grad(y, leaves, gy_dev[0])[4]
+    else:
+        y, _ = op(*leaves)
+        for again in range(2 if call == "again" else 1):
+            gu = torch.autograd.grad(y, leaves, gy_dev[0], retain_graph=True)[4]
+    want = oracle.backward_c(*ref, gy_ref[0], 64)[4].reshape(-1)
+    unit = 2.0 ** (np.floor(np.log2(np.abs(want))) - 7)
+    worst = (np.abs(to_np(gu).reshape(-1) - want) / unit).max()
+    print("gu %s T=%d H=%d: %.3f units" % (call, T, H, worst), flush=True)
+    assert worst <= 0.5 + 4.6 / T ** 0.5
+
+
 def test_training_pair_in_time_segments_with_fallback_segments(op, oracle):
     # segments whose decay the tile scaling cannot represent are redone by the exact per-timestep
     # code in every pass (forward passes, both backward passes); decay exactly 0 and exactly 1
