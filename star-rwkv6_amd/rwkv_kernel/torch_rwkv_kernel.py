@@ -258,6 +258,7 @@ class RWKVKernelOperator:
         arguments: the fixed token-shift mix of rwkv6_model.py:136 and of the channel-mix layer
         (:57-60).  bf16 tensors on the GPU, ``mix`` one value per channel.  Not part of the reference's operator."""
         assert x.is_contiguous() and x.dim() == 3 and mix.numel() == x.shape[2]
+        assert mix.device == x.device, "x and mix must be on one device"
         assert self.shift_mix_supported(x, 32), "shift_mix_x takes bf16 tensors on the GPU, channels a multiple of 64"
         return _ShiftMixX.apply(x, mix.reshape(x.shape[2]))
 
@@ -272,6 +273,7 @@ class RWKVKernelOperator:
         assert x.is_contiguous() and mix_x.numel() == C
         R = w2t.shape[2]
         assert a.shape == (5 * R, C) and w2t.shape == (5, C, R) and bias.shape == (5, C)
+        assert x.device == mix_x.device == a.device == w2t.device == bias.device, "x and the mixers' parameters must be on one device"
         assert self.shift_mix_supported(x, R), "shift_mix takes bf16 tensors on the GPU with rank 32 or 64"
         return self._torch.shift_mix(x, mix_x.reshape(C), a, w2t, bias)
 

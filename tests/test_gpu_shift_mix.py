@@ -212,6 +212,20 @@ def test_unsupported_shapes_are_refused(lib):
     assert rc == 1          # WKV6_ERR_ARG
 
 
+def test_parameters_on_another_device_are_refused():
+    """The kernels take addresses: a parameter left in host memory must not get that far."""
+    import rwkv_kernel
+    op = rwkv_kernel.RWKVKernelOperator(64, 64)
+    dev, _ = _inputs(2, 9, 128, 32, 3)
+    args = [dev[k] for k in ("x", "mix_x", "a", "w2t", "bias")]
+    assert len(op.shift_mix(*args)) == 5
+    for i in range(1, 5):
+        with pytest.raises(AssertionError, match="one device"):
+            op.shift_mix(*[t.cpu() if i == j else t for j, t in enumerate(args)])
+    with pytest.raises(AssertionError, match="one device"):
+        op.shift_mix_x(args[0], args[1].cpu())
+
+
 def test_full_size_known_answers(lib):
     """At the benchmark's layer shape (B=8, T=1024, C=2048, rank 32), where a float64 reference of
     everything is too slow: cases whose exact answer needs no arithmetic.  Coefficient 0 (W = 0,
