@@ -289,16 +289,23 @@ struct ShiftMix : torch::autograd::Function<ShiftMix> {
   }
 };
 
+// (B, H, N, N)
+at::DimVector state_shape(const Dims &d) {
+  TORCH_CHECK(d.H > 0, "wkv6: tensors without channels have no state");   // (the size per head below divides by it)
+  return {d.B, d.H, d.C / d.H, d.C / d.H};
+}
+
 // Stateful forward without a gradient (rwkv_kernel/torch_rwkv_kernel.py:76-95 of the reference): y and the final state.
 // An undefined map with an initial state means row b starts from s0[b].
 std::pair<Tensor, Tensor> forward_with_state(int64_t H, const Tensor &map, const Tensor &r, const Tensor &k, const Tensor &v,
                                              const Tensor &w, const Tensor &u, const Tensor &s0, int64_t algo, ScalarType st) {
   const at::NoGradGuard no_grad;
   const c10::DeviceGuard guard(r.device());
-  const auto [B, T, C, H_] = dims_of(r, H);
+  const Dims d = dims_of(r, H);
+  const auto [B, T, C, H_] = d;
   const int code = code_of(r.scalar_type());
   const Tensor y = carve(r, {{{B, T, C}, out_type(r.scalar_type()), 5}})[0];
-  const Tensor ys = at::empty({B, H, C / H, C / H}, r.options().dtype(st));
+  const Tensor ys = at::empty(state_shape(d), r.options().dtype(st));
   // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
   const size_t n = wkv6_forward_workspace_bytes(code, algo, B, T, C, H);
   const Tensor ws = bytes(r, n);
@@ -314,12 +321,13 @@ std::pair<Tensor, Tensor> forward_gn_gate(int64_t H, const Tensor &map, const Te
                                           const Tensor &offset, double eps, bool want_state) {
   const at::NoGradGuard no_grad;
   const c10::DeviceGuard guard(r.device());
-  const auto [B, T, C, H_] = dims_of(r, H);
+  const Dims d = dims_of(r, H);
+  const auto [B, T, C, H_] = d;
   const int code = code_of(r.scalar_type());
   const Tensor sc = scale.to(r.device(), at::kFloat).contiguous(), of = offset.to(r.device(), at::kFloat).contiguous();
   const ScalarType st = s0.defined() ? s0.scalar_type() : at::kFloat;
   const Tensor res = carve(r, {{{B, T, C}, r.scalar_type(), 5}})[0];
-  const Tensor ys = want_state ? at::empty({B, H, C / H, C / H}, r.options().dtype(st)) : Tensor();
+  const Tensor ys = want_state ? at::empty(state_shape(d), r.options().dtype(st)) : Tensor();
   const size_t n = wkv6_forward_workspace_bytes(code, kChunk, B, T, C, H);
   const Tensor ws = bytes(r, n);
   check(wkv6_forward_gn_gate_ex(stream_of(r), code, code_of(st), B, T, C, H, s0.defined(), static_cast<const int64_t *>(in(map)), in(r),
@@ -332,7 +340,8 @@ std::pair<Tensor, Tensor> forward_gn_gate(int64_t H, const Tensor &map, const Te
 
 // r, k, v, w and u as the kernels take them, with nothing left for the Python layer to check or to change.
 bool plain(int64_t N, const Tensor &r, const Tensor &k, const Tensor &v, const Tensor &w, const Tensor &u) {
-  if (r.dim() != 3 || !r.is_cuda() || code_of(r.scalar_type()) < 0 || r.size(2) % N != 0 || u.numel() != r.size(2)) return false;
+  if (r.dim() != 3 || !r.is_cuda() || code_of(r.scalar_type()) < 0 || r.size(2) == 0 || r.size(2) % N != 0 || u.numel() != r.size(2))
+    return false;
   for (const Tensor *t : {&r, &k, &v, &w, &u})
     if (t->device() != r.device() || t->scalar_type() != r.scalar_type() || !t->is_contiguous()) return false;
   return k.sizes() == r.sizes() && v.sizes() == r.sizes() && w.sizes() == r.sizes();

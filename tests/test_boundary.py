@@ -93,6 +93,17 @@ def test_torch_flavour_argument_checks(restore_backend):
         op(torch.zeros(2, 4, 100), x, x, x, u)  # C % head_size
 
 
+def test_state_of_tensors_without_channels_is_an_error():
+    from rwkv_kernel import _native
+    m = _native.load_torch()
+    for dt in (torch.float32, torch.bfloat16):
+        z, u = torch.zeros(2, 3, 0, dtype=dt), torch.zeros(0, 64, dtype=dt)
+        with pytest.raises(RuntimeError, match="without channels"):
+            m.forward_with_state(0, None, z, z, z, z, u, None, 0, _native.F32)
+        with pytest.raises(RuntimeError, match="without channels"):
+            m.forward_gn_gate(0, None, z, z, z, z, u, None, z, u, u, 64e-5, True)
+
+
 class _Var:
     def __init__(self, value):
         self.value = value

@@ -119,6 +119,18 @@ def test_transforms_stay_refused(op):
         torch.func.jvp(lambda r: op(r, *ins[1:])[0], (ins[0],), (ins[0],))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_tensors_without_elements_are_refused(op, dtype):
+    for B, T, C in ((2, 3, 0), (0, 3, 64), (2, 0, 64)):
+        z, u = torch.zeros(B, T, C, dtype=dtype, device="cuda"), torch.zeros(C // 64, 64, dtype=dtype, device="cuda")
+        sc = torch.zeros(C, device="cuda")
+        for kw in ({}, {"return_state": True}):
+            with pytest.raises(Exception):
+                op(z, z, z, z, u, **kw)
+            with pytest.raises(Exception):
+                op.forward_gn_gate(z, z, z, z, u, z, sc, sc, **kw)
+
+
 def test_input_side_gradients_of_some_outputs(op):
     B, T, C, R = 2, 40, 128, 32
     mk = lambda *s: torch.randn(*s, device="cuda") * 0.2
