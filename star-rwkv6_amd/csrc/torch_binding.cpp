@@ -103,6 +103,12 @@ std::vector<Tensor> carve(const Tensor &like, std::initializer_list<Piece> piece
   return res;
 }
 
+// The gradient of a parameter gets an allocation of its own: torch takes it over as the parameter's .grad as it is, where it
+// stays for as long as the caller keeps gradients, and with it whatever shares its block.
+Tensor parameter_gradient(const Tensor &like, at::IntArrayRef shape, ScalarType type) {
+  return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
+}
+
 bool any_requires_grad(std::initializer_list<const Tensor *> ts) {
   for (const Tensor *t : ts)
     if (t->defined() && t->requires_grad()) return true;
@@ -123,10 +129,10 @@ std::vector<Tensor> wkv6_grads(const Dims &d, int algo, const Tensor &r, const T
   const int code = code_of(r.scalar_type());
   const ScalarType ot = out_type(r.scalar_type());
   const at::DimVector big{B, T, C};
-  std::vector<Tensor> g = carve(r, {{big, ot, 7}, {big, ot, 8}, {big, ot, 9}, {big, ot, 10}, {at::DimVector(u.sizes()), ot, 0}, {{B, C}, ot, 0}});
-  const Tensor gu_rows = g[5];
-  g.pop_back();
+  std::vector<Tensor> g = carve(r, {{big, ot, 7}, {big, ot, 8}, {big, ot, 9}, {big, ot, 10}, {{B, C}, ot, 0}});
+  const Tensor gu_rows = std::move(g[4]);
   if (saved.defined()) {
+    g[4] = parameter_gradient(r, u.sizes(), ot);
     // the batch sum of u's gradient (rwkv_kernel/torch_rwkv_kernel.py:73 of the reference) comes out of the same launch
     check(wkv6_backward_saved_sum(stream_of(r), code, algo, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gy), out(g[0]),
                                   out(g[1]), out(g[2]), out(g[3]), out(gu_rows), out(g[4]), out(saved), saved.numel()));
@@ -233,13 +239,14 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
     const Tensor gout = grads[0].contiguous();
     const ScalarType t = r.scalar_type();
     const Tensor gy = carve(r, {{{B, T, C}, t, 5}})[0];
-    const auto g = carve(r, {{{B, T, C}, t, 6}, {at::DimVector(s[6].sizes()), at::kFloat, 0}, {at::DimVector(s[7].sizes()), at::kFloat, 0}});
+    const Tensor ggate = carve(r, {{{B, T, C}, t, 6}})[0];
+    const Tensor gscale = parameter_gradient(r, s[6].sizes(), at::kFloat), goffset = parameter_gradient(r, s[7].sizes(), at::kFloat);
     check(wkv6_gn_gate_backward(stream_of(r), code_of(t), B, T, C, H, in(gout), in(s[8]), in_f(s[9]), in(s[5]), in_f(s[6]), in_f(s[7]),
-                                out(gy), out(g[0]), out_f(g[1]), out_f(g[2])));
+                                out(gy), out(ggate), out_f(gscale), out_f(goffset)));
     auto w = wkv6_grads(d, kChunk, r, s[1], s[2], s[3], s[4], gy, take(ctx));
-    return {w[0], w[1], w[2], w[3], w[4], g[0],
-            g[1].to(static_cast<ScalarType>(ctx->saved_data["scale_type"].toInt())),
-            g[2].to(static_cast<ScalarType>(ctx->saved_data["offset_type"].toInt())), Tensor(), Tensor()};
+    return {w[0], w[1], w[2], w[3], w[4], ggate,
+            gscale.to(static_cast<ScalarType>(ctx->saved_data["scale_type"].toInt())),
+            goffset.to(static_cast<ScalarType>(ctx->saved_data["offset_type"].toInt())), Tensor(), Tensor()};
   }
 };
 
@@ -277,15 +284,17 @@ struct ShiftMix : torch::autograd::Function<ShiftMix> {
     const ScalarType t = x.scalar_type(), wt = static_cast<ScalarType>(ctx->saved_data["weight_type"].toInt());
     const int code = code_of(t);
     for (Tensor &g : grads) g = g.to(t).contiguous();
-    const auto g = carve(x, {{{B, T, C}, t, 6}, {{5 * R, C}, wt, 0}, {{5, C, R}, wt, 0}, {{5, C}, at::kFloat, 0}, {{C}, at::kFloat, 0}});
+    const Tensor gx = carve(x, {{{B, T, C}, t, 6}})[0];
+    const Tensor gmix = parameter_gradient(x, {C}, at::kFloat), ga = parameter_gradient(x, {5 * R, C}, wt),
+                 gw2t = parameter_gradient(x, {5, C, R}, wt), gbias = parameter_gradient(x, {5, C}, at::kFloat);
     const size_t n = wkv6_shift_mix_backward_workspace_bytes(code, B, T, C, R);
     const Tensor ws = bytes(x, n);
     check(wkv6_shift_mix_backward(stream_of(x), code, code_of(wt), B, T, C, R, in(x), in_f(mx), in_f(b32), in(weights), in(h),
-                                  in(grads[0]), in(grads[1]), in(grads[2]), in(grads[3]), in(grads[4]), out(g[0]), out_f(g[4]),
-                                  out(g[1]), out(g[2]), out_f(g[3]), out(ws), n));
+                                  in(grads[0]), in(grads[1]), in(grads[2]), in(grads[3]), in(grads[4]), out(gx), out_f(gmix),
+                                  out(ga), out(gw2t), out_f(gbias), out(ws), n));
     const auto types = ctx->saved_data["types"].toIntVector();
     const auto as = [&](const Tensor &v, int i) { return v.to(static_cast<ScalarType>(types[i])); };
-    return {g[0], as(g[4], 0), as(g[1], 1), as(g[2], 2), as(g[3], 3)};
+    return {gx, as(gmix, 0), as(ga, 1), as(gw2t, 2), as(gbias, 3)};
   }
 };
 

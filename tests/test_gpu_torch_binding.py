@@ -119,6 +119,36 @@ def test_transforms_stay_refused(op):
         torch.func.jvp(lambda r: op(r, *ins[1:])[0], (ins[0],), (ins[0],))
 
 
+@pytest.mark.parametrize("again", [False, True])
+def test_parameters_gradients_hold_nothing_else(op, again):
+    """torch takes a parameter's gradient over as it is: its storage is the parameter's own size, to the allocator's
+    rounding at most, and not a block that also holds gradients of the size of the activations."""
+    B, T, H, R = 4, 96, 4, 32
+    C = H * 64
+    mk = lambda *s: (torch.randn(*s, device="cuda") * 0.2).requires_grad_(True)
+
+    def check(params, out, g):
+        for i in range(2 if again else 1):           # (a second backward over one graph goes another way)
+            for q in params:
+                q.grad = None
+            out.backward(g, retain_graph=again)
+        for q in params:
+            assert q.grad.shape == q.shape and q.grad.dtype == q.dtype
+            assert q.grad.untyped_storage().nbytes() <= q.numel() * q.element_size() + 512
+
+    for dtype in DTYPES:
+        ins = _inputs(B, T, H, dtype, grad=True)
+        y = op(*ins)[0]
+        check(ins[4:], y, torch.randn_like(y))
+    ins = _inputs(B, T, H, torch.bfloat16, grad=True)
+    gate, sc, of = mk(B, T, C).bfloat16(), mk(H, 64), mk(C)
+    out = op.forward_gn_gate(*ins, gate, sc, of)[0]
+    check([ins[4], sc, of], out, torch.randn_like(out))
+    ps = [mk(C), mk(5 * R, C), mk(5, C, R), mk(5, C)]
+    outs = torch.stack(op.shift_mix(mk(B, T, C).bfloat16(), *ps))
+    check(ps, outs, torch.randn_like(outs))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_tensors_without_elements_are_refused(op, dtype):
     for B, T, C in ((2, 3, 0), (0, 3, 64), (2, 0, 64)):
