@@ -250,6 +250,13 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
   }
 };
 
+// A parameter as the kernels read it: of this type, contiguous and on a 16-byte boundary.  (One that already has the type and
+// is contiguous may be a view into a flat buffer of parameters, anywhere in it.)
+Tensor laid_out(const Tensor &t, ScalarType type) {
+  const Tensor c = t.to(type).contiguous();
+  return reinterpret_cast<uintptr_t>(c.const_data_ptr()) % 16 == 0 ? c : c.clone();
+}
+
 // The layer's input side (rwkv6_model.py:134-146 of the reference) with gradients, bf16: x -> (xr, xk, xv, xw, xg).
 struct ShiftMix : torch::autograd::Function<ShiftMix> {
   static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &mix_x, const Tensor &a, const Tensor &w2t,
@@ -259,7 +266,8 @@ struct ShiftMix : torch::autograd::Function<ShiftMix> {
     const int code = code_of(x.scalar_type());
     const Tensor mx = mix_x.to(at::kFloat).contiguous(), b32 = bias.to(at::kFloat).contiguous();
     const ScalarType wt = a.scalar_type() == w2t.scalar_type() && a.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat;
-    const Tensor aw = a.to(wt).contiguous(), ww = w2t.to(wt).contiguous();
+    // (bf16 second weights are handed through, and refused off a 16-byte boundary, like x and the biases)
+    const Tensor aw = laid_out(a, wt), ww = w2t.scalar_type() == at::kBFloat16 ? w2t.to(wt).contiguous() : laid_out(w2t, wt);
     const int64_t nw = wkv6_shift_mix_weights_bytes(C, R);
     const ScalarType t = x.scalar_type();
     const at::DimVector big{B, T, C};

@@ -212,6 +212,29 @@ def test_unsupported_shapes_are_refused(lib):
     assert rc == 1          # WKV6_ERR_ARG
 
 
+@pytest.mark.parametrize("shift", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("adt,wdt", [(torch.float32, torch.float32), (BF16, BF16), (BF16, torch.float32)])
+def test_weights_may_lie_anywhere_in_a_flat_buffer(adt, wdt, shift):
+    import rwkv_kernel
+    op = rwkv_kernel.RWKVKernelOperator(64, 64)
+    dev, _ = _inputs(2, 9, 128, 32, 4)
+
+    def results(place, shift2):
+        args = [place(dev["x"], 0), place(dev["mix_x"], 0), place(dev["a"].to(adt), shift), place(dev["w2t"].to(wdt), shift2), place(dev["bias"], 0)]
+        outs = op.shift_mix(*args)
+        return list(outs) + list(torch.autograd.grad(outs, args, [dev["x"]] * 5))
+
+    def anywhere(t, elements):
+        return torch.empty(t.numel() + elements, dtype=t.dtype, device="cuda")[elements:].view(t.shape).copy_(t).requires_grad_(True)
+
+    shift2 = shift if wdt == torch.float32 else 0
+    for got, want in zip(results(anywhere, shift2), results(lambda t, _: t.clone().requires_grad_(True), 0)):
+        assert torch.equal(got, want)
+    if wdt == BF16 and shift % 8:      # (handed through to the kernel, which reads 16 bytes at a time)
+        with pytest.raises(Exception):
+            results(anywhere, shift)
+
+
 def test_parameters_on_another_device_are_refused():
     """The kernels take addresses: a parameter left in host memory must not get that far."""
     import rwkv_kernel
