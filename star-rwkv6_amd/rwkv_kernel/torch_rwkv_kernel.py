@@ -168,6 +168,14 @@ class RWKVKernelOperator:
         self.normal_kernenl = _WKV6
         self.kernel_with_state = _forward_with_state
 
+    def __getstate__(self):
+        """Copies and pickles leave the native module out (a module can be neither) and find it again."""
+        return {k: v for k, v in self.__dict__.items() if k != "_torch"}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._torch = _native.load_torch()
+
     def _check(self, r, k, v, w, u, init_state, state_map):
         """Argument checks shared by every entry; returns (B, T, C, H, N, u, init_state, state_map)."""
         B, T, C = r.shape

@@ -1,8 +1,10 @@
 """The Python surface mirrors the reference's rwkv_kernel package (names, signature, errors).
 CPU only: the portable flavour is compared with the oracle; the torch flavour is exercised up to
 its argument checks (its kernels need the GPU)."""
+import copy
 import importlib
 import os
+import pickle
 import sys
 
 import numpy as np
@@ -91,6 +93,16 @@ def test_torch_flavour_argument_checks(restore_backend):
         op(x, x, x, x, u)                       # tensors must live on the GPU (torch_rwkv_kernel.py:107-111)
     with pytest.raises(AssertionError):
         op(torch.zeros(2, 4, 100), x, x, x, u)  # C % head_size
+
+
+def test_operator_objects_can_be_copied_and_pickled(restore_backend):
+    # a model that holds one is deep-copied for weight averaging, and saved whole
+    op = _fresh_import("torch").RWKVKernelOperator(64, 1024)
+    op.algo = 2
+    for other in (copy.copy(op), copy.deepcopy(op), pickle.loads(pickle.dumps(op))):
+        assert (type(other), other.head_size, other.max_sequence_length, other.algo) == (type(op), 64, 1024, 2)
+        with pytest.raises(AssertionError):
+            other(*[torch.zeros(2, 4, 128)] * 4, torch.zeros(2, 64))      # (as far as a call gets without a GPU)
 
 
 def test_state_of_tensors_without_channels_is_an_error():
