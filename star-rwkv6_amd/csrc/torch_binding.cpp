@@ -374,6 +374,13 @@ const Tensor *tensor(const py::object &o) { return THPVariable_Check(o.ptr()) ? 
 
 py::object wrap(const Tensor &t) { return t.defined() ? py::reinterpret_steal<py::object>(THPVariable_Wrap(t)) : py::none(); }
 
+// Whatever Python takes for true or false (pybind11's bool refuses lists, texts and other objects with a length).
+bool truth(const py::object &o) {
+  const int t = PyObject_IsTrue(o.ptr());
+  if (t < 0) throw py::error_already_set();
+  return t != 0;
+}
+
 py::tuple wrap(const std::pair<Tensor, Tensor> &p) { return py::make_tuple(wrap(p.first), wrap(p.second)); }
 
 // Runs f without the interpreter's lock.  A Python error that torch has put into a C++ exception is restored as it was.
@@ -389,11 +396,11 @@ template <typename F> auto unlocked(F &&f) {
 }
 
 py::object try_call(int64_t N, int64_t algo, const py::object &r_, const py::object &k_, const py::object &v_, const py::object &w_,
-                    const py::object &u_, bool return_state, const py::object &s0_) {
+                    const py::object &u_, const py::object &return_state_, const py::object &s0_) {
   const Tensor *r = tensor(r_), *k = tensor(k_), *v = tensor(v_), *w = tensor(w_), *u = tensor(u_), *s0 = tensor(s0_);
   if (!r || !k || !v || !w || !u || !plain(N, *r, *k, *v, *w, *u)) return py::none();
   const int64_t H = r->size(2) / N;
-  if (!return_state) {
+  if (!truth(return_state_)) {
     if (!s0_.is_none()) return py::none();
     return py::make_tuple(wrap(unlocked([&] { return Wkv6::apply(*r, *k, *v, *w, *u, H, algo); })), py::none());
   }
@@ -405,8 +412,8 @@ py::object try_call(int64_t N, int64_t algo, const py::object &r_, const py::obj
 }
 
 py::object try_gn_gate(int64_t N, const py::object &r_, const py::object &k_, const py::object &v_, const py::object &w_,
-                       const py::object &u_, const py::object &gate_, const py::object &scale_, const py::object &offset_, double eps,
-                       bool return_state, const py::object &s0_) {
+                       const py::object &u_, const py::object &gate_, const py::object &scale_, const py::object &offset_,
+                       const py::object &eps_, const py::object &return_state_, const py::object &s0_) {
   const Tensor *r = tensor(r_), *k = tensor(k_), *v = tensor(v_), *w = tensor(w_), *u = tensor(u_), *s0 = tensor(s0_);
   const Tensor *gate = tensor(gate_), *scale = tensor(scale_), *offset = tensor(offset_);
   if (!r || !k || !v || !w || !u || !gate || !scale || !offset || !plain(N, *r, *k, *v, *w, *u)) return py::none();
@@ -417,6 +424,8 @@ py::object try_gn_gate(int64_t N, const py::object &r_, const py::object &k_, co
     return py::none();
   const Tensor state = s0 ? *s0 : Tensor();
   if (s0 ? !plain_state(N, *r, state) : !s0_.is_none()) return py::none();
+  const bool return_state = truth(return_state_);
+  const double eps = py::float_(eps_);
   if (at::GradMode::is_enabled() && any_requires_grad({r, k, v, w, u, gate, scale, offset})) {
     if (return_state || s0 || !wkv6_forward_gn_gate_save_supported(code_of(r->scalar_type()), B, T, C, H)) return py::none();
     return py::make_tuple(wrap(unlocked([&] { return Wkv6GnGate::apply(*r, *k, *v, *w, *u, *gate, *scale, *offset, H, eps); })), py::none());

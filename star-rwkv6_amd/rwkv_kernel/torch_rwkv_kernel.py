@@ -309,7 +309,7 @@ class RWKVKernelOperator:
                 assert x.is_contiguous()
             lib = _native.load()
             if lib.wkv6_forward_gn_gate_save_supported(_DTYPE_CODE[r.dtype], B, T, C, H):
-                return self._torch.wkv6_gn_gate(r, k, v, w, u, gate, gn_scale.to(r.device), gn_offset.to(r.device), H, epsilon), None
+                return self._torch.wkv6_gn_gate(r, k, v, w, u, gate, gn_scale.to(r.device), gn_offset.to(r.device), H, float(epsilon)), None
             # (a shape the fused training kernels do not take, e.g. a sequence too long for the chunk form: unfused calls)
             y, _ = self(r, k, v, w, u)
             z = torch.nn.functional.layer_norm(y.float().view(B, T, H, N), (N,), eps=epsilon).view(B, T, C)
@@ -318,4 +318,4 @@ class RWKVKernelOperator:
         init_state, state_map = self._resolve_state(B, r, init_state, state_map)
         for x in (r, k, v, w, u, gate):
             assert x.is_contiguous()
-        return self._torch.forward_gn_gate(H, state_map, r, k, v, w, u, init_state, gate, gn_scale, gn_offset, epsilon, bool(return_state))
+        return self._torch.forward_gn_gate(H, state_map, r, k, v, w, u, init_state, gate, gn_scale, gn_offset, float(epsilon), bool(return_state))

@@ -1,7 +1,9 @@
 """The torch flavour's native calls against the general way through the checks of the Python layer, and what autograd
 offers around a node: a second backward, saved-tensor hooks, inference mode, other streams; transforms stay refused."""
 import types
+from fractions import Fraction
 
+import numpy as np
 import pytest
 import torch
 
@@ -147,6 +149,21 @@ def test_parameters_gradients_hold_nothing_else(op, again):
     ps = [mk(C), mk(5 * R, C), mk(5, C, R), mk(5, C)]
     outs = torch.stack(op.shift_mix(mk(B, T, C).bfloat16(), *ps))
     check(ps, outs, torch.randn_like(outs))
+
+
+def test_flags_and_numbers_of_any_type(op):
+    """return_state is anything with a truth, epsilon anything with a value, as in a Python signature."""
+    ins = _inputs(2, 33, 2, torch.bfloat16)
+    gate, p = ins[0], torch.ones(128, device="cuda")
+    want = {s: op(*ins, return_state=s) for s in (False, True)}
+    fused = {s: op.forward_gn_gate(*ins, gate, p, p, 0.25, return_state=s) for s in (False, True)}
+    for flag in (0, 1, None, [], [0], "", "yes", torch.tensor(True), torch.zeros(1).cuda(), np.bool_(True), object()):
+        _same(op(*ins, return_state=flag), want[bool(flag)])
+        _same(op.forward_gn_gate(*ins, gate, p, p, 0.25, return_state=flag), fused[bool(flag)])
+    for eps in (np.float32(0.25), torch.tensor(0.25), Fraction(1, 4), "0.25"):
+        _same(op.forward_gn_gate(*ins, gate, p, p, eps, return_state=True), fused[True])
+    with pytest.raises(Exception):
+        op(*ins, return_state=torch.zeros(2))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
