@@ -754,24 +754,25 @@ constexpr int kMostSegments = 16;
 // state of the backward pass obeys (the gradient arriving at the end of segment p is what segment
 // p + 1 sends into its incoming state: its own contribution plus D_{p+1} times what arrives at its end).
 // kFactors: dsum holds two factors of each segment's decay, [2][pairs][64], instead of its exponent's four parts.
-template <typename Ts, bool kReverse, int kMost, bool kFactors>
-__global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
+template <typename Ts, bool kReverse, int P, bool kFactors>
+__global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
                                                             const float *__restrict__ dsum, float *__restrict__ states, Ts *__restrict__ sT)   // sT: the final state, or null
 {
     // Thread: four value columns i0..i0+3 of one key row j of one (batch, head): 1024 threads per pair,
     // gridDim.x * 256 = B * H * 1024.  states[(b*P + seg), h] holds U on entry and the segment's
-    // incoming state on exit (P <= kMost segments).  All P loads are issued before the chain is walked (their addresses do
-    // not depend on it): the kernel takes about two memory round trips instead of 2 P.
+    // incoming state on exit.  All P loads are issued before the chain is walked (their addresses do
+    // not depend on it): the kernel takes about two memory round trips instead of 2 P.  For that P has to be known to the
+    // compiler: loops of up to 16 steps with a way out at a run-time P kept x and d in 272 bytes of scratch memory (a prompt of
+    // B1 T4096 H8, 16 segments: 43 us), and with steps past P that change nothing it took 32 us (so: 27.5 us).
     const int e = blockIdx.x * 256 + threadIdx.x;
     const int i0 = (e & 15) * 4, j = (e >> 4) & 63, bh = e >> 10;
     const int b = bh / H, h = bh - b * H;
     const int64_t np = (int64_t)(gridDim.x >> 2) * P;   // pairs of all segments
     auto pair_of_step = [&](int n) { return ((int64_t)b * P + (kReverse ? P - 1 - n : n)) * H + h; };   // step n of the walk
-    float4 x[kMost];
-    float d[kMost];
+    float4 x[P];
+    float d[P];
 #pragma unroll
-    for (int n = 0; n < kMost; ++n) {
-        if (n >= P) break;
+    for (int n = 0; n < P; ++n) {
         const int64_t vp = pair_of_step(n);
         x[n] = *reinterpret_cast<const float4 *>(states + (vp * kN + j) * kN + i0);
         if (kFactors) d[n] = dsum[vp * kN + j] * dsum[(np + vp) * kN + j];
@@ -783,27 +784,24 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, int P, const 
         load4(s0 + ((row * H + h) * kN + j) * kN + i0, S);
     }
 #pragma unroll
-    for (int n = 0; n < kMost; ++n) {
-        if (n >= P) break;
+    for (int n = 0; n < P; ++n) {
         const float dd = kFactors ? d[n] : exp2_fast(-d[n]);
         *reinterpret_cast<float4 *>(states + (pair_of_step(n) * kN + j) * kN + i0) = make_float4(S[0], S[1], S[2], S[3]);
         S[0] = fmaf(S[0], dd, x[n].x); S[1] = fmaf(S[1], dd, x[n].y); S[2] = fmaf(S[2], dd, x[n].z); S[3] = fmaf(S[3], dd, x[n].w);
     }
     if (sT) store4(sT + (((int64_t)b * H + h) * kN + j) * kN + i0, S[0], S[1], S[2], S[3]);
 }
-template <typename Ts, bool kReverse, bool kFactors = false>
+template <typename Ts, bool kReverse, bool kFactors = false, int N = kMostSegments>
 static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, const Ts *s0, const int64_t *map,
                                const float *dsum, float *states, Ts *sT)
 {
-    const dim3 grid((unsigned)(B * H * 4)), block(256);
-    if (P < 2 || P > kMostSegments) return hipErrorInvalidValue;
-    auto run = [&](auto most) {
-        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, decltype(most)::value, kFactors>), grid, block, 0, st, (int)H, P, s0, map, dsum, states, sT);
-    };
-    if (P <= 4) run(std::integral_constant<int, 4>{});
-    else if (P <= 8) run(std::integral_constant<int, 8>{});
-    else run(std::integral_constant<int, kMostSegments>{});
-    return hipGetLastError();
+    if constexpr (N < 2) {
+        return hipErrorInvalidValue;
+    } else {
+        if (P != N) return launch_chain<Ts, kReverse, kFactors, N - 1>(st, P, B, H, s0, map, dsum, states, sT);
+        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, N, kFactors>), dim3((unsigned)(B * H * 4)), dim3(256), 0, st, (int)H, s0, map, dsum, states, sT);
+        return hipGetLastError();
+    }
 }
 
 // Segments of a sequence of T tokens when `pairs` (batch, head) pairs share the chip: as many as still fit it once, each a

@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import struct
+import subprocess
 
 import pytest
 
@@ -135,3 +136,38 @@ def test_missing_library_fails_loudly(native, monkeypatch):
     monkeypatch.setattr(native, "LIB_PATH", "/nonexistent/libwkv6_gfx950.so")
     with pytest.raises(native.WKV6Error):
         native.load()
+
+
+def _scratch_bytes(library, directory):
+    """Bytes of scratch memory per lane of every kernel in the library, from its code objects' own notes."""
+    blob = open(library, "rb").read()
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at, found = blob.find(magic), {}
+    while at >= 0:
+        (entries,) = struct.unpack_from("<Q", blob, at + len(magic))
+        pos = at + len(magic) + 8
+        for _ in range(entries):
+            offset, size, n = struct.unpack_from("<QQQ", blob, pos)
+            ident = blob[pos + 24:pos + 24 + n]
+            pos += 24 + n
+            if size == 0 or b"gfx" not in ident:
+                continue
+            path = directory / "code_object"
+            path.write_bytes(blob[at + offset:at + offset + size])
+            notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
+            for kernel in notes.split("- .agpr_count")[1:]:
+                name = re.search(r"\n    \.name:\s+(\S+)", kernel).group(1)
+                found[name] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", kernel).group(1))
+        at = blob.find(magic, at + len(magic))
+    return found
+
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs ROCm's llvm-readelf")
+def test_state_chain_keeps_its_values_in_registers(native, tmp_path):
+    """The chain over a sequence's segments has everything it loads in flight at once, which only works from registers;
+    a loop that does not unroll puts the values into scratch memory (and takes twice the time)."""
+    kernels = {k: v for k, v in _scratch_bytes(native.LIB_PATH, tmp_path).items() if "segment_chain_kernel" in k}
+    assert kernels and not any(kernels.values()), kernels

@@ -10,7 +10,7 @@ from _util import cast_inputs, check_close, out_dtype, to_np
 
 pytestmark = pytest.mark.gpu
 
-SCAN, CHUNK = 1, 2
+AUTO, SCAN, CHUNK = 0, 1, 2
 DTYPES = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
 
 
@@ -871,6 +871,22 @@ def test_prompt_in_time_segments_of_any_length(op, oracle, T, H, sdt):
     check_close("sT", sT, sT_ref, torch.bfloat16)
     check_close("sT fused", oT, sT_ref, torch.bfloat16)
     check_close("out", out, oracle.group_norm_gate_np(y_ref, gate_ref[0], scale.numpy(), offset.numpy(), N), torch.bfloat16)
+
+
+@pytest.mark.parametrize("P", range(2, 17))
+def test_every_number_of_segments(op, oracle, P):
+    """The state chain is built for each number of segments: forward, reverse and (prompts) from and to a bf16 state, in
+    bf16, and in fp32, whose segments' decays are factors."""
+    H, T = {2: (100, 2048), 3: (80, 2048)}.get(P, (1, 256 * P))     # (few segments only where more would not fit)
+    _case(op, oracle, 1, T, H, 500 + P, torch.bfloat16, CHUNK)
+    _case(op, oracle, 1, T, H, 600 + P, torch.float32, AUTO)
+    if P >= 6:
+        ins = oracle.make_inputs(1, 192 * P, 2, 64, 700 + P, with_state=True)
+        dev, ref = cast_inputs(ins[:5] + [ins[6]], torch.bfloat16)
+        y, sT = op(*dev[:5], return_state=True, init_state=dev[5])
+        y_ref, sT_ref = oracle.forward_c(*ref[:5], 64, ref[5])
+        check_close("y", y, y_ref, torch.bfloat16)
+        check_close("sT", sT, sT_ref, torch.bfloat16)
 
 
 def test_segments_add_up_the_bonus_gradient_unrounded(op, oracle):
