@@ -55,7 +55,7 @@ struct BlockFwdArgs {
     int T, H, B;
     int bstep;               // batch rows between two pairs of a workgroup (B: one pair per workgroup)
     int slice;               // chunks of a pair's slice of `ckpt` (those of the longest row)
-    RowCut cut;              // rows that are time segments (one pair per workgroup and kRagged)
+    RowCut cut;              // kCut: how the rows lie in the sequences (one pair per workgroup)
     const bf16_t *r, *k, *v, *w, *u;
     const void *s0;          // initial state (B or n_state, H, 64, 64) [key][value] in Ts, or null
     const int64_t *map;      // batch row -> state row, or null
@@ -412,7 +412,9 @@ __device__ __forceinline__ void block_output_stage_in_place(const BlockFwdArgs &
     }
 }
 
-template <typename Ts, bool kSave, bool kRagged, bool kFuse>
+// kCut: rows that are time segments (of true fp32 states).  Built apart: asked at run time, the other ragged launches, whose
+// pointers then depend on it, took 2 % longer (prompts of B8 T999 H40: 63.1 us, so 61.7).
+template <typename Ts, bool kSave, bool kRagged, bool kFuse, bool kCut>
 __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -424,7 +426,7 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pair0 = (int)blockIdx.x;
-    if (kRagged && a.cut.segments) {
+    if (kCut) {
         const RowView rv = row_view(a.cut, pair0 / a.H, a.T);
         const int64_t n = rv.shift * a.H * kN;
         a.T = rv.tokens;
@@ -487,16 +489,22 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     a.gate = (const bf16_t *)gate; a.gn_scale = gn_scale; a.gn_offset = gn_offset; a.gn_eps = gn_eps; a.out = (bf16_t *)out; a.stats = stats;
-    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag) -> hipError_t {
+    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto cut_tag) -> hipError_t {
         constexpr bool kFuse = decltype(fuse_tag)::value;
-        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse>;
+        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(cut_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockFwdLdsT<kFuse>::kBytes);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlockFwdThreads), BlockFwdLdsT<kFuse>::kBytes, st, a);
         return hipGetLastError();
     };
     auto launch_ts = [&](auto ts_tag, auto save_tag, auto fuse_tag) -> hipError_t {
-        return (T % kBlockTokens) != 0 || cut.segments ? launch(ts_tag, save_tag, std::true_type{}, fuse_tag) : launch(ts_tag, save_tag, std::false_type{}, fuse_tag);
+        const std::true_type yes;
+        const std::false_type no;
+        if (cut.segments) {
+            if constexpr (std::is_same<decltype(ts_tag), float>::value) return launch(ts_tag, save_tag, yes, fuse_tag, yes);
+            else return hipErrorInvalidValue;
+        }
+        return (T % kBlockTokens) != 0 ? launch(ts_tag, save_tag, yes, fuse_tag, no) : launch(ts_tag, save_tag, no, fuse_tag, no);
     };
     const bool save = saved_states != nullptr;
     if (gate != nullptr) {
