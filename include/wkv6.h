@@ -243,8 +243,9 @@ size_t wkv6_backward_workspace_bytes(int dtype, int64_t B, int64_t T, int64_t C,
  * point of the call -- code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc -- and neither the library nor anything it calls allocates or frees memory here (the
  * first call on a device looks the array's address up once).  Shapes whose
- * wkv6_backward_workspace_bytes() exceeds WKV6_STATIC_SCRATCH_BYTES run on the per-timestep kernels
- * if their workspace (4 bytes per element of r) fits, and are refused with WKV6_ERR_WORKSPACE
+ * wkv6_backward_workspace_bytes() exceeds WKV6_STATIC_SCRATCH_BYTES run in one piece instead of time
+ * segments if that fits (same results to rounding), else on the per-timestep kernels if their
+ * workspace (4 bytes per element of r) fits, and are refused with WKV6_ERR_WORKSPACE
  * otherwise (the benchmark shape B=8 T=1024 C=2048 needs exactly the array's size, as bf16 on the
  * chunked kernels and as fp32 on the per-timestep ones).  All calls
  * on one GPU share the one array: two calls whose kernels overlap in time on the same GPU

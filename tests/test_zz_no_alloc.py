@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _pair(lib, native, B, T, H, dtype, seed):
+def _pair(lib, native, B, T, H, dtype, seed, algo=None):
     N = 64
     C = H * N
     code = {torch.bfloat16: native.BF16, torch.float32: native.F32}[dtype]
@@ -28,6 +28,12 @@ def _pair(lib, native, B, T, H, dtype, seed):
     want = outs()
     native.check(lib.wkv6_backward(st, code, B, T, C, H, P(r), P(k), P(v), P(w), P(u), P(gy), *[P(x) for x in want], P(ws), n))
     got = outs()
+    if algo is not None:
+        m = lib.wkv6_backward_workspace_bytes_ex(code, algo, B, T, C, H)
+        ws2 = torch.empty(max(m, 16), dtype=torch.uint8, device="cuda")
+        native.check(lib.wkv6_backward_ex(st, code, algo, B, T, C, H, P(r), P(k), P(v), P(w), P(u), P(gy), *[P(x) for x in got], P(ws2), m))
+        torch.cuda.synchronize()
+        return got, want
 
     def call():
         native.check(lib.wkv6_backward_static(st, code, B, T, C, H, P(r), P(k), P(v), P(w), P(u), P(gy), *[P(x) for x in got]))
@@ -88,6 +94,24 @@ def test_static_scratch_backward_takes_the_smaller_workspace_when_only_that_fits
     torch.cuda.synchronize()
     for name, a, b in zip("gr gk gv gw gu".split(), got, want):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 8191, 32), (2, 4001, 32), (1, 8192, 32)])
+def test_static_scratch_backward_runs_in_one_piece_where_segments_do_not_fit(B, T, H):
+    # a long sequence of few pairs: its segments' states (72 MiB) do not fit the array, the chunk states alone (64 MiB) do,
+    # and the call stays on the chunked kernels, which differ from the per-timestep ones by bf16 operands
+    from rwkv_kernel import _native
+
+    lib = _native.load()
+    torch.cuda.set_device(0)
+    C = H * 64
+    assert lib.wkv6_backward_workspace_bytes(_native.BF16, B, T, C, H) > _native.STATIC_SCRATCH_BYTES
+    got, want = _pair(lib, _native, B, T, H, torch.bfloat16, 7)
+    exact, _ = _pair(lib, _native, B, T, H, torch.bfloat16, 7, algo=_native.ALGO_SCAN)
+    for name, a, b, c in zip("gr gk gv gw gu".split(), got, want, exact):
+        assert float((a.float() - b.float()).norm() / b.float().norm()) <= 1e-2, name
+        assert float((a.float() - c.float()).norm() / c.float().norm()) <= 1e-2, name
+        assert not torch.equal(a, c), name
 
 
 def test_static_scratch_backward_refuses_what_does_not_fit():
