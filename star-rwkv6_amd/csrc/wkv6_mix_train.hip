@@ -863,12 +863,14 @@ hipError_t shift_mix_forward(hipStream_t st, int weight_dtype, int64_t B, int64_
     return shift_mix_five(st, B, T, C, R, x, h, w.w, bias, out);
 }
 
-// how the tokens are cut for mix_grads_kernel: runs of two ranges each, enough workgroups for the chip and no more (a
-// partial of every weight gradient per run)
+// how the tokens are cut for mix_grads_kernel: runs of two ranges each, as many as the chip holds at once and no more (a
+// partial of every weight gradient per run; and a workgroup's LDS leaves no room for a second one on its compute unit, so
+// that one workgroup too many is a second round of full length).  Backward at 8192 tokens, one run less than needed to give
+// every compute unit something / one more than fits: H12 68 / 91 us, H24 104 / 137, H40 198 / 251, H48 231 / 300.
 struct MixCut {
     int nruns, steps;
     MixCut(int64_t n, int64_t C) {
-        const int64_t groups = C / 64, want = (compute_units() + groups - 1) / groups;      // runs that fill the chip once
+        const int64_t groups = C / 64, fit = compute_units() / groups, want = fit > 1 ? fit : 1;   // runs that the chip holds at once
         const int64_t most = (n + 2 * kGradTok - 1) / (2 * kGradTok);                       // runs of one step per range
         const int64_t runs = want < most ? want : most;
         steps = (int)((n + runs * 2 * kGradTok - 1) / (runs * 2 * kGradTok));

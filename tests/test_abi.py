@@ -138,6 +138,19 @@ def test_missing_library_fails_loudly(native, monkeypatch):
         native.load()
 
 
+@pytest.mark.parametrize("H", [1, 3, 8, 12, 24, 32, 40, 48, 64, 100, 257])
+@pytest.mark.parametrize("tokens", [1, 100, 8192, 200000])
+def test_input_side_backward_is_one_round_of_workgroups(native, H, tokens):
+    """A workgroup of the weight gradients' kernel has a compute unit to itself (its LDS), so one workgroup too many is a
+    second round of full length.  Their number follows from the workspace: per run of tokens a partial of both weights'
+    gradients (160 rows each), two of the biases' (5) and of the mix's, and two times two rows at the ranges' ends."""
+    lib, C, R = native.load(), H * 64, 32
+    gpre = (tokens * 5 * R * 2 + 255) // 256 * 256
+    runs, rest = divmod(lib.wkv6_shift_mix_backward_workspace_bytes(native.BF16, 1, tokens, C, R) - gpre, C * 4 * (160 + 160 + 2 * 5 + 2 + 4))
+    assert rest == 0 and runs >= 1
+    assert runs == 1 or runs * H <= 256
+
+
 def _scratch_bytes(library, directory):
     """Bytes of scratch memory per lane of every kernel in the library, from its code objects' own notes."""
     blob = open(library, "rb").read()
