@@ -110,12 +110,18 @@ template <int R, bool kGrads> struct MixBlock {
 };
 
 // The five outputs of a 16-token block go through LDS ([mixer][token][128 channels], two blocks in turn) so that every
-// store covers whole 256-byte pieces of rows, and past the caches: nothing reads them before they would be evicted.
+// store covers whole 256-byte pieces of rows.
 // Bound by the stores: at B8 T1024 C2048 R32 52 us with 64-byte pieces stored straight from the MFMA layout, 40 us so
-// (the same traffic with nothing computed: 32 us); and x, no longer displaced by them, is still in the last-level cache
-// when the backward begins (60 -> 50 us for its first kernel).
+// (the same traffic with nothing computed: 32 us).
+// Large outputs go past the caches (kPast): what reads them next, the layer's projections, finds them in memory either way,
+// and x, no longer displaced by them, is still in the last-level cache when the backward begins (60 -> 50 us for its
+// first kernel).  Up to a quarter of that cache (256 MB) they stay: the projections then read them from there.  This kernel
+// and five C x C projections, ordinary stores against past the caches: 5 MB of outputs (C1024) 78.5 / 87.5 us, 21 MB (C512)
+// 81.1 / 87.6, 61 MB (C2048) 183.7 / 187.0, 84 MB (C4096) 408 / 402, 168 MB (C2048) 359 / 352; a step of the model (168 MB)
+// 134.6 / 134.1 ms.
+constexpr int64_t kMixCached = (int64_t)64 << 20;   // bytes of outputs
 constexpr int kMixOutPitch = 128 + 8;   // elements: eight token rows on eight different bank groups
-template <int R>
+template <int R, bool kPast>
 __global__ __launch_bounds__(256) void shift_mix5_fwd_kernel(int64_t n_tok, int T, int C,
         const bf16_t *__restrict__ x, const bf16_t *__restrict__ h, const bf16_t *__restrict__ w2t, const float *__restrict__ bias,
         bf16_t *__restrict__ o0, bf16_t *__restrict__ o1, bf16_t *__restrict__ o2, bf16_t *__restrict__ o3, bf16_t *__restrict__ o4)
@@ -162,8 +168,11 @@ __global__ __launch_bounds__(256) void shift_mix5_fwd_kernel(int64_t n_tok, int 
         if (mine && n0 + 4 * wave + g < n_tok) {
             const size_t e = (size_t)(n0 + 4 * wave + g) * C + cw + 8 * l16;
 #pragma unroll
-            for (int s = 0; s < kMixers; ++s)
-                __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(&rows[tb & 1][s][4 * wave + g][8 * l16]), reinterpret_cast<u32x4 *>(outs[s] + e));
+            for (int s = 0; s < kMixers; ++s) {
+                const u32x4 row = *reinterpret_cast<const u32x4 *>(&rows[tb & 1][s][4 * wave + g][8 * l16]);
+                if (kPast) __builtin_nontemporal_store(row, reinterpret_cast<u32x4 *>(outs[s] + e));
+                else *reinterpret_cast<u32x4 *>(outs[s] + e) = row;
+            }
         }
         if (!more) break;
     }
@@ -342,7 +351,9 @@ hipError_t shift_mix_five(hipStream_t st, int64_t B, int64_t T, int64_t C, int64
         hipLaunchKernelGGL(kernel, mix5_grid(n, C), dim3(256), 0, st, n, (int)T, (int)C, (const bf16_t *)x, (const bf16_t *)h,
                            (const bf16_t *)w2t, bias, (bf16_t *)out[0], (bf16_t *)out[1], (bf16_t *)out[2], (bf16_t *)out[3], (bf16_t *)out[4]);
     };
-    if (R == 32) launch(shift_mix5_fwd_kernel<32>); else launch(shift_mix5_fwd_kernel<64>);
+    const bool past = n * C * kMixers * (int64_t)sizeof(bf16_t) > kMixCached;
+    if (R == 32) past ? launch(shift_mix5_fwd_kernel<32, true>) : launch(shift_mix5_fwd_kernel<32, false>);
+    else past ? launch(shift_mix5_fwd_kernel<64, true>) : launch(shift_mix5_fwd_kernel<64, false>);
     return hipGetLastError();
 }
 

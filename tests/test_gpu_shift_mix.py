@@ -354,6 +354,27 @@ def test_calls_replay_in_a_hip_graph(lib):
                 assert torch.equal(t, eager[n]), (rep, n)
 
 
+@pytest.mark.parametrize("R", [32, 64])
+def test_outputs_past_the_caches_are_the_same(lib, R):
+    """More than 64 MiB of outputs are stored past the caches, fewer through them: sequence by sequence (the second way)
+    gives what all of them at once (the first) give, bit for bit."""
+    from rwkv_kernel import _native
+    B, T, C = 3, 2185, 1088                      # 68.0 MiB together; no multiple of a workgroup's tokens or channels
+    dev, _ = _inputs(B, T, C, R, 6)
+    h = torch.tanh(torch.randn(B, T, 5, R, device="cuda")).to(BF16)
+
+    def five(x, h):
+        outs = [torch.full_like(x, float("nan")) for _ in range(5)]
+        _native.check(lib.wkv6_shift_mix_five(_stream(), _native.BF16, x.shape[0], T, C, R, x.data_ptr(), h.data_ptr(),
+                                              dev["w2t"].data_ptr(), dev["bias"].data_ptr(), *[o.data_ptr() for o in outs]))
+        return outs
+
+    assert 10 * B * T * C > 64 << 20 > 10 * T * C
+    apart = [five(dev["x"][b:b + 1], h[b:b + 1]) for b in range(B)]
+    for i, out in enumerate(five(dev["x"], h)):
+        assert torch.equal(out, torch.cat([a[i] for a in apart]))
+
+
 @pytest.mark.parametrize("B,T,C", [(2, 64, 128), (3, 37, 64), (5, 1, 192), (1, 300, 320)])
 def test_fixed_mix_on_its_own(B, T, C):
     """op.shift_mix_x: x + xx * mix and its gradients (the backward kernel with no gp / gxx) against
