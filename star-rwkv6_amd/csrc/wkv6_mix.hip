@@ -109,29 +109,29 @@ template <int R, bool kGrads> struct MixBlock {
     }
 };
 
-// The five outputs of a 16-token block go through LDS ([mixer][token][128 channels], two blocks in turn) so that every
-// store covers whole 256-byte pieces of rows.
-// Bound by the stores: at B8 T1024 C2048 R32 52 us with 64-byte pieces stored straight from the MFMA layout, 40 us so
-// (the same traffic with nothing computed: 32 us).
-// Large outputs go past the caches (kPast): what reads them next, the layer's projections, finds them in memory either way,
-// and x, no longer displaced by them, is still in the last-level cache when the backward begins (60 -> 50 us for its
-// first kernel).  Up to a quarter of that cache (256 MB) they stay: the projections then read them from there.  This kernel
-// and five C x C projections, ordinary stores against past the caches: 5 MB of outputs (C1024) 78.5 / 87.5 us, 21 MB (C512)
-// 81.1 / 87.6, 61 MB (C2048) 183.7 / 187.0, 84 MB (C4096) 408 / 402, 168 MB (C2048) 359 / 352; a step of the model (168 MB)
-// 134.6 / 134.1 ms.
+// Bound by the stores.  kStaged: the five outputs of a 16-token block go through LDS ([mixer][token][128 channels], two blocks
+// in turn) so that every store covers whole 256-byte pieces of rows, and past the caches: what reads such outputs next, the
+// layer's projections, finds them in memory either way, and x, no longer displaced by them, is still in the last-level cache when
+// the backward begins (60 -> 50 us for its first kernel).  Otherwise 64-byte pieces straight from the MFMA layout, into the caches.
+// Staged for rank 32 and more than a quarter of that cache (256 MB) of outputs.  This kernel alone / with five C x C projections
+// behind it, direct against staged, R32: 42 MB (T2048 C2048) 19.6 / 137.8 us against 18.5 / 143.4, 84 MB (T4096 C2048) 28.3 / 208.2
+// against 25.0 / 208.8, 168 MB (T8192 C2048) 46.7 / 374 against 43.3 / 364 (a step of the model: 134.6 ms through the caches, 134.1
+// past them).  R64, whose weights fill the registers: 42 MB 27.0 / 144.4 against 27.3 / 152.2, 168 MB 74.6 / 390 against 74.9 / 387.
+// Two workgroups per compute unit have to fit their registers: with 264 of them at rank 64 there is room for one, 97 us.
 constexpr int64_t kMixCached = (int64_t)64 << 20;   // bytes of outputs
 constexpr int kMixOutPitch = 128 + 8;   // elements: eight token rows on eight different bank groups
-template <int R, bool kPast>
-__global__ __launch_bounds__(256) void shift_mix5_fwd_kernel(int64_t n_tok, int T, int C,
+template <int R, bool kStaged>
+__global__ __launch_bounds__(256, 2) void shift_mix5_fwd_kernel(int64_t n_tok, int T, int C,
         const bf16_t *__restrict__ x, const bf16_t *__restrict__ h, const bf16_t *__restrict__ w2t, const float *__restrict__ bias,
         bf16_t *__restrict__ o0, bf16_t *__restrict__ o1, bf16_t *__restrict__ o2, bf16_t *__restrict__ o3, bf16_t *__restrict__ o4)
 {
-    __shared__ __align__(16) bf16_t rows[2][kMixers][16][kMixOutPitch];
+    __shared__ __align__(16) bf16_t rows[2][kMixers][kStaged ? 16 : 1][kMixOutPitch];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
     const int ncg = (C + kMixGroupCh - 1) / kMixGroupCh;   // workgroups side by side over the channels: neighbours share token rows
     const int cw = (int)(blockIdx.x % ncg) * kMixGroupCh, c0 = cw + wave * kMixWaveCh;
     const int64_t first = (int64_t)(blockIdx.x / ncg) * (16 * kMixTokBlocks);
     const bool live = c0 < C;
+    if (!kStaged && !live) return;   // (staged: a wave without channels of its own still stores rows)
     MixWeights<R> wt;
     MixBlock<R, false> cur, nxt;
     bf16_t *const outs[kMixers] = {o0, o1, o2, o3, o4};
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void shift_mix5_fwd_kernel(int64_t n_tok, int 
         wt.load(w2t, bias, C, c0, l16, g);
         cur.load(first, n_tok, T, C, c0, l16, g, x, h, none);
     }
-    // stored by this lane: token row 4 wave + g of the block, channels 8 l16 .. of the workgroup's 128
+    // staged: stored by this lane are token row 4 wave + g of the block, channels 8 l16 .. of the workgroup's 128
     const bool mine = cw + 8 * l16 < C;
     for (int tb = 0; tb < kMixTokBlocks; ++tb) {
         const int64_t n0 = first + 16 * tb, n1 = n0 + 16;
@@ -160,18 +160,18 @@ __global__ __launch_bounds__(256) void shift_mix5_fwd_kernel(int64_t n_tok, int 
 #pragma unroll
                     for (int e = 0; e < 4; ++e) o[m][e] = fmaf(xx[m][e], acc[e], xv[m][e]);
                 }
-                store8(&rows[tb & 1][s][l16][wave * kMixWaveCh + 8 * g], o);
+                if (kStaged) store8(&rows[tb & 1][s][l16][wave * kMixWaveCh + 8 * g], o);
+                else if (cur.valid) store8(outs[s] + cur.e0, o);
             }
             cur = nxt;
         }
-        __syncthreads();   // (the block two before has left this buffer: its stores' reads were behind the last barrier)
-        if (mine && n0 + 4 * wave + g < n_tok) {
-            const size_t e = (size_t)(n0 + 4 * wave + g) * C + cw + 8 * l16;
+        if (kStaged) {
+            __syncthreads();   // (the block two before has left this buffer: its stores' reads were behind the last barrier)
+            if (mine && n0 + 4 * wave + g < n_tok) {
+                const size_t e = (size_t)(n0 + 4 * wave + g) * C + cw + 8 * l16;
 #pragma unroll
-            for (int s = 0; s < kMixers; ++s) {
-                const u32x4 row = *reinterpret_cast<const u32x4 *>(&rows[tb & 1][s][4 * wave + g][8 * l16]);
-                if (kPast) __builtin_nontemporal_store(row, reinterpret_cast<u32x4 *>(outs[s] + e));
-                else *reinterpret_cast<u32x4 *>(outs[s] + e) = row;
+                for (int s = 0; s < kMixers; ++s)
+                    __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(&rows[tb & 1][s][4 * wave + g][8 * l16]), reinterpret_cast<u32x4 *>(outs[s] + e));
             }
         }
         if (!more) break;
@@ -351,9 +351,9 @@ hipError_t shift_mix_five(hipStream_t st, int64_t B, int64_t T, int64_t C, int64
         hipLaunchKernelGGL(kernel, mix5_grid(n, C), dim3(256), 0, st, n, (int)T, (int)C, (const bf16_t *)x, (const bf16_t *)h,
                            (const bf16_t *)w2t, bias, (bf16_t *)out[0], (bf16_t *)out[1], (bf16_t *)out[2], (bf16_t *)out[3], (bf16_t *)out[4]);
     };
-    const bool past = n * C * kMixers * (int64_t)sizeof(bf16_t) > kMixCached;
-    if (R == 32) past ? launch(shift_mix5_fwd_kernel<32, true>) : launch(shift_mix5_fwd_kernel<32, false>);
-    else past ? launch(shift_mix5_fwd_kernel<64, true>) : launch(shift_mix5_fwd_kernel<64, false>);
+    if (R == 64) launch(shift_mix5_fwd_kernel<64, false>);
+    else if (n * C * kMixers * (int64_t)sizeof(bf16_t) > kMixCached) launch(shift_mix5_fwd_kernel<32, true>);
+    else launch(shift_mix5_fwd_kernel<32, false>);
     return hipGetLastError();
 }
 
