@@ -450,6 +450,8 @@ PYBIND11_MODULE(_wkv6_torch, m) {
     return unlocked([&] { return Wkv6GnGate::apply(r, k, v, w, u, gate, scale, offset, H, eps); });
   });
   m.def("shift_mix", [](const Tensor &x, const Tensor &mix_x, const Tensor &a, const Tensor &w2t, const Tensor &bias) {
+    for (const Tensor *t : {&mix_x, &a, &w2t, &bias})
+      TORCH_CHECK(t->device() == x.device(), "wkv6: x and the mixers' parameters must be on one device");   // (the kernels take addresses)
     const variable_list o = unlocked([&] { return ShiftMix::apply(x, mix_x, a, w2t, bias); });
     return py::make_tuple(wrap(o[0]), wrap(o[1]), wrap(o[2]), wrap(o[3]), wrap(o[4]));
   });

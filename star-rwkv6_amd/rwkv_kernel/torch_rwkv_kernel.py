@@ -281,7 +281,6 @@ class RWKVKernelOperator:
         assert x.is_contiguous() and mix_x.numel() == C
         R = w2t.shape[2]
         assert a.shape == (5 * R, C) and w2t.shape == (5, C, R) and bias.shape == (5, C)
-        assert x.device == mix_x.device == a.device == w2t.device == bias.device, "x and the mixers' parameters must be on one device"
         assert self.shift_mix_supported(x, R), "shift_mix takes bf16 tensors on the GPU with rank 32 or 64"
         return self._torch.shift_mix(x, mix_x.reshape(C), a, w2t, bias)
 

@@ -243,7 +243,7 @@ def test_parameters_on_another_device_are_refused():
     args = [dev[k] for k in ("x", "mix_x", "a", "w2t", "bias")]
     assert len(op.shift_mix(*args)) == 5
     for i in range(1, 5):
-        with pytest.raises(AssertionError, match="one device"):
+        with pytest.raises(RuntimeError, match="one device"):
             op.shift_mix(*[t.cpu() if i == j else t for j, t in enumerate(args)])
     with pytest.raises(AssertionError, match="one device"):
         op.shift_mix_x(args[0], args[1].cpu())
