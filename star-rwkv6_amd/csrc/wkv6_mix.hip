@@ -113,11 +113,12 @@ template <int R, bool kGrads> struct MixBlock {
 // in turn) so that every store covers whole 256-byte pieces of rows, and past the caches: what reads such outputs next, the
 // layer's projections, finds them in memory either way, and x, no longer displaced by them, is still in the last-level cache when
 // the backward begins (60 -> 50 us for its first kernel).  Otherwise 64-byte pieces straight from the MFMA layout, into the caches.
-// Staged for rank 32 and more than a quarter of that cache (256 MB) of outputs.  This kernel alone / with five C x C projections
-// behind it, direct against staged, R32: 42 MB (T2048 C2048) 19.6 / 137.8 us against 18.5 / 143.4, 84 MB (T4096 C2048) 28.3 / 208.2
+// Staged for more than a quarter of that cache (256 MB) of outputs.  This kernel alone / with five C x C projections behind it,
+// direct against staged, R32: 42 MB (T2048 C2048) 19.6 / 137.8 us against 18.5 / 143.4, 84 MB (T4096 C2048) 28.3 / 208.2
 // against 25.0 / 208.8, 168 MB (T8192 C2048) 46.7 / 374 against 43.3 / 364 (a step of the model: 134.6 ms through the caches, 134.1
-// past them).  R64, whose weights fill the registers: 42 MB 27.0 / 144.4 against 27.3 / 152.2, 168 MB 74.6 / 390 against 74.9 / 387.
-// Two workgroups per compute unit have to fit their registers: with 264 of them at rank 64 there is room for one, 97 us.
+// past them).  R64: 42 MB 27.0 / 144.4 against 27.3 / 152.2, 168 MB 74.6 / 390 against 74.9 / 387, forward and backward of the
+// call 449 against 425.  Two workgroups per compute unit have to fit their registers: with the 264 that rank 64 takes unasked there
+// is room for one, 96 us.
 constexpr int64_t kMixCached = (int64_t)64 << 20;   // bytes of outputs
 constexpr int kMixOutPitch = 128 + 8;   // elements: eight token rows on eight different bank groups
 template <int R, bool kStaged>
@@ -351,9 +352,9 @@ hipError_t shift_mix_five(hipStream_t st, int64_t B, int64_t T, int64_t C, int64
         hipLaunchKernelGGL(kernel, mix5_grid(n, C), dim3(256), 0, st, n, (int)T, (int)C, (const bf16_t *)x, (const bf16_t *)h,
                            (const bf16_t *)w2t, bias, (bf16_t *)out[0], (bf16_t *)out[1], (bf16_t *)out[2], (bf16_t *)out[3], (bf16_t *)out[4]);
     };
-    if (R == 64) launch(shift_mix5_fwd_kernel<64, false>);
-    else if (n * C * kMixers * (int64_t)sizeof(bf16_t) > kMixCached) launch(shift_mix5_fwd_kernel<32, true>);
-    else launch(shift_mix5_fwd_kernel<32, false>);
+    const bool staged = n * C * kMixers * (int64_t)sizeof(bf16_t) > kMixCached;
+    if (R == 32) staged ? launch(shift_mix5_fwd_kernel<32, true>) : launch(shift_mix5_fwd_kernel<32, false>);
+    else staged ? launch(shift_mix5_fwd_kernel<64, true>) : launch(shift_mix5_fwd_kernel<64, false>);
     return hipGetLastError();
 }
 

@@ -356,8 +356,8 @@ def test_calls_replay_in_a_hip_graph(lib):
 
 @pytest.mark.parametrize("R", [32, 64])
 def test_outputs_past_the_caches_are_the_same(lib, R):
-    """At rank 32 more than 64 MiB of outputs go through LDS and past the caches, fewer straight into them: sequence by
-    sequence (the second way) gives what all of them at once (the first) give, bit for bit."""
+    """More than 64 MiB of outputs go through LDS and past the caches, fewer straight into them: sequence by sequence (the
+    second way) gives what all of them at once (the first) give, bit for bit."""
     from rwkv_kernel import _native
     B, T, C = 3, 2185, 1088                      # 68.0 MiB together; no multiple of a workgroup's tokens or channels
     dev, _ = _inputs(B, T, C, R, 6)
