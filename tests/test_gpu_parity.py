@@ -890,7 +890,7 @@ def test_every_number_of_segments(op, oracle, P):
 
 
 def test_segments_add_up_the_bonus_gradient_unrounded(op, oracle):
-    # gu of a sequence in segments is rounded to bf16 once: half an ulp (2^-9 relative) of every value, no more but
+    # gu of a sequence in segments is rounded to bf16 once: half an ulp (up to 2^-8 relative) of every value, no more but
     # for the operands' own rounding, whose share falls with the 1031 tokens that are summed
     B, T, H = 1, 1031, 4
     ins = oracle.make_inputs(B, T, H, 64, 5)
@@ -909,9 +909,9 @@ def test_segments_round_the_bonus_gradient_once(op, oracle, T, H, wild, call):
     """gu of a bf16 sequence in segments (tile form, one redone segment, block form) in the training pair, in a second
     backward over one graph, with gradients through the state and as the row of the batch: half a unit in the last place
     from the exact sum, plus what the terms bring along.  A term r k <v,gy> is formed from four bf16 operands (r and k
-    times a scale factor, and the factors), each off by up to 2^-9, by 2^-9 / sqrt 3 in the root mean square: 2.3e-3
-    together.  Over T terms of one sign, products of half normals ((E x^2)^(1/2) / E x <= 1.6), that is 3.6e-3 / sqrt T of
-    the sum and, where a unit is smallest (2^-8 of the value), 0.92 / sqrt T units; five times that is allowed."""
+    times a scale factor, and the factors), each off by up to 2^-8, by 1.7e-3 in the root mean square: 3.3e-3 together.  Over
+    T terms of one sign, products of half normals ((E x^2)^(1/2) / E x <= 1.6), that is 5.2e-3 / sqrt T of the sum and,
+    where a unit is smallest (2^-8 of the value), 1.33 / sqrt T units; four times that is allowed."""
     from rwkv_kernel import _native
 
     ins = oracle.make_inputs(1, T, H, 64, 5)
@@ -942,7 +942,7 @@ def test_segments_round_the_bonus_gradient_once(op, oracle, T, H, wild, call):
     unit = 2.0 ** (np.floor(np.log2(np.abs(want))) - 7)
     worst = (np.abs(to_np(gu).reshape(-1) - want) / unit).max()
     print("gu %s T=%d H=%d: %.3f units" % (call, T, H, worst), flush=True)
-    assert worst <= 0.5 + 4.6 / T ** 0.5
+    assert worst <= 0.5 + 5.3 / T ** 0.5
 
 
 def test_training_pair_in_time_segments_with_fallback_segments(op, oracle):
