@@ -351,9 +351,10 @@ hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B
 // states-only pass over all segments at once, the chain, and the saving forward from every segment's true state.  The
 // decay of a segment is carried as the product of its chunks' e^{c_32} themselves, not as an exponent.
 // Without segments a pair's chunks follow each other in one workgroup whatever else is idle.  Forward and backward, before and
-// now: fp32 B1 T8191 H32 2317 -> 449 us, B2 T2048 H16 580 -> 129, B1 T1031 H64 307 -> 144, B2 T1024 H64 (128 pairs, not
-// taken by the rule: two segments only from 2048 tokens on) 310 -> 269 from the kernels alone; fp16 B1 T5003 H8 1420 -> 181, B4
-// T2100 H32 704 -> 520.
+// now: fp32 B1 T8191 H32 2317 -> 441 us, B2 T2048 H16 580 -> 126, B1 T1031 H64 307 -> 144; fp16 B1 T5003 H8 1420 -> 167, B4
+// T2100 H32 704 -> 521.  Two or three segments only from 2048 tokens on, as in the bf16 forms; below, where the line has not been
+// looked for, they would gain as well: fp32 pair in one piece / in segments, B2 T1024 H64 276 / 235 us, B2 T1999 H64 534 / 441,
+// B3 T1024 H24 258 / 172.
 // ------------------------------------------------------------------------------------------
 int chunk32_train_segments(int64_t B, int64_t T, int64_t H, int64_t *L) {
     if (T < 1024) return 1;

@@ -808,9 +808,9 @@ static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, cons
 // Segments of a sequence of T tokens when `pairs` (batch, head) pairs share the chip: as many as still fit it once, each a
 // whole number of chunks and at least `least` of them; the last one ends with the sequence.  (Segments that had to
 // divide the sequence left training at all other lengths to one workgroup per pair; a prompt's tokens behind its equal
-// segments took a pass of their own.  Forward and backward at H32: B1 T8191 771 -> 193 us, B1 T2049 211 -> 93, B4 T4001
-// 427 -> 338; H8 B1 T5003 475 -> 110; prompts of H32: T1337 38 -> 24.5 us, T1024 37 -> 23 (six segments of three chunks
-// instead of four of four), T3000 with the output stage 57 -> 37.)
+// segments took a pass of their own.  Forward and backward at H32: B1 T8191 771 -> 176 us, B1 T2049 211 -> 87, B4 T4001
+// 427 -> 326; H8 B1 T5003 475 -> 88; prompts of H32: T1337 38 -> 23 us, T1024 37 -> 22 (six segments of three chunks
+// instead of four of four), T3000 with the output stage 57 -> 36.)
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
     const int64_t chunks = (T + CL - 1) / CL, fit = compute_units() / pairs;
     const int64_t most = fit < kMostSegments ? fit : kMostSegments;
@@ -891,7 +891,9 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 // ------------------------------------------------------------------------------------------
 static int train_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
     // (two state-only passes at 0.7 of a forward each on top of the forward and the backward: 1.5
-    // times the work on P times the workgroups, and three small kernels)
+    // times the work on P times the workgroups, and three small kernels.  Two or three segments only from 2048 tokens on;
+    // below they would gain less, but gain: kernels in one piece / in segments, B2 T1024 H64 109 / 104 us, B2 T1999 H64 214 / 174,
+    // B3 T1024 H24 107 / 87)
     if (T < 1024) return 1;
     const int P = plan_segments(B * H, T, 4, L);
     return T >= 2048 || P >= 4 ? P : 1;

@@ -11,7 +11,8 @@
 // a lane's channels stay the same over all its tokens, so the sums for scale and offset stay in registers.  Four tokens'
 // rows are in flight per wave.  What is not read again soon (gout, y, gate, ggate) goes past the caches, gy is the next
 // kernel's input (the gate's own backward, which reads ggate next, takes as long with it in the caches: within 3 % either way from 256 to 16384
-// tokens of H32).  B8 T1024 H32, 168 MB: 32.5 us = 5.2 TB/s (one head per wave, 2 bytes per lane: 49 us).
+// tokens of H32).  B8 T1024 H32, 168 MB: 31 us = 5.5 TB/s behind the forward that
+// wrote y, 41 us with nothing of it cached (one head per wave, 2 bytes per lane: 49 and 55 us).
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
 

@@ -14,8 +14,9 @@
 // workgroup, so the gradients g_s are read twice: mix_reduce_kernel<grad> takes whole rows of a few tokens (gpre
 // complete, nothing to combine between workgroups), mix_grads_kernel takes 64 channels of many tokens (the weight
 // gradients stay in accumulators, one partial per workgroup).
-// B8 T1024 C2048 R32, forward and backward: 195 us of kernels; as four elementwise kernels around six library products
-// (gcoef written and read twice, x_mix written and read) 504 us, of which 235 us the skinny products.
+// B8 T1024 C2048, forward and backward: 182 us of kernels at R32 (x and the gradients read twice more than once: 501 MB in, 232 MB
+// out), 431 us at R64; R32 as four elementwise kernels around six library products (gcoef written and read twice, x_mix
+// written and read) 504 us, of which 235 us the skinny products.
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
 #include "wkv6_mfma.h"
@@ -137,8 +138,9 @@ __device__ __forceinline__ float tanh_bf16(float x) {
 // One workgroup takes all channels of 32 tokens (16 at R = 64: the accumulators), so nothing is left to combine; its
 // eight waves take 32-channel chunks in turn and add up through LDS at the end.  The weights' fragments come from L2 once
 // per workgroup (16 tokens per workgroup, i.e. twice that traffic: 30 and 73 us instead of 21 and 50).  A chunk's x and
-// g are fetched while the chunk before it is worked on.  B8 T1024 C2048 R32: 21 us forward, latencies of a launch of one
-// workgroup per compute unit (12 us with nothing fetched in the loop); 50 us backward for 201 MB read.
+// g are fetched while the chunk before it is worked on.  B8 T1024 C2048 in a pass, R32: 17 us forward, latencies of a launch of one
+// workgroup per compute unit (12 us with nothing fetched in the loop); 41 us backward for 204 MB read, part of it still in the
+// last-level cache.  R64: 39 and 58 us.
 // ------------------------------------------------------------------------------------------
 constexpr int kReduceWaves = 8;
 template <int R> struct MixReduce {
@@ -302,9 +304,10 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
 //   W waves:   gcoef, transposed through a tile of their own in LDS (the transposing read), for gW and gbias;
 //   A waves:   x_mix, the same way, for gA; they also bring the h and gpre rows that all roles read from LDS.
 // (The roles read the same x and g: the later reads find the lines in L1 or L2.  One wave doing everything had a SIMD to
-// itself for its 440 registers and every LDS and MFMA latency in the open: 84 us at B8 T1024 C2048 R32 against 74 so.  The
+// itself for its 440 registers and every LDS and MFMA latency in the open: 84 us at B8 T1024 C2048 R32 against 75 so.  The
 // traffic alone, 256 MB, would take 50 us; the roles alone take 45, 44 and 32 us: vector instructions and LDS on top.)
-// R = 64: a second launch without gx waves (kGx false) does the other half of the rank's columns.
+// R = 64: a second launch without gx waves (kGx false) does the other half of the rank's columns: 181 + 63 us, with 39 registers
+// of the first in scratch memory (3 at R = 32).
 // ------------------------------------------------------------------------------------------
 constexpr int kGradTok = 32;
 template <int R, bool kGx> struct MixGrads {
