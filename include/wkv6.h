@@ -290,7 +290,7 @@ int wkv6_backward_saved(void *stream, int dtype, int algo, int64_t B, int64_t T,
 
 /* wkv6_backward_saved with the batch sum of gu fused in: gu (B,C) still receives the per-batch
  * partials, gu_sum (C elements, output type) their sum over the batch, added up in fp32 from the
- * stored partials -- the value `gu = torch.sum(gu, 0)` gives the caller in
+ * stored partials (where a sequence runs in segments: from the segments' unrounded fp32 rows) -- the value `gu = torch.sum(gu, 0)` gives the caller in
  * rwkv_kernel/torch_rwkv_kernel.py:73 (rwkv_kernel/jax_rwkv_kernel.py:166), without the extra
  * kernel.  `saved` must come from wkv6_forward_save of the same shape (it carries per-head arrival
  * counters, which the call leaves ready for another backward on the same buffer). */

@@ -5,7 +5,7 @@
     y, state = op(r, k, v, w, u, return_state=False, init_state=None, state_map=None)
 
 The flavour is picked by the KERAS_BACKEND environment variable, which must be set, exactly as
-the reference does (rwkv_kernel/__init__.py:2-11): "torch" -> torch autograd.Function over the
+the reference does (rwkv_kernel/__init__.py:2-11): "torch" -> native torch autograd nodes over the
 gfx950 library, "jax" -> jax custom_vjp over the same library's XLA custom-call targets, anything
 else -> the portable python-loop operator, which is also always exported as OPSKernelOperator.
 
