@@ -300,6 +300,15 @@ int wkv6_backward_saved_sum(void *stream, int dtype, int algo, int64_t B, int64_
                             void *gr, void *gk, void *gv, void *gw, void *gu, void *gu_sum,
                             void *saved, size_t saved_bytes);
 
+/* The same with the type of gr, gk, gv, gw and gu_sum as an argument: the output type, or for fp16 tensors WKV6_F16, the fp32
+ * gradients rounded once where they are stored (gu keeps its fp32 partials); fp16 gradients only on the full-precision chunk
+ * form (WKV6_ERR_UNSUPPORTED elsewhere: WKV6_ALGO_CHUNK, WKV6_ALGO_SCAN, shapes with wkv6_saved_bytes() = 0). */
+int wkv6_backward_saved_sum_ex(void *stream, int dtype, int grad_dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H,
+                               const void *r, const void *k, const void *v, const void *w, const void *u,
+                               const void *gy,
+                               void *gr, void *gk, void *gv, void *gw, void *gu, void *gu_sum,
+                               void *saved, size_t saved_bytes);
+
 /* Backward with gradients through the state (no counterpart in the reference, whose backward is
  * defined for the stateless call only, rwkv_kernel/torch_rwkv_kernel.py:100-168; it is what carrying
  * the state across calls, rwkv_kernel/__init__.py:14-38, needs for truncated back-propagation over

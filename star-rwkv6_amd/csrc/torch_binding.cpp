@@ -129,13 +129,16 @@ std::vector<Tensor> wkv6_grads(const Dims &d, int algo, const Tensor &r, const T
   const int code = code_of(r.scalar_type());
   const ScalarType ot = out_type(r.scalar_type());
   const at::DimVector big{B, T, C};
-  std::vector<Tensor> g = carve(r, {{big, ot, 7}, {big, ot, 8}, {big, ot, 9}, {big, ot, 10}, {{B, C}, ot, 0}});
+  // torch hands the gradient of an fp16 tensor on as fp16 whatever a node returns, in a kernel per gradient: the library
+  // rounds where it stores them, where its kernels can
+  const ScalarType gt = saved.defined() && algo != kChunk ? r.scalar_type() : ot;
+  std::vector<Tensor> g = carve(r, {{big, gt, 7}, {big, gt, 8}, {big, gt, 9}, {big, gt, 10}, {{B, C}, ot, 0}});
   const Tensor gu_rows = std::move(g[4]);
   if (saved.defined()) {
-    g[4] = parameter_gradient(r, u.sizes(), ot);
+    g[4] = parameter_gradient(r, u.sizes(), gt);
     // the batch sum of u's gradient (rwkv_kernel/torch_rwkv_kernel.py:73 of the reference) comes out of the same launch
-    check(wkv6_backward_saved_sum(stream_of(r), code, algo, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gy), out(g[0]),
-                                  out(g[1]), out(g[2]), out(g[3]), out(gu_rows), out(g[4]), out(saved), saved.numel()));
+    check(wkv6_backward_saved_sum_ex(stream_of(r), code, code_of(gt), algo, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gy),
+                                     out(g[0]), out(g[1]), out(g[2]), out(g[3]), out(gu_rows), out(g[4]), out(saved), saved.numel()));
     return g;
   }
   const size_t n = wkv6_backward_workspace_bytes_ex(code, algo, B, T, C, H);

@@ -488,7 +488,9 @@ static int backward_segments_impl(void *stream, int dtype, int algo, int64_t B, 
 static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                          void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, size_t workspace_bytes,
-                         bool states_ready, void *gu_sum = nullptr, bool one_piece = false) {
+                         bool states_ready, void *gu_sum = nullptr, bool one_piece = false, int grad_dtype = -1) {
+    // grad_dtype: type of gr, gk, gv, gw and gu_sum where it is not the output type (the full-precision chunk form's training pair only)
+    if (grad_dtype < 0) grad_dtype = out_type(dtype);
     int rc = check_shape_any(dtype, B, T, C, H);
     if (rc != WKV6_OK && rc != kSmallHead) return rc;
     if (!r || !k || !v || !w || !u || !gy || !gr || !gk || !gv || !gw || !gu) return WKV6_ERR_ARG;
@@ -501,7 +503,7 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
     if (rc == kSmallHead) {
         if (algo == WKV6_ALGO_CHUNK) return WKV6_ERR_UNSUPPORTED;
         rc = finish(wkv6::generic_backward(st, dtype, B, T, H, C / H, r, k, v, w, u, nullptr, gy, nullptr, gr, gk, gv, gw, gu, nullptr, workspace));
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
+        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
         return rc;
     }
     if (train_chunk32(dtype, algo, B, T, H)) {
@@ -512,11 +514,11 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
         }
         if (states_ready && train_segments32(dtype, algo, B, T, H) > 1) {
             if (workspace_bytes < wkv6_saved_bytes(dtype, algo, B, T, C, H)) return WKV6_ERR_WORKSPACE;
-            rc = finish(wkv6::chunk32_backward_saved_segments(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+            rc = finish(wkv6::chunk32_backward_saved_segments(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
         } else {
-            rc = finish(wkv6::chunk32_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+            rc = finish(wkv6::chunk32_backward(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
         }
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
+        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
         return rc;
     }
     if (algo == WKV6_ALGO_CHUNK && !chunk_possible(dtype, T, C)) return WKV6_ERR_UNSUPPORTED;
@@ -524,7 +526,7 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     if (!chunk) {
         rc = finish(wkv6::scan_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
+        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
         return rc;
     }
     if (!states_ready && !one_piece && train_segments(dtype, algo, B, T, C, H) > 1) {
@@ -593,6 +595,21 @@ int wkv6_backward_saved_sum(void *stream, int dtype, int algo, int64_t B, int64_
                          need > 0, gu_sum);
 }
 
+int wkv6_backward_saved_sum_ex(void *stream, int dtype, int grad_dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H,
+                               const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
+                               void *gr, void *gk, void *gv, void *gw, void *gu, void *gu_sum,
+                               void *saved, size_t saved_bytes) {
+    if (grad_dtype == out_type(dtype))
+        return wkv6_backward_saved_sum(stream, dtype, algo, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, gu_sum, saved, saved_bytes);
+    const int rc = check_shape(dtype, B, T, C, H);
+    if (rc != WKV6_OK) return rc;
+    if (!gu_sum || grad_dtype != dtype || algo < WKV6_ALGO_AUTO || algo > WKV6_ALGO_CHUNK) return WKV6_ERR_ARG;
+    if (!train_chunk32(dtype, algo, B, T, H)) return WKV6_ERR_UNSUPPORTED;
+    if (saved_bytes < wkv6_saved_bytes(dtype, algo, B, T, C, H)) return WKV6_ERR_WORKSPACE;
+    return backward_impl(stream, dtype, algo, B, T, C, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, saved, saved_bytes, true, gu_sum,
+                         false, grad_dtype);
+}
+
 // where the pairs' final states sit in the workspace of a full-precision backward with state gradients
 static size_t state32_offset(int64_t B, int64_t T, int64_t H) { return (wkv6::chunk32_saved_bytes(B, T, H) + 255) & ~(size_t)255; }
 
@@ -635,7 +652,7 @@ int wkv6_backward_with_state(void *stream, int dtype, int algo, int64_t B, int64
         float *sT = gsT ? reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + state32_offset(B, T, H)) : nullptr;
         const hipError_t e = wkv6::chunk32_forward(st, dtype, WKV6_F32, B, T, H, r, k, v, w, u, s0, nullptr, nullptr, sT, workspace);
         if (e != hipSuccess) return finish(e);
-        return finish(wkv6::chunk32_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, s0, gsT, sT, gs0));
+        return finish(wkv6::chunk32_backward(st, dtype, wkv6::kF32, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace, s0, gsT, sT, gs0));
     }
     const bool chunk = algo == WKV6_ALGO_CHUNK || (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     if (!chunk)

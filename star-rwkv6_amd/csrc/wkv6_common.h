@@ -76,7 +76,18 @@ __device__ __forceinline__ void store4(float *p, float a, float b, float c, floa
 __device__ __forceinline__ void store4(bf16_t *p, float a, float b, float c, float d) {
     *reinterpret_cast<uint2 *>(p) = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
 }
+// fp32 -> fp16, round to nearest even, of the value as fp32 holds it (left to itself the compiler rounds the result of a
+// multiply-add to fp16 in the same instruction, which is another value where the fp32 one is a tie)
+__device__ __forceinline__ f16_t to_f16(float a) {
+    asm("" : "+v"(a));
+    return (_Float16)a;
+}
+__device__ __forceinline__ void store4(f16_t *p, float a, float b, float c, float d) {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<h4 *>(p) = (h4){to_f16(a), to_f16(b), to_f16(c), to_f16(d)};
+}
 __device__ __forceinline__ void store1(float *p, float a) { *p = a; }
+__device__ __forceinline__ void store1(f16_t *p, float a) { *p = to_f16(a); }
 __device__ __forceinline__ void store1(bf16_t *p, float a) {
     *reinterpret_cast<uint16_t *>(p) = (uint16_t)pack_bf16x2(a, 0.f);
 }

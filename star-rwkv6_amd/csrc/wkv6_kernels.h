@@ -133,7 +133,8 @@ hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B
 
 // saved_states: what chunk32_forward left (the pair's slice also serves the per-timestep pass of a pair
 // whose decay left the chunk form's reach); gu (B, C)
-hipError_t chunk32_backward(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+// grad_dtype: type of gr, gk, gv, gw: kF32, or kF16 for fp16 tensors
+hipError_t chunk32_backward(hipStream_t st, int dtype, int grad_dtype, int64_t B, int64_t T, int64_t H,
                             const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                             void *gr, void *gk, void *gv, void *gw, void *gu, void *saved_states,
                             // gradients through the state ((B,H,64,64) fp32 [key][value]; sT = the forward's final state,
@@ -157,7 +158,7 @@ C32Segments chunk32_segments_layout(int64_t B, int64_t T, int64_t H, void *saved
 hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
                                          const void *r, const void *k, const void *v, const void *w, const void *u,
                                          void *y, void *saved);
-hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
+hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int grad_dtype, int64_t B, int64_t T, int64_t H,
                                            const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                                            void *gr, void *gk, void *gv, void *gw, void *gu, void *saved);
 
@@ -202,8 +203,8 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse);
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
 RowCut cut_of(int P, int64_t L, int64_t T);
-template <typename T>
-hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T_, int64_t H, const float *gu_rows, T *gu, T *gw, bool zero_first, bool zero_last);
+template <typename E, typename Eg>
+hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, E *gu, Eg *gw, bool zero_first, bool zero_last);
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
 hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -280,7 +281,7 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
 // in_dtype kF16 (needs states_ready): r, k, w, u fp16, v and gy their bf16 copies, v_orig / gy_orig the
 // caller's fp16 v and fp32 gy, gradients fp32
 
-// sum over the batch of (B, C) partials -> (C), both in the output type (for the paths without a fused sum)
-hipError_t sum_over_batch(hipStream_t st, int out_dtype, int64_t B, int64_t C, const void *partials, void *sum);
+// sum over the batch of (B, C) partials -> (C), both in the output type, or fp32 partials and an fp16 sum (for the paths without a fused sum)
+hipError_t sum_over_batch(hipStream_t st, int out_dtype, int sum_dtype, int64_t B, int64_t C, const void *partials, void *sum);
 
 }  // namespace wkv6

@@ -168,11 +168,11 @@ typedef ScanBwdALdsT<4> ScanBwdALds;
 // first element ((B,T,C) layout: pstride = C; a private [T][64] block: pstride = 64).
 // The first NW waves work (wave q owns value columns [64/NW q, 64/NW (q+1)); NW <= 16; the first
 // 256 threads also stage the tiles and finish the rows); further threads only keep the barriers company.
-template <typename Tin, typename Tout, int NW = 4>
+template <typename Tin, typename Tout, int NW = 4, typename Tg = Tout>   // Tg: type of gr (deduced)
 __device__ __forceinline__ void scan_bwd_a_body(ScanBwdALdsT<NW> &L, int b, int h, int T, int H,
         const Tin *__restrict__ r, const Tin *__restrict__ k, const Tin *__restrict__ v,
         const Tin *__restrict__ w, const Tin *__restrict__ u, const Tout *__restrict__ gy,
-        Tout *__restrict__ gr, Tout *__restrict__ gu, float *__restrict__ wsP, int64_t pstride,
+        Tg *__restrict__ gr, Tout *__restrict__ gu, float *__restrict__ wsP, int64_t pstride,
         const float *__restrict__ s0 = nullptr, const float *__restrict__ gsT = nullptr, float *fT = nullptr,
         float *__restrict__ gu_row = nullptr)   // gu_row: takes the pair's 64 values of gu unrounded, in the place of gu
 {
@@ -344,12 +344,12 @@ typedef ScanBwdBLdsT<4> ScanBwdBLds;
 // The first 2 NWR waves of the workgroup work: NWR in the K role, then NWR in the V role, each
 // owning 64/NWR value columns / key rows; the first 512 threads also stage the tiles and finish the
 // rows.  P addressed as in sweep A.
-template <typename Tin, typename Tout, int NWR = 4>
+template <typename Tin, typename Tout, int NWR = 4, typename Tg = Tout>   // Tg: type of gk, gv, gw (deduced)
 __device__ __forceinline__ void scan_bwd_b_body(ScanBwdBLdsT<NWR> &L, int b, int h, int T, int H,
         const Tin *__restrict__ r, const Tin *__restrict__ k, const Tin *__restrict__ v,
         const Tin *__restrict__ w, const Tin *__restrict__ u, const Tout *__restrict__ gy,
         const float *__restrict__ wsP, int64_t pstride,
-        Tout *__restrict__ gk, Tout *__restrict__ gv, Tout *__restrict__ gw,
+        Tg *__restrict__ gk, Tg *__restrict__ gv, Tg *__restrict__ gw,
         const float *__restrict__ gsT = nullptr, const float *fT = nullptr, float *__restrict__ gs0 = nullptr,
         bool first_decay_unused = true)
 {

@@ -347,3 +347,37 @@ def test_random_shapes_against_the_oracle_and_the_per_timestep_kernels(op, oracl
         for a, b in zip(outs[AUTO], outs[SCAN]):
             assert torch.isfinite(a.float()).all()
             assert rel(a, b) <= tol, (case, rel(a, b))
+
+
+@pytest.mark.parametrize("B,T,H,big,wild", [(1, 64, 1, False, False), (2, 65, 2, False, False), (3, 200, 2, True, False), (2, 95, 3, False, True),
+                                            (1, 1100, 3, False, False), (1, 1100, 2, False, True), (5, 128, 60, False, False)])
+def test_fp16_gradients_are_the_fp32_ones_rounded_once(lib, oracle, B, T, H, big, wild):
+    # wkv6_backward_saved_sum_ex with grad_dtype WKV6_F16 against the fp32 gradients converted by torch, bit for bit: ragged ends,
+    # time segments, a pair redone per timestep, values past fp16's range, more pairs than compute units
+    from rwkv_kernel import _native
+
+    C = H * N
+    ins = oracle.make_inputs(B, T, H, N, 34)
+    if wild:
+        ins[3][0, T // 2:T // 2 + 40, :N] = 2.0
+    dev, _ = cast_inputs(ins[:5], torch.float16)
+    r, k, v, w, u = dev
+    gy = torch.randn(B, T, C, device="cuda", generator=torch.Generator(device="cuda").manual_seed(2)) * (3000.0 if big else 1.0)
+    st = torch.cuda.current_stream().cuda_stream
+    P = lambda t: t.data_ptr()
+    n = lib.wkv6_saved_bytes(_native.F16, AUTO, B, T, C, H)
+    res = []
+    for code, dt in ((_native.F32, torch.float32), (_native.F16, torch.float16)):
+        y = torch.empty(B, T, C, device="cuda")
+        buf = torch.empty(n, dtype=torch.uint8, device="cuda")
+        outs = [torch.empty(B, T, C, dtype=dt, device="cuda") for _ in range(4)] + [torch.empty(B, C, device="cuda"), torch.empty(C, dtype=dt, device="cuda")]
+        _native.check(lib.wkv6_forward_save(st, _native.F16, AUTO, B, T, C, H, P(r), P(k), P(v), P(w), P(u), P(y), P(buf), n))
+        _native.check(lib.wkv6_backward_saved_sum_ex(st, _native.F16, code, AUTO, B, T, C, H, P(r), P(k), P(v), P(w), P(u), P(gy), *[P(o) for o in outs], P(buf), n))
+        res.append(outs)
+    torch.cuda.synchronize()
+    for name, a, b in zip("gr gk gv gw gu gu_sum".split(), *res):
+        assert torch.equal(a.to(b.dtype), b), name
+    assert not big or any(bool(torch.isinf(x).any()) for x in res[1][:4])
+    bad = lib.wkv6_backward_saved_sum_ex(st, _native.F16, _native.F16, CHUNK, B, T, C, H, *[P(x) for x in (r, k, v, w, u, gy)], *[P(o) for o in res[1]], P(buf), n)
+    assert bad == 2 and lib.wkv6_backward_saved_sum_ex(st, _native.F32, _native.F16, AUTO, B, T, C, H, *[P(x) for x in (r, k, v, w, u, gy)],
+                                                       *[P(o) for o in res[1]], P(buf), n) == 1
