@@ -10,6 +10,7 @@
 // a state S entering a block acts through g1 o S, and leaves it as g2 o (g1 o S + K~^T V).
 #pragma once
 #include "wkv6_mfma.h"
+#include "wkv6_kernels.h"
 
 namespace wkv6 {
 
@@ -220,6 +221,73 @@ __device__ __forceinline__ bool block_prepare(const unsigned char *raw_r, const 
         emit(tile_off(16 * p + 4 * g + e, 4 * l16), xr, xk, al, ew2[e]);
     }
     return __builtin_amdgcn_ballot_w64(!ok) == 0ull;
+}
+
+// ------------------------------------------------------------------------------------------
+// Rows that are time segments: the state segment `row` of head h starts from (kReverse: the gradient arriving at its end), from
+// what the segments before it (behind it) leave alone, by 512 threads (t) into `lds` ([key][value] fp32) and c.start.
+// A thread has eight value columns of one key row and up to seven segments' loads in flight (eight spilled registers in one
+// kernel), so a chain takes one to three round trips to memory, during which the loading waves bring and prepare the first chunk anyway.  With the chain as a kernel
+// between the two passes (and a kernel for gu behind the backward) / so: prompt of B1 T1337 H32 27.4 / 24.3 us, training pair
+// T2049 77.2 / 68.8, T8192 169.5 / 162.4, B2 T4096 H16 102.7 / 95.7.
+// ------------------------------------------------------------------------------------------
+template <bool kReverse>
+__device__ __forceinline__ void chain_start(const SegmentChain &c, int row, int H, int h, int t, float *lds)
+{
+    const int b = row / c.P, s = row - b * c.P, steps = kReverse ? c.P - 1 - s : s;
+    const int64_t from = ((int64_t)b * c.P + (kReverse ? c.P - 1 : 0)) * H + h;     // the segment the walk begins with
+    const float *alone = c.alone + from * (kN * kN), *decay = c.decay + from * kN;  // (uniform; the lane's part of the addresses: 8 t, t >> 3)
+    const int64_t pairs = kReverse ? -H : H;                                        // ... and its stride
+    float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (!kReverse && c.first) {
+        const int64_t e = ((c.map ? c.map[b] : (int64_t)b) * H + h) * (kN * kN) + 8 * t;
+        float lo[4], hi[4];
+        if (c.bf16) { load4(reinterpret_cast<const bf16_t *>(c.first) + e, lo); load4(reinterpret_cast<const bf16_t *>(c.first) + e + 4, hi); }
+        else { load4(reinterpret_cast<const float *>(c.first) + e, lo); load4(reinterpret_cast<const float *>(c.first) + e + 4, hi); }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { S[i] = lo[i]; S[4 + i] = hi[i]; }
+    }
+    constexpr int kAtOnce = 7;
+    for (int n0 = 0; n0 < steps; n0 += kAtOnce) {   // (steps and everything that depends on it: the same for the whole workgroup)
+        f32x4 x[kAtOnce][2];
+        float d[kAtOnce];
+#pragma unroll
+        for (int n = 0; n < kAtOnce; ++n)
+            if (n0 + n < steps) {
+                const float *p = alone + (n0 + n) * pairs * (kN * kN);
+                x[n][0] = *reinterpret_cast<const f32x4 *>(p + 8 * t);
+                x[n][1] = *reinterpret_cast<const f32x4 *>(p + 8 * t + 4);
+                d[n] = decay[(n0 + n) * pairs * kN + (t >> 3)];
+            }
+#pragma unroll
+        for (int n = 0; n < kAtOnce; ++n)
+            if (n0 + n < steps) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) S[i] = fmaf(S[i], d[n], x[n][i >> 2][i & 3]);
+            }
+    }
+    const f32x4 lo = {S[0], S[1], S[2], S[3]}, hi = {S[4], S[5], S[6], S[7]};
+    *reinterpret_cast<f32x4 *>(lds + 8 * t) = lo;
+    *reinterpret_cast<f32x4 *>(lds + 8 * t + 4) = hi;
+    float *out = c.start + ((int64_t)row * H + h) * (kN * kN) + 8 * t;
+    *reinterpret_cast<f32x4 *>(out) = lo;
+    *reinterpret_cast<f32x4 *>(out + 4) = hi;
+    if (!kReverse && c.last && s == c.P - 1) {
+        // the sequence's final state, one more step of the same walk (the state that the second pass itself ends with is 1.18
+        // times as far from float64: its blocks scale k from their middle, the first pass's tiles towards their end)
+        const int64_t own = (int64_t)row * H + h, e = ((int64_t)b * H + h) * (kN * kN) + 8 * t;
+        const f32x4 x0 = *reinterpret_cast<const f32x4 *>(c.alone + own * (kN * kN) + 8 * t), x1 = *reinterpret_cast<const f32x4 *>(c.alone + own * (kN * kN) + 8 * t + 4);
+        const float d = c.decay[own * kN + (t >> 3)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) S[i] = fmaf(S[i], d, i < 4 ? x0[i & 3] : x1[i & 3]);
+        if (c.bf16) {
+            store4(reinterpret_cast<bf16_t *>(c.last) + e, S[0], S[1], S[2], S[3]);
+            store4(reinterpret_cast<bf16_t *>(c.last) + e + 4, S[4], S[5], S[6], S[7]);
+        } else {
+            store4(reinterpret_cast<float *>(c.last) + e, S[0], S[1], S[2], S[3]);
+            store4(reinterpret_cast<float *>(c.last) + e + 4, S[4], S[5], S[6], S[7]);
+        }
+    }
 }
 
 }  // namespace wkv6

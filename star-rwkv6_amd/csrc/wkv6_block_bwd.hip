@@ -58,6 +58,7 @@ struct BlockBwdArgs {
     int bstep;        // batch rows between two pairs of a workgroup (B: one pair per workgroup)
     int slice;        // chunks of a pair's slice of `ckpt` (those of the longest row)
     RowCut cut;       // rows that are time segments (!kMulti and kRagged)
+    SegmentChain chain;   // kSegments: what they start from; gsT and gs0 are not used, s0 holds the states that the segments start from
     const bf16_t *r, *k, *v, *w, *u, *gy;
     bf16_t *gr, *gk, *gv, *gw, *gu;
     float *gu_rows;   // null, or (rows, C): takes every row's gu unrounded, in the place of gu (rows that are time segments; !kMulti)
@@ -93,7 +94,7 @@ typedef volatile int __attribute__((address_space(3))) *LdsFlag;
 // Wave (q, HALF): key channels j = 16q .. 16q+15, block HALF of the visit (tokens 32 HALF .. +31):
 // gr, gk, gw, gu.  Gj[m]: reverse state, rows i = block_row_channel(m, g) + rr, column j = 16q + l16.
 // ------------------------------------------------------------------------------------------
-template <int HALF, bool kMulti, bool kRagged>
+template <int HALF, bool kMulti, bool kRagged, bool kSegments>
 __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned char *smem, const int *s_wild, int pair0, int q, int lane)
 {
     const int T = a.T, H = a.H;
@@ -109,9 +110,11 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
     char *gr_h = reinterpret_cast<char *>(a.gr + base0), *gk_h = reinterpret_cast<char *>(a.gk + base0), *gw_h = reinterpret_cast<char *>(a.gw + base0);
     f32x4 Gj[4];
     // the reverse state a pair starts from: zero, or the gradient arriving at its final state ([key j][value i])
-    const float *const gsT = kMulti ? nullptr : a.gsT;   // (state gradients: one pair per workgroup only)
-    float *const gs0 = kMulti ? nullptr : a.gs0;
-    const bool has_s0 = !kMulti && a.s0 != nullptr;
+    const float *const gsT = kMulti || kSegments ? nullptr : a.gsT;   // (state gradients: one pair per workgroup only)
+    float *const gs0 = kMulti || kSegments ? nullptr : a.gs0;
+    // whether a state enters the row, and a gradient arrives at its end
+    const bool has_s0 = kSegments ? b0 % a.chain.P != 0 : !kMulti && a.s0 != nullptr;
+    const bool has_gsT = kSegments ? b0 % a.chain.P != a.chain.P - 1 : gsT != nullptr;
     auto start_G = [&](int slot_) {
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -119,7 +122,13 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
             if (gsT) Gj[m] = *reinterpret_cast<const f32x4 *>(gsT + (int64_t)((b0 + slot_ * a.bstep) * H + h) * (kN * kN) + col * kN + block_row_channel(m, g));
         }
     };
-    start_G(0);
+    if (kSegments) {   // (the tiles of g2 o G are free until the first visit)
+        float *start = reinterpret_cast<float *>(smem + BlockBwdLds::kGt);
+        chain_start<true>(a.chain, b0, H, h, 256 * HALF + 64 * q + lane, start);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 4; ++m) Gj[m] = *reinterpret_cast<const f32x4 *>(start + col * kN + block_row_channel(m, g));
+    } else start_G(0);
     float u4[4];
     load4(a.u + h * kN + 16 * q + 4 * g, u4);   // u of this lane's four channels 16q + 4g + rr
     float gu_acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -134,8 +143,8 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
             const float4 x = *reinterpret_cast<const float4 *>(rows), y = *reinterpret_cast<const float4 *>(rows + kN);
             const float t0 = x.x + y.x, t1 = x.y + y.y, t2 = x.z + y.z, t3 = x.w + y.w;
             const int64_t e = (int64_t)(b0 + done * a.bstep) * C + h * kN + 16 * q + 4 * g;
-            if (!kMulti && a.gu_rows) {   // one pair per workgroup: its row is the sum
-                *reinterpret_cast<float4 *>(a.gu_rows + e) = make_float4(t0, t1, t2, t3);
+            if (kSegments || (!kMulti && a.gu_rows)) {   // one pair per workgroup: its row is the sum
+                if (!kSegments) *reinterpret_cast<float4 *>(a.gu_rows + e) = make_float4(t0, t1, t2, t3);
                 *reinterpret_cast<float4 *>(gu_lds + 4 * kN + 16 * q + 4 * g) = make_float4(t0, t1, t2, t3);
                 return;
             }
@@ -364,7 +373,7 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
             // balance leaves rounding residue there)
             // (with an initial state / a gradient arriving at the final state they are not zero)
             if ((HALF == 0 && n == 0 && c == 0 && l16 == 0 && !has_s0) ||
-                ((kRagged ? c * kBlockTokens + (n == 0 ? R0 : R1) + l16 == T - 1 : (HALF == 1 && n == 1 && c == nchunk - 1 && l16 == 15)) && !gsT)) {
+                ((kRagged ? c * kBlockTokens + (n == 0 ? R0 : R1) + l16 == T - 1 : (HALF == 1 && n == 1 && c == nchunk - 1 && l16 == 15)) && !has_gsT)) {
                 gwo[0] = gwo[1] = gwo[2] = gwo[3] = 0.f;
             }
             packed[0][n][0] = pack_bf16x2(gro[0], gro[1]); packed[0][n][1] = pack_bf16x2(gro[2], gro[3]);
@@ -476,7 +485,7 @@ __device__ __forceinline__ void block_bwd_gv(const unsigned char *smem, bf16_t *
 // ------------------------------------------------------------------------------------------
 // Producer wave p: loads, operand preparation of tokens 16p..16p+15, then the gv role.
 // ------------------------------------------------------------------------------------------
-template <bool kMulti, bool kRagged>
+template <bool kMulti, bool kRagged, bool kSegments>
 __device__ __forceinline__ void block_bwd_producer(const BlockBwdArgs &a, unsigned char *smem, int *s_wild, int pair0, int p, int lane)
 {
     const int T = a.T, H = a.H;
@@ -580,6 +589,7 @@ __device__ __forceinline__ void block_bwd_producer(const BlockBwdArgs &a, unsign
     issue_rkw();
     if (nvisit > 1) issue_rkw();
     prepare(nvisit > 1 ? kRkwLoads : 0);
+    if (kSegments) __syncthreads();   // (the chain's barrier)
     for (int it = 0; it < nvisit; ++it) {
         __syncthreads();
         // free again: every tile of visit it-1
@@ -602,7 +612,9 @@ __device__ __forceinline__ void block_bwd_producer(const BlockBwdArgs &a, unsign
 
 constexpr int kBlockBwdThreads = 12 * 64;
 
-template <bool kMulti, bool kRagged>   // kMulti: a workgroup takes several pairs, one after the other; kRagged: T is no multiple of 64
+// kMulti: a workgroup takes several pairs, one after the other; kRagged: T is no multiple of 64; kSegments: rows are time
+// segments that find their arriving gradient themselves, and the last workgroup of a head leaves gu of every sequence
+template <bool kMulti, bool kRagged, bool kSegments>
 __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -624,9 +636,9 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
         move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.gy, n);
         move_rows(a.gr, n); move_rows(a.gk, n); move_rows(a.gv, n); move_rows(a.gw, n);
     }
-    if (wave < 4) block_bwd_producer<kMulti, kRagged>(a, smem, s_wild, pair0, wave, lane);
-    else if (wave < 8) block_bwd_xw<0, kMulti, kRagged>(a, smem, s_wild, pair0, wave - 4, lane);
-    else block_bwd_xw<1, kMulti, kRagged>(a, smem, s_wild, pair0, wave - 8, lane);
+    if (wave < 4) block_bwd_producer<kMulti, kRagged, kSegments>(a, smem, s_wild, pair0, wave, lane);
+    else if (wave < 8) block_bwd_xw<0, kMulti, kRagged, kSegments>(a, smem, s_wild, pair0, wave - 4, lane);
+    else block_bwd_xw<1, kMulti, kRagged, kSegments>(a, smem, s_wild, pair0, wave - 8, lane);
     const int b0 = pair0 / a.H, h = pair0 - b0 * a.H;
     const int npw = kMulti ? (a.B - b0 + a.bstep - 1) / a.bstep : 1;
     const int64_t slice = (int64_t)a.slice * (kN * kN), C = (int64_t)a.H * kN;
@@ -649,6 +661,10 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
         const int64_t so = (int64_t)(b * a.H + h) * (kN * kN) + z;
         const float *s0p = !kMulti && a.s0 ? a.s0 + so : nullptr, *gsTp = !kMulti && a.gsT ? a.gsT + so : nullptr;
         float *gs0p = !kMulti && a.gs0 ? a.gs0 + so : nullptr;
+        if (kSegments) {
+            s0p = b0 % a.chain.P ? a.s0 + so : nullptr;
+            gsTp = b0 % a.chain.P != a.chain.P - 1 ? a.chain.start + so : nullptr;
+        }
         const bool states = s0p || gsTp || gs0p;
         __syncthreads();
         scan_bwd_a_body<bf16_t, bf16_t>(*reinterpret_cast<ScanBwdALds *>(smem), b, h, a.T, a.H, a.r + z, a.k + z, a.v + z, a.w + z, a.u + z, a.gy + z,
@@ -666,7 +682,7 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
     int lane_id = tid;
     asm volatile("" : "+v"(lane_id));
     float part = 0.f;
-    if (a.gu_sum != nullptr && lane_id < kN) {
+    if ((kSegments || a.gu_sum != nullptr) && lane_id < kN) {
         part = s_gu_wg[lane_id];
         for (int slot = 0; slot < npw; ++slot)   // the redone pairs' rows, as the second pass stored them
             if (s_wild[slot]) {
@@ -678,7 +694,7 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
     // workgroup of the head.  They travel as written-through (agent scope) stores into the unused second half of
     // the workspace slice of each workgroup's first pair, completed before the arrival counter is bumped; no
     // fence, which would write back the whole L2.
-    if (a.gu_sum != nullptr) {
+    if (kSegments || a.gu_sum != nullptr) {
         __shared__ int s_last;
         const int nparts = a.bstep;   // workgroups of this head (first pairs h, h + H, ..)
         if (tid < kN) {          // wave 0
@@ -688,11 +704,22 @@ __global__ __launch_bounds__(kBlockBwdThreads) void block_bwd_kernel(BlockBwdArg
                 s_last = __hip_atomic_fetch_add(a.arrivals + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
         }
         __syncthreads();
-        if (s_last && tid < kN) {
-            float acc = 0.f;
-            for (int j = 0; j < nparts; ++j)
-                acc += __hip_atomic_load(a.ckpt + (int64_t)(h + j * a.H) * slice + slice / 2 + lane_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            store1(a.gu_sum + h * kN + lane_id, acc);
+        if (s_last) {
+            float *rows = reinterpret_cast<float *>(smem);
+            const float *first = a.ckpt + h * slice + slice / 2;
+            if (kSegments) {   // a sequence's gu from its segments, unrounded until here; then the sum over the batch
+                float acc = 0.f;
+                for (int b = 0; b < nparts / a.chain.P; ++b) {
+                    const float one = sum_partial_rows<12>(first + (int64_t)b * a.chain.P * a.H * slice, a.H * slice, a.chain.P, rows, wave, lane_id & 63);
+                    if (tid < kN) store1(a.gu + b * C + h * kN + lane_id, one);
+                    acc += one;
+                    __syncthreads();
+                }
+                if (a.gu_sum && tid < kN) store1(a.gu_sum + h * kN + lane_id, acc);
+            } else {
+                const float acc = sum_partial_rows<12>(first, a.H * slice, nparts, rows, wave, lane_id & 63);
+                if (tid < kN) store1(a.gu_sum + h * kN + lane_id, acc);
+            }
             if (tid == 0) __hip_atomic_store(a.arrivals + h, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // armed again
         }
     }
@@ -703,10 +730,10 @@ bool block_backward_applies(int64_t B, int64_t T, int64_t H) { return block_forw
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
-                          const float *s0, const float *gsT, float *gs0, RowCut cut, float *gu_rows)
+                          const float *s0, const float *gsT, float *gs0, RowCut cut, float *gu_rows, SegmentChain chain)
 {
     BlockBwdArgs a = {};
-    a.cut = cut; a.gu_rows = gu_rows;
+    a.cut = cut; a.gu_rows = gu_rows; a.chain = chain;
     a.slice = (int)((T + kBlockTokens - 1) / kBlockTokens);
     a.T = (int)T; a.H = (int)H; a.B = (int)B;
     const int64_t grid = block_grid(B, H);
@@ -719,16 +746,20 @@ hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
     a.ckpt = (float *)workspace;
     a.arrivals = reinterpret_cast<int *>(reinterpret_cast<char *>(workspace) + chunk_backward_workspace_bytes(B, T, H));
     const bool multi = B * H > grid, ragged = (T % kBlockTokens) != 0 || cut.segments;
-    if ((cut.segments || gu_rows) && multi) return hipErrorInvalidValue;
-    auto launch = [&](auto multi_tag, auto ragged_tag) -> hipError_t {
-        constexpr auto kern = block_bwd_kernel<decltype(multi_tag)::value, decltype(ragged_tag)::value>;
+    if ((cut.segments || gu_rows || chain.P) && multi) return hipErrorInvalidValue;
+    if (chain.P && (gsT || gs0 || !s0 || !gu_rows || !gu)) return hipErrorInvalidValue;
+    auto launch = [&](auto multi_tag, auto ragged_tag, auto segments_tag) -> hipError_t {
+        constexpr auto kern = block_bwd_kernel<decltype(multi_tag)::value, decltype(ragged_tag)::value, decltype(segments_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockBwdLds::kBytes);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlockBwdThreads), BlockBwdLds::kBytes, st, a);
         return hipGetLastError();
     };
-    if (multi) return ragged ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
-    return ragged ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
+    const std::true_type yes;
+    const std::false_type no;
+    if (chain.P) return ragged ? launch(no, yes, yes) : launch(no, no, yes);
+    if (multi) return ragged ? launch(yes, yes, no) : launch(yes, no, no);
+    return ragged ? launch(no, yes, no) : launch(no, no, no);
 }
 
 }  // namespace wkv6

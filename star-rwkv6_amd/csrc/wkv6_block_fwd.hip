@@ -55,7 +55,8 @@ struct BlockFwdArgs {
     int T, H, B;
     int bstep;               // batch rows between two pairs of a workgroup (B: one pair per workgroup)
     int slice;               // chunks of a pair's slice of `ckpt` (those of the longest row)
-    RowCut cut;              // kCut: how the rows lie in the sequences (one pair per workgroup)
+    RowCut cut;              // kSegments: how the rows lie in the sequences, and what they start from (one pair per workgroup; s0, map and
+    SegmentChain chain;      // sT are not used)
     const bf16_t *r, *k, *v, *w, *u;
     const void *s0;          // initial state (B or n_state, H, 64, 64) [key][value] in Ts, or null
     const int64_t *map;      // batch row -> state row, or null
@@ -83,7 +84,7 @@ __device__ __forceinline__ float sum_row8(float x) {
 // Consumer wave q: value columns i = 16q + l16.
 // State S[m]: rows j = block_row_channel(m, g) + rr, column i.
 // ------------------------------------------------------------------------------------------
-template <typename Ts, bool kSave, bool kFuse>
+template <typename Ts, bool kSave, bool kFuse, bool kSegments>
 __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsigned char *smem, int pair0, int q, int lane)
 {
     const int T = a.T, H = a.H;
@@ -104,16 +105,24 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) Snext[m][rr] = load1(p + (block_row_channel(m, g) + rr) * kN);
     };
-    if (a.s0 != nullptr) request_state(0);
+    if (kSegments) {   // (the staging tiles are free until the first visit is under way)
+        float *start = reinterpret_cast<float *>(smem + BlockFwdLds::kYStage);
+        chain_start<false>(a.chain, b0, H, h, 64 * q + lane, start);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) Snext[m][rr] = start[(block_row_channel(m, g) + rr) * kN + 16 * q + l16];
+    } else if (a.s0 != nullptr) request_state(0);
     if (kSave && b0 == 0 && q == 0 && lane == 0 && a.arrivals) a.arrivals[h] = 0;
     int c = 0, slot = 0;   // visit `it` is chunk c of pair number `slot`
     for (int it = 0; it < nvisit; ++it) {
         __syncthreads();
         if (c == 0) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) S[m] = a.s0 != nullptr ? Snext[m] : (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < 4; ++m) S[m] = kSegments || a.s0 != nullptr ? Snext[m] : (f32x4){0.f, 0.f, 0.f, 0.f};
         }
-        if (a.s0 != nullptr && c == nchunk - 1 && slot + 1 < npw) request_state(slot + 1);
+        if (!kSegments && a.s0 != nullptr && c == nchunk - 1 && slot + 1 < npw) request_state(slot + 1);
         const unsigned char *rt = smem + BlockFwdLds::kOp + (it & 1) * 2 * kTileBytes, *kt = rt + kTileBytes;
         const float *vec = reinterpret_cast<const float *>(smem + BlockFwdLds::kVec + (it & 1) * kBlockVecBytes);
         const float *ruk = vec + 4 * kN;
@@ -188,7 +197,7 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
         }
         __builtin_amdgcn_sched_barrier(0);
         if (++c == nchunk) {
-            if (a.sT != nullptr) {   // the pair's final state
+            if (!kSegments && a.sT != nullptr) {   // the pair's final state
                 Ts *p = reinterpret_cast<Ts *>(a.sT) + ((int64_t)(b0 + slot * a.bstep) * H + h) * (kN * kN) + 16 * q + l16;
 #pragma unroll
                 for (int m = 0; m < 4; ++m)
@@ -208,7 +217,7 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
 // One function: both walk the same visits with the same cursors and lane mapping.
 // ------------------------------------------------------------------------------------------
 constexpr int kBlockFwdLoads = 1, kBlockFwdStores = 2;
-template <bool kSave, bool kRagged, bool kFuse, int kRole>
+template <bool kSave, bool kRagged, bool kFuse, bool kSegments, int kRole>
 __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsigned char *smem, int *s_wild, int pair0, int p, int lane)
 {
     const int T = a.T, H = a.H;
@@ -221,6 +230,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
     const uint32_t rowbytes = (uint32_t)C * 2u;
     const uint32_t lds0 = lds_address(smem);
     typedef BlockFwdLdsT<kFuse> BlockFwdLds;
+    if (kSegments && kRole == kBlockFwdStores) chain_start<false>(a.chain, b0, H, h, 256 + 64 * p + lane, reinterpret_cast<float *>(smem + BlockFwdLds::kYStage));
     // first element of the workgroup's pair number `slot` in a (B,T,C) tensor
     auto pair_base = [&](int slot) { return (int64_t)(b0 + slot * a.bstep) * T * C + (int64_t)h * kN; };
     // this lane's part of an 8-row block: row (lane >> 3), 16-byte piece swizzled with the row
@@ -375,6 +385,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
         if (kVAhead > 2 && nvisit > 2) issue_v();
         prepare(nvisit > 2);
     }
+    if (kSegments) __syncthreads();   // (the chain's barrier)
     for (int it = 0; it < nvisit; ++it) {
         __syncthreads();
         // free again: the raw v block of visit it-1; the staging tiles of visit it-1 are complete
@@ -412,9 +423,9 @@ __device__ __forceinline__ void block_output_stage_in_place(const BlockFwdArgs &
     }
 }
 
-// kCut: rows that are time segments (of true fp32 states).  Built apart: asked at run time, the other ragged launches, whose
+// kSegments: rows that are time segments.  Built apart: asked at run time, the other ragged launches, whose
 // pointers then depend on it, took 2 % longer (prompts of B8 T999 H40: 63.1 us, so 61.7).
-template <typename Ts, bool kSave, bool kRagged, bool kFuse, bool kCut>
+template <typename Ts, bool kSave, bool kRagged, bool kFuse, bool kSegments>
 __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -426,16 +437,16 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pair0 = (int)blockIdx.x;
-    if (kCut) {
+    if (kSegments && kRagged) {
         const RowView rv = row_view(a.cut, pair0 / a.H, a.T);
         const int64_t n = rv.shift * a.H * kN;
         a.T = rv.tokens;
         move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.y, n);
         if (kFuse) { move_rows(a.gate, n); move_rows(a.out, n); move_rows(a.stats, rv.shift * a.H * 2); }
     }
-    if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
-    else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse>(a, smem, pair0, wave - 4, lane);
-    else block_fwd_producer<kSave, kRagged, kFuse, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
+    if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
+    else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse, kSegments>(a, smem, pair0, wave - 4, lane);
+    else block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
     // exact second pass for the pairs of which 16 tokens left the range the scaled operands can hold
     __threadfence_block();
     __syncthreads();
@@ -445,7 +456,8 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
         if (!s_wild[slot]) continue;   // (uniform over the workgroup)
         __syncthreads();
         scan_fwd_body<bf16_t, bf16_t, Ts>(*reinterpret_cast<ScanFwdLds *>(smem), b0 + slot * a.bstep, h, a.T, a.H, a.r, a.k, a.v, a.w, a.u,
-                                          reinterpret_cast<const Ts *>(a.s0), a.map, kFuse ? a.out : a.y, reinterpret_cast<Ts *>(a.sT), false);
+                                          kSegments ? reinterpret_cast<const Ts *>(a.chain.start) : reinterpret_cast<const Ts *>(a.s0), kSegments ? nullptr : a.map,
+                                          kFuse ? a.out : a.y, kSegments ? nullptr : reinterpret_cast<Ts *>(a.sT), false);
         if (kFuse) {
             __threadfence_block();
             __syncthreads();
@@ -476,22 +488,23 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H) {
 static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                        const void *r, const void *k, const void *v, const void *w, const void *u,
                                        const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
-                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats, RowCut cut)
+                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats, RowCut cut,
+                                       const SegmentChain &chain)
 {
     BlockFwdArgs a = {};
-    a.cut = cut;
+    a.cut = cut; a.chain = chain;
     a.slice = (int)((T + kBlockTokens - 1) / kBlockTokens);
     a.T = (int)T; a.H = (int)H; a.B = (int)B;
     const int64_t grid = block_grid(B, H);
     a.bstep = B * H <= grid ? (int)B : (int)(grid / H);
-    if (cut.segments && B * H > grid) return hipErrorInvalidValue;
+    if ((cut.segments && !chain.P) || (chain.P && (B * H > grid || s0 || map || sT))) return hipErrorInvalidValue;
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     a.gate = (const bf16_t *)gate; a.gn_scale = gn_scale; a.gn_offset = gn_offset; a.gn_eps = gn_eps; a.out = (bf16_t *)out; a.stats = stats;
-    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto cut_tag) -> hipError_t {
+    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag) -> hipError_t {
         constexpr bool kFuse = decltype(fuse_tag)::value;
-        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(cut_tag)::value>;
+        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(segments_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockFwdLdsT<kFuse>::kBytes);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlockFwdThreads), BlockFwdLdsT<kFuse>::kBytes, st, a);
@@ -500,8 +513,8 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
     auto launch_ts = [&](auto ts_tag, auto save_tag, auto fuse_tag) -> hipError_t {
         const std::true_type yes;
         const std::false_type no;
-        if (cut.segments) {
-            if constexpr (std::is_same<decltype(ts_tag), float>::value) return launch(ts_tag, save_tag, yes, fuse_tag, yes);
+        if (chain.P) {   // (segments are whole chunks where they divide the sequence evenly)
+            if constexpr (std::is_same<decltype(ts_tag), float>::value) return cut.segments ? launch(ts_tag, save_tag, yes, fuse_tag, yes) : launch(ts_tag, save_tag, no, fuse_tag, yes);
             else return hipErrorInvalidValue;
         }
         return (T % kBlockTokens) != 0 ? launch(ts_tag, save_tag, yes, fuse_tag, no) : launch(ts_tag, save_tag, no, fuse_tag, no);
@@ -518,19 +531,19 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
 
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut)
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut, SegmentChain chain)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters,
-                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, cut);
+                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, cut, chain);
 }
 
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut)
+                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut, SegmentChain chain)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, saved_states != nullptr,
-                                gate, gn_scale, gn_offset, gn_eps, out, stats, cut);
+                                gate, gn_scale, gn_offset, gn_eps, out, stats, cut, chain);
 }
 
 }  // namespace wkv6

@@ -668,11 +668,9 @@ __global__ __launch_bounds__(kBwdWaves * 64) void chunk_bwd_kernel(BwdArgs a)
                 s_last = __hip_atomic_fetch_add(a.arrivals + h, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
         }
         __syncthreads();
-        if (s_last && tid < kN) {
-            float acc = 0.f;
-            for (int j = 0; j < nparts; ++j)
-                acc += __hip_atomic_load(a.ckpt + (int64_t)(h + j * a.H) * slice + slice / 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            store1(reinterpret_cast<Tout *>(a.gu_sum) + h * kN + tid, acc);
+        if (s_last) {
+            const float acc = sum_partial_rows<kBwdWaves>(a.ckpt + h * slice + slice / 2, a.H * slice, nparts, reinterpret_cast<float *>(smem), wave, lane);
+            if (tid < kN) store1(reinterpret_cast<Tout *>(a.gu_sum) + h * kN + tid, acc);
             if (tid == 0) __hip_atomic_store(a.arrivals + h, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // armed again
         }
     }
@@ -789,10 +787,16 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
     // (1) What each segment alone sends back into its incoming state: G_0 = sum_t (prod_{s<t} d_s) r_t^T gy_t.
     // That is the state the FORWARD recurrence builds from zero over the segment read back to front
     // with r in the place of k and gy in the place of v, so the forward kernel's state-only pass does it.
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
+    const bool block = block_backward_applies(rows, L, H);
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
+    if (block) {   // (2), (3) and the sums over the segments in one launch
+        SegmentChain c;
+        c.P = s.P; c.alone = s.alone; c.decay = s.decay; c.start = s.gstates;
+        return block_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, saved, gu_sum, s.states, nullptr, nullptr, s.cut, s.gu_rows, c);
+    }
     // (2) chained backwards in time: the gradient arriving at the end of every segment
-    if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates)) != hipSuccess) return e;
+    if ((e = segment_chain_reverse(st, s.P, B, H, s.decay, s.gstates)) != hipSuccess) return e;
     // (3) every segment again, between its true incoming state and its true arriving gradient
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, nullptr, saved, true, gu_sum,
                        s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut, s.gu_rows);
@@ -811,14 +815,14 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
-    if ((e = segment_chain_forward(st, s.P, B, H, s.dsum, s.states, s0)) != hipSuccess) return e;
+    if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, s0)) != hipSuccess) return e;
     e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, nullptr, nullptr, saved, nullptr, false, false, s.cut);
     if (e != hipSuccess) return e;
     e = chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
-    if ((e = segment_chain_reverse(st, s.P, B, H, s.dsum, s.gstates, gsT, gs0)) != hipSuccess) return e;
+    if ((e = segment_chain_reverse(st, s.P, B, H, s.decay, s.gstates, gsT, gs0)) != hipSuccess) return e;
     e = chunk_backward(st, rows, L, H, r, k, v, w, u, gy, gr, gk, gv, gw, nullptr, saved, true, nullptr,
                        s.states, s.gstates, nullptr, kBF16, nullptr, nullptr, s.cut, s.gu_rows);
     if (e != hipSuccess) return e;

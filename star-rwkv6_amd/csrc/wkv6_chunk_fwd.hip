@@ -46,7 +46,8 @@ struct FwdLds {
     static constexpr int kBytes0 = kOp + 2 * kOpBytes;
     // only WITHOUT the fused output stage: [2] K^ = K~ g, k decayed to the END of its tile (exponents <= 0)
     static constexpr int kKg = kBytes0;
-    static constexpr int kBytes = kKg + 2 * kTileBytes;
+    static constexpr int kDecay = kKg + 2 * kTileBytes;                 // [4 tiles][64] floats: see FwdArgs::decay
+    static constexpr int kBytes = kDecay + 4 * kN * 4;
     // only with the fused output stage (group norm and gate):
     static constexpr int kYStage = kBytes0;                             // [2 visit parities] y of one chunk, bf16
     static constexpr int kRawG = kYStage + 2 * kTileBytes;              // [4] raw gate tiles (visit & 3)
@@ -73,7 +74,7 @@ struct FwdArgs {
     int reverse;     // 1: the time axis is read back to front (row T-1-t in the place of row t)
     int slice;       // chunks of a pair's slice of `ckpt` (those of the longest row)
     RowCut cut;      // rows that are time segments (one pair per workgroup and kRagged)
-    float *dsum;     // null, or [4 tiles][pairs][64]: per pair, log2(e) * sum of exp(w) over the tokens of tile p of every chunk
+    float *decay;    // null, or [pairs][64]: per pair exp(-sum of exp(w) over its tokens) (one pair per workgroup, no output stage)
     const bf16_t *r, *k, *v, *w, *u;   // 16-bit elements: bf16, or fp16 with v a bf16 copy (see OutOf)
     const void *v_orig;                // v as the caller holds it (the exact per-timestep pass reads this one)
     const void *s0;
@@ -438,10 +439,8 @@ __device__ __forceinline__ void fwd_producer(const FwdArgs &a, unsigned char *sm
             const float tot = transpose_reduce16(pr, lane);
             if ((lane & 3) == 0) reinterpret_cast<float *>(op + FwdLds::kOpRuk)[16 * p + ((lane >> 2) & 15)] = tot;
         }
-        if (pp_c + 1 == nchunk && a.dsum != nullptr && part == 0) {   // the pair's total decay, this wave's tiles
-            a.dsum[((int64_t)p * a.nitems + (bh0 + pp_n * stride)) * kN + ch] = dacc;
-            dacc = 0.f;
-        }
+        if (!kMulti && !kFuse && pp_c + 1 == nchunk)   // the exponent of the pair's decay, this wave's tiles
+            reinterpret_cast<float *>(smem + FwdLds::kDecay)[p * kN + ch] = dacc;
         if (++pp_c == nchunk && kMulti) {   // the next preparation opens the next pair: its head's u
             pp_c = 0; ++pp_n;
             if (pp_n < n_my) {
@@ -546,6 +545,10 @@ __global__ __launch_bounds__(kFwdThreads) void chunk_fwd_kernel(FwdArgs a)
     // (workgroups sharing a pair all see the same flags and all redo the whole pair: the same values)
     __threadfence_block();   // workgroup scope is enough (and a device-scope fence would write back the L2)
     __syncthreads();
+    if (!kMulti && !kFuse && a.decay && part == 0 && threadIdx.x < kN) {
+        const float *e = reinterpret_cast<const float *>(smem + FwdLds::kDecay) + threadIdx.x;
+        a.decay[(int64_t)bh0 * kN + threadIdx.x] = exp2_fast(-((e[0] + e[kN]) + (e[2 * kN] + e[3 * kN])));
+    }
     const int stride = (int)gridDim.x;
     const int n_my = kMulti ? (a.nitems - bh0 + stride - 1) / stride : 1;
     for (int n = 0; n < n_my; ++n) {
@@ -619,13 +622,13 @@ static unsigned forward_grid(int64_t pairs, bool *multi, int *split) {
 
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *dsum, bool reverse,
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, bool reverse,
                          bool counters, RowCut cut)
 {
-    if (y != nullptr && dsum == nullptr && !reverse && block_forward_applies(B, T, H))
+    if (y != nullptr && decay == nullptr && !reverse && block_forward_applies(B, T, H))
         return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters, cut);
     FwdArgs a = {};
-    a.dsum = dsum;
+    a.decay = decay;
     a.reverse = reverse;
     a.cut = cut;
     a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
@@ -635,7 +638,7 @@ hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, 
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     bool multi;
     const unsigned grid = forward_grid(B * H, &multi, &a.split);
-    if (cut.segments && multi) return hipErrorInvalidValue;
+    if ((cut.segments || decay) && multi) return hipErrorInvalidValue;
     const bool save = saved_states != nullptr, ragged = (T % CL) != 0 || cut.segments;
     return state_dtype == kF32 ? launch_fwd<float>(st, a, save, ragged, multi, grid)
                                : launch_fwd<bf16_t>(st, a, save, ragged, multi, grid);
@@ -745,19 +748,19 @@ hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_
 // affine, S_out = D o S_in + U with D[j] = exp(-sum_t exp(w_t[j])) over the segment and U the state
 // the segment builds from zero, so: (A) every segment runs from a zero state (all segments at once;
 // a (B,T,C) tensor cut into P equal segments IS a (B*P, T/P, C) tensor, and RowCut stands for other lengths; no y in this pass) and leaves
-// U and, from the producer waves, the exponent of D; (B) a tiny kernel chains the P affine maps per pair,
-// leaving each segment's true incoming state where its U was (and the final state); (C) every
-// segment runs again from its true state and writes y.  Twice the forward work on P times the
+// U and, from the producer waves, D; (B) the P affine maps of a pair are chained, at the start of the second pass in
+// the block form (chain_start), by a tiny kernel that leaves each segment's true incoming state where its U was (and the final
+// state) in the others; (C) every segment runs again from its true state and writes y.  Twice the forward work on P times the
 // workgroups.
 // ------------------------------------------------------------------------------------------
 constexpr int kMostSegments = 16;
 // kReverse: the same chain walked from the last segment to the first, which is what the reverse
 // state of the backward pass obeys (the gradient arriving at the end of segment p is what segment
 // p + 1 sends into its incoming state: its own contribution plus D_{p+1} times what arrives at its end).
-// kFactors: dsum holds two factors of each segment's decay, [2][pairs][64], instead of its exponent's four parts.
-template <typename Ts, bool kReverse, int P, bool kFactors>
+// kFactors: `decay` holds one or two factors of each segment's decay, [kFactors][pairs][64].
+template <typename Ts, bool kReverse, int P, int kFactors>
 __global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__restrict__ s0, const int64_t *__restrict__ map,
-                                                            const float *__restrict__ dsum, float *__restrict__ states, Ts *__restrict__ sT)   // sT: the final state, or null
+                                                            const float *__restrict__ decay, float *__restrict__ states, Ts *__restrict__ sT)   // sT: the final state, or null
 {
     // Thread: four value columns i0..i0+3 of one key row j of one (batch, head): 1024 threads per pair,
     // gridDim.x * 256 = B * H * 1024.  states[(b*P + seg), h] holds U on entry and the segment's
@@ -776,8 +779,8 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__r
     for (int n = 0; n < P; ++n) {
         const int64_t vp = pair_of_step(n);
         x[n] = *reinterpret_cast<const float4 *>(states + (vp * kN + j) * kN + i0);
-        if (kFactors) d[n] = dsum[vp * kN + j] * dsum[(np + vp) * kN + j];
-        else d[n] = (dsum[vp * kN + j] + dsum[(np + vp) * kN + j]) + (dsum[(2 * np + vp) * kN + j] + dsum[(3 * np + vp) * kN + j]);
+        d[n] = decay[vp * kN + j];
+        if (kFactors == 2) d[n] *= decay[(np + vp) * kN + j];
     }
     float S[4] = {0.f, 0.f, 0.f, 0.f};
     if (s0) {
@@ -786,21 +789,21 @@ __global__ __launch_bounds__(256) void segment_chain_kernel(int H, const Ts *__r
     }
 #pragma unroll
     for (int n = 0; n < P; ++n) {
-        const float dd = kFactors ? d[n] : exp2_fast(-d[n]);
+        const float dd = d[n];
         *reinterpret_cast<float4 *>(states + (pair_of_step(n) * kN + j) * kN + i0) = make_float4(S[0], S[1], S[2], S[3]);
         S[0] = fmaf(S[0], dd, x[n].x); S[1] = fmaf(S[1], dd, x[n].y); S[2] = fmaf(S[2], dd, x[n].z); S[3] = fmaf(S[3], dd, x[n].w);
     }
     if (sT) store4(sT + (((int64_t)b * H + h) * kN + j) * kN + i0, S[0], S[1], S[2], S[3]);
 }
-template <typename Ts, bool kReverse, bool kFactors = false, int N = kMostSegments>
+template <typename Ts, bool kReverse, int kFactors = 1, int N = kMostSegments>
 static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, const Ts *s0, const int64_t *map,
-                               const float *dsum, float *states, Ts *sT)
+                               const float *decay, float *states, Ts *sT)
 {
     if constexpr (N < 2) {
         return hipErrorInvalidValue;
     } else {
-        if (P != N) return launch_chain<Ts, kReverse, kFactors, N - 1>(st, P, B, H, s0, map, dsum, states, sT);
-        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, N, kFactors>), dim3((unsigned)(B * H * 4)), dim3(256), 0, st, (int)H, s0, map, dsum, states, sT);
+        if (P != N) return launch_chain<Ts, kReverse, kFactors, N - 1>(st, P, B, H, s0, map, decay, states, sT);
+        hipLaunchKernelGGL((segment_chain_kernel<Ts, kReverse, N, kFactors>), dim3((unsigned)(B * H * 4)), dim3(256), 0, st, (int)H, s0, map, decay, states, sT);
         return hipGetLastError();
     }
 }
@@ -848,8 +851,8 @@ int chunk_forward_segments(int64_t B, int64_t T, int64_t H) {
 }
 size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H) {
     const int P = chunk_forward_segments(B, T, H);
-    // per segment and pair a state and the decay exponents
-    return P <= 1 ? 0 : (size_t)(B * P * H) * (kN * kN + 4 * kN) * sizeof(float);
+    // per segment and pair two states (what it leaves alone, what it starts from) and the decay
+    return P <= 1 ? 0 : (size_t)(B * P * H) * (2 * kN * kN + kN) * sizeof(float);
 }
 
 // With `gate` the second pass runs the fused output stage (y = out then).
@@ -862,26 +865,32 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
     const int P = forward_segments_plan(B, T, H, &L);
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
-    float *states = (float *)workspace, *dsum = states + rows * H * kN * kN;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, dsum, false, true, cut);
+    float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
     if (e != hipSuccess) return e;
-    e = state_dtype == kF32 ? launch_chain<float, false>(st, P, B, H, (const float *)s0, map, dsum, states, (float *)sT)
-                            : launch_chain<bf16_t, false>(st, P, B, H, (const bf16_t *)s0, map, dsum, states, (bf16_t *)sT);
+    if (block_forward_applies(rows, L, H)) {   // the chain at the start of the second pass
+        SegmentChain c;
+        c.P = P; c.alone = states; c.decay = decay; c.first = s0; c.map = map; c.last = sT; c.bf16 = state_dtype != kF32; c.start = start;
+        return gate ? block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr, nullptr, nullptr, nullptr, cut, c)
+                    : block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, nullptr, true, cut, c);
+    }
+    e = state_dtype == kF32 ? launch_chain<float, false>(st, P, B, H, (const float *)s0, map, decay, states, (float *)sT)
+                            : launch_chain<bf16_t, false>(st, P, B, H, (const bf16_t *)s0, map, decay, states, (bf16_t *)sT);
     if (e != hipSuccess) return e;
     return gate ? chunk_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr, cut)
                 : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, states, nullptr, y, nullptr, nullptr, nullptr, false, true, cut);
 }
 
-hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
+hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states,
                                  const float *arriving, float *leaving) {
-    return launch_chain<float, true>(st, P, B, H, arriving, nullptr, dsum, states, leaving);
+    return launch_chain<float, true>(st, P, B, H, arriving, nullptr, decay, states, leaving);
 }
 hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse) {
-    return reverse ? launch_chain<float, true, true>(st, P, B, H, nullptr, nullptr, decay, states, nullptr)
-                   : launch_chain<float, false, true>(st, P, B, H, nullptr, nullptr, decay, states, nullptr);
+    return reverse ? launch_chain<float, true, 2>(st, P, B, H, nullptr, nullptr, decay, states, nullptr)
+                   : launch_chain<float, false, 2>(st, P, B, H, nullptr, nullptr, decay, states, nullptr);
 }
-hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states, const float *s0) {
-    return launch_chain<float, false>(st, P, B, H, s0, nullptr, dsum, states, nullptr);
+hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, const float *s0) {
+    return launch_chain<float, false>(st, P, B, H, s0, nullptr, decay, states, nullptr);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -909,22 +918,31 @@ TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra
     s.cut = cut_of(s.P, s.L, T);
     const size_t pairs = (size_t)(B * s.P * H);
     s.states = reinterpret_cast<float *>(extra);
-    s.dsum = s.states + pairs * kN * kN;
-    s.gstates = s.dsum + pairs * 4 * kN;
-    s.gu_rows = s.gstates + pairs * kN * kN;
-    s.bytes = (pairs * (2 * kN * kN + 4 * kN) + pairs * kN) * sizeof(float);
+    s.gstates = s.states + pairs * kN * kN;
+    s.alone = s.gstates + pairs * kN * kN;
+    s.decay = s.alone + pairs * kN * kN;
+    s.gu_rows = s.decay + pairs * kN;
+    s.bytes = pairs * (3 * kN * kN + 2 * kN) * sizeof(float);
     return s;
 }
 
+// The second pass of the saving forward, from what the first one left in `alone` and `decay`.
+static SegmentChain train_chain(const TrainSegments &s, float *start) {
+    SegmentChain c;
+    c.P = s.P; c.alone = s.alone; c.decay = s.decay; c.start = start;
+    return c;
+}
 hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                        const void *r, const void *k, const void *v, const void *w, const void *u,
                                        void *y, void *saved, void *extra)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
+    const bool block = block_forward_applies(rows, L, H);
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
-    if ((e = launch_chain<float, false>(st, s.P, B, H, nullptr, nullptr, s.dsum, s.states, nullptr)) != hipSuccess) return e;
+    if (block) return block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, saved, true, s.cut, train_chain(s, s.states));
+    if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, nullptr)) != hipSuccess) return e;
     return chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, y, nullptr, saved, nullptr, false, true, s.cut);
 }
 
@@ -937,9 +955,11 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.dsum, false, true, s.cut);
+    const bool block = block_forward_applies(rows, L, H);
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
-    if ((e = launch_chain<float, false>(st, s.P, B, H, nullptr, nullptr, s.dsum, s.states, nullptr)) != hipSuccess) return e;
+    if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states));
+    if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, nullptr)) != hipSuccess) return e;
     return fused_save_from(st, rows, L, H, r, k, v, w, u, s.states, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, s.cut);
 }
 

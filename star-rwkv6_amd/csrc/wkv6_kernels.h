@@ -87,11 +87,25 @@ template <typename P> __device__ __forceinline__ void move_rows(P *&p, int64_t e
     if (p) p += elements;
 }
 
+// How the rows of a launch, the P segments of each sequence, come by the state they start from (the block-form kernels; the
+// tile form and the full-precision form are handed the states by segment_chain_kernel): from what every segment leaves alone,
+// started from zero, and the decay over it.
+struct SegmentChain {
+    int P = 0;                        // segments of a sequence (0: every row is a sequence of its own)
+    const float *alone = nullptr;     // [rows][H][64][64] (fp32, [key][value])
+    const float *decay = nullptr;     // [rows][H][64]
+    const void *first = nullptr;      // forward: the states the sequences start from, or null (zero); type of `last`
+    const int64_t *map = nullptr;     // ... batch row -> row of `first`, or null
+    void *last = nullptr;             // forward: the sequences' final states [B][H][64][64], or null
+    bool bf16 = false;                // `first` and `last` are bf16 (otherwise fp32)
+    float *start = nullptr;           // [rows][H][64][64]: receives what every segment starts from
+};
+
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states,
-                         float *dsum = nullptr,    // dsum: see chunk_forward_segments_run
+                         float *decay = nullptr,   // see FwdArgs
                          bool reverse = false,     // the time axis read back to front (no y)
                          bool counters = true,     // saved_states ends with the per-head counters of the fused gu sum (zeroed here)
                          RowCut cut = RowCut());
@@ -104,21 +118,26 @@ int64_t block_grid(int64_t B, int64_t H);
 bool block_forward_applies(int64_t B, int64_t T, int64_t H);
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut = RowCut());
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
+                         RowCut cut = RowCut(), SegmentChain chain = SegmentChain());   // (rows that are segments: cut and chain, s0 = map = sT = null)
 
 // the block-form forward with the layer's output stage fused in (see chunk_forward_fused / chunk_forward_fused_save):
 // y and stats may be null (inference), saved_states null without a backward to follow
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut = RowCut());
+                               void *out, void *y, float *stats, void *sT, void *saved_states,
+                               RowCut cut = RowCut(), SegmentChain chain = SegmentChain());
 bool block_backward_applies(int64_t B, int64_t T, int64_t H);
 // workspace: the chunk-start states as a forward pass leaves them, followed by the per-head counters; gu_sum may be null
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                           const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                           void *gr, void *gk, void *gv, void *gw, void *gu, void *workspace, void *gu_sum,
                           const float *s0 = nullptr, const float *gsT = nullptr, float *gs0 = nullptr, RowCut cut = RowCut(),
-                          float *gu_rows = nullptr);   // gu_rows: see chunk_backward; one pair per workgroup
+                          float *gu_rows = nullptr,    // gu_rows: see chunk_backward; one pair per workgroup
+                          // rows that are segments: gu (sequences, C) and gu_sum from all of them, gu_rows as scratch, gw zero at the
+                          // ends of the sequences; s0 = what the forward's segments started from, gsT = gs0 = null
+                          SegmentChain chain = SegmentChain());
 
 // --- full-precision chunk form (wkv6_chunk32_fwd.hip, wkv6_chunk32_bwd.hip): fp32 and fp16 tensors on the
 // fp32 matrix instructions, chunks of 32 tokens, fp32 states; any T (the last chunk may be short).
@@ -188,8 +207,9 @@ struct TrainSegments {
     int64_t L;          // tokens of a segment (the last one of a sequence may be shorter)
     RowCut cut;         // how the kernels find them
     float *states;      // [B*P][H][64][64] state entering each segment
-    float *dsum;        // decay exponents of each segment (as chunk_forward leaves them)
+    float *decay;       // [B*P][H][64] decay over each segment
     float *gstates;     // [B*P][H][64][64] gradient arriving at the end of each segment
+    float *alone;       // [B*P][H][64][64] (block form) what each segment leaves alone, forward or backward in time
     float *gu_rows;     // [B*P][C] gu of each segment
     size_t bytes;       // size of the block
 };
@@ -198,14 +218,14 @@ TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra
 // states[(b*P + seg), h]: on entry what each segment builds alone, on exit what enters it (forward: the
 // state, from s0 or zero; reverse: the gradient arriving at its end, from `arriving` or zero, and
 // `leaving` receives what leaves the first segment, dL/dS_0).
-hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states, const float *s0);
+hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, const float *s0);
 // the same with the segments' decays as two factors each, [2][B*P][H][64]
 hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse);
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
 RowCut cut_of(int P, int64_t L, int64_t T);
 template <typename E, typename Eg>
 hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, E *gu, Eg *gw, bool zero_first, bool zero_last);
-hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *dsum, float *states,
+hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
 hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                          const void *r, const void *k, const void *v, const void *w, const void *u,

@@ -1161,3 +1161,58 @@ def test_training_pair_replays_in_a_hip_graph(op, oracle, B, T, H):
         torch.cuda.synchronize()
         for name, t in outs.items():
             assert torch.equal(t, eager[name]), (rep, name)
+
+
+@pytest.mark.parametrize("B,T,H,sdt,wild", [(1, 3072, 16, torch.float32, False), (2, 4096, 8, torch.bfloat16, True), (1, 2880, 17, torch.float32, True),
+                                            (1, 1500, 32, torch.bfloat16, False), (1, 1025, 43, torch.float32, False)])
+def test_prompt_whose_second_pass_finds_its_states_itself(op, oracle, B, T, H, sdt, wild):
+    # block form, 16 (more than two groups of seven at once), 16, 15, 8 and 5 segments, even and ragged; states by map, in both
+    # types; redone segments in the middle and at the end of a sequence
+    N = 64
+    ins = oracle.make_inputs(B, T, H, N, 63, with_state=True)
+    if wild:
+        ins[3][B - 1, T // 2:T // 2 + 20, 5:25] = 6.0
+        ins[3][0, T - 9:T - 1, 20:40] = 6.0
+    dev, ref = cast_inputs(ins[:5], torch.bfloat16)
+    s_dev, s_ref = cast_inputs([ins[6][:B]], sdt)
+    s_dev, s_ref, smap = s_dev[0].flip(0).contiguous(), s_ref[0], list(range(B))[::-1]
+    gate_dev, gate_ref = cast_inputs([torch.randn(B, T, H * N, generator=torch.Generator().manual_seed(5))], torch.bfloat16)
+    one, zero = torch.ones(H, N, device="cuda"), torch.zeros(H, N, device="cuda")
+    op.algo = CHUNK
+    y, sT = op(*dev, return_state=True, init_state=s_dev, state_map=smap)
+    out, oT = op.forward_gn_gate(*dev, gate_dev[0], one, zero, return_state=True, init_state=s_dev, state_map=smap)
+    y_ref, sT_ref = oracle.forward_c(*ref, N, s_ref)
+    check_close("y", y, y_ref, torch.bfloat16)
+    for s in (sT, oT):
+        assert s.dtype == sdt
+        check_close("sT", s, sT_ref, torch.bfloat16)
+    check_close("out", out, oracle.group_norm_gate_np(y_ref, gate_ref[0], one.cpu().numpy(), zero.cpu().numpy(), N), torch.bfloat16)
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 4096, 16), (2, 3000, 12), (3, 2048, 11)])
+def test_training_pair_of_many_segments_in_block_form(op, oracle, B, T, H):
+    # 16, 10 and 7 segments to a sequence; u's gradient by row and over the batch out of the backward's launch, twice over one buffer
+    from rwkv_kernel import _native
+
+    lib, C = _native.load(), H * 64
+    ins = oracle.make_inputs(B, T, H, 64, 65)
+    dev, ref = cast_inputs(ins[:5], torch.bfloat16)
+    gy_dev, gy_ref = cast_inputs(ins[5:6], torch.bfloat16)
+    buf = torch.empty(lib.wkv6_saved_bytes(_native.BF16, CHUNK, B, T, C, H), dtype=torch.uint8, device="cuda")
+    st, P = torch.cuda.current_stream().cuda_stream, lambda t: t.data_ptr()
+    y = torch.empty_like(dev[0])
+    _native.check(lib.wkv6_forward_save(st, _native.BF16, CHUNK, B, T, C, H, *map(P, dev), P(y), P(buf), buf.numel()))
+    g_ref, res = oracle.backward_c(*ref, gy_ref[0], 64), []
+    for _ in range(2):
+        outs = [torch.full_like(y, float("nan")) for _ in range(4)]
+        gu, gus = (torch.full(s, float("nan"), dtype=torch.bfloat16, device="cuda") for s in ((B, C), (C,)))
+        _native.check(lib.wkv6_backward_saved_sum(st, _native.BF16, CHUNK, B, T, C, H, *map(P, dev), P(gy_dev[0]), *map(P, outs), P(gu), P(gus), P(buf), buf.numel()))
+        res.append(outs + [gu, gus])
+    check_close("y", y, oracle.forward_c(*ref, 64)[0], torch.bfloat16)
+    for name, g, want in zip("gr gk gv gw".split(), res[0], g_ref):
+        check_close(name, g, want, torch.bfloat16, is_grad=True)
+    assert float(res[0][3][:, 0].abs().max()) == 0.0 and float(res[0][3][:, -1].abs().max()) == 0.0
+    check_close("gu", to_np(res[0][5]).reshape(H, 64), g_ref[4], torch.bfloat16, is_grad=True)
+    check_close("gu rows", to_np(res[0][4]).sum(0).reshape(H, 64), g_ref[4], torch.bfloat16, is_grad=True)
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
