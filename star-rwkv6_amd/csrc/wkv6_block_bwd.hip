@@ -212,9 +212,7 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
                 for (int m = 0; m < 4; ++m) gq[pp][m] = la.frag_tok_rows(gyt, m, 32 * blk + 16 * pp);
             }
 #pragma unroll
-            for (int pp = 0; pp < 2; ++pp)
-#pragma unroll
-                for (int m = 0; m < 4; ++m) Gj[m] = mfma16(gq[pp][m], rtq[pp], Gj[m]);
+            for (int m = 0; m < 4; ++m) Gj[m] = mfma32(both16(gq[0][m], gq[1][m]), both16(rtq[0], rtq[1]), Gj[m]);
             settle(Gj[0], Gj[1], Gj[2], Gj[3]);
             pend = g1c;
         };
@@ -253,9 +251,7 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
 #pragma unroll
                 for (int m = 0; m < 4; ++m) { Sv[m][0] *= g1c0; Sv[m][1] *= g1c0; Sv[m][2] *= g1c0; Sv[m][3] *= g1c0; }
 #pragma unroll
-                for (int pp = 0; pp < 2; ++pp)
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) Sv[m] = mfma16(vq[pp][m], ktq[pp], Sv[m]);
+                for (int m = 0; m < 4; ++m) Sv[m] = mfma32(both16(vq[0][m], vq[1][m]), both16(ktq[0], ktq[1]), Sv[m]);
                 settle(Sv[0], Sv[1], Sv[2], Sv[3]);
 #pragma unroll
                 for (int m = 0; m < 4; ++m) { Sv[m][0] *= g2c0; Sv[m][1] *= g2c0; Sv[m][2] *= g2c0; Sv[m][3] *= g2c0; }
@@ -324,11 +320,9 @@ __device__ __forceinline__ void block_bwd_xw(const BlockBwdArgs &a, unsigned cha
                 T00[rr] = (l16 > x) ? T00[rr] : 0.f; T11[rr] = (l16 > x) ? T11[rr] : 0.f;      // rows s, column t: t > s
             }
             X1[0] = mfma16(kq0, pack4(T00), zero);
-            X1[1] = mfma16(kq0, pack4(T01), zero);
-            W1[0] = mfma16(rq0, pack4(D00), zero);
+            X1[1] = mfma32(both16(kq0, kq1), acc_as_operand(T01, T11), zero);
+            W1[0] = mfma32(both16(rq0, rq1), acc_as_operand(D00, D10), zero);
             W1[1] = mfma16(rq1, pack4(D11), zero);
-            X1[1] = mfma16(kq1, pack4(T11), X1[1]);
-            W1[0] = mfma16(rq1, pack4(D10), W1[0]);
         }
         settle(X0[0], X0[1], W0[0], W0[1]);
         settle(X1[0], X1[1], W1[0], W1[1]);
@@ -471,8 +465,7 @@ __device__ __forceinline__ void block_bwd_gv(const unsigned char *smem, bf16_t *
             A00[rr] = (x > l16) ? A00[rr] : ((x == l16) ? ruk0 : 0.f);
             A11[rr] = (x > l16) ? A11[rr] : ((x == l16) ? ruk1 : 0.f);
         }
-        f32x4 V0 = mfma16(gyq0, pack4(A00), zero), V1 = mfma16(gyq1, pack4(A11), zero);
-        V0 = mfma16(gyq1, pack4(A10), V0);
+        f32x4 V0 = mfma32(both16(gyq0, gyq1), acc_as_operand(A00, A10), zero), V1 = mfma16(gyq1, pack4(A11), zero);
         settle(GV0, GV1, V0, V1);
         // 16 bytes per lane: token (g odd ? R1 : R0) + l16, channels 16q + 8 (g >> 1) .. +7
         const int tok = c * kBlockTokens + R0 + 16 * (g & 1) + l16;

@@ -171,9 +171,9 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
                     A00[rr] = (l16 > s_) ? A00[rr] : ((l16 == s_) ? ruk0 : 0.f);
                     A11[rr] = (l16 > s_) ? A11[rr] : ((l16 == s_) ? ruk1 : 0.f);
                 }
-                Y0 = mfma16(vf0, pack4(A00), Y0);
-                Y1 = mfma16(vf0, pack4(A01), Y1);
-                Y1 = mfma16(vf1, pack4(A11), Y1);
+                const bf16x8 vf = both16(vf0, vf1);
+                Y0 = mfma32(vf, both16(pack4(A00), make_s16x4(0u, 0u)), Y0);
+                Y1 = mfma32(vf, acc_as_operand(A01, A11), Y1);
                 settle(Y0, Y1);
                 *reinterpret_cast<uint2 *>(ys + tile_off(r0, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y0[0], Y0[1]), pack_bf16x2(Y0[2], Y0[3]));
                 *reinterpret_cast<uint2 *>(ys + tile_off(r1, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y1[0], Y1[1]), pack_bf16x2(Y1[2], Y1[3]));
@@ -188,9 +188,7 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
                     for (int m = 0; m < 4; ++m) kq[pp][m] = block_frag_tok_rows(kt, m, 32 * blk + 16 * pp, l16, g);
                 }
 #pragma unroll
-                for (int pp = 0; pp < 2; ++pp)
-#pragma unroll
-                    for (int m = 0; m < 4; ++m) S[m] = mfma16(kq[pp][m], vf[pp], S[m]);
+                for (int m = 0; m < 4; ++m) S[m] = mfma32(both16(kq[0][m], kq[1][m]), both16(vf[0], vf[1]), S[m]);
             }
             settle(S[0], S[1], S[2], S[3]);
             scale(vec + (2 * blk + 1) * kN);   // g2 of the block

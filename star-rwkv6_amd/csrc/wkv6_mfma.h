@@ -174,6 +174,12 @@ __device__ __forceinline__ bf16x8 frag_global(const void *base, uint32_t rowbyte
     const uint2 hi = *reinterpret_cast<const uint2 *>(b + (rowbyte + 2u * (uint32_t)(32 * h + 16 + 4 * g)));
     return make_bf16x8(lo.x, lo.y, hi.x, hi.y);
 }
+// The fragments of two 16-token groups as one operand of a 16x16x32 MFMA over their 32 tokens: the k-slots of lane group g are
+// then 4g .. 4g+3 of either group, and two operands built so agree.  (A 16x16x16 MFMA takes as long as a 16x16x32 one.)
+__device__ __forceinline__ bf16x8 both16(const s16x4 &a, const s16x4 &b) {
+    const u32x2 x = __builtin_bit_cast(u32x2, a), y = __builtin_bit_cast(u32x2, b);
+    return make_bf16x8(x[0], x[1], y[0], y[1]);
+}
 __device__ __forceinline__ s16x4 pack4(const f32x4 &a) {
     return make_s16x4(pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]));
 }
