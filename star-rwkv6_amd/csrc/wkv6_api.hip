@@ -503,7 +503,7 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
     if (rc == kSmallHead) {
         if (algo == WKV6_ALGO_CHUNK) return WKV6_ERR_UNSUPPORTED;
         rc = finish(wkv6::generic_backward(st, dtype, B, T, H, C / H, r, k, v, w, u, nullptr, gy, nullptr, gr, gk, gv, gw, gu, nullptr, workspace));
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
+        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
         return rc;
     }
     if (train_chunk32(dtype, algo, B, T, H)) {
@@ -514,19 +514,17 @@ static int backward_impl(void *stream, int dtype, int algo, int64_t B, int64_t T
         }
         if (states_ready && train_segments32(dtype, algo, B, T, H) > 1) {
             if (workspace_bytes < wkv6_saved_bytes(dtype, algo, B, T, C, H)) return WKV6_ERR_WORKSPACE;
-            rc = finish(wkv6::chunk32_backward_saved_segments(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
-        } else {
-            rc = finish(wkv6::chunk32_backward(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
+            return finish(wkv6::chunk32_backward_saved_segments(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, gu_sum, workspace));
         }
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
-        return rc;
+        return finish(wkv6::chunk32_backward(st, dtype, grad_dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace,
+                                             nullptr, nullptr, nullptr, nullptr, wkv6::RowCut(), false, gu_sum));
     }
     if (algo == WKV6_ALGO_CHUNK && !chunk_possible(dtype, T, C)) return WKV6_ERR_UNSUPPORTED;
     const bool chunk = algo == WKV6_ALGO_CHUNK ||
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     if (!chunk) {
         rc = finish(wkv6::scan_backward(st, dtype, B, T, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, workspace));
-        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), grad_dtype, B, C, gu, gu_sum));
+        if (rc == WKV6_OK && gu_sum) rc = finish(wkv6::sum_over_batch(st, out_type(dtype), B, C, gu, gu_sum));
         return rc;
     }
     if (!states_ready && !one_piece && train_segments(dtype, algo, B, T, C, H) > 1) {

@@ -61,6 +61,16 @@ struct C32BwdArgs {
     float *gs0;
     int slice;      // chunks of a pair's slice of `saved` (those of the longest row)
     RowCut cut;     // rows that are time segments
+    int P;          // ... of which so many make a sequence (0: every row is a sequence)
+    // Sums of gu, by the last workgroup of a head to arrive (null: not wanted): every row leaves its part, written through, at
+    // parts + row * part_row + head * part_head; arrivals[head * arrival_step] counts.  Without segments both lie in the pairs'
+    // slices of `saved`, in the place of the first chunk's state, which is zero and not read.
+    float *parts;
+    int64_t part_row, part_head;
+    int *arrivals;
+    int64_t arrival_step;
+    void *gu_sum;     // (C) in Tg, or null
+    float *gu_seq;    // with segments: (sequences, C)
 };
 
 // kOnlyG: only the reverse state is wanted (gs0): the value waves update it, everything else is left out.  (A pair that is
@@ -94,6 +104,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
     const Tin *u = reinterpret_cast<const Tin *>(a.u);
     const Tout *gy = reinterpret_cast<const Tout *>(a.gy);
     float *const ck = a.saved + (int64_t)pair * a.slice * (kN * kN);
+    const bool first_row = a.P ? b % a.P == 0 : a.s0 == nullptr, last_row = a.P && b % a.P == a.P - 1;
+    __shared__ float s_gu[kN];   // the row's gu
     // step s handles chunk nchunk - 1 - s
 
     if (wave >= 8) {
@@ -334,7 +346,15 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) St[jb][e] = p0[jb * 1024 + e * 4];
         };
-        load_state(nchunk - 1);
+        const int lowest = a.s0 ? 0 : 1;   // the state before a sequence's first token is zero where none is given
+        auto next_state = [&](int c) {     // the state of chunk c - 1, where there is one
+            if (c > lowest) load_state(c - 1);
+            else {
+#pragma unroll
+                for (int jb = 0; jb < 4; ++jb) St[jb] = zero;
+            }
+        };
+        next_state(nchunk);
         __syncthreads();
         for (int s = 0; s < nchunk; ++s) {
             const int c = nchunk - 1 - s, buf = s & 1;
@@ -386,7 +406,7 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
                 }
                 Z[x] *= e_mid;
             }
-            if (c > 0) load_state(c - 1);
+            next_state(c);
             f32x4 rp[2], kp[2];   // R', K'; element e: token 16x + 4g + e, channel col
 #pragma unroll
             for (int x = 0; x < 2; ++x)
@@ -453,7 +473,8 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
                 }
                 // (a zero initial state: the first decay reaches no output, its gradient is zero and not
                 // what rounding leaves of two equal sums)
-                if (x == 0 && a.s0 == nullptr && c == 0 && n == 0) o_w = zero;
+                if (x == 0 && first_row && c == 0 && n == 0) o_w = zero;
+                if (last_row && c == nchunk - 1 && c * kC32 + 16 * x + n == T - 1) o_w = zero;   // (nor does the last one of a sequence in segments)
                 if (full || 16 * x < left) store4(gw + out0 + 16 * x * C + lane_off, o_w[0], o_w[1], o_w[2], o_w[3]);
             }
             __syncthreads();
@@ -461,27 +482,63 @@ __global__ __launch_bounds__(768) void chunk32_bwd_kernel(C32BwdArgs a)
         // gu: the lanes of a row hold the tokens n (mod 16) of every chunk
 #pragma unroll
         for (int e = 0; e < 4; ++e) gu_acc[e] = row_sum16(gu_acc[e]);
-        if (n < 4) store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + ch + n, n == 0 ? gu_acc[0] : n == 1 ? gu_acc[1] : n == 2 ? gu_acc[2] : gu_acc[3]);
+        if (n < 4) {
+            const float x = n == 0 ? gu_acc[0] : n == 1 ? gu_acc[1] : n == 2 ? gu_acc[2] : gu_acc[3];
+            store1(reinterpret_cast<Tout *>(a.gu) + (int64_t)b * C + h * kN + ch + n, x);
+            s_gu[ch + n] = x;
+        }
     }
     __syncthreads();
     // a pair whose decay left the reach: once more, one timestep at a time (the pair's slice of the saved
-    // states, T/32 x 64 x 64 floats, is large enough for the T x 64 workspace of that pass)
+    // states, T/32 x 64 x 64 floats, is large enough for the T x 64 workspace of that pass behind the first chunk's state,
+    // whose place may hold parts and counters)
     __shared__ float s_ft[kN];
     if (L.wild[0] | L.wild[1] | L.wild[2] | L.wild[3]) {
         const int64_t so = (int64_t)pair * (kN * kN);
-        const float *s0p = a.s0 ? a.s0 + so : nullptr, *gsTp = a.gsT ? a.gsT + so : nullptr;
+        const float *s0p = a.s0 && !first_row ? a.s0 + so : nullptr, *gsTp = a.gsT && !last_row ? a.gsT + so : nullptr;
         float *gs0p = a.gs0 ? a.gs0 + so : nullptr;
+        float *const wsP = ck + kN * kN;
         const bool states = s0p || gsTp || gs0p;
         __syncthreads();
         scan_bwd_a_body<Tin, Tout>(reinterpret_cast<C32BwdSmem *>(c32_smem)->scan_a, b, h, T, H, r, k, v, w, u, gy,
-                                   reinterpret_cast<Tg *>(a.gr), reinterpret_cast<Tout *>(a.gu), ck, kN,
+                                   reinterpret_cast<Tg *>(a.gr), reinterpret_cast<Tout *>(a.gu), wsP, kN,
                                    s0p, gsTp, states ? s_ft : nullptr);
         __threadfence_block();
         __syncthreads();
-        scan_bwd_b_body<Tin, Tout>(reinterpret_cast<C32BwdSmem *>(c32_smem)->scan_b, b, h, T, H, r, k, v, w, u, gy, ck, kN,
+        scan_bwd_b_body<Tin, Tout>(reinterpret_cast<C32BwdSmem *>(c32_smem)->scan_b, b, h, T, H, r, k, v, w, u, gy, wsP, kN,
                                    reinterpret_cast<Tg *>(a.gk), reinterpret_cast<Tg *>(a.gv), reinterpret_cast<Tg *>(a.gw),
                                    gsTp, states ? s_ft : nullptr, gs0p, s0p == nullptr);
+        __threadfence_block();
+        __syncthreads();
+        if (wave == 8) s_gu[lane] = reinterpret_cast<const Tout *>(a.gu)[(int64_t)b * C + h * kN + lane];
     }
+    if (kOnlyG) return;
+    // (these arguments are read anew from the argument block: kept in scalar registers across the chunks they spill others that
+    // the loops use)
+    const C32BwdArgs __attribute__((address_space(4))) *z = (const C32BwdArgs __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(z));
+    if (z->parts == nullptr) return;
+    __shared__ int s_last;
+    const int rows = (int)gridDim.x / H;
+    if (wave == 8) {   // (a loading wave: it has no stores of gradients to wait for)
+        __hip_atomic_store(z->parts + b * z->part_row + h * z->part_head + lane, s_gu[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (written before it is counted)
+        if (lane == 0) s_last = __hip_atomic_fetch_add(z->arrivals + h * z->arrival_step, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == rows - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the last workgroup of the head: rows of a sequence first (one each without segments), then the sequences
+    float *part = reinterpret_cast<float *>(c32_smem), *first = z->parts + h * z->part_head;
+    const int per = z->P ? z->P : rows;
+    float sum = 0.f;
+    for (int s = 0; s < rows / per; ++s) {
+        const float one = sum_partial_rows<12>(first + (int64_t)s * per * z->part_row, z->part_row, per, part, wave, lane);
+        if (z->P && tid < kN) z->gu_seq[(int64_t)s * C + h * kN + tid] = one;
+        sum += one;
+        __syncthreads();
+    }
+    if (z->gu_sum && tid < kN) store1(reinterpret_cast<Tg *>(z->gu_sum) + h * kN + tid, sum);
+    if (tid == 0) __hip_atomic_store(z->arrivals + h * z->arrival_step, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // armed again
 }
 
 template <typename Tin, typename Tout, typename Tg, bool kOnlyG>
@@ -496,11 +553,24 @@ static hipError_t launch(hipStream_t st, int64_t B, const C32BwdArgs &a) {
 hipError_t chunk32_backward(hipStream_t st, int dtype, int grad_dtype, int64_t B, int64_t T, int64_t H,
                             const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
                             void *gr, void *gk, void *gv, void *gw, void *gu, void *saved_states,
-                            const float *s0, const float *gsT, const float *sT, float *gs0, RowCut cut, bool only_gs0)
+                            const float *s0, const float *gsT, const float *sT, float *gs0, RowCut cut, bool only_gs0, void *gu_sum,
+                            const C32Segments *seg)
 {
     if (grad_dtype != kF32 && (grad_dtype != kF16 || dtype != kF16)) return hipErrorInvalidValue;
     if (gsT != nullptr && sT == nullptr) return hipErrorInvalidValue;   // (the anchor of the decay gradient needs S_T)
-    C32BwdArgs a;
+    C32BwdArgs a = {};
+    if (seg) {
+        a.P = seg->P; a.parts = seg->gu_rows; a.part_row = H * kN; a.part_head = kN;
+        a.arrivals = seg->arrivals; a.arrival_step = 1;
+        a.gu_sum = gu_sum; a.gu_seq = (float *)gu;
+        gu = seg->gu_rows;
+    } else if (gu_sum) {
+        if (s0 || gsT || gs0) return hipErrorInvalidValue;   // (the first chunk's state is in use)
+        const int64_t slice = (T + kC32 - 1) / kC32 * (kN * kN);
+        a.parts = reinterpret_cast<float *>(saved_states) + kN; a.part_row = H * slice; a.part_head = slice;
+        a.arrivals = reinterpret_cast<int *>(saved_states); a.arrival_step = slice;
+        a.gu_sum = gu_sum;
+    }
     a.cut = cut; a.slice = (int)((T + kC32 - 1) / kC32);
     a.s0 = s0; a.gsT = gsT; a.sT = sT; a.gs0 = gs0;
     a.T = (int)T; a.H = (int)H;
@@ -517,7 +587,7 @@ hipError_t chunk32_backward(hipStream_t st, int dtype, int grad_dtype, int64_t B
 
 hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int grad_dtype, int64_t B, int64_t T, int64_t H,
                                            const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
-                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *saved)
+                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *gu_sum, void *saved)
 {
     const C32Segments s = chunk32_segments_layout(B, T, H, saved);
     const int64_t rows = B * s.P;
@@ -527,11 +597,8 @@ hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int grad_d
                                     s.states, nullptr, nullptr, s.gstates, s.cut, true);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_factors(st, s.P, B, H, s.decay, s.gstates, true)) != hipSuccess) return e;
-    e = chunk32_backward(st, dtype, grad_dtype, rows, s.L, H, r, k, v, w, u, gy, gr, gk, gv, gw, s.gu_rows, s.chunks,
-                         s.states, s.gstates, s.ends, nullptr, s.cut);
-    if (e != hipSuccess) return e;
-    return grad_dtype == kF16 ? segments_finish(st, s.P, B, T, H, s.gu_rows, (float *)gu, (f16_t *)gw, true, true)
-                              : segments_finish(st, s.P, B, T, H, s.gu_rows, (float *)gu, (float *)gw, true, true);
+    return chunk32_backward(st, dtype, grad_dtype, rows, s.L, H, r, k, v, w, u, gy, gr, gk, gv, gw, gu, s.chunks,
+                            s.states, s.gstates, s.ends, nullptr, s.cut, false, gu_sum, &s);
 }
 
 }  // namespace wkv6

@@ -49,6 +49,7 @@ struct C32FwdArgs {
     float *saved;   // [pair][chunk][4096] chunk-start states in fragment order (null: not kept)
     int slice;      // chunks of a pair's slice of `saved` (those of the longest row)
     RowCut cut;     // rows that are time segments
+    int *arrivals;  // null, or per head: the counters of the backward's sums of gu, zeroed here
     float *decay;   // null, or (states only) [2][pair][64]: the decay of the whole row, as the product of the two loading groups' chunks
 };
 
@@ -225,6 +226,7 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
                 if (t < T) store4(y + base + (int64_t)t * C + ch, o[0], o[1], o[2], o[3]);
             }
         };
+        if (a.arrivals && b == 0 && tid == 0) a.arrivals[h] = 0;
         float *saved = a.saved ? a.saved + (int64_t)pair * a.slice * (kN * kN) + (q * 4) * 256 + lane * 4 : nullptr;
         __syncthreads();
         for (int c = 0; c < nchunk; ++c) {
@@ -333,11 +335,12 @@ static hipError_t launch(hipStream_t st, int64_t B, const C32FwdArgs &a) {
 
 hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B, int64_t T, int64_t H,
                            const void *r, const void *k, const void *v, const void *w, const void *u,
-                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, RowCut cut)
+                           const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, RowCut cut,
+                           int *arrivals)
 {
     (void)state_dtype;   // fp32 and fp16 tensors keep fp32 states
     C32FwdArgs a;
-    a.cut = cut; a.decay = decay; a.slice = (int)((T + kC32 - 1) / kC32);
+    a.cut = cut; a.decay = decay; a.arrivals = arrivals; a.slice = (int)((T + kC32 - 1) / kC32);
     a.T = (int)T; a.H = (int)H;
     a.r = r; a.k = k; a.v = v; a.w = w; a.u = u; a.s0 = s0; a.map = map; a.y = y; a.sT = sT;
     a.saved = reinterpret_cast<float *>(saved_states);
@@ -373,7 +376,8 @@ C32Segments chunk32_segments_layout(int64_t B, int64_t T, int64_t H, void *saved
     s.gstates = s.ends + pairs * kN * kN;
     s.decay = s.gstates + pairs * kN * kN;
     s.gu_rows = s.decay + 2 * pairs * kN;
-    s.bytes = reinterpret_cast<char *>(s.gu_rows + pairs * kN) - reinterpret_cast<char *>(s.chunks);
+    s.arrivals = reinterpret_cast<int *>(s.gu_rows + pairs * kN);
+    s.bytes = reinterpret_cast<char *>(s.arrivals + H) - reinterpret_cast<char *>(s.chunks);
     return s;
 }
 hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, int64_t T, int64_t H,
@@ -385,7 +389,7 @@ hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, i
     hipError_t e = chunk32_forward(st, dtype, kF32, rows, s.L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_factors(st, s.P, B, H, s.decay, s.states, false)) != hipSuccess) return e;
-    return chunk32_forward(st, dtype, kF32, rows, s.L, H, r, k, v, w, u, s.states, nullptr, y, s.ends, s.chunks, nullptr, s.cut);
+    return chunk32_forward(st, dtype, kF32, rows, s.L, H, r, k, v, w, u, s.states, nullptr, y, s.ends, s.chunks, nullptr, s.cut, s.arrivals);
 }
 
 }  // namespace wkv6

@@ -684,22 +684,20 @@ size_t chunk_saved_bytes(int64_t B, int64_t T, int64_t H) {
     return chunk_backward_workspace_bytes(B, T, H) + (((size_t)H * sizeof(int) + 255) & ~(size_t)255);
 }
 
-template <typename T, typename E>
-__global__ void sum_over_batch_kernel(int B, int C, const T *__restrict__ p, E *__restrict__ out) {
+template <typename T>
+__global__ void sum_over_batch_kernel(int B, int C, const T *__restrict__ p, T *__restrict__ out) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= C) return;
     float acc = 0.f;
     for (int b = 0; b < B; ++b) acc += load1(p + (int64_t)b * C + c);
     store1(out + c, acc);
 }
-hipError_t sum_over_batch(hipStream_t st, int out_dtype, int sum_dtype, int64_t B, int64_t C, const void *partials, void *sum) {
+hipError_t sum_over_batch(hipStream_t st, int out_dtype, int64_t B, int64_t C, const void *partials, void *sum) {
     const dim3 grid((unsigned)((C + 255) / 256)), block(256);
-    if (sum_dtype == kF16)
-        hipLaunchKernelGGL((sum_over_batch_kernel<float, f16_t>), grid, block, 0, st, (int)B, (int)C, (const float *)partials, (f16_t *)sum);
-    else if (out_dtype == kBF16)
-        hipLaunchKernelGGL((sum_over_batch_kernel<bf16_t, bf16_t>), grid, block, 0, st, (int)B, (int)C, (const bf16_t *)partials, (bf16_t *)sum);
+    if (out_dtype == kBF16)
+        hipLaunchKernelGGL(sum_over_batch_kernel<bf16_t>, grid, block, 0, st, (int)B, (int)C, (const bf16_t *)partials, (bf16_t *)sum);
     else
-        hipLaunchKernelGGL((sum_over_batch_kernel<float, float>), grid, block, 0, st, (int)B, (int)C, (const float *)partials, (float *)sum);
+        hipLaunchKernelGGL(sum_over_batch_kernel<float>, grid, block, 0, st, (int)B, (int)C, (const float *)partials, (float *)sum);
     return hipGetLastError();
 }
 
@@ -749,13 +747,12 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
     return ragged ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
-// Training pair in time segments, last step: gu of a batch row = sum over its segments, which come unrounded (up to 16 of
+// bf16 training pair in time segments, last step where the rows did not do it themselves (block form): gu of a batch row = sum over its segments, which come unrounded (up to 16 of
 // them rounded to bf16 first made gu's error 1.05 to 1.17 times that of one piece, T 1100 to 5003); the decay
 // gradient at the first and the last token of a sequence is zero by definition
 // (rwkv_kernels.cu:381,406), where the kernels, given explicit states, leave rounding residue.
-template <typename E, typename Eg>
 __global__ void segments_finish_kernel(int P, int64_t T, int C, const float *__restrict__ gu_rows,
-                                       E *__restrict__ gu, Eg *__restrict__ gw, bool zero_first, bool zero_last)
+                                       bf16_t *__restrict__ gu, bf16_t *__restrict__ gw, bool zero_first, bool zero_last)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
     if (c >= C) return;
@@ -766,16 +763,13 @@ __global__ void segments_finish_kernel(int P, int64_t T, int C, const float *__r
     if (zero_last) store1(gw + ((int64_t)b * T + T - 1) * C + c, 0.f);
 }
 
-template <typename E, typename Eg>
-hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, E *gu, Eg *gw, bool zero_first, bool zero_last)
+static hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, bf16_t *gu, bf16_t *gw, bool zero_first, bool zero_last)
 {
     const int C = (int)(H * kN);
-    hipLaunchKernelGGL((segments_finish_kernel<E, Eg>), dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
+    hipLaunchKernelGGL(segments_finish_kernel, dim3((unsigned)((C + 255) / 256), (unsigned)B), dim3(256), 0, st,
                        P, T, C, gu_rows, gu, gw, zero_first, zero_last);
     return hipGetLastError();
 }
-template hipError_t segments_finish<float, float>(hipStream_t, int, int64_t, int64_t, int64_t, const float *, float *, float *, bool, bool);
-template hipError_t segments_finish<float, f16_t>(hipStream_t, int, int64_t, int64_t, int64_t, const float *, float *, f16_t *, bool, bool);
 
 hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                          const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,

@@ -113,4 +113,20 @@ __device__ __forceinline__ float load1(const bf16_t *p) {
 }
 __device__ __forceinline__ float load1(const f16_t *p) { return (float)*p; }
 
+// What the last workgroup of a head makes of the head's partial rows of gu (64 floats each, written through by the others): row j
+// at `first + j * stride`, summed over j.  Wave w of kWaves takes rows w, w + kWaves, ..; the caller's 64 lanes of wave 0 get the
+// sum.  (These loads pass by the caches, about a microsecond each: one wave that adds row after row waits for them one by
+// one: with eight rows a training pair took 1.2 us longer at B8 T1024 H32 and 2.5 at B1 T8192 H32.)  part: kWaves rows of 64 floats in LDS.
+template <int kWaves>
+__device__ __forceinline__ float sum_partial_rows(const float *first, int64_t stride, int rows, float *part, int wave, int lane) {
+    float acc = 0.f;
+    for (int j = wave; j < rows; j += kWaves) acc += __hip_atomic_load(first + j * stride + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    part[wave * kN + lane] = acc;
+    __syncthreads();
+    float sum = 0.f;
+    if (wave == 0)
+        for (int j = 0; j < min(rows, kWaves); ++j) sum += part[j * kN + lane];
+    return sum;
+}
+
 }  // namespace wkv6

@@ -148,8 +148,9 @@ hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B
                            const void *r, const void *k, const void *v, const void *w, const void *u,
                            const void *s0, const int64_t *map, void *y, void *sT, void *saved_states,
                            float *decay = nullptr,   // [2][pair][64]: two factors of each row's decay
-                           RowCut cut = RowCut());
+                           RowCut cut = RowCut(), int *arrivals = nullptr);   // arrivals: see C32FwdArgs
 
+struct C32Segments;
 // saved_states: what chunk32_forward left (the pair's slice also serves the per-timestep pass of a pair
 // whose decay left the chunk form's reach); gu (B, C)
 // grad_dtype: type of gr, gk, gv, gw: kF32, or kF16 for fp16 tensors
@@ -159,7 +160,10 @@ hipError_t chunk32_backward(hipStream_t st, int dtype, int grad_dtype, int64_t B
                             // gradients through the state ((B,H,64,64) fp32 [key][value]; sT = the forward's final state,
                             // needed with gsT); the saved states come from a forward that started from s0
                             const float *s0 = nullptr, const float *gsT = nullptr, const float *sT = nullptr, float *gs0 = nullptr,
-                            RowCut cut = RowCut(), bool only_gs0 = false);   // only_gs0: nothing but gs0 is wanted
+                            RowCut cut = RowCut(), bool only_gs0 = false,   // only_gs0: nothing but gs0 is wanted
+                            // gu_sum (may be null; without states): (C) in grad_dtype, the sum of gu over the batch
+                            // seg: the rows are segments: gu (sequences, C) and gu_sum from all of them, gw zero at the sequences' ends
+                            void *gu_sum = nullptr, const C32Segments *seg = nullptr);
 
 // The training pair in time segments; what the forward leaves for the backward in `saved` (the first part as chunk32_forward).
 struct C32Segments {
@@ -170,6 +174,7 @@ struct C32Segments {
     float *states, *ends, *gstates;   // [B*P][H][64][64]: state entering and leaving each segment, gradient arriving at its end
     float *decay;      // [2][B*P][H][64]
     float *gu_rows;    // [B*P][C]
+    int *arrivals;     // [H]
     size_t bytes;
 };
 int chunk32_train_segments(int64_t B, int64_t T, int64_t H, int64_t *L);
@@ -179,7 +184,7 @@ hipError_t chunk32_forward_save_segments(hipStream_t st, int dtype, int64_t B, i
                                          void *y, void *saved);
 hipError_t chunk32_backward_saved_segments(hipStream_t st, int dtype, int grad_dtype, int64_t B, int64_t T, int64_t H,
                                            const void *r, const void *k, const void *v, const void *w, const void *u, const void *gy,
-                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *saved);
+                                           void *gr, void *gk, void *gv, void *gw, void *gu, void *gu_sum, void *saved);
 
 // fp16 tensors on the chunked kernels (training pair only: y and the gradients are fp32).  r, k, w stay
 // fp16 (the kernels unpack them exactly); v and gy are consumed as bf16 MFMA operands, so the caller
@@ -223,8 +228,6 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse);
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
 RowCut cut_of(int P, int64_t L, int64_t T);
-template <typename E, typename Eg>
-hipError_t segments_finish(hipStream_t st, int P, int64_t B, int64_t T, int64_t H, const float *gu_rows, E *gu, Eg *gw, bool zero_first, bool zero_last);
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
 hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -301,7 +304,7 @@ hipError_t chunk_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
 // in_dtype kF16 (needs states_ready): r, k, w, u fp16, v and gy their bf16 copies, v_orig / gy_orig the
 // caller's fp16 v and fp32 gy, gradients fp32
 
-// sum over the batch of (B, C) partials -> (C), both in the output type, or fp32 partials and an fp16 sum (for the paths without a fused sum)
-hipError_t sum_over_batch(hipStream_t st, int out_dtype, int sum_dtype, int64_t B, int64_t C, const void *partials, void *sum);
+// sum over the batch of (B, C) partials -> (C), both in the output type (for the paths without a fused sum)
+hipError_t sum_over_batch(hipStream_t st, int out_dtype, int64_t B, int64_t C, const void *partials, void *sum);
 
 }  // namespace wkv6
