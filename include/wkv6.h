@@ -273,8 +273,8 @@ size_t wkv6_backward_workspace_bytes_ex(int dtype, int algo, int64_t B, int64_t 
  * chunk form: the fp32 state at every 32-token chunk start), and the backward that consumes it and therefore
  * skips its own forward state sweep.  `saved` is caller-owned device memory of wkv6_saved_bytes()
  * bytes (0 = this path saves nothing; pass NULL), must be left untouched between the two calls,
- * and serves the backward as its workspace too.  A long sequence (T >= 1024) of so few (batch, head)
- * pairs that they fill at most half of the compute units runs as 2 to 16 time segments side by side in
+ * and serves the backward as its workspace too.  A sequence (bf16 from T = 705 on, fp32 and fp16 from 320) of so few
+ * (batch, head) pairs that they fill at most half of the compute units runs as 2 to 16 time segments side by side in
  * both calls, whatever its length (same results to rounding); wkv6_saved_bytes() includes what that keeps.
  * No counterpart in the reference, whose backward
  * recomputes everything from the inputs (rwkv_kernel/torch_rwkv_kernel.py:33 saves only r,k,v,w,u). */

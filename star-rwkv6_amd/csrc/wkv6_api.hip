@@ -108,7 +108,9 @@ size_t wkv6_forward_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, i
     const bool chunk = (algo == WKV6_ALGO_CHUNK && chunk_possible(dtype, T, C)) ||
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     // optional: with it, a long sequence of few (batch, head) pairs runs as time segments side by side
-    return chunk ? wkv6::chunk_forward_segments_workspace_bytes(B, T, H) : 0;
+    if (!chunk) return 0;
+    const size_t plain = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, false), fused = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, true);
+    return plain > fused ? plain : fused;
 }
 
 static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
@@ -140,7 +142,7 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
     if (!chunk)
         return finish(wkv6::scan_forward(st, dtype, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys));
     if (!saved && workspace && aligned16(workspace)) {
-        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H);
+        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, false);
         if (need > 0 && workspace_bytes >= need)
             return finish(wkv6::chunk_forward_segments_run(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, workspace));
     }
@@ -185,7 +187,7 @@ int wkv6_forward_gn_gate_ex(void *stream, int dtype, int state_dtype,
                                                has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
                                                gate, gn_scale, gn_offset, gn_eps, out, ys));
     if (workspace && aligned16(workspace)) {   // optional: few pairs, long sequence -> time segments side by side
-        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H);
+        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, true);
         if (need > 0 && workspace_bytes >= need)
             return finish(wkv6::chunk_forward_segments_run((hipStream_t)stream, state_dtype, B, T, H, r, k, v, w, u,
                                                            has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,

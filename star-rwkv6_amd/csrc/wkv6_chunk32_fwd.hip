@@ -353,16 +353,15 @@ hipError_t chunk32_forward(hipStream_t st, int dtype, int state_dtype, int64_t B
 // The training pair of a long sequence of few pairs in time segments, as in the bf16 forms (wkv6_chunk_fwd.hip): a
 // states-only pass over all segments at once, the chain, and the saving forward from every segment's true state.  The
 // decay of a segment is carried as the product of its chunks' e^{c_32} themselves, not as an exponent.
-// Without segments a pair's chunks follow each other in one workgroup whatever else is idle.  Forward and backward, before and
-// now: fp32 B1 T8191 H32 2317 -> 441 us, B2 T2048 H16 580 -> 126, B1 T1031 H64 307 -> 144; fp16 B1 T5003 H8 1420 -> 167, B4
-// T2100 H32 704 -> 521.  Two or three segments only from 2048 tokens on, as in the bf16 forms; below, where the line has not been
-// looked for, they would gain as well: fp32 pair in one piece / in segments, B2 T1024 H64 276 / 235 us, B2 T1999 H64 534 / 441,
-// B3 T1024 H24 258 / 172.
+// Without segments a pair's chunks follow each other in one workgroup whatever else is idle.  From 320 tokens on, two or three
+// segments from 384 (four launches more: 18 us of host time on top of 65).  fp32 pair of kernels in one piece / in segments:
+// B1 T320 H8 89 / 49 us, T512 H8 134 / 51, B4 T512 H16 138 / 86, B1 T1000 H8 251 / 57; with two segments B2 T320 H48 95 / 101, T384
+// 110 / 102, T512 140 / 124, T1000 267 / 217; longer ones B1 T8191 H32 2317 / 441, B2 T2048 H16 580 / 126.
 // ------------------------------------------------------------------------------------------
 int chunk32_train_segments(int64_t B, int64_t T, int64_t H, int64_t *L) {
-    if (T < 1024) return 1;
-    const int P = plan_segments(B * H, T, 4, L);
-    return T >= 2048 || P >= 4 ? P : 1;
+    if (T < 320) return 1;
+    const int P = plan_segments(B * H, T, 1, L);
+    return P >= 4 || T >= 384 ? P : 1;
 }
 C32Segments chunk32_segments_layout(int64_t B, int64_t T, int64_t H, void *saved) {
     C32Segments s;

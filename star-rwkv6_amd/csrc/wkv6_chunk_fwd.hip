@@ -810,10 +810,9 @@ static hipError_t launch_chain(hipStream_t st, int P, int64_t B, int64_t H, cons
 
 // Segments of a sequence of T tokens when `pairs` (batch, head) pairs share the chip: as many as still fit it once, each a
 // whole number of chunks and at least `least` of them; the last one ends with the sequence.  (Segments that had to
-// divide the sequence left training at all other lengths to one workgroup per pair; a prompt's tokens behind its equal
-// segments took a pass of their own.  Forward and backward at H32: B1 T8191 771 -> 176 us, B1 T2049 211 -> 87, B4 T4001
-// 427 -> 326; H8 B1 T5003 475 -> 88; prompts of H32: T1337 38 -> 23 us, T1024 37 -> 22 (six segments of three chunks
-// instead of four of four), T3000 with the output stage 57 -> 36.)
+// divide the sequence left training at all other lengths to one workgroup per pair: forward and backward at H32 T8191 771 ->
+// 176 us, H8 T5003 475 -> 88.  At least three chunks of a prompt and four in training, as long as the chain was a launch of its
+// own, / one: training pair bf16 B1 T1400 H16 67.8 / 44.4, T1900 H8 66.8 / 44.4, fp32 B1 T1400 H8 116 / 77, prompt T1337 H8 23.2 / 19.2.)
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L) {
     const int64_t chunks = (T + CL - 1) / CL, fit = compute_units() / pairs;
     const int64_t most = fit < kMostSegments ? fit : kMostSegments;
@@ -829,28 +828,38 @@ RowCut cut_of(int P, int64_t L, int64_t T) {
     return c;
 }
 
-static int forward_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
-    // (two passes over T / P tokens and two more launches against one pass over T: nothing to gain
-    // below four segments or on short sequences)
-    if (T < 1024) return 1;
+// The second pass of the segments, `rows` of them: in block form from a quarter of the chip on (half of it, in one piece:
+// the tile form's two workgroups to a pair save nothing that the chain at the start and whole rows do not save as well; training pair of
+// B1 H8 T1000 46.6 us as tiles / 36.8, T4000 73.8 / 63.0, H4 T768 38.8 / 31.2).  Fewer rows still run the tile form, whose y is, but
+// for the chain's rounding, that of a call in one piece.
+bool segments_in_block_form(int64_t rows, int64_t H) { return 4 * rows * H >= compute_units(); }
+
+// Prompts, in one piece / in segments: B1 T256 H16 17.7 / 17.5 us, T384 H8 17.7 / 16.6, H64 21.2 / 18.8, T512 H32 22.4 / 17.4, T1000
+// H16 36.5 / 20.1, H64 38.1 / 27.8; three segments H72 T384 19.5 / 19.5, T512 23.4 / 22.6; two H128 T1024 38.0 / 39.9, T2048
+// 65.0 / 61.4.  With the output stage, whose first pass leaves it out, three H72 T384 23.2 / 20.3; two H128 T384 25.1 / 24.8 (B8 H8
+// 23.2 / 24.4), T512 30.1 / 28.3, T2048 90.2 / 66.1.
+static bool prompt_takes(int P, int64_t T, bool fused) {
+    return P >= 4 ? T >= 384 : P == 3 ? T >= (fused ? 384 : 512) : P == 2 && T >= (fused ? 512 : 2048);
+}
+static int forward_segments_plan(int64_t B, int64_t T, int64_t H, bool fused, int64_t *L) {
     if (B == 1) {
-        const int P = plan_segments(H, T, 3, L);
+        int P = plan_segments(H, T, 1, L);
+        if (segments_in_block_form(P, H)) return prompt_takes(P, T, fused) ? P : 1;
+        P = T >= 1024 ? plan_segments(H, T, 3, L) : 1;
         return P >= 4 ? P : 1;
     }
     // (the interface promises segments to batches whose length divides evenly, and no workspace to others)
-    for (int P = kMostSegments; P >= 4; P >>= 1)
-        if (B * H * P <= compute_units() && T % (P * CL) == 0 && T / P >= 4 * CL) {
+    for (int P = kMostSegments; P >= 2; P >>= 1)
+        if (B * H * P <= compute_units() && T % (P * CL) == 0 &&
+            (segments_in_block_form(B * P, H) ? prompt_takes(P, T, fused) : T >= 1024 && P >= 4 && T / P >= 4 * CL)) {
             *L = T / P;
             return P;
         }
     return 1;
 }
-int chunk_forward_segments(int64_t B, int64_t T, int64_t H) {
+size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused) {
     int64_t L;
-    return forward_segments_plan(B, T, H, &L);
-}
-size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H) {
-    const int P = chunk_forward_segments(B, T, H);
+    const int P = forward_segments_plan(B, T, H, fused, &L);
     // per segment and pair two states (what it leaves alone, what it starts from) and the decay
     return P <= 1 ? 0 : (size_t)(B * P * H) * (2 * kN * kN + kN) * sizeof(float);
 }
@@ -862,13 +871,13 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps)
 {
     int64_t L = 0;
-    const int P = forward_segments_plan(B, T, H, &L);
+    const int P = forward_segments_plan(B, T, H, gate != nullptr, &L);
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
     float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;
     hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
     if (e != hipSuccess) return e;
-    if (block_forward_applies(rows, L, H)) {   // the chain at the start of the second pass
+    if (segments_in_block_form(rows, H)) {   // the chain at the start of the second pass
         SegmentChain c;
         c.P = P; c.alone = states; c.decay = decay; c.first = s0; c.map = map; c.last = sT; c.bf16 = state_dtype != kF32; c.start = start;
         return gate ? block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr, nullptr, nullptr, nullptr, cut, c)
@@ -898,13 +907,17 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 // keeps every segment's incoming state and decay exponents for the backward, whose reverse state
 // is chained the same way (see chunk_backward_saved_segments).
 // ------------------------------------------------------------------------------------------
+// From 705 tokens on: below, the two more launches cost a caller whose host is what takes the time (60 us of autograd and 9
+// for them) what the kernels gain.  Pair of kernels in one piece / in segments: B1 T512 H8 57.9 / 30.7 us, T768 H8 80.7 / 33.1, H40
+// 82.1 / 43.1, T1000 H16 108 / 39, B2 T1000 H12 108 / 47.  Two or three segments from 833 on (B2 H48 T1000 113 / 92, T1900 197 / 145;
+// T768 84.8 / 71.2, but without saved states B5 T768 H24 75.7 / 78.3, T1000 101.8 / 97.8).
 static int train_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
-    // (two state-only passes at 0.7 of a forward each on top of the forward and the backward: 1.5
-    // times the work on P times the workgroups, and three small kernels.  Two or three segments only from 2048 tokens on;
-    // below they would gain less, but gain: kernels in one piece / in segments, B2 T1024 H64 109 / 104 us, B2 T1999 H64 214 / 174,
-    // B3 T1024 H24 107 / 87)
+    if (T <= 704) return 1;
+    int P = plan_segments(B * H, T, 1, L);
+    if (segments_in_block_form(B * P, H)) return P >= 4 || T > 832 ? P : 1;
+    // (tile form: two state-only passes at 0.7 of a forward each on top of the forward and the backward, and three small kernels)
     if (T < 1024) return 1;
-    const int P = plan_segments(B * H, T, 4, L);
+    P = plan_segments(B * H, T, 4, L);
     return T >= 2048 || P >= 4 ? P : 1;
 }
 int chunk_train_segments(int64_t B, int64_t T, int64_t H) {
@@ -938,7 +951,7 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
-    const bool block = block_forward_applies(rows, L, H);
+    const bool block = segments_in_block_form(rows, H);
     hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, saved, true, s.cut, train_chain(s, s.states));
@@ -955,7 +968,7 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
-    const bool block = block_forward_applies(rows, L, H);
+    const bool block = segments_in_block_form(rows, H);
     hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states));

@@ -195,9 +195,8 @@ hipError_t chunk_forward_save_f16(hipStream_t st, int64_t B, int64_t T, int64_t 
                                   void *y, void *saved_states);
 
 // Few pairs, long sequence: the forward as P time segments side by side (two passes joined by the
-// affine map of a segment's state).  chunk_forward_segments = P for the shape (1 = does not apply).
-int chunk_forward_segments(int64_t B, int64_t T, int64_t H);
-size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H);
+// affine map of a segment's state).  The workspace's size is 0 where that does not apply to the shape.
+size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused);   // fused: with the output stage
 hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                       const void *r, const void *k, const void *v, const void *w, const void *u,
                                       const void *s0, const int64_t *map, void *y, void *sT, void *workspace,
@@ -227,6 +226,7 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 // the same with the segments' decays as two factors each, [2][B*P][H][64]
 hipError_t segment_chain_factors(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states, bool reverse);
 int plan_segments(int64_t pairs, int64_t T, int64_t least, int64_t *L);
+bool segments_in_block_form(int64_t rows, int64_t H);   // the form of the second pass of the bf16 pair and of prompts
 RowCut cut_of(int P, int64_t L, int64_t T);
 hipError_t segment_chain_reverse(hipStream_t st, int P, int64_t B, int64_t H, const float *decay, float *states,
                                  const float *arriving = nullptr, float *leaving = nullptr);
