@@ -746,7 +746,7 @@ hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_
 // With fewer (batch, head) pairs than half the compute units most of the chip would idle while each
 // pair walks its sequence alone.  The map from a segment's incoming state to its outgoing state is
 // affine, S_out = D o S_in + U with D[j] = exp(-sum_t exp(w_t[j])) over the segment and U the state
-// the segment builds from zero, so: (A) every segment runs from a zero state (all segments at once;
+// the segment builds from zero, so: (A) every segment runs from a zero state (block form: wkv6_state.hip; all segments at once;
 // a (B,T,C) tensor cut into P equal segments IS a (B*P, T/P, C) tensor, and RowCut stands for other lengths; no y in this pass) and leaves
 // U and, from the producer waves, D; (B) the P affine maps of a pair are chained, at the start of the second pass in
 // the block form (chain_start), by a tiny kernel that leaves each segment's true incoming state where its U was (and the final
@@ -875,7 +875,8 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
     float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
+    hipError_t e = segments_in_block_form(rows, H) ? segment_states(st, rows, L, H, k, v, w, states, decay, false, cut)
+        : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
     if (e != hipSuccess) return e;
     if (segments_in_block_form(rows, H)) {   // the chain at the start of the second pass
         SegmentChain c;
@@ -952,7 +953,8 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, s.alone, s.decay, false, s.cut)
+        : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, saved, true, s.cut, train_chain(s, s.states));
     if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, nullptr)) != hipSuccess) return e;
@@ -969,7 +971,8 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, block ? s.alone : s.states, nullptr, s.decay, false, true, s.cut);
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, s.alone, s.decay, false, s.cut)
+        : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states));
     if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, nullptr)) != hipSuccess) return e;

@@ -101,6 +101,11 @@ struct SegmentChain {
     float *start = nullptr;           // [rows][H][64][64]: receives what every segment starts from
 };
 
+// First pass over the segments (wkv6_state.hip, bf16): the state each row of at most L tokens builds from zero and the decay over it
+// (may be null); reverse: the rows read back to front
+hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w,
+                          float *states, float *decay, bool reverse, RowCut cut);
+
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
