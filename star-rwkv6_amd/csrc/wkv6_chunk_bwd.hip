@@ -782,7 +782,7 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
     // That is the state the FORWARD recurrence builds from zero over the segment read back to front
     // with r in the place of k and gy in the place of v, so the forward kernel's state-only pass does it.
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, r, gy, w, s.alone, nullptr, true, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, r, gy, w, u, s.alone, nullptr, true, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) {   // (2), (3) and the sums over the segments in one launch
@@ -813,13 +813,13 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
     // (what a segment leaves alone: state_kernel, as in the training pair; forward and backward of B1 T8192 H32 through the torch flavour
     // 226 to 234 us with the tile form's state-only passes, 216 so)
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, s.states, s.decay, false, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.states, s.decay, false, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, s0)) != hipSuccess) return e;
     e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, s.states, nullptr, nullptr, nullptr, saved, nullptr, false, false, s.cut);
     if (e != hipSuccess) return e;
-    e = block ? segment_states(st, rows, L, H, r, gy, w, s.gstates, nullptr, true, s.cut)
+    e = block ? segment_states(st, rows, L, H, r, gy, w, u, s.gstates, nullptr, true, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     if ((e = segment_chain_reverse(st, s.P, B, H, s.decay, s.gstates, gsT, gs0)) != hipSuccess) return e;

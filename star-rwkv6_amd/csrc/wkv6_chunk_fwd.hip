@@ -875,7 +875,7 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
     float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;
-    hipError_t e = segments_in_block_form(rows, H) ? segment_states(st, rows, L, H, k, v, w, states, decay, false, cut)
+    hipError_t e = segments_in_block_form(rows, H) ? segment_states(st, rows, L, H, k, v, w, u, states, decay, false, cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
     if (e != hipSuccess) return e;
     if (segments_in_block_form(rows, H)) {   // the chain at the start of the second pass
@@ -953,7 +953,7 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, s.alone, s.decay, false, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, saved, true, s.cut, train_chain(s, s.states));
@@ -971,7 +971,7 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, s.alone, s.decay, false, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states));

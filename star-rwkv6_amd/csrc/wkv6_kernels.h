@@ -103,7 +103,7 @@ struct SegmentChain {
 
 // First pass over the segments (wkv6_state.hip, bf16): the state each row of at most L tokens builds from zero and the decay over it
 // (may be null); reverse: the rows read back to front
-hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w,
+hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w, const void *u,
                           float *states, float *decay, bool reverse, RowCut cut);
 
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
