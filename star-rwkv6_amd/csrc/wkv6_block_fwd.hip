@@ -171,9 +171,9 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
                     A00[rr] = (l16 > s_) ? A00[rr] : ((l16 == s_) ? ruk0 : 0.f);
                     A11[rr] = (l16 > s_) ? A11[rr] : ((l16 == s_) ? ruk1 : 0.f);
                 }
-                const bf16x8 vf = both16(vf0, vf1);
-                Y0 = mfma32(vf, both16(pack4(A00), make_s16x4(0u, 0u)), Y0);
-                Y1 = mfma32(vf, acc_as_operand(A01, A11), Y1);
+                // (the first group by itself: with zeros against the second group's v an infinity there would reach back to it as 0 x inf)
+                Y0 = mfma16(vf0, pack4(A00), Y0);
+                Y1 = mfma32(both16(vf0, vf1), acc_as_operand(A01, A11), Y1);
                 settle(Y0, Y1);
                 *reinterpret_cast<uint2 *>(ys + tile_off(r0, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y0[0], Y0[1]), pack_bf16x2(Y0[2], Y0[3]));
                 *reinterpret_cast<uint2 *>(ys + tile_off(r1, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y1[0], Y1[1]), pack_bf16x2(Y1[2], Y1[3]));
