@@ -239,11 +239,9 @@ __device__ __forceinline__ void chain_start(const SegmentChain &c, int row, int 
     const float *alone = c.alone + from * (kN * kN), *decay = c.decay + from * kN;  // (uniform; the lane's part of the addresses: 8 t, t >> 3)
     const int64_t pairs = kReverse ? -H : H;                                        // ... and its stride
     float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (!kReverse && c.first) {
-        const int64_t e = ((c.map ? c.map[b] : (int64_t)b) * H + h) * (kN * kN) + 8 * t;
-        float lo[4], hi[4];
-        if (c.bf16) { load4(reinterpret_cast<const bf16_t *>(c.first) + e, lo); load4(reinterpret_cast<const bf16_t *>(c.first) + e + 4, hi); }
-        else { load4(reinterpret_cast<const float *>(c.first) + e, lo); load4(reinterpret_cast<const float *>(c.first) + e + 4, hi); }
+    if (!kReverse && c.given) {
+        const float *p = c.start + from * (kN * kN) + 8 * t;
+        const f32x4 lo = *reinterpret_cast<const f32x4 *>(p), hi = *reinterpret_cast<const f32x4 *>(p + 4);
 #pragma unroll
         for (int i = 0; i < 4; ++i) { S[i] = lo[i]; S[4 + i] = hi[i]; }
     }
@@ -269,9 +267,11 @@ __device__ __forceinline__ void chain_start(const SegmentChain &c, int row, int 
     const f32x4 lo = {S[0], S[1], S[2], S[3]}, hi = {S[4], S[5], S[6], S[7]};
     *reinterpret_cast<f32x4 *>(lds + 8 * t) = lo;
     *reinterpret_cast<f32x4 *>(lds + 8 * t + 4) = hi;
-    float *out = c.start + ((int64_t)row * H + h) * (kN * kN) + 8 * t;
-    *reinterpret_cast<f32x4 *>(out) = lo;
-    *reinterpret_cast<f32x4 *>(out + 4) = hi;
+    if (kReverse || !c.given || s > 0) {   // (a given state is there, and other segments read it)
+        float *out = c.start + ((int64_t)row * H + h) * (kN * kN) + 8 * t;
+        *reinterpret_cast<f32x4 *>(out) = lo;
+        *reinterpret_cast<f32x4 *>(out + 4) = hi;
+    }
     if (!kReverse && c.last && s == c.P - 1) {
         // the sequence's final state, one more step of the same walk (the state that the second pass itself ends with is 1.18
         // times as far from float64: its blocks scale k from their middle, the first pass's tiles towards their end)

@@ -875,15 +875,18 @@ hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
     float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;
-    hipError_t e = segments_in_block_form(rows, H) ? segment_states(st, rows, L, H, k, v, w, u, states, decay, false, cut)
-        : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
-    if (e != hipSuccess) return e;
     if (segments_in_block_form(rows, H)) {   // the chain at the start of the second pass
+        GivenStates given;
+        given.states = s0; given.map = map; given.bf16 = state_dtype != kF32; given.P = P; given.start = start;
+        const hipError_t e = segment_states(st, rows, L, H, k, v, w, u, states, decay, false, cut, given);
+        if (e != hipSuccess) return e;
         SegmentChain c;
-        c.P = P; c.alone = states; c.decay = decay; c.first = s0; c.map = map; c.last = sT; c.bf16 = state_dtype != kF32; c.start = start;
+        c.P = P; c.alone = states; c.decay = decay; c.given = s0 != nullptr; c.last = sT; c.bf16 = state_dtype != kF32; c.start = start;
         return gate ? block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, y, nullptr, nullptr, nullptr, nullptr, cut, c)
                     : block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, nullptr, true, cut, c);
     }
+    hipError_t e = chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, states, nullptr, decay, false, true, cut);
+    if (e != hipSuccess) return e;
     e = state_dtype == kF32 ? launch_chain<float, false>(st, P, B, H, (const float *)s0, map, decay, states, (float *)sT)
                             : launch_chain<bf16_t, false>(st, P, B, H, (const bf16_t *)s0, map, decay, states, (bf16_t *)sT);
     if (e != hipSuccess) return e;

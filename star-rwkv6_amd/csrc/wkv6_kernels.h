@@ -94,17 +94,25 @@ struct SegmentChain {
     int P = 0;                        // segments of a sequence (0: every row is a sequence of its own)
     const float *alone = nullptr;     // [rows][H][64][64] (fp32, [key][value])
     const float *decay = nullptr;     // [rows][H][64]
-    const void *first = nullptr;      // forward: the states the sequences start from, or null (zero); type of `last`
-    const int64_t *map = nullptr;     // ... batch row -> row of `first`, or null
+    bool given = false;               // forward: `start` of every sequence's first segment holds the state it starts from (otherwise zero)
     void *last = nullptr;             // forward: the sequences' final states [B][H][64][64], or null
-    bool bf16 = false;                // `first` and `last` are bf16 (otherwise fp32)
+    bool bf16 = false;                // `last` is bf16 (otherwise fp32)
     float *start = nullptr;           // [rows][H][64][64]: receives what every segment starts from
 };
 
+// The states the sequences start from, which the first pass leaves as fp32 in the place of the first segments' `start`: the second
+// pass stores the final states, and a caller's final states may lie where the given ones do.
+struct GivenStates {
+    const void *states = nullptr;     // (n_state, H, 64, 64), or null: zero
+    const int64_t *map = nullptr;     // batch row -> row of `states`, or null: the same
+    bool bf16 = false;                // otherwise fp32
+    int P = 1;                        // segments of a sequence
+    float *start = nullptr;           // as in SegmentChain
+};
 // First pass over the segments (wkv6_state.hip, bf16): the state each row of at most L tokens builds from zero and the decay over it
 // (may be null); reverse: the rows read back to front
 hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w, const void *u,
-                          float *states, float *decay, bool reverse, RowCut cut);
+                          float *states, float *decay, bool reverse, RowCut cut, const GivenStates &given = GivenStates());
 
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,

@@ -39,6 +39,7 @@ struct StateArgs {
     const bf16_t *k, *v, *w;
     const bf16_t *u;             // (read by the pass one timestep at a time, for a y that it does not write)
     float *states, *decay;       // [rows][H][64 key][64 value], [rows][H][64] (may be null)
+    GivenStates given;
 };
 
 __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
@@ -129,6 +130,21 @@ __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
     } else {
         // ---------------- consumer waves ----------------
         const int q = wave - 4, g = lane >> 4, l16 = lane & 15;
+        // the given state of a sequence's first segment: 16 of the 4096 elements to a thread, asked for here and left behind the chunks
+        const bool give = a.given.states && row % a.given.P == 0;
+        const int first = 4 * (64 * q + lane);
+        float given[4][4];
+        if (give) {
+            const int b = row / a.given.P;
+            const int64_t from = ((a.given.map ? a.given.map[b] : (int64_t)b) * a.H + h) * (kN * kN) + first;
+            if (a.given.bf16) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) load4(reinterpret_cast<const bf16_t *>(a.given.states) + from + 1024 * i, given[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) load4(reinterpret_cast<const float *>(a.given.states) + from + 1024 * i, given[i]);
+            }
+        }
         f32x4 S[4];   // S[m][rr]: key row 16m + 4g + rr, value column 16q + l16
 #pragma unroll
         for (int m = 0; m < 4; ++m) S[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -148,6 +164,10 @@ __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
                 for (int m = 0; m < 4; ++m) S[m] = mfma16(kf[m], vf, S[m]);
                 settle(S[0], S[1], S[2], S[3]);
             }
+        }
+        if (give) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) store4(a.given.start + (int64_t)pair * (kN * kN) + first + 1024 * i, given[i][0], given[i][1], given[i][2], given[i][3]);
         }
         if (!s_wild) {   // (complete: the last chunk was prepared before the last barrier)
             float *out = a.states + (int64_t)pair * (kN * kN) + 16 * q + l16;
@@ -170,12 +190,12 @@ __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
 }
 
 hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w, const void *u,
-                          float *states, float *decay, bool reverse, RowCut cut)
+                          float *states, float *decay, bool reverse, RowCut cut, const GivenStates &given)
 {
     StateArgs a = {};
     a.T = (int)L; a.H = (int)H; a.reverse = reverse; a.cut = cut;
     a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
-    a.states = states; a.decay = decay;
+    a.states = states; a.decay = decay; a.given = given;
     const hipError_t e = allow_dynamic_lds<state_kernel>(StateLds::kBytes);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(state_kernel, dim3((unsigned)(rows * H)), dim3(512), StateLds::kBytes, st, a);
