@@ -85,7 +85,7 @@ __device__ __forceinline__ float sum_row8(float x) {
 // State S[m]: rows j = block_row_channel(m, g) + rr, column i.
 // ------------------------------------------------------------------------------------------
 template <typename Ts, bool kSave, bool kFuse, bool kSegments>
-__device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsigned char *smem, int pair0, int q, int lane)
+__device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsigned char *smem, const int *s_wild, int pair0, int q, int lane)
 {
     const int T = a.T, H = a.H;
     const int g = lane >> 4, l16 = lane & 15;
@@ -195,7 +195,9 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
         }
         __builtin_amdgcn_sched_barrier(0);
         if (++c == nchunk) {
-            if (!kSegments && a.sT != nullptr) {   // the pair's final state
+            // the pair's final state (not of a pair that is redone: its initial one, which may lie in the same place, is still needed;
+            // the flag is complete, the pair's last chunk was prepared in front of the visit's barrier)
+            if (!kSegments && a.sT != nullptr && !s_wild[slot]) {
                 Ts *p = reinterpret_cast<Ts *>(a.sT) + ((int64_t)(b0 + slot * a.bstep) * H + h) * (kN * kN) + 16 * q + l16;
 #pragma unroll
                 for (int m = 0; m < 4; ++m)
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
         if (kFuse) { move_rows(a.gate, n); move_rows(a.out, n); move_rows(a.stats, rv.shift * a.H * 2); }
     }
     if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
-    else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse, kSegments>(a, smem, pair0, wave - 4, lane);
+    else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse, kSegments>(a, smem, s_wild, pair0, wave - 4, lane);
     else block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
     // exact second pass for the pairs of which 16 tokens left the range the scaled operands can hold
     __threadfence_block();

@@ -55,3 +55,11 @@ def _compare(oracle, dt, sdt, B, T, H, fused=False, identity=False, strong=False
 def test_time_segments(oracle, B, T, H, strong, sdt, fused, identity):
     # 8, 7, 16, 5 and 4 segments in block form: the last one of a sequence ends while others may still start
     assert _compare(oracle, BF16, sdt, B, T, H, fused, identity, strong, CHUNK) > 0
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("sdt", [F32, BF16])
+@pytest.mark.parametrize("B,T,H", [(5, 64, 32), (9, 150, 32), (70, 70, 4)])
+def test_pairs_redone_per_timestep_in_block_form(oracle, B, T, H, sdt, fused):
+    # one pair to a workgroup, two of them, ragged; every other head holds a decay out of reach
+    _compare(oracle, BF16, sdt, B, T, H, fused, strong=True, algo=CHUNK)
