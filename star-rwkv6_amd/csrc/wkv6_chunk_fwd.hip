@@ -97,7 +97,7 @@ struct FwdArgs {
 // scaling), group 0 produces y for tiles 0 and 2, group 1 for tiles 1 and 3.
 // ------------------------------------------------------------------------------------------
 template <typename Tin, typename Ts, bool kSave, bool kRagged, bool kMulti, bool kFuse, int GRP>
-__device__ __forceinline__ void fwd_consumer(const FwdArgs &a, const unsigned char *smem, int bh0, int q, int lane)
+__device__ __forceinline__ void fwd_consumer(const FwdArgs &a, const unsigned char *smem, const int *s_wild, int bh0, int q, int lane)
 {
     const int T = a.T, H = a.H;
     const int g = lane >> 4, l16 = lane & 15;
@@ -242,7 +242,9 @@ __device__ __forceinline__ void fwd_consumer(const FwdArgs &a, const unsigned ch
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (a.sT != nullptr && GRP == 0) {
+        // (not of a pair that is redone: its initial state, which may lie in the same place, is still needed; the flag is complete, the
+        // pair's last chunk was prepared in front of its barrier)
+        if (a.sT != nullptr && GRP == 0 && !s_wild[n]) {
             Ts *p = reinterpret_cast<Ts *>(a.sT) + (int64_t)bh * kN * kN + 16 * q + l16;
 #pragma unroll
             for (int m = 0; m < 4; ++m)
@@ -538,11 +540,12 @@ __global__ __launch_bounds__(kFwdThreads) void chunk_fwd_kernel(FwdArgs a)
         fwd_producer<Tin, kSave, kRagged, kMulti, kFuse, kNoR>(a, smem, s_wild, bh0, part, wave, lane);
     } else {
         const int cw = wave - 4, grp = cw / nq, q = part * nq + (cw - grp * nq);
-        if (grp == 0) fwd_consumer<Tin, Ts, kSave, kRagged, kMulti, kFuse, 0>(a, smem, bh0, q, lane);
-        else fwd_consumer<Tin, Ts, kSave, kRagged, kMulti, kFuse, 1>(a, smem, bh0, q, lane);
+        if (grp == 0) fwd_consumer<Tin, Ts, kSave, kRagged, kMulti, kFuse, 0>(a, smem, s_wild, bh0, q, lane);
+        else fwd_consumer<Tin, Ts, kSave, kRagged, kMulti, kFuse, 1>(a, smem, s_wild, bh0, q, lane);
     }
     // exact second pass for every pair of this workgroup that had a tile leave the representable range
-    // (workgroups sharing a pair all see the same flags and all redo the whole pair: the same values)
+    // (workgroups sharing a pair all see the same flags; each leaves its own value columns, which do not depend on the others: those
+    // of the initial state may have been overwritten by now)
     __threadfence_block();   // workgroup scope is enough (and a device-scope fence would write back the L2)
     __syncthreads();
     if (!kMulti && !kFuse && a.decay && part == 0 && threadIdx.x < kN) {
@@ -558,7 +561,8 @@ __global__ __launch_bounds__(kFwdThreads) void chunk_fwd_kernel(FwdArgs a)
         typedef typename OutOf<Tin>::type Tout;
         auto in = [](const void *p) { return reinterpret_cast<const Tin *>(p); };
         scan_fwd_body<Tin, Tout, Ts>(*reinterpret_cast<ScanFwdLds *>(smem), bh / a.H, bh % a.H, a.T, a.H, in(a.r), in(a.k), in(a.v_orig), in(a.w), in(a.u),
-                                     reinterpret_cast<const Ts *>(a.s0), a.map, reinterpret_cast<Tout *>(kFuse ? a.out : a.y), reinterpret_cast<Ts *>(a.sT), a.reverse != 0);
+                                     reinterpret_cast<const Ts *>(a.s0), a.map, reinterpret_cast<Tout *>(kFuse ? a.out : a.y), reinterpret_cast<Ts *>(a.sT), a.reverse != 0,
+                                     part * 16 * nq, (part + 1) * 16 * nq);
         if (kFuse) {
             __threadfence_block();
             __syncthreads();

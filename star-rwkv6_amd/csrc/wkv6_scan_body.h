@@ -42,7 +42,8 @@ __device__ __forceinline__ void scan_fwd_body(ScanFwdLdsT<NW> &L, int b, int h, 
         const Tin *__restrict__ r, const Tin *__restrict__ k, const Tin *__restrict__ v,
         const Tin *__restrict__ w, const Tin *__restrict__ u,
         const Ts *__restrict__ s0, const int64_t *__restrict__ map,
-        Tout *__restrict__ y, Ts *__restrict__ sT, bool reverse = false)   // reverse: timestep t reads row T-1-t (no y then)
+        Tout *__restrict__ y, Ts *__restrict__ sT, bool reverse = false,   // reverse: timestep t reads row T-1-t (no y then)
+        int first_col = 0, int end_col = kN)   // the value columns (first_col a multiple of four, as is end_col) that are written
 {
     auto &s_r = L.s_r; auto &s_k = L.s_k; auto &s_d = L.s_d; auto &s_v = L.s_v;
     auto &s_part = L.s_part; auto &s_ruk = L.s_ruk; auto &s_u = L.s_u;
@@ -138,13 +139,13 @@ __device__ __forceinline__ void scan_fwd_body(ScanFwdLdsT<NW> &L, int b, int h, 
                     const float4 c = *reinterpret_cast<const float4 *>(&s_part[qq][t][c4]);
                     a.x += c.x; a.y += c.y; a.z += c.z; a.w += c.w;
                 }
-                if (y) store4(y + base + (int64_t)(t0 + t) * C + c4, a.x, a.y, a.z, a.w);
+                if (y && c4 >= first_col && c4 < end_col) store4(y + base + (int64_t)(t0 + t) * C + c4, a.x, a.y, a.z, a.w);
             }
         }
         // the next tile's LDS writes touch s_r/s_k/s_v/s_d/s_ruk only, all readers of which are
         // past the barrier above; s_part is rewritten only after the barrier that follows them.
     }
-    if (sT != nullptr) {
+    if (sT != nullptr && lane >= first_col && lane < end_col) {
         Ts *p = sT + (((int64_t)b * H + h) * kN + RW * q) * kN + lane;
 #pragma unroll
         for (int jj = 0; jj < RW; ++jj) store1(p + jj * kN, s[jj]);

@@ -63,3 +63,12 @@ def test_time_segments(oracle, B, T, H, strong, sdt, fused, identity):
 def test_pairs_redone_per_timestep_in_block_form(oracle, B, T, H, sdt, fused):
     # one pair to a workgroup, two of them, ragged; every other head holds a decay out of reach
     _compare(oracle, BF16, sdt, B, T, H, fused, strong=True, algo=CHUNK)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("sdt", [F32, BF16])
+@pytest.mark.parametrize("B,T,H", [(4, 150, 32), (3, 100, 32), (2, 320, 5), (1, 50, 2), (3, 64, 100)])
+def test_pairs_redone_per_timestep_in_tile_form(oracle, B, T, H, sdt, fused):
+    # a pair shared by two workgroups, by four (whole chunks, and shorter than one; with the output stage always one), and several pairs to
+    # a workgroup
+    _compare(oracle, BF16, sdt, B, T, H, fused, strong=True, algo=CHUNK)
