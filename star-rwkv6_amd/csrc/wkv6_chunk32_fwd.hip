@@ -78,6 +78,13 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
     const Tin *u = reinterpret_cast<const Tin *>(a.u);
     Tout *y = reinterpret_cast<Tout *>(a.y);
 
+    auto redo = [&]() {   // behind the barrier that follows the last chunk
+        int any = 0;
+#pragma unroll
+        for (int i = 0; i < 4 * kGroups; ++i) any |= L.wild[i];
+        return any != 0;
+    };
+
     if (wave >= 4) {
         // ---------------- loading waves ----------------
         const int grp = (wave - 4) >> 2, p = (wave - 4) & 3, t16 = lane & 15, ch = 16 * p + 4 * (lane >> 4);
@@ -198,6 +205,7 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
         if (lane == 0) L.wild[wave - 4] = any;
         if (!kOut && a.decay && t16 == 0)
             *reinterpret_cast<f32x4 *>(a.decay + ((int64_t)grp * gridDim.x + pair) * kN + ch) = (f32x4){decay[0], decay[1], decay[2], decay[3]};
+        __syncthreads();
     } else {
         // ---------------- computing waves ----------------
         const int q = wave, n = lane & 15, g = lane >> 4;
@@ -296,7 +304,9 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
             __syncthreads();
         }
         if (kOut && y) store_y(nchunk - 1);
-        if (a.sT) {
+        __syncthreads();   // (the loading waves' flags)
+        // the final state (not of a pair that is redone: its initial one, which may lie in the same place, is still needed)
+        if (a.sT && !redo()) {
             StateT *p0 = reinterpret_cast<StateT *>(a.sT) + (int64_t)pair * (kN * kN) + 16 * q + n;
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib)
@@ -304,12 +314,8 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
                 for (int e = 0; e < 4; ++e) store1(p0 + (16 * ib + 4 * g + e) * kN, S[ib][e]);
         }
     }
-    __syncthreads();
     // a pair whose decay left the reach: once more, one timestep at a time
-    int wild_any = 0;
-#pragma unroll
-    for (int i = 0; i < 4 * kGroups; ++i) wild_any |= L.wild[i];
-    if (wild_any && (kOut || a.sT)) {   // (its chunk states are not used: the backward takes the same way out)
+    if ((kOut || a.sT) && redo()) {   // (its chunk states are not used: the backward takes the same way out)
         __syncthreads();
         scan_fwd_body<Tin, Tout, Ts, 8>(reinterpret_cast<C32FwdSmem *>(c32_smem)->scan, b, h, T, H, r, k, v, w, u,
                                         reinterpret_cast<const Ts *>(a.s0), a.map, y, reinterpret_cast<Ts *>(a.sT));

@@ -72,3 +72,16 @@ def test_pairs_redone_per_timestep_in_tile_form(oracle, B, T, H, sdt, fused):
     # a pair shared by two workgroups, by four (whole chunks, and shorter than one; with the output stage always one), and several pairs to
     # a workgroup
     _compare(oracle, BF16, sdt, B, T, H, fused, strong=True, algo=CHUNK)
+
+
+@pytest.mark.parametrize("dt", [F32, F16])
+@pytest.mark.parametrize("B,T,H", [(2, 64, 3), (3, 203, 32), (2, 1100, 4)])
+def test_pairs_redone_per_timestep_in_full_precision(oracle, B, T, H, dt):
+    _compare(oracle, dt, F32, B, T, H, strong=True)
+
+
+@pytest.mark.parametrize("dt,sdt", [(F32, F32), (F16, F32), (BF16, F32), (BF16, BF16)])
+@pytest.mark.parametrize("B,T,H", [(9, 1, 5), (3, 20, 4), (8, 128, 32)])
+def test_calls_in_one_piece(oracle, B, T, H, dt, sdt):
+    # a single timestep, the per-timestep kernels and the chunk forms, no pair redone
+    _compare(oracle, dt, sdt, B, T, H)
