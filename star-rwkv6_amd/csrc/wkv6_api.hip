@@ -658,7 +658,11 @@ int wkv6_backward_with_state(void *stream, int dtype, int algo, int64_t B, int64
     if (!chunk)
         return finish(wkv6::scan_backward_state(st, dtype, B, T, H, r, k, v, w, u, s0, gy, gsT, gr, gk, gv, gw, gu, gs0, workspace));
     const int P = train_segments(dtype, algo, B, T, C, H);
-    if (P > 1) {
+    // Seven launches in segments against two in one piece, and the torch flavour's step through the state spends 160 to 190 us of host
+    // time on the rest: B2 T1000 H24 165 us in one piece / 171 in segments, B1 T1024 H32 187 / 184, two segments B2 T1024 H64 163 / 187,
+    // T2048 229 / 219.  (The plain backward, called directly, gains from 705 tokens on as the pair does: B1 T705 H8 70.6 / 34.0 us,
+    // T1000 H64 95.5 / 54.4, two segments B5 T900 H24 92.0 / 83.4, B2 T1023 H64 98.2 / 85.4.)
+    if (P > 1 && (T >= 2048 || (T >= 1024 && P >= 4))) {
         char *extra = reinterpret_cast<char *>(workspace) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_backward_state_segments(st, B, T, H, r, k, v, w, u, s0, gy, gsT, gr, gk, gv, gw, gu, gs0,
                                                           workspace, extra));

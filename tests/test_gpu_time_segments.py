@@ -1,4 +1,6 @@
 """Time segments of bf16 sequences: what a segment hands to the next one."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -80,3 +82,30 @@ def test_gradient_of_the_state_behind_strong_decays_stays_fp32(op, oracle, B, T,
     want = oracle.backward_state_c(*ref, gy_ref[0], N, s_ref, to_np(gs))[5]
     assert rel_l2(to_np(got), want) <= 2.0 ** -20
     assert np.isfinite(to_np(sT)).all()
+
+
+@pytest.mark.parametrize("B,T,H,launches", [(1, 1023, 8, 2), (2, 1000, 24, 2), (1, 1024, 8, 7), (2, 2047, 64, 2), (2, 2048, 64, 7)])
+def test_backward_through_the_state_in_segments_where_its_launches_pay(oracle, B, T, H, launches):
+    from rwkv_kernel import _native
+
+    lib, C = _native.load(), H * N
+    r, k, v, w, u, gy = (x.bfloat16().cuda().contiguous() for x in oracle.make_inputs(B, T, H, N, 76))
+    s0, gs = (torch.randn(B, H, N, N, device="cuda") for _ in range(2))
+    outs, gu, gs0 = [torch.empty_like(r) for _ in range(4)], torch.empty(B, C, dtype=torch.bfloat16, device="cuda"), torch.empty_like(s0)
+    n = lib.wkv6_backward_with_state_workspace_bytes(_native.BF16, 0, B, T, C, H)
+    ws = torch.empty(int(n), dtype=torch.uint8, device="cuda")
+    P = lambda t: t.data_ptr()
+
+    def call():
+        _native.check(lib.wkv6_backward_with_state(torch.cuda.current_stream().cuda_stream, _native.BF16, 0, B, T, C, H, *map(P, (r, k, v, w, u, s0, gy, gs)),
+                                                   *map(P, outs), P(gu), P(gs0), P(ws), n))
+
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    nodes = ctypes.c_size_t()
+    hip = ctypes.CDLL(next(x.split()[-1] for x in open("/proc/self/maps") if "libamdhip64" in x))   # the one that torch runs on
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert nodes.value == launches
