@@ -440,7 +440,8 @@ int wkv6_forward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64
 static size_t segments_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
     const int P = train_segments(dtype, algo, B, T, C, H);
     if (P <= 1) return 0;
-    return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H) + wkv6::train_segments_layout(B, T, H, nullptr).bytes;
+    const wkv6::TrainSegments seg = wkv6::train_segments_layout(B, T, H, nullptr);
+    return saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, seg.L, C, H) + seg.bytes_unsaved;
 }
 
 // Workspace of a backward in one piece, whatever the sequence's length.

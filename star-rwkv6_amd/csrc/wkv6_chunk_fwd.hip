@@ -940,10 +940,11 @@ TrainSegments train_segments_layout(int64_t B, int64_t T, int64_t H, void *extra
     const size_t pairs = (size_t)(B * s.P * H);
     s.states = reinterpret_cast<float *>(extra);
     s.gstates = s.states + pairs * kN * kN;
-    s.alone = s.gstates + pairs * kN * kN;
-    s.decay = s.alone + pairs * kN * kN;
+    s.decay = s.gstates + pairs * kN * kN;
     s.gu_rows = s.decay + pairs * kN;
-    s.bytes = pairs * (3 * kN * kN + 2 * kN) * sizeof(float);
+    s.alone = s.gu_rows + pairs * kN;
+    s.bytes_unsaved = pairs * (2 * kN * kN + 2 * kN) * sizeof(float);
+    s.bytes = s.bytes_unsaved + pairs * kN * kN * sizeof(float);
     return s;
 }
 

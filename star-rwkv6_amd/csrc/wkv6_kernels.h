@@ -226,8 +226,9 @@ struct TrainSegments {
     float *states;      // [B*P][H][64][64] state entering each segment
     float *decay;       // [B*P][H][64] decay over each segment
     float *gstates;     // [B*P][H][64][64] gradient arriving at the end of each segment
-    float *alone;       // [B*P][H][64][64] (block form) what each segment leaves alone, forward or backward in time
     float *gu_rows;     // [B*P][C] gu of each segment
+    float *alone;       // [B*P][H][64][64] (training pair in block form) what each segment leaves alone, forward or backward in time
+    size_t bytes_unsaved;   // size of the block without `alone` (a backward without saved states)
     size_t bytes;       // size of the block
 };
 int chunk_train_segments(int64_t B, int64_t T, int64_t H);

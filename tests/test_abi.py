@@ -87,6 +87,18 @@ def test_argument_validation_returns_status_codes(native):
     assert lib.wkv6_forward_with_state(None, native.BF16, 2, 16, 128, 2, 1, None, *args[:5], None, fake, fake) == 1
 
 
+def test_backward_in_segments_keeps_two_states_to_a_segment(native):
+    # a backward without saved states has no use for the third one of the training pair, which put lengths that the library's
+    # own array (64 MiB) can hold in segments out of its reach: with 16 segments to B1 H16, 16 x 16 x 16 KiB = 4 MiB of 64.1
+    lib, scratch = native.load(), 64 << 20
+    for T, H in ((12492, 16), (13312, 16), (6656, 32)):
+        assert 0 < lib.wkv6_backward_workspace_bytes(native.BF16, 1, T, H * 64, H) <= scratch
+    seg = lambda B, T, H, P, chunks: P * B * H * (chunks * 64 * 64 + 2 * 64 * 64 + 2 * 64) * 4   # chunk states; states and vectors of a segment
+    for B, T, H, P, chunks in ((1, 4096, 8, 16, 4), (1, 12492, 16, 16, 13), (2, 900, 8, 15, 1)):
+        assert lib.wkv6_backward_workspace_bytes(native.BF16, B, T, H * 64, H) - seg(B, T, H, P, chunks) == 256   # (and the counters of up to 64 heads)
+        assert lib.wkv6_saved_bytes(native.BF16, native.ALGO_AUTO, B, T, H * 64, H) - seg(B, T, H, P, chunks) >= P * B * H * 64 * 64 * 4
+
+
 def test_misaligned_pointers_are_refused_by_the_fused_entry_points(native):
     """The token-shift, low-rank-mixer and group-norm entry points use 16-byte vector accesses on every
     tensor argument: a pointer off a 16-byte boundary is WKV6_ERR_ARG before anything is launched, as in
