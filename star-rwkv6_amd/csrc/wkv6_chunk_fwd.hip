@@ -629,8 +629,9 @@ hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, 
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, bool reverse,
                          bool counters, RowCut cut)
 {
-    if (y != nullptr && decay == nullptr && !reverse && block_forward_applies(B, T, H))
-        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters, cut);
+    // (rows that are segments and find their states here, not in the chain, are fewer than the block form takes: segments_in_block_form)
+    if (y != nullptr && decay == nullptr && !reverse && !cut.segments && block_forward_applies(B, T, H))
+        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters);
     FwdArgs a = {};
     a.decay = decay;
     a.reverse = reverse;
@@ -692,8 +693,8 @@ hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale,
                                const float *gn_offset, float gn_eps, void *out, void *sT, RowCut cut)
 {
-    if (block_forward_applies(B, T, H))
-        return block_forward_fused(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, gate, gn_scale, gn_offset, gn_eps, out, nullptr, nullptr, sT, nullptr, cut);
+    if (!cut.segments && block_forward_applies(B, T, H))
+        return block_forward_fused(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, gate, gn_scale, gn_offset, gn_eps, out, nullptr, nullptr, sT, nullptr);
     FwdArgs a = {};
     a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
@@ -718,8 +719,8 @@ static hipError_t fused_save_from(hipStream_t st, int64_t B, int64_t T, int64_t 
                                   const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
                                   void *out, void *y, float *stats, void *saved_states, RowCut cut = RowCut())
 {
-    if (block_forward_applies(B, T, H))
-        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states, cut);
+    if (!cut.segments && block_forward_applies(B, T, H))
+        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states);
     FwdArgs a = {};
     a.s0 = s0;
     a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
