@@ -136,6 +136,8 @@ def test_state_in_out(op, oracle, dt, T):
 
 def test_state_split_consistency_fp32(op, oracle):
     # op(T1+T2) == op(T1) -> op(T2, init_state): bit-identical in fp32 state
+    # (on the per-timestep kernels: the chunk form's scaling depends on where a chunk starts)
+    op.algo = SCAN
     B, T, H, N = 2, 96, 2, 64
     ins = oracle.make_inputs(B, T, H, N, 22)
     dev, _ = cast_inputs(ins[:5], torch.float32)
