@@ -64,7 +64,7 @@ enum {
                             that much from what wkv6_forward returns for the same inputs.  In
                             either chunk form a (batch, head) pair whose decay goes beyond what the
                             operand scaling can hold is redone with the exact per-timestep code
-                            inside the same launch                                             */
+                            inside the same launch (of a sequence in time segments: the segment)  */
 };
 
 const char *wkv6_status_string(int status);
@@ -91,7 +91,7 @@ int wkv6_forward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64
  * rwkv_kernel/jax_kernel/rwkv_kernels.cu:165-190).  has_init_state==0: s and state_map ignored,
  * zero initial state.  has_init_state!=0: S_0[b] = s[state_map[b]] (state_map NULL = identity);
  * state_map values must lie in [0, rows of s) -- validated by the caller on the host.
- * s and ys are in the output type.  ys may alias s only when state_map is the identity. */
+ * s and ys are in the output type.  ys may alias s (ys = s) only when state_map is the identity. */
 int wkv6_forward_with_state(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
                             int has_init_state, const int64_t *state_map,
                             const void *r, const void *k, const void *v, const void *w, const void *u,
@@ -273,9 +273,12 @@ size_t wkv6_backward_workspace_bytes_ex(int dtype, int algo, int64_t B, int64_t 
  * chunk form: the fp32 state at every 32-token chunk start), and the backward that consumes it and therefore
  * skips its own forward state sweep.  `saved` is caller-owned device memory of wkv6_saved_bytes()
  * bytes (0 = this path saves nothing; pass NULL), must be left untouched between the two calls,
- * and serves the backward as its workspace too.  A sequence (bf16 from T = 705 on, fp32 and fp16 from 320) of so few
- * (batch, head) pairs that they fill at most half of the compute units runs as 2 to 16 time segments side by side in
- * both calls, whatever its length (same results to rounding); wkv6_saved_bytes() includes what that keeps.
+ * and serves the backward as its workspace too.  Sequences of so few (batch, head) pairs that they fill at most half of
+ * the compute units may run as 2 to 16 time segments side by side in both calls, whatever their length (same results to
+ * rounding): with four segments or more bf16 from T = 705 on and fp32 / fp16 from 320, with two or three from 833 and 384,
+ * bf16 whose segments fill less than a quarter of the compute units from 1024 (2048).  wkv6_saved_bytes() includes what that
+ * keeps, three fp32 states to a segment and head besides the chunk states: 8.5 MB at bf16 B1 T1000 H8, where one piece
+ * keeps 2.1.
  * No counterpart in the reference, whose backward
  * recomputes everything from the inputs (rwkv_kernel/torch_rwkv_kernel.py:33 saves only r,k,v,w,u). */
 size_t wkv6_saved_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);

@@ -1,6 +1,6 @@
 // WKV6 forward in block form for gfx950 (bf16 MFMA for the dense products, fp32 state), for bf16
-// tensors and more than half a (batch, head) pair per compute unit (a sequence length that is no
-// multiple of 64 leaves the last chunk with tokens past the end: kRagged).  The tile form in wkv6_chunk_fwd.hip (state advanced every 16 tokens) serves every
+// tensors and more than half a (batch, head) pair per compute unit, or a quarter where the rows are time segments (a sequence
+// length that is no multiple of 64 leaves the last chunk with tokens past the end: kRagged).  The tile form in wkv6_chunk_fwd.hip (state advanced every 16 tokens) serves every
 // other case.  Notation and the operand scaling are in wkv6_block.h.
 //
 // One workgroup per pair; with more pairs than compute units one workgroup per compute unit, which runs

@@ -811,7 +811,7 @@ hipError_t chunk_backward_state_segments(hipStream_t st, int64_t B, int64_t T, i
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     // (what a segment leaves alone: state_kernel, as in the training pair; forward and backward of B1 T8192 H32 through the torch flavour
-    // 226 to 234 us with the tile form's state-only passes, 216 so)
+    // 237 us with the tile form's state-only passes, 225 so)
     const bool block = segments_in_block_form(rows, H);
     hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.states, s.decay, false, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);

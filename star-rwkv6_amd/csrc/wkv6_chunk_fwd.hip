@@ -913,13 +913,15 @@ hipError_t segment_chain_forward(hipStream_t st, int P, int64_t B, int64_t H, co
 
 // ------------------------------------------------------------------------------------------
 // The same for the training pair (saving forward, backward from the saved states): the forward
-// keeps every segment's incoming state and decay exponents for the backward, whose reverse state
+// keeps every segment's incoming state and the decay over it for the backward, whose reverse state
 // is chained the same way (see chunk_backward_saved_segments).
 // ------------------------------------------------------------------------------------------
-// From 705 tokens on: below, the two more launches cost a caller whose host is what takes the time (60 us of autograd and 9
-// for them) what the kernels gain.  Pair of kernels in one piece / in segments: B1 T512 H8 57.9 / 30.7 us, T768 H8 80.7 / 33.1, H40
-// 82.1 / 43.1, T1000 H16 108 / 39, B2 T1000 H12 108 / 47.  Two or three segments from 833 on (B2 H48 T1000 113 / 92, T1900 197 / 145;
-// T768 84.8 / 71.2, but without saved states B5 T768 H24 75.7 / 78.3, T1000 101.8 / 97.8).
+// The pair of kernels gains at every length, in one piece / in segments: B1 T512 H8 57.9 / 30.7 us, T768 H8 80.7 / 33.1, H40 82.1 / 43.1,
+// T1000 H16 108 / 39, B2 T1000 H12 108 / 47; two segments B2 H48 T768 84.8 / 71.2, T1000 113 / 92, T1900 197 / 145.  But a step through
+// the torch flavour takes 75 us of host time with the two more launches and 65 without, so below 705 tokens, where one piece takes less
+// than that, a caller who waits for each step would lose: B1 T705 H8 79.4 / 73.8 us, B2 T740 H12 81.5 / 75.8, B1 T768 H32 77.5 / 78.4, T800 H16
+// 86.8 / 77.3.  Two or three segments from 833 on: the backward without saved states, which takes the same plan, loses with them before
+// (B5 T768 H24 75.7 / 78.3, T1000 101.8 / 97.8).
 static int train_segments_plan(int64_t B, int64_t T, int64_t H, int64_t *L) {
     if (T <= 704) return 1;
     int P = plan_segments(B * H, T, 1, L);
