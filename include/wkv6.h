@@ -106,6 +106,14 @@ int wkv6_forward_with_state_ex(void *stream, int dtype, int state_dtype, int alg
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s, void *y, void *ys,
                                void *workspace, size_t workspace_bytes);
+/* The same call and results, for a caller whose next use of r, k, v and w is the backward: large calls
+ * otherwise read them past the caches.  No counterpart in the reference. */
+int wkv6_forward_with_state_for_backward(void *stream, int dtype, int state_dtype, int algo,
+                                         int64_t B, int64_t T, int64_t C, int64_t H,
+                                         int has_init_state, const int64_t *state_map,
+                                         const void *r, const void *k, const void *v, const void *w, const void *u,
+                                         const void *s, void *y, void *ys,
+                                         void *workspace, size_t workspace_bytes);
 /* Optional workspace of wkv6_forward_ex / wkv6_forward_with_state_ex (0 = none useful).  Where it is
  * non-zero -- a long bf16 sequence with so few (batch, head) pairs that most of the chip would idle --
  * passing that many bytes lets the forward run as time segments side by side (same results to

@@ -318,7 +318,8 @@ at::DimVector state_shape(const Dims &d) {
 // Stateful forward without a gradient (rwkv_kernel/torch_rwkv_kernel.py:76-95 of the reference): y and the final state.
 // An undefined map with an initial state means row b starts from s0[b].
 std::pair<Tensor, Tensor> forward_with_state(int64_t H, const Tensor &map, const Tensor &r, const Tensor &k, const Tensor &v,
-                                             const Tensor &w, const Tensor &u, const Tensor &s0, int64_t algo, ScalarType st) {
+                                             const Tensor &w, const Tensor &u, const Tensor &s0, int64_t algo, ScalarType st,
+                                             bool backward_follows = false) {
   const at::NoGradGuard no_grad;
   const c10::DeviceGuard guard(r.device());
   const Dims d = dims_of(r, H);
@@ -329,9 +330,9 @@ std::pair<Tensor, Tensor> forward_with_state(int64_t H, const Tensor &map, const
   // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
   const size_t n = wkv6_forward_workspace_bytes(code, algo, B, T, C, H);
   const Tensor ws = bytes(r, n);
-  check(wkv6_forward_with_state_ex(stream_of(r), code, code_of(st), algo, B, T, C, H, s0.defined(),
-                                   static_cast<const int64_t *>(in(map)), in(r), in(k), in(v), in(w), in(u), in(s0), out(y), out(ys),
-                                   out(ws), n));
+  const auto forward = backward_follows ? wkv6_forward_with_state_for_backward : wkv6_forward_with_state_ex;
+  check(forward(stream_of(r), code, code_of(st), algo, B, T, C, H, s0.defined(), static_cast<const int64_t *>(in(map)), in(r), in(k),
+                in(v), in(w), in(u), in(s0), out(y), out(ys), out(ws), n));
   return {y, ys};
 }
 
@@ -459,10 +460,11 @@ PYBIND11_MODULE(_wkv6_torch, m) {
     return py::make_tuple(wrap(o[0]), wrap(o[1]), wrap(o[2]), wrap(o[3]), wrap(o[4]));
   });
   m.def("forward_with_state", [](int64_t H, const std::optional<Tensor> &map, const Tensor &r, const Tensor &k, const Tensor &v,
-                                 const Tensor &w, const Tensor &u, const std::optional<Tensor> &s0, int64_t algo, int state_code) {
+                                 const Tensor &w, const Tensor &u, const std::optional<Tensor> &s0, int64_t algo, int state_code,
+                                 bool backward_follows) {
     const ScalarType st = state_code == WKV6_F32 ? at::kFloat : state_code == WKV6_F16 ? at::kHalf : at::kBFloat16;
-    return wrap(unlocked([&] { return forward_with_state(H, given(map), r, k, v, w, u, given(s0), algo, st); }));
-  });
+    return wrap(unlocked([&] { return forward_with_state(H, given(map), r, k, v, w, u, given(s0), algo, st, backward_follows); }));
+  }, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg("backward_follows") = false);
   m.def("forward_gn_gate", [](int64_t H, const std::optional<Tensor> &map, const Tensor &r, const Tensor &k, const Tensor &v, const Tensor &w,
                               const Tensor &u, const std::optional<Tensor> &s0, const Tensor &gate, const Tensor &scale,
                               const Tensor &offset, double eps, bool want_state) {

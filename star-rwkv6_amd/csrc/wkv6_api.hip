@@ -118,7 +118,7 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
                         int has_init_state, const int64_t *state_map,
                         const void *r, const void *k, const void *v, const void *w, const void *u,
                         const void *s, void *y, void *ys, void *saved,
-                        void *workspace = nullptr, size_t workspace_bytes = 0) {
+                        void *workspace = nullptr, size_t workspace_bytes = 0, bool keep_inputs = false) {
     int rc = check_shape_any(dtype, B, T, C, H);
     if (rc != WKV6_OK && rc != kSmallHead) return rc;
     if (!r || !k || !v || !w || !u || !y) return WKV6_ERR_ARG;
@@ -146,7 +146,7 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
         if (need > 0 && workspace_bytes >= need)
             return finish(wkv6::chunk_forward_segments_run(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, workspace));
     }
-    return finish(wkv6::chunk_forward(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, saved));
+    return finish(wkv6::chunk_forward(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, saved, nullptr, false, true, wkv6::RowCut(), keep_inputs));
 }
 
 int wkv6_forward_with_state_ex(void *stream, int dtype, int state_dtype, int algo,
@@ -156,6 +156,15 @@ int wkv6_forward_with_state_ex(void *stream, int dtype, int state_dtype, int alg
                                const void *s, void *y, void *ys, void *workspace, size_t workspace_bytes) {
     return forward_impl(stream, dtype, state_dtype, algo, B, T, C, H, has_init_state, state_map, r, k, v, w, u, s, y, ys,
                         nullptr, workspace, workspace_bytes);
+}
+
+int wkv6_forward_with_state_for_backward(void *stream, int dtype, int state_dtype, int algo,
+                                         int64_t B, int64_t T, int64_t C, int64_t H,
+                                         int has_init_state, const int64_t *state_map,
+                                         const void *r, const void *k, const void *v, const void *w, const void *u,
+                                         const void *s, void *y, void *ys, void *workspace, size_t workspace_bytes) {
+    return forward_impl(stream, dtype, state_dtype, algo, B, T, C, H, has_init_state, state_map, r, k, v, w, u, s, y, ys,
+                        nullptr, workspace, workspace_bytes, true);
 }
 
 int wkv6_forward_gn_gate(void *stream, int dtype, int state_dtype,

@@ -217,7 +217,7 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
 // One function: both walk the same visits with the same cursors and lane mapping.
 // ------------------------------------------------------------------------------------------
 constexpr int kBlockFwdLoads = 1, kBlockFwdStores = 2;
-template <bool kSave, bool kRagged, bool kFuse, bool kSegments, int kRole>
+template <bool kSave, bool kRagged, bool kFuse, bool kSegments, int kStream, int kRole>
 __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsigned char *smem, int *s_wild, int pair0, int p, int lane)
 {
     const int T = a.T, H = a.H;
@@ -264,7 +264,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
         const uint32_t vv = lds0 + BlockFwdLds::kRawV + (cv.it % (BlockFwdLds::kVAhead + 1)) * kTileBytes + 16 * p * kTileRow;
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk)
-            load_rows8_to_lds(vb, row_offset(cv.c * kBlockTokens + 16 * p + 8 * blk + lrow), vv + 8 * blk * kTileRow);
+            load_rows8_to_lds<kStream != 0>(vb, row_offset(cv.c * kBlockTokens + 16 * p + 8 * blk + lrow), vv + 8 * blk * kTileRow);
         issued += 2;
         ++cv.it;
         if (++cv.c == nchunk) { cv.c = 0; ++cv.slot; vb = a.v + pair_base(cv.slot); }
@@ -274,9 +274,9 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk) {
             const uint32_t o = row_offset(cr.c * kBlockTokens + 16 * p + 8 * blk + lrow);
-            load_rows8_to_lds(wb, o, raw + 2 * kTileBytes + 8 * blk * kTileRow);
-            load_rows8_to_lds(rb, o, raw + 8 * blk * kTileRow);
-            load_rows8_to_lds(kb_, o, raw + kTileBytes + 8 * blk * kTileRow);
+            load_rows8_to_lds<kStream != 0>(wb, o, raw + 2 * kTileBytes + 8 * blk * kTileRow);
+            load_rows8_to_lds<kStream != 0>(rb, o, raw + 8 * blk * kTileRow);
+            load_rows8_to_lds<kStream != 0>(kb_, o, raw + kTileBytes + 8 * blk * kTileRow);
         }
         issued += 6;
         if (cr.it & 1) mark_odd = issued; else mark_even = issued;
@@ -294,7 +294,7 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
         const uint32_t gg = lds0 + BlockFwdLds::kGate + (cg.it & 1) * kTileBytes + 16 * p * kTileRow;
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk)
-            load_rows8_to_lds(gtb, row_offset(cg.c * kBlockTokens + 16 * p + 8 * blk + lrow), gg + 8 * blk * kTileRow);
+            load_rows8_to_lds<kStream != 0>(gtb, row_offset(cg.c * kBlockTokens + 16 * p + 8 * blk + lrow), gg + 8 * blk * kTileRow);
         issued += 2;
         if (cg.it & 1) mark_gate_odd = issued; else mark_gate_even = issued;
         ++cg.it;
@@ -329,7 +329,12 @@ __device__ __forceinline__ void block_fwd_producer(const BlockFwdArgs &a, unsign
                 if (a.stats && (lane & 7) == 0 && (!kRagged || tok < T))
                     *reinterpret_cast<float2 *>(a.stats + (((int64_t)(b0 + co.slot * a.bstep) * T + tok) * H + h) * 2) = make_float2(mean, rstd);
             }
-            if (!kRagged || tok < T) *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(yb) + o) = x;
+            if (!kRagged || tok < T) {
+                u32x4 *to = reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(yb) + o);
+                const u32x4 row16 = {x.x, x.y, x.z, x.w};
+                if (kStream == 2) __builtin_nontemporal_store(row16, to);
+                else *to = row16;
+            }
             if (kSave) {
                 const uint4 s = *reinterpret_cast<const uint4 *>(ss + row * kTileRow + (lane & 7) * 16);
                 *reinterpret_cast<uint4 *>(ckb + ((uint32_t)co.c * (uint32_t)(kN * kN * 2) + (uint32_t)(row * kTileRow) + lpiece)) = s;
@@ -423,9 +428,12 @@ __device__ __forceinline__ void block_output_stage_in_place(const BlockFwdArgs &
     }
 }
 
+// kStream: a call without a backward and with large tensors (past_caches): 1: r, k, v, w and the gate are read without keeping
+// their lines.  What such a call reads it reads once, and lines that stay behind only push out others.  2: y (or out) is written so, too.
+// (Two kernels: asked at run time, the two kinds of store became one.)
 // kSegments: rows that are time segments.  Built apart: asked at run time, the other ragged launches, whose
 // pointers then depend on it, took 2 % longer (prompts of B8 T999 H40: 63.1 us, so 61.7).
-template <typename Ts, bool kSave, bool kRagged, bool kFuse, bool kSegments>
+template <typename Ts, bool kSave, bool kRagged, bool kFuse, bool kSegments, int kStream>
 __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -444,9 +452,9 @@ __global__ __launch_bounds__(kBlockFwdThreads) void block_fwd_kernel(BlockFwdArg
         move_rows(a.r, n); move_rows(a.k, n); move_rows(a.v, n); move_rows(a.w, n); move_rows(a.y, n);
         if (kFuse) { move_rows(a.gate, n); move_rows(a.out, n); move_rows(a.stats, rv.shift * a.H * 2); }
     }
-    if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
+    if (wave < 4) block_fwd_producer<kSave, kRagged, kFuse, kSegments, kStream, kBlockFwdLoads>(a, smem, s_wild, pair0, wave, lane);
     else if (wave < 8) block_fwd_consumer<Ts, kSave, kFuse, kSegments>(a, smem, s_wild, pair0, wave - 4, lane);
-    else block_fwd_producer<kSave, kRagged, kFuse, kSegments, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
+    else block_fwd_producer<kSave, kRagged, kFuse, kSegments, kStream, kBlockFwdStores>(a, smem, s_wild, pair0, wave - 8, lane);
     // exact second pass for the pairs of which 16 tokens left the range the scaled operands can hold
     __threadfence_block();
     __syncthreads();
@@ -484,12 +492,23 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H) {
     return 2 * pairs > cus && block_grid(B, H) > 0 && T * H * kN < (1LL << 31);
 }
 
+// kStream of a call that no backward follows: from 28 MiB a tensor 1, from 64 MiB 2.  Prompts, kept / 1 / 2, us: B64 T512 H32 with the output
+// stage 186.4 / 179.1 / 152.3 (5.7 TB/s), without 151.8 / 146.6 / 132.3; B16 T1024 (64 MiB) 83.9 / 71.8 / 70.8; B8 T1024 (32 MiB) 43.3 / 38.1,
+// with the output stage 51.3 / 45.8; B8 T900 (28.1 MiB) 40.0 / 37.8.  Below, inputs that other work left in the last-level cache are lost by 1: 23 MiB a
+// tensor (B5 T1184) 38.2 / 38.4, 8 MiB (B6 T350) 16.8 / 17.8; and so is an output by 2: call and a product that reads its y together, B8 T1024
+// 64.1 / 60.4 / 62.2; B16 T1024 109.0 / 99.2 / 101.2 and B64 T512 195.0 / 171.6 / 175.4, where the call by itself gains more.  With a
+// backward that reads the inputs again (keep_inputs) they stay: B8 T1024 through the state 167.3 / 169.1, the training pair 124.5 / 126.9.
+static int past_caches(int64_t B, int64_t T, int64_t H) {
+    const int64_t bytes = B * T * H * kN * 2;
+    return bytes >= (64LL << 20) ? 2 : bytes >= (28LL << 20) ? 1 : 0;
+}
+
 // gate != null: the fused output stage (out = (group norm of y) * gate; y and stats only where given)
 static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                        const void *r, const void *k, const void *v, const void *w, const void *u,
                                        const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
                                        const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats, RowCut cut,
-                                       const SegmentChain &chain)
+                                       const SegmentChain &chain, bool keep_inputs = false)
 {
     BlockFwdArgs a = {};
     a.cut = cut; a.chain = chain;
@@ -502,13 +521,21 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     a.gate = (const bf16_t *)gate; a.gn_scale = gn_scale; a.gn_offset = gn_offset; a.gn_eps = gn_eps; a.out = (bf16_t *)out; a.stats = stats;
-    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag) -> hipError_t {
+    auto launch_as = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag, auto stream_tag) -> hipError_t {
         constexpr bool kFuse = decltype(fuse_tag)::value;
-        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(segments_tag)::value>;
+        constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(segments_tag)::value, decltype(stream_tag)::value>;
         hipError_t e = allow_dynamic_lds<kern>(BlockFwdLdsT<kFuse>::kBytes);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlockFwdThreads), BlockFwdLdsT<kFuse>::kBytes, st, a);
         return hipGetLastError();
+    };
+    auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag) -> hipError_t {
+        if constexpr (!decltype(save_tag)::value && !decltype(segments_tag)::value)
+            switch (keep_inputs ? 0 : past_caches(B, T, H)) {
+            case 1: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 1>{});
+            case 2: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 2>{});
+            }
+        return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 0>{});
     };
     auto launch_ts = [&](auto ts_tag, auto save_tag, auto fuse_tag) -> hipError_t {
         const std::true_type yes;
@@ -531,10 +558,11 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
 
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
-                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut, SegmentChain chain)
+                         const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters, RowCut cut, SegmentChain chain,
+                         bool keep_inputs)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters,
-                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, cut, chain);
+                                nullptr, nullptr, nullptr, 0.f, nullptr, nullptr, cut, chain, keep_inputs);
 }
 
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,

@@ -627,11 +627,11 @@ static unsigned forward_grid(int64_t pairs, bool *multi, int *split) {
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, float *decay, bool reverse,
-                         bool counters, RowCut cut)
+                         bool counters, RowCut cut, bool keep_inputs)
 {
     // (rows that are segments and find their states here, not in the chain, are fewer than the block form takes: segments_in_block_form)
     if (y != nullptr && decay == nullptr && !reverse && !cut.segments && block_forward_applies(B, T, H))
-        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters);
+        return block_forward(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, counters, RowCut(), SegmentChain(), keep_inputs);
     FwdArgs a = {};
     a.decay = decay;
     a.reverse = reverse;

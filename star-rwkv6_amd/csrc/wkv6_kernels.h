@@ -121,7 +121,7 @@ hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, 
                          float *decay = nullptr,   // see FwdArgs
                          bool reverse = false,     // the time axis read back to front (no y)
                          bool counters = true,     // saved_states ends with the per-head counters of the fused gu sum (zeroed here)
-                         RowCut cut = RowCut());
+                         RowCut cut = RowCut(), bool keep_inputs = false);   // keep_inputs: a backward will read them again
 
 // --- block form (wkv6_block_fwd.hip, wkv6_block_bwd.hip): a 64-token chunk as one block of the
 // recurrence; bf16 tensors, T a multiple of 64, between half a pair and one pair per compute unit.
@@ -132,7 +132,8 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H);
 hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                          const void *r, const void *k, const void *v, const void *w, const void *u,
                          const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
-                         RowCut cut = RowCut(), SegmentChain chain = SegmentChain());   // (rows that are segments: cut and chain, s0 = map = sT = null)
+                         RowCut cut = RowCut(), SegmentChain chain = SegmentChain(),   // (rows that are segments: cut and chain, s0 = map = sT = null)
+                         bool keep_inputs = false);   // a backward will read them again
 
 // the block-form forward with the layer's output stage fused in (see chunk_forward_fused / chunk_forward_fused_save):
 // y and stats may be null (inference), saved_states null without a backward to follow

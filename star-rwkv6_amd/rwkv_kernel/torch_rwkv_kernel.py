@@ -94,13 +94,13 @@ class _ShiftMixX(torch.autograd.Function):
             return gx, gmx.to(ctx.mix_dtype)
 
 
-def _forward_with_state(B, T, C, H, state_map, r, k, v, w, u, init_state, algo=_native.ALGO_AUTO, state_dtype=None):
+def _forward_with_state(B, T, C, H, state_map, r, k, v, w, u, init_state, algo=_native.ALGO_AUTO, state_dtype=None, backward_follows=False):
     """Stateful forward, no gradient (rwkv_kernel/torch_rwkv_kernel.py:76-95)."""
     # state_map None with an init_state means the identity map (row b starts from init_state[b])
     assert init_state is not None or state_map is None, "state_map needs init_state"
     assert state_map is None or state_map.dtype == torch.int64
     sdt = init_state.dtype if init_state is not None else (state_dtype or _out_dtype(r.dtype))
-    return _native.load_torch().forward_with_state(H, state_map, r, k, v, w, u, init_state, algo, _DTYPE_CODE[sdt])
+    return _native.load_torch().forward_with_state(H, state_map, r, k, v, w, u, init_state, algo, _DTYPE_CODE[sdt], backward_follows)
 
 
 class _WKV6State(torch.autograd.Function):
@@ -115,7 +115,7 @@ class _WKV6State(torch.autograd.Function):
         ctx.algo = algo
         ctx.has_s0 = s0 is not None
         ctx.set_materialize_grads(False)   # an unused output arrives as None, not as a tensor of zeros
-        y, sT = _forward_with_state(B, T, C, H, None, r, k, v, w, u, s0, algo, state_dtype=torch.float32)
+        y, sT = _forward_with_state(B, T, C, H, None, r, k, v, w, u, s0, algo, state_dtype=torch.float32, backward_follows=True)
         ctx.save_for_backward(r, k, v, w, u, *((s0,) if s0 is not None else ()))
         return y, sT
 

@@ -1,0 +1,51 @@
+"""Large calls without a backward read their inputs and write their output past the caches: the same bits as smaller calls."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+N = 64
+MIB = 2 ** 20
+
+
+@pytest.fixture(scope="module")
+def op():
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    import rwkv_kernel
+
+    return rwkv_kernel.RWKVKernelOperator(N, 16384)
+
+
+# A pair's result does not depend on the pairs around it, so the first `few` rows by themselves, a call that stays below the limits
+# (28 MiB a tensor for what is read, 64 MiB for what is written), have to be what they are among all rows.
+@pytest.mark.parametrize("B,few,T,H,sdt", [(9, 8, 800, 32, torch.float32),      # read past the caches, 28.1 MiB; several pairs to a workgroup
+                                           (8, 7, 897, 32, torch.bfloat16),     # one pair to a workgroup and a chunk of one token, 28.0 MiB
+                                           (20, 8, 820, 32, torch.float32),     # written past them, too: 64.1 MiB, a ragged end
+                                           (65, 16, 320, 24, torch.float32),    # 60.9 MiB: read only; heads that do not divide the chip
+                                           (37, 8, 448, 32, None)])             # 64.75 MiB, without a state
+@pytest.mark.parametrize("fused", [False, True])
+def test_large_calls_give_the_bits_of_small_ones(op, B, few, T, H, sdt, fused):
+    assert few * T * H * N * 2 < 28 * MIB <= B * T * H * N * 2
+    g = torch.Generator(device="cuda").manual_seed(B)
+
+    def normal(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=g, device="cuda").to(dtype)
+
+    C = H * N
+    r, k, v = (normal(B, T, C) for _ in range(3))
+    w = (torch.rand(B, T, C, generator=g, device="cuda") * 7 - 6).bfloat16()
+    w[2, T // 2:, :N] = 6.0    # a pair that is redone one timestep at a time
+    u = normal(H, N)
+    s0 = None if sdt is None else normal(B, H, N, N, dtype=sdt)
+    gate, scale, offset = normal(B, T, C), normal(H, N, dtype=torch.float32), normal(H, N, dtype=torch.float32)
+
+    def call(n):
+        ins = [x[:n].contiguous() for x in (r, k, v, w)]
+        state = None if s0 is None else s0[:n].contiguous()
+        if fused:
+            return op.forward_gn_gate(*ins, u, gate[:n].contiguous(), scale, offset, return_state=True, init_state=state)
+        return op(*ins, u, return_state=True, init_state=state)
+
+    y, s = call(B)
+    y_few, s_few = call(few)
+    assert torch.equal(y[:few], y_few) and torch.equal(s[:few], s_few)
