@@ -120,6 +120,9 @@ int wkv6_forward_with_state_for_backward(void *stream, int dtype, int state_dtyp
  * rounding); without it the call works as always.  Batches need T to divide into equal segments
  * of whole 64-token chunks; a single sequence (B = 1) may have any length. */
 size_t wkv6_forward_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);
+/* The same for batches of any length: a call that is given this many bytes (>= those above) runs as time segments, the last
+ * of every sequence shorter, also where no equal ones divide T. */
+size_t wkv6_forward_workspace_bytes_any_length(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H);
 
 /* Forward (inference) with the layer's output stage fused in; y itself is not written:
  *     out[b,t,h,:] = (layer_norm(y[b,t,h,:], gn_eps) * gn_scale[h,:] + gn_offset[h,:]) * gate[b,t,h,:]

@@ -184,7 +184,7 @@ struct Wkv6 : torch::autograd::Function<Wkv6> {
     } else {
       y = carve(r, {yp})[0];
       // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
-      const size_t n = wkv6_forward_workspace_bytes(code, algo, B, T, C, H);
+      const size_t n = wkv6_forward_workspace_bytes_any_length(code, algo, B, T, C, H);
       const Tensor ws = bytes(r, n);
       check(wkv6_forward_ex(stream_of(r), code, algo, B, T, C, H, in(r), in(k), in(v), in(w), in(u), out(y), out(ws), n));
     }
@@ -328,7 +328,7 @@ std::pair<Tensor, Tensor> forward_with_state(int64_t H, const Tensor &map, const
   const Tensor y = carve(r, {{{B, T, C}, out_type(r.scalar_type()), 5}})[0];
   const Tensor ys = at::empty(state_shape(d), r.options().dtype(st));
   // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
-  const size_t n = wkv6_forward_workspace_bytes(code, algo, B, T, C, H);
+  const size_t n = wkv6_forward_workspace_bytes_any_length(code, algo, B, T, C, H);
   const Tensor ws = bytes(r, n);
   const auto forward = backward_follows ? wkv6_forward_with_state_for_backward : wkv6_forward_with_state_ex;
   check(forward(stream_of(r), code, code_of(st), algo, B, T, C, H, s0.defined(), static_cast<const int64_t *>(in(map)), in(r), in(k),
@@ -349,7 +349,7 @@ std::pair<Tensor, Tensor> forward_gn_gate(int64_t H, const Tensor &map, const Te
   const ScalarType st = s0.defined() ? s0.scalar_type() : at::kFloat;
   const Tensor res = carve(r, {{{B, T, C}, r.scalar_type(), 5}})[0];
   const Tensor ys = want_state ? at::empty(state_shape(d), r.options().dtype(st)) : Tensor();
-  const size_t n = wkv6_forward_workspace_bytes(code, kChunk, B, T, C, H);
+  const size_t n = wkv6_forward_workspace_bytes_any_length(code, kChunk, B, T, C, H);
   const Tensor ws = bytes(r, n);
   check(wkv6_forward_gn_gate_ex(stream_of(r), code, code_of(st), B, T, C, H, s0.defined(), static_cast<const int64_t *>(in(map)), in(r),
                                 in(k), in(v), in(w), in(u), in(s0), in(gate), in_f(sc), in_f(of), static_cast<float>(eps), out(res),

@@ -103,14 +103,31 @@ int wkv6_supports_head_size(int64_t N) { return N == 64 || wkv6::generic_head_si
 int wkv6_last_status(void) { return g_last_status; }
 int wkv6_last_hip_error(void) { return g_last_hip_error; }
 
-size_t wkv6_forward_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
+static size_t forward_workspace(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H, bool any_length) {
     if (check_shape(dtype, B, T, C, H) != WKV6_OK) return 0;
     const bool chunk = (algo == WKV6_ALGO_CHUNK && chunk_possible(dtype, T, C)) ||
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     // optional: with it, a long sequence of few (batch, head) pairs runs as time segments side by side
     if (!chunk) return 0;
-    const size_t plain = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, false), fused = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, true);
+    const size_t plain = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, false, any_length);
+    const size_t fused = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, true, any_length);
     return plain > fused ? plain : fused;
+}
+size_t wkv6_forward_workspace_bytes(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
+    return forward_workspace(dtype, algo, B, T, C, H, false);
+}
+size_t wkv6_forward_workspace_bytes_any_length(int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H) {
+    return forward_workspace(dtype, algo, B, T, C, H, true);
+}
+
+// What a workspace is enough for: 0 one piece, 1 the segments of wkv6_forward_workspace_bytes, 2 those of any length.
+static int segments_that_fit(const void *workspace, size_t bytes, int64_t B, int64_t T, int64_t H, bool fused) {
+    if (!workspace || !aligned16(workspace)) return 0;
+    for (int which = 2; which >= 1; --which) {
+        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, fused, which == 2);
+        if (need > 0 && bytes >= need) return which;
+    }
+    return 0;
 }
 
 static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
@@ -141,11 +158,8 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
                        (algo == WKV6_ALGO_AUTO && chunk_eligible(dtype, T, C));
     if (!chunk)
         return finish(wkv6::scan_forward(st, dtype, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys));
-    if (!saved && workspace && aligned16(workspace)) {
-        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, false);
-        if (need > 0 && workspace_bytes >= need)
-            return finish(wkv6::chunk_forward_segments_run(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, workspace));
-    }
+    if (const int segments = saved ? 0 : segments_that_fit(workspace, workspace_bytes, B, T, H, false))
+        return finish(wkv6::chunk_forward_segments_run(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, workspace, segments == 2));
     return finish(wkv6::chunk_forward(st, state_dtype, B, T, H, r, k, v, w, u, s_in, map_in, y, ys, saved, nullptr, false, true, wkv6::RowCut(), keep_inputs));
 }
 
@@ -195,13 +209,11 @@ int wkv6_forward_gn_gate_ex(void *stream, int dtype, int state_dtype,
         return finish(wkv6::step_forward_fused((hipStream_t)stream, state_dtype, B, H, r, k, v, w, u,
                                                has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
                                                gate, gn_scale, gn_offset, gn_eps, out, ys));
-    if (workspace && aligned16(workspace)) {   // optional: few pairs, long sequence -> time segments side by side
-        const size_t need = wkv6::chunk_forward_segments_workspace_bytes(B, T, H, true);
-        if (need > 0 && workspace_bytes >= need)
-            return finish(wkv6::chunk_forward_segments_run((hipStream_t)stream, state_dtype, B, T, H, r, k, v, w, u,
-                                                           has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
-                                                           out, ys, workspace, gate, gn_scale, gn_offset, gn_eps));
-    }
+    // optional: few pairs, long sequence -> time segments side by side
+    if (const int segments = segments_that_fit(workspace, workspace_bytes, B, T, H, true))
+        return finish(wkv6::chunk_forward_segments_run((hipStream_t)stream, state_dtype, B, T, H, r, k, v, w, u,
+                                                       has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
+                                                       out, ys, workspace, segments == 2, gate, gn_scale, gn_offset, gn_eps));
     return finish(wkv6::chunk_forward_fused((hipStream_t)stream, state_dtype, B, T, H, r, k, v, w, u,
                                             has_init_state ? s : nullptr, has_init_state ? state_map : nullptr,
                                             gate, gn_scale, gn_offset, gn_eps, out, ys));

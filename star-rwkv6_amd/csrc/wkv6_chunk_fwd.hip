@@ -839,21 +839,24 @@ RowCut cut_of(int P, int64_t L, int64_t T) {
 // for the chain's rounding, that of a call in one piece.
 bool segments_in_block_form(int64_t rows, int64_t H) { return 4 * rows * H >= compute_units(); }
 
-// Prompts, in one piece / in segments: B1 T256 H16 17.7 / 17.5 us, T384 H8 17.7 / 16.6, H64 21.2 / 18.8, T512 H32 22.4 / 17.4, T1000
-// H16 36.5 / 20.1, H64 38.1 / 27.8; three segments H72 T384 19.5 / 19.5, T512 23.4 / 22.6; two H128 T1024 38.0 / 39.9, T2048
-// 65.0 / 61.4.  With the output stage, whose first pass leaves it out, three H72 T384 23.2 / 20.3; two H128 T384 25.1 / 24.8 (B8 H8
-// 23.2 / 24.4), T512 30.1 / 28.3, T2048 90.2 / 66.1.
+// Prompts, in one piece / in segments, us.  Four segments and more pay from the first length that has them: B1 H32 T200 11.2 / 10.6, T300
+// 13.0 / 10.9, B2 H16 T330 14.7 / 11.2, T520 19.8 / 13.3, B2 T1000 H8 30.8 / 13.1, B3 T4097 H12 114 / 41.  Three: B3 H28 T330 15.4 / 16.3, T450 18.8 /
+// 19.0, T530 20.5 / 19.4, T700 24.0 / 21.4.  Two: B2 H64 T800 28.7 / 30.8, T1100 37.4 / 37.3, B4 H32 T1500 49.2 / 47.6, T2200 68.8 / 66.0.
+// With the output stage, which the first pass leaves out: four B1 H32 T200 14.6 / 11.7, B2 T2052 H16 102 / 25; three B3 H28 T200 15.3 / 16.0,
+// T260 18.3 / 16.8; two B2 H64 T330 22.5 / 19.3, T500 28.9 / 23.0.
 static bool prompt_takes(int P, int64_t T, bool fused) {
-    return P >= 4 ? T >= 384 : P == 3 ? T >= (fused ? 384 : 512) : P == 2 && T >= (fused ? 512 : 2048);
+    return P >= 4 || (P == 3 ? T >= (fused ? 256 : 512) : P == 2 && T >= (fused ? 320 : 1280));
 }
-static int forward_segments_plan(int64_t B, int64_t T, int64_t H, bool fused, int64_t *L) {
-    if (B == 1) {
-        int P = plan_segments(H, T, 1, L);
-        if (segments_in_block_form(P, H)) return prompt_takes(P, T, fused) ? P : 1;
-        P = T >= 1024 ? plan_segments(H, T, 3, L) : 1;
+// any_length: a batch's length need not divide into the segments, either.  Without it (wkv6_forward_workspace_bytes, which promises
+// no workspace then) a batch of prompts ran as segments only where 16, 8, 4 or 2 equal ones of whole chunks make its length,
+// and otherwise on one or two workgroups a pair.
+static int forward_segments_plan(int64_t B, int64_t T, int64_t H, bool fused, bool any_length, int64_t *L) {
+    if (B == 1 || any_length) {
+        int P = plan_segments(B * H, T, 1, L);
+        if (P > 1 && segments_in_block_form(B * P, H)) return prompt_takes(P, T, fused) ? P : 1;
+        P = T >= 1024 ? plan_segments(B * H, T, 3, L) : 1;
         return P >= 4 ? P : 1;
     }
-    // (the interface promises segments to batches whose length divides evenly, and no workspace to others)
     for (int P = kMostSegments; P >= 2; P >>= 1)
         if (B * H * P <= compute_units() && T % (P * CL) == 0 &&
             (segments_in_block_form(B * P, H) ? prompt_takes(P, T, fused) : T >= 1024 && P >= 4 && T / P >= 4 * CL)) {
@@ -862,9 +865,9 @@ static int forward_segments_plan(int64_t B, int64_t T, int64_t H, bool fused, in
         }
     return 1;
 }
-size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused) {
+size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused, bool any_length) {
     int64_t L;
-    const int P = forward_segments_plan(B, T, H, fused, &L);
+    const int P = forward_segments_plan(B, T, H, fused, any_length, &L);
     // per segment and pair two states (what it leaves alone, what it starts from) and the decay
     return P <= 1 ? 0 : (size_t)(B * P * H) * (2 * kN * kN + kN) * sizeof(float);
 }
@@ -872,11 +875,11 @@ size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, b
 // With `gate` the second pass runs the fused output stage (y = out then).
 hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                       const void *r, const void *k, const void *v, const void *w, const void *u,
-                                      const void *s0, const int64_t *map, void *y, void *sT, void *workspace,
+                                      const void *s0, const int64_t *map, void *y, void *sT, void *workspace, bool any_length,
                                       const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps)
 {
     int64_t L = 0;
-    const int P = forward_segments_plan(B, T, H, gate != nullptr, &L);
+    const int P = forward_segments_plan(B, T, H, gate != nullptr, any_length, &L);
     const int64_t rows = B * P;
     const RowCut cut = cut_of(P, L, T);
     float *states = (float *)workspace, *start = states + rows * H * kN * kN, *decay = start + rows * H * kN * kN;

@@ -210,10 +210,11 @@ hipError_t chunk_forward_save_f16(hipStream_t st, int64_t B, int64_t T, int64_t 
 
 // Few pairs, long sequence: the forward as P time segments side by side (two passes joined by the
 // affine map of a segment's state).  The workspace's size is 0 where that does not apply to the shape.
-size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused);   // fused: with the output stage
+// fused: with the output stage; any_length: batches of a length that does not divide evenly, too
+size_t chunk_forward_segments_workspace_bytes(int64_t B, int64_t T, int64_t H, bool fused, bool any_length);
 hipError_t chunk_forward_segments_run(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                       const void *r, const void *k, const void *v, const void *w, const void *u,
-                                      const void *s0, const int64_t *map, void *y, void *sT, void *workspace,
+                                      const void *s0, const int64_t *map, void *y, void *sT, void *workspace, bool any_length,
                                       const void *gate = nullptr, const float *gn_scale = nullptr,
                                       const float *gn_offset = nullptr, float gn_eps = 0.f);
 
