@@ -15,7 +15,7 @@
 // complete, nothing to combine between workgroups), mix_grads_kernel takes 64 channels of many tokens (the weight
 // gradients stay in accumulators, one partial per workgroup).
 // B8 T1024 C2048, forward and backward: 182 us of kernels at R32 (x and the gradients read twice more than once: 501 MB in, 232 MB
-// out), 431 us at R64; R32 as four elementwise kernels around six library products (gcoef written and read twice, x_mix
+// out), 393 us at R64; R32 as four elementwise kernels around six library products (gcoef written and read twice, x_mix
 // written and read) 504 us, of which 235 us the skinny products.
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
@@ -306,15 +306,19 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
 // (The roles read the same x and g: the later reads find the lines in L1 or L2.  One wave doing everything had a SIMD to
 // itself for its 440 registers and every LDS and MFMA latency in the open: 84 us at B8 T1024 C2048 R32 against 75 so.  The
 // traffic alone, 256 MB, would take 50 us; the roles alone take 45, 44 and 32 us: vector instructions and LDS on top.)
-// R = 64: a second launch without gx waves (kGx false) does the other half of the rank's columns: 181 + 63 us, with 39 registers
-// of the first in scratch memory (3 at R = 32).
+// R = 64: the W and A waves hold accumulators for half of the rank's columns, a second launch without gx waves (kGx false) does the
+// other half.  The gx waves need all of them: a step of the first launch has two parts of 160 columns (32 of each mixer) that go
+// through the same two tiles as at R = 32, and gxx and gxm take each part's share (both are linear in it).  B8 T1024 C2048: 143 + 60 us.
+// (Tiles of all 320 columns fit once: filled from memory between two barriers in every step, 181 + 63 us.  Now 15 registers of the first
+// launch are in scratch memory, 3 at R = 32.)
 // ------------------------------------------------------------------------------------------
 constexpr int kGradTok = 32;
 template <int R, bool kGx> struct MixGrads {
     static constexpr int kThreads = kGx ? 768 : 512;
-    static constexpr int kCols = kMix * (kGx ? R : 32);      // columns of h and gpre the launch reads
+    static constexpr int kParts = kGx ? R / 32 : 1;          // parts of a step: 32 columns of each mixer go through the tiles at a time
+    static constexpr int kCols = kMix * 32;
     static constexpr int kPitch = kCols + 8;                 // elements per token row of their tiles: 8 rows on 8 different bank groups
-    static constexpr int kBufs = kCols == 160 ? 2 : 1;       // (two of 320 columns do not fit: filled between two barriers instead)
+    static constexpr int kBufs = 2;
     static constexpr int kStagePitch = 40;
     static constexpr bool kLdsA = R == 32;                   // A's fragments in LDS, too (R = 64: from L2)
     static constexpr int kTile = kGradTok * kPitch * 2;      // bytes of one range's rows
@@ -414,32 +418,26 @@ __device__ __forceinline__ void store8(float *p, const float (&v)[8]) {
     *reinterpret_cast<f32x4 *>(p + 4) = (f32x4){v[4], v[5], v[6], v[7]};
 }
 
-// Rows of h or gpre for a range's tile: 128 threads, four per token, 32 columns at a time
+// Rows of h or gpre for a range's tile: 128 threads, four per token, 32 columns (of one mixer) at a time.  `r0`: the first of them
 template <int R, bool kGx> struct MixTile {
-    static constexpr int kPieces = MixGrads<R, kGx>::kCols / 32;
-    u32x4 v[kPieces];
-    __device__ __forceinline__ void fetch(const MixGradArgs &p, const bf16_t *src, int64_t first_tok, int step, int tid) {
+    u32x4 v[kMix];
+    __device__ __forceinline__ void fetch(const MixGradArgs &p, const bf16_t *src, int64_t first_tok, int step, int r0, int tid) {
         const int64_t t0 = uniform64(min(first_tok + step * kGradTok, p.n_tok - 1)), rest = p.n_tok - 1 - t0;
-        const uint32_t o = (uint32_t)(min(tid >> 2, (int)(rest < kGradTok ? rest : kGradTok)) * (kMix * R) + (tid & 3) * 8 + (kGx ? 0 : p.r0)) * 2u;
-        const char *b = reinterpret_cast<const char *>(src + t0 * (kMix * R));
+        const uint32_t o = (uint32_t)(min(tid >> 2, (int)(rest < kGradTok ? rest : kGradTok)) * (kMix * R) + (tid & 3) * 8 + (kGx ? 0 : r0)) * 2u;
+        const char *b = reinterpret_cast<const char *>(src + t0 * (kMix * R) + (kGx ? r0 : 0));
 #pragma unroll
-        for (int j = 0; j < kPieces; ++j) v[j] = *reinterpret_cast<const u32x4 *>(b + o + j * (kGx ? 64 : 2 * R));
+        for (int j = 0; j < kMix; ++j) v[j] = *reinterpret_cast<const u32x4 *>(b + o + j * 2 * R);
     }
     __device__ __forceinline__ void put(bf16_t *tile, int tid) const {
 #pragma unroll
-        for (int j = 0; j < kPieces; ++j)
+        for (int j = 0; j < kMix; ++j)
             *reinterpret_cast<u32x4 *>(tile + (tid >> 2) * MixGrads<R, kGx>::kPitch + (tid & 3) * 8 + 32 * j) = v[j];
     }
 };
-// where a range's h (which = 0) or gpre (1) rows of a step are
-template <int R, bool kGx> __device__ __forceinline__ bf16_t *mix_tile(unsigned char *smem, int step, int rg, int which) {
+// where a range's h (which = 0) or gpre (1) rows are of part number `turn` (step * kParts + part)
+template <int R, bool kGx> __device__ __forceinline__ bf16_t *mix_tile(unsigned char *smem, int turn, int rg, int which) {
     typedef MixGrads<R, kGx> L;
-    return reinterpret_cast<bf16_t *>(smem + L::kTiles + (((L::kBufs == 2 ? step & 1 : 0) * 2 + rg) * 2 + which) * L::kTile);
-}
-// the barriers at the head of a step: its rows are in LDS behind them
-template <int R, bool kGx> __device__ __forceinline__ void mix_step_begins() {
-    __syncthreads();
-    if (MixGrads<R, kGx>::kBufs == 1) __syncthreads();   // (the A waves fill the only buffer in between)
+    return reinterpret_cast<bf16_t *>(smem + L::kTiles + (((turn & 1) * 2 + rg) * 2 + which) * L::kTile);
 }
 // operand fragment with the k-slots along a step's 32 tokens: column n0 + l16 of a tile.  A lane group's four slots are
 // tokens two apart: with 20 banks from row to row, their four 32-byte pieces then lie on all 32 different banks.
@@ -458,12 +456,15 @@ template <int R>
 __device__ __forceinline__ void mix_gx_wave(const MixGradArgs &p, unsigned char *smem, int range, int rg, int cg, int half, int lane)
 {
     typedef MixGrads<R, true> L;
-    constexpr int KW = R / 32, KA = kMix * R / 32, kPitch = L::kPitch;
+    constexpr int kParts = L::kParts, kPitch = L::kPitch;
     const int l16 = lane & 15, g = lane >> 4, C = p.C;
     const bf16_t *wf = reinterpret_cast<const bf16_t *>(smem + L::kW), *af = reinterpret_cast<const bf16_t *>(smem + L::kA);
     const float *bias_l = reinterpret_cast<const float *>(smem + L::kBias) + 32 * half + 8 * g;
     const float *mix_l = reinterpret_cast<const float *>(smem + L::kMixX) + 32 * half + 8 * g;
     const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
+    // (R = 64) A's columns of the workgroup, and the lane's place in them: tile 2 half, the other tile's rows are four channels on
+    const char *a_cols = reinterpret_cast<const char *>(p.a_t + (size_t)cg * 64 * (kMix * R));
+    const uint32_t a_off = (uint32_t)(mix_frag_channel(2 * half, l16) * (kMix * R) + 8 * g) * 2u;
     MixWalk wk(p, range, cg * 64 + half * 32, lane);
 #pragma unroll
     for (int s = 0; s < kMix; ++s) wk.fetch_g(s);
@@ -474,71 +475,82 @@ __device__ __forceinline__ void mix_gx_wave(const MixGradArgs &p, unsigned char 
         *reinterpret_cast<bf16x8 *>(reinterpret_cast<char *>(p.gx + base) + o) = pack_operand(v);
     };
     for (int step = 0; step < p.steps; ++step) {
-        mix_step_begins<R, true>();
-        const bf16_t *ht = mix_tile<R, true>(smem, step, rg, 0), *gt = mix_tile<R, true>(smem, step, rg, 1);
         const int next = min(step + 1, p.steps - 1);
         const int64_t cur_base = wk.base, step_tok = first_tok + step * kGradTok;
         const uint32_t cur_off[2] = {wk.off[0], wk.off[1]};
         float xx[2][8], gsum[2][8], gxx[2][8];
-        {
+        f32x4 xm[2][2];   // gxm, the same lane order as coef
+        auto take_x = [&]() {
             float xv[2][8];
             wk.x_and_xx(xv, xx);
-        }
-        wk.aim(next);
-        wk.fetch_x();
+            if (kParts == 1) wk.aim(next);
+            wk.fetch_x();
+        };
 #pragma unroll
-        for (int s = 0; s < kMix; ++s) {
-            f32x4 cf[2][2];
-            bf16x8 wfr[2][KW];
+        for (int part = 0; part < kParts; ++part) {
+            __syncthreads();
+            const bf16_t *ht = mix_tile<R, true>(smem, step * kParts + part, rg, 0), *gt = mix_tile<R, true>(smem, step * kParts + part, rg, 1);
+            if (kParts == 1) take_x();
+            else if (part == kParts - 1) wk.aim(next);
+            if (part > 0) {   // (as loaded: not the values unpacked for the part before, twice the registers)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                cf[0][m] = cf[1][m] = *reinterpret_cast<const f32x4 *>(bias_l + 64 * s + 4 * m);
+                for (int s = 0; s < kMix; ++s)
 #pragma unroll
-                for (int kk = 0; kk < KW; ++kk)
-                    wfr[m][kk] = *reinterpret_cast<const bf16x8 *>(wf + (size_t)(((s * KW + kk) * 4 + 2 * half + m) * 64 + lane) * 8);
+                    for (int b = 0; b < 2; ++b) asm volatile("" : "+v"(wk.gr[s][b].a.x), "+v"(wk.gr[s][b].a.y), "+v"(wk.gr[s][b].a.z), "+v"(wk.gr[s][b].a.w));
             }
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+            for (int s = 0; s < kMix; ++s) {
+                f32x4 cf[2][2];
+                bf16x8 wfr[2];
 #pragma unroll
-                for (int kk = 0; kk < KW; ++kk) {
-                    const bf16x8 hr = *reinterpret_cast<const bf16x8 *>(ht + (16 * b + l16) * kPitch + s * R + 32 * kk + 8 * g);
-#pragma unroll
-                    for (int m = 0; m < 2; ++m) cf[b][m] = mfma32(wfr[m][kk], hr, cf[b][m]);
+                for (int m = 0; m < 2; ++m) {
+                    cf[0][m] = cf[1][m] = part == 0 ? *reinterpret_cast<const f32x4 *>(bias_l + 64 * s + 4 * m) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                    wfr[m] = *reinterpret_cast<const bf16x8 *>(wf + (size_t)(((s * kParts + part) * 4 + 2 * half + m) * 64 + lane) * 8);
                 }
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                float gv[8];
-                wk.gr[s][b].to_float(gv);
+                for (int b = 0; b < 2; ++b) {
+                    const bf16x8 hr = *reinterpret_cast<const bf16x8 *>(ht + (16 * b + l16) * kPitch + s * 32 + 8 * g);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    gsum[b][e] = s == 0 ? gv[e] : gsum[b][e] + gv[e];
-                    gxx[b][e] = s == 0 ? gv[e] * cf[b][e >> 2][e & 3] : fmaf(gv[e], cf[b][e >> 2][e & 3], gxx[b][e]);
+                    for (int m = 0; m < 2; ++m) cf[b][m] = mfma32(wfr[m], hr, cf[b][m]);
                 }
-                pin8(gsum[b]);   // (or the sums sink to their use behind the branches below, with every g still in registers)
-                pin8(gxx[b]);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    float gv[8];
+                    wk.gr[s][b].to_float(gv);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        if (part == kParts - 1) gsum[b][e] = s == 0 ? gv[e] : gsum[b][e] + gv[e];
+                        gxx[b][e] = part == 0 && s == 0 ? gv[e] * cf[b][e >> 2][e & 3] : fmaf(gv[e], cf[b][e >> 2][e & 3], gxx[b][e]);
+                    }
+                    if (part == kParts - 1) pin8(gsum[b]);   // (or the sums sink to their use behind the branches below, with every g still in registers)
+                    pin8(gxx[b]);
+                }
+                if (part == kParts - 1) wk.fetch_g(s);
+                if (s & 1) __builtin_amdgcn_sched_barrier(0);
             }
-            wk.fetch_g(s);
-            if (s & 1) __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        f32x4 xm[2][2];   // gxm, the same lane order as coef
+            __builtin_amdgcn_sched_barrier(0);
+            if (part == 0) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b) xm[b][0] = xm[b][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < KA; ++kk) {
-            bf16x8 afr[2];
-#pragma unroll
-            for (int m = 0; m < 2; ++m)
-                afr[m] = L::kLdsA ? *reinterpret_cast<const bf16x8 *>(af + (size_t)((kk * 4 + 2 * half + m) * 64 + lane) * 8)
-                                  : *reinterpret_cast<const bf16x8 *>(p.a_t + (size_t)(cg * 64 + mix_frag_channel(2 * half + m, l16)) * (kMix * R) + 32 * kk + 8 * g);
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const bf16x8 gq = *reinterpret_cast<const bf16x8 *>(gt + (16 * b + l16) * kPitch + 32 * kk + 8 * g);
-#pragma unroll
-                for (int m = 0; m < 2; ++m) xm[b][m] = mfma32(afr[m], gq, xm[b][m]);
+                for (int b = 0; b < 2; ++b) xm[b][0] = xm[b][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
-            if (kk & 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < kMix; ++s) {
+                const int kk = s * kParts + part;   // 32 of A's stacked rows
+                bf16x8 afr[2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    afr[m] = L::kLdsA ? *reinterpret_cast<const bf16x8 *>(af + (size_t)((kk * 4 + 2 * half + m) * 64 + lane) * 8)
+                                      : *reinterpret_cast<const bf16x8 *>(a_cols + a_off + m * 4 * (kMix * R) * 2 + 64 * kk);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const bf16x8 gq = *reinterpret_cast<const bf16x8 *>(gt + (16 * b + l16) * kPitch + 32 * s + 8 * g);
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) xm[b][m] = mfma32(afr[m], gq, xm[b][m]);
+                }
+                if (s & 1) __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        if (kParts > 1) take_x();   // (here, not ahead of the products: xx is not needed before, and its sixteen registers are)
         float o[2][8], mx[8];
         load8(mix_l, mx);
 #pragma unroll
@@ -617,8 +629,6 @@ __device__ __forceinline__ void mix_w_wave(const MixGradArgs &p, unsigned char *
     typedef MixGrads<R, kGx> L;
     const int l16 = lane & 15, g = lane >> 4, C = p.C;
     bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + (2 * rg + half) * kGradTok * L::kStagePitch;
-    const int col0 = kGx ? p.r0 : 0;                          // of a mixer's columns in the tile
-    constexpr int kMixCols = kGx ? R : 32;
     f32x4 acc[4 * kMix];                                      // (s, rank tile, channel tile): rows = rank, columns = channels
     f32x4 acc_b[2];                                           // row s: gbias of mixer s
 #pragma unroll
@@ -630,8 +640,8 @@ __device__ __forceinline__ void mix_w_wave(const MixGradArgs &p, unsigned char *
 #pragma unroll
     for (int s = 0; s < kAhead; ++s) wk.fetch_g(s);
     for (int step = 0; step < p.steps; ++step) {
-        mix_step_begins<R, kGx>();
-        const bf16_t *ht = mix_tile<R, kGx>(smem, step, rg, 0);
+        __syncthreads();
+        const bf16_t *ht = mix_tile<R, kGx>(smem, step * L::kParts, rg, 0);   // (the part with this launch's columns)
         float xx[2][8];
         {
             float xv[2][8];
@@ -653,7 +663,7 @@ __device__ __forceinline__ void mix_w_wave(const MixGradArgs &p, unsigned char *
             const bf16x8 gc[2] = {mix_frag_tokens(stage, L::kStagePitch, 0, l16, g), mix_frag_tokens(stage, L::kStagePitch, 16, l16, g)};
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const bf16x8 hq = mix_frag_tokens(ht, L::kPitch, s * kMixCols + col0 + 16 * i, l16, g);
+                const bf16x8 hq = mix_frag_tokens(ht, L::kPitch, s * 32 + 16 * i, l16, g);
 #pragma unroll
                 for (int j = 0; j < 2; ++j) acc[4 * s + 2 * i + j] = mfma32(hq, gc[j], acc[4 * s + 2 * i + j]);
             }
@@ -664,6 +674,7 @@ __device__ __forceinline__ void mix_w_wave(const MixGradArgs &p, unsigned char *
             if (s & 1) __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if (L::kParts == 2) __syncthreads();   // (the other part is the gx waves')
     }
     if (p.r0 == 0) {
 #pragma unroll
@@ -682,33 +693,26 @@ __device__ __forceinline__ void mix_a_wave(const MixGradArgs &p, unsigned char *
     const int l16 = lane & 15, g = lane >> 4, tid = half * 64 + lane, C = p.C;
     const float *mix_l = reinterpret_cast<const float *>(smem + L::kMixX) + 32 * half + 8 * g;
     bf16_t *stage = reinterpret_cast<bf16_t *>(smem + L::kStage) + (4 + 2 * rg + half) * kGradTok * L::kStagePitch;
-    const int col0 = kGx ? p.r0 : 0;
-    constexpr int kMixCols = kGx ? R : 32;
     f32x4 acc[4 * kMix];                                      // (s, rank tile, channel tile): rows = channels, columns = rank
 #pragma unroll
     for (int i = 0; i < 4 * kMix; ++i) acc[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int64_t first_tok = (int64_t)range * p.steps * kGradTok;
     MixTile<R, kGx> tile;
-    auto fill = [&](const bf16_t *src, int from, int step, int which) {
-        tile.fetch(p, src, first_tok, from, tid);
-        tile.put(mix_tile<R, kGx>(smem, step, rg, which), tid);
-    };
-    if (L::kBufs == 2) {
-        fill(p.h, 0, 0, 0);
-        fill(p.gpre, 0, 0, 1);
-    }
+    constexpr int kParts = L::kParts;
+    const int r0 = kGx ? 0 : p.r0;
+    tile.fetch(p, p.h, first_tok, 0, r0, tid);
+    tile.put(mix_tile<R, kGx>(smem, 0, rg, 0), tid);
+    tile.fetch(p, p.gpre, first_tok, 0, r0, tid);
+    tile.put(mix_tile<R, kGx>(smem, 0, rg, 1), tid);
     MixWalk wk(p, range, cg * 64 + half * 32, lane);
-    for (int step = 0; step < p.steps; ++step) {
+    // one part of a step, the tiles of the part behind it brought meanwhile
+    auto take = [&](auto part, int step) {
+        constexpr int kPart = decltype(part)::value;
         __syncthreads();
         const int next = min(step + 1, p.steps - 1);
-        if (L::kBufs == 1) {
-            fill(p.h, step, step, 0);
-            fill(p.gpre, step, step, 1);
-            __syncthreads();
-        } else {
-            tile.fetch(p, p.h, first_tok, next, tid);
-        }
-        {
+        const int bstep = kPart + 1 < kParts ? step : next, br0 = kParts == 2 ? 32 * (1 - kPart) : r0;
+        tile.fetch(p, p.h, first_tok, bstep, br0, tid);
+        if constexpr (kPart == 0) {
             float xv[2][8], xx[2][8], mx[8];
             wk.x_and_xx(xv, xx);
             wk.aim(next);
@@ -721,20 +725,24 @@ __device__ __forceinline__ void mix_a_wave(const MixGradArgs &p, unsigned char *
                 *reinterpret_cast<bf16x8 *>(stage + (16 * b + l16) * L::kStagePitch + 8 * g) = pack_operand(xv[b]);
             }
         }
-        if (L::kBufs == 2) {
-            tile.put(mix_tile<R, kGx>(smem, step + 1, rg, 0), tid);
-            tile.fetch(p, p.gpre, first_tok, next, tid);
-        }
-        const bf16x8 xt[2] = {mix_frag_tokens(stage, L::kStagePitch, 0, l16, g), mix_frag_tokens(stage, L::kStagePitch, 16, l16, g)};
-        const bf16_t *gt = mix_tile<R, kGx>(smem, step, rg, 1);
+        tile.put(mix_tile<R, kGx>(smem, step * kParts + kPart + 1, rg, 0), tid);
+        tile.fetch(p, p.gpre, first_tok, bstep, br0, tid);
+        if constexpr (kPart == 0) {
+            const bf16x8 xt[2] = {mix_frag_tokens(stage, L::kStagePitch, 0, l16, g), mix_frag_tokens(stage, L::kStagePitch, 16, l16, g)};
+            const bf16_t *gt = mix_tile<R, kGx>(smem, step * kParts + kPart, rg, 1);
 #pragma unroll
-        for (int i = 0; i < 2 * kMix; ++i) {
-            const bf16x8 gq = mix_frag_tokens(gt, L::kPitch, (i >> 1) * kMixCols + col0 + 16 * (i & 1), l16, g);
+            for (int i = 0; i < 2 * kMix; ++i) {
+                const bf16x8 gq = mix_frag_tokens(gt, L::kPitch, 16 * i, l16, g);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[2 * i + j] = mfma32(xt[j], gq, acc[2 * i + j]);
-            if (i % 5 == 4) __builtin_amdgcn_sched_barrier(0);
+                for (int j = 0; j < 2; ++j) acc[2 * i + j] = mfma32(xt[j], gq, acc[2 * i + j]);
+                if (i % 5 == 4) __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        if (L::kBufs == 2) tile.put(mix_tile<R, kGx>(smem, step + 1, rg, 1), tid);
+        tile.put(mix_tile<R, kGx>(smem, step * kParts + kPart + 1, rg, 1), tid);
+    };
+    for (int step = 0; step < p.steps; ++step) {
+        take(std::integral_constant<int, 0>{}, step);
+        if constexpr (kParts == 2) take(std::integral_constant<int, 1>{}, step);
     }
     mix_fold(acc, reinterpret_cast<f32x4 *>(smem) + (half * 40 + 20) * 64, p.part_a, ((size_t)(run * (C / 64) + cg) * 2 + half) * 20, rg, lane);
 }
