@@ -170,6 +170,16 @@ int wkv6_gn_gate_backward(void *stream, int dtype, int64_t B, int64_t T, int64_t
                           const void *gout, const void *y, const float *stats, const void *gate,
                           const float *gn_scale, const float *gn_offset,
                           void *gy, void *ggate, float *gscale, float *goffset);
+/* The same pair without the launch that zeroes gscale and goffset: the forward does it on the way, and the (first) backward
+ * adds to what it left. */
+int wkv6_forward_gn_gate_save_sums(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                                   const void *r, const void *k, const void *v, const void *w, const void *u,
+                                   const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
+                                   void *out, void *y, float *stats, void *saved, size_t saved_bytes, float *gscale, float *goffset);
+int wkv6_gn_gate_backward_sums(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                               const void *gout, const void *y, const float *stats, const void *gate,
+                               const float *gn_scale, const float *gn_offset,
+                               void *gy, void *ggate, float *gscale, float *goffset);
 
 /* The INPUT side of the layer around the operator (no counterpart in the reference, which leaves it
  * to framework kernels): the token shift and the five low-rank mixers of rwkv6_model.py:134-146 that

@@ -151,13 +151,13 @@ std::vector<Tensor> wkv6_grads(const Dims &d, int algo, const Tensor &r, const T
 
 // The saved chunk states, handed from the forward to the first backward.  A second backward over the same graph
 // (retain_graph) finds none, since their counters are used up, and runs the plain backward.  (torch holds the node's
-// lock while a backward runs.)
-void keep(AutogradContext *ctx, const Tensor &saved) {
-  if (saved.defined()) ctx->saved_data["states"] = saved;
+// lock while a backward runs.)  The same goes for sums that the forward cleared.
+void keep(AutogradContext *ctx, const Tensor &saved, const char *name = "states") {
+  if (saved.defined()) ctx->saved_data[name] = saved;
 }
 
-Tensor take(AutogradContext *ctx) {
-  auto it = ctx->saved_data.find("states");
+Tensor take(AutogradContext *ctx, const char *name = "states") {
+  auto it = ctx->saved_data.find(name);
   if (it == ctx->saved_data.end()) return Tensor();
   Tensor t = it->second.toTensor();
   ctx->saved_data.erase(it);
@@ -221,9 +221,14 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
     // out and what stays for the backward lie in blocks of their own: an output that a caller keeps holds nothing else
     const Tensor res = carve(r, {{{B, T, C}, r.scalar_type(), 5}})[0];
     const auto t = carve(r, {{{B, T, C}, r.scalar_type(), 6}, {{nsave}, at::kByte, 7}, {{B, T, H, 2}, at::kFloat, 0}});
-    check(wkv6_forward_gn_gate_save(stream_of(r), code, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gate), in_f(sc), in_f(of),
-                                    static_cast<float>(eps), out(res), out(t[0]), out_f(t[2]), out(t[1]), nsave));
+    // the norm's gradients, which this forward clears for the first backward to add to
+    const Tensor gscale = parameter_gradient(r, sc.sizes(), at::kFloat), goffset = parameter_gradient(r, of.sizes(), at::kFloat);
+    check(wkv6_forward_gn_gate_save_sums(stream_of(r), code, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gate), in_f(sc), in_f(of),
+                                         static_cast<float>(eps), out(res), out(t[0]), out_f(t[2]), out(t[1]), nsave, out_f(gscale),
+                                         out_f(goffset)));
     keep(ctx, t[1]);
+    keep(ctx, gscale, "gscale");
+    keep(ctx, goffset, "goffset");
     ctx->saved_data["H"] = H;
     ctx->saved_data["scale_type"] = static_cast<int64_t>(scale.scalar_type());
     ctx->saved_data["offset_type"] = static_cast<int64_t>(offset.scalar_type());
@@ -243,9 +248,14 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
     const ScalarType t = r.scalar_type();
     const Tensor gy = carve(r, {{{B, T, C}, t, 5}})[0];
     const Tensor ggate = carve(r, {{{B, T, C}, t, 6}})[0];
-    const Tensor gscale = parameter_gradient(r, s[6].sizes(), at::kFloat), goffset = parameter_gradient(r, s[7].sizes(), at::kFloat);
-    check(wkv6_gn_gate_backward(stream_of(r), code_of(t), B, T, C, H, in(gout), in(s[8]), in_f(s[9]), in(s[5]), in_f(s[6]), in_f(s[7]),
-                                out(gy), out(ggate), out_f(gscale), out_f(goffset)));
+    Tensor gscale = take(ctx, "gscale"), goffset = take(ctx, "goffset");
+    const auto norm_backward = gscale.defined() ? wkv6_gn_gate_backward_sums : wkv6_gn_gate_backward;
+    if (!gscale.defined()) {   // a second backward over the same graph
+      gscale = parameter_gradient(r, s[6].sizes(), at::kFloat);
+      goffset = parameter_gradient(r, s[7].sizes(), at::kFloat);
+    }
+    check(norm_backward(stream_of(r), code_of(t), B, T, C, H, in(gout), in(s[8]), in_f(s[9]), in(s[5]), in_f(s[6]), in_f(s[7]), out(gy),
+                        out(ggate), out_f(gscale), out_f(goffset)));
     auto w = wkv6_grads(d, kChunk, r, s[1], s[2], s[3], s[4], gy, take(ctx));
     return {w[0], w[1], w[2], w[3], w[4], ggate,
             gscale.to(static_cast<ScalarType>(ctx->saved_data["scale_type"].toInt())),

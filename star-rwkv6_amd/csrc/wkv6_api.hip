@@ -227,10 +227,11 @@ int wkv6_forward_gn_gate_save_supported(int dtype, int64_t B, int64_t T, int64_t
     return check_shape(dtype, B, T, C, H) == WKV6_OK && dtype == WKV6_BF16 && chunk_possible(dtype, T, C);
 }
 
-int wkv6_forward_gn_gate_save(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+static int forward_gn_gate_save(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
                               const void *r, const void *k, const void *v, const void *w, const void *u,
                               const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                              void *out, void *y, float *stats, void *saved, size_t saved_bytes) {
+                              void *out, void *y, float *stats, void *saved, size_t saved_bytes,
+                                wkv6::GnSums sums) {
     int rc = check_shape(dtype, B, T, C, H);
     if (rc != WKV6_OK) return rc;
     if (dtype != WKV6_BF16 || !chunk_possible(dtype, T, C)) return WKV6_ERR_UNSUPPORTED;
@@ -244,23 +245,54 @@ int wkv6_forward_gn_gate_save(void *stream, int dtype, int64_t B, int64_t T, int
     if (P > 1) {   // few pairs, long sequence: time segments side by side, the output stage in their second pass
         char *extra = reinterpret_cast<char *>(saved) + saved_base_bytes(dtype, WKV6_ALGO_CHUNK, B * P, wkv6::train_segments_layout(B, T, H, nullptr).L, C, H);
         return finish(wkv6::chunk_forward_fused_save_segments((hipStream_t)stream, B, T, H, r, k, v, w, u, gate, gn_scale, gn_offset,
-                                                              gn_eps, out, y, stats, saved, extra));
+                                                              gn_eps, out, y, stats, saved, extra, sums));
     }
     return finish(wkv6::chunk_forward_fused_save((hipStream_t)stream, B, T, H, r, k, v, w, u, gate, gn_scale, gn_offset, gn_eps,
-                                                 out, y, stats, saved));
+                                                 out, y, stats, saved, sums));
 }
 
-int wkv6_gn_gate_backward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+int wkv6_forward_gn_gate_save(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                              const void *r, const void *k, const void *v, const void *w, const void *u,
+                              const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
+                              void *out, void *y, float *stats, void *saved, size_t saved_bytes) {
+    return forward_gn_gate_save(stream, dtype, B, T, C, H, r, k, v, w, u, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, saved_bytes, wkv6::GnSums());
+}
+
+int wkv6_forward_gn_gate_save_sums(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                                   const void *r, const void *k, const void *v, const void *w, const void *u,
+                                   const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
+                                   void *out, void *y, float *stats, void *saved, size_t saved_bytes, float *gscale, float *goffset) {
+    if (!gscale || !goffset) return WKV6_ERR_ARG;
+    wkv6::GnSums sums;
+    sums.scale = gscale; sums.offset = goffset;
+    return forward_gn_gate_save(stream, dtype, B, T, C, H, r, k, v, w, u, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, saved_bytes, sums);
+}
+
+static int gn_gate_backward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
                           const void *gout, const void *y, const float *stats, const void *gate,
                           const float *gn_scale, const float *gn_offset,
-                          void *gy, void *ggate, float *gscale, float *goffset) {
+                          void *gy, void *ggate, float *gscale, float *goffset, bool cleared) {
     int rc = check_shape(dtype, B, T, C, H);
     if (rc != WKV6_OK) return rc;
     if (dtype != WKV6_BF16) return WKV6_ERR_UNSUPPORTED;
     if (!gout || !y || !stats || !gate || !gn_scale || !gn_offset || !gy || !ggate || !gscale || !goffset) return WKV6_ERR_ARG;
     if (!aligned16(gout) || !aligned16(y) || !aligned16(stats) || !aligned16(gate) || !aligned16(gn_scale) || !aligned16(gn_offset) ||
         !aligned16(gy) || !aligned16(ggate) || !aligned16(gscale) || !aligned16(goffset)) return WKV6_ERR_ARG;
-    return finish(wkv6::gn_gate_backward((hipStream_t)stream, B, T, H, gout, y, stats, gate, gn_scale, gn_offset, gy, ggate, gscale, goffset));
+    return finish(wkv6::gn_gate_backward((hipStream_t)stream, B, T, H, gout, y, stats, gate, gn_scale, gn_offset, gy, ggate, gscale, goffset, cleared));
+}
+
+int wkv6_gn_gate_backward(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                          const void *gout, const void *y, const float *stats, const void *gate,
+                          const float *gn_scale, const float *gn_offset,
+                          void *gy, void *ggate, float *gscale, float *goffset) {
+    return gn_gate_backward(stream, dtype, B, T, C, H, gout, y, stats, gate, gn_scale, gn_offset, gy, ggate, gscale, goffset, false);
+}
+
+int wkv6_gn_gate_backward_sums(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
+                               const void *gout, const void *y, const float *stats, const void *gate,
+                               const float *gn_scale, const float *gn_offset,
+                               void *gy, void *ggate, float *gscale, float *goffset) {
+    return gn_gate_backward(stream, dtype, B, T, C, H, gout, y, stats, gate, gn_scale, gn_offset, gy, ggate, gscale, goffset, true);
 }
 
 static int check_mix(int dtype, int64_t B, int64_t T, int64_t C, int64_t R) {

@@ -70,6 +70,7 @@ struct BlockFwdArgs {
     float gn_eps;
     bf16_t *out;
     float *stats;            // null, or (B, T, H, 2): mean and 1/sqrt(var + eps) per (token, head) for the backward
+    GnSums sums;             // (kSave)
 };
 
 // sum over the 8 lanes that hold one 128-byte row (lanes 8k .. 8k+7), result in each of them
@@ -115,6 +116,7 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
             for (int rr = 0; rr < 4; ++rr) Snext[m][rr] = start[(block_row_channel(m, g) + rr) * kN + 16 * q + l16];
     } else if (a.s0 != nullptr) request_state(0);
     if (kSave && b0 == 0 && q == 0 && lane == 0 && a.arrivals) a.arrivals[h] = 0;
+    if (kSave && kFuse && b0 == 0 && q == 0) clear_sums(a.sums, h, lane);
     int c = 0, slot = 0;   // visit `it` is chunk c of pair number `slot`
     for (int it = 0; it < nvisit; ++it) {
         __syncthreads();
@@ -428,7 +430,7 @@ __device__ __forceinline__ void block_output_stage_in_place(const BlockFwdArgs &
     }
 }
 
-// kStream: a call without a backward and with large tensors (past_caches): 1: r, k, v, w and the gate are read without keeping
+// kStream: large tensors, and no backward or one that comes late (past_caches): 1: r, k, v, w and the gate are read without keeping
 // their lines.  What such a call reads it reads once, and lines that stay behind only push out others.  2: y (or out) is written so, too.
 // (Two kernels: asked at run time, the two kinds of store became one.)
 // kSegments: rows that are time segments.  Built apart: asked at run time, the other ragged launches, whose
@@ -492,12 +494,14 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H) {
     return 2 * pairs > cus && block_grid(B, H) > 0 && T * H * kN < (1LL << 31);
 }
 
-// kStream of a call that no backward follows: from 28 MiB a tensor 1, from 64 MiB 2.  Prompts, kept / 1 / 2, us: B64 T512 H32 with the output
+// kStream: from 28 MiB a tensor 1, from 64 MiB 2.  Prompts, kept / 1 / 2, us: B64 T512 H32 with the output
 // stage 186.4 / 179.1 / 152.3 (5.7 TB/s), without 151.8 / 146.6 / 132.3; B16 T1024 (64 MiB) 83.9 / 71.8 / 70.8; B8 T1024 (32 MiB) 43.3 / 38.1,
 // with the output stage 51.3 / 45.8; B8 T900 (28.1 MiB) 40.0 / 37.8.  Below, inputs that other work left in the last-level cache are lost by 1: 23 MiB a
 // tensor (B5 T1184) 38.2 / 38.4, 8 MiB (B6 T350) 16.8 / 17.8; and so is an output by 2: call and a product that reads its y together, B8 T1024
 // 64.1 / 60.4 / 62.2; B16 T1024 109.0 / 99.2 / 101.2 and B64 T512 195.0 / 171.6 / 175.4, where the call by itself gains more.  With a
 // backward that reads the inputs again (keep_inputs) they stay: B8 T1024 through the state 167.3 / 169.1, the training pair 124.5 / 126.9.
+// The saving forward with the output stage reads past them as well: five tensors written and three more read lie between it and the
+// operator's backward (forward and backward B8 T1024 170.7 / 167.4, B16 T512 165.6 / 163.0, B34 T570 H12 171.9 / 167.9).
 static int past_caches(int64_t B, int64_t T, int64_t H) {
     const int64_t bytes = B * T * H * kN * 2;
     return bytes >= (64LL << 20) ? 2 : bytes >= (28LL << 20) ? 1 : 0;
@@ -508,7 +512,7 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
                                        const void *r, const void *k, const void *v, const void *w, const void *u,
                                        const void *s0, const int64_t *map, void *y, void *sT, void *saved_states, bool counters,
                                        const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps, void *out, float *stats, RowCut cut,
-                                       const SegmentChain &chain, bool keep_inputs = false)
+                                       const SegmentChain &chain, bool keep_inputs = false, GnSums sums = GnSums())
 {
     BlockFwdArgs a = {};
     a.cut = cut; a.chain = chain;
@@ -521,6 +525,7 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
     a.s0 = s0; a.map = map; a.y = (bf16_t *)y; a.sT = sT; a.ckpt = (float *)saved_states;
     a.arrivals = saved_states && counters ? reinterpret_cast<int *>(reinterpret_cast<char *>(saved_states) + chunk_backward_workspace_bytes(B, T, H)) : nullptr;
     a.gate = (const bf16_t *)gate; a.gn_scale = gn_scale; a.gn_offset = gn_offset; a.gn_eps = gn_eps; a.out = (bf16_t *)out; a.stats = stats;
+    a.sums = sums;
     auto launch_as = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag, auto stream_tag) -> hipError_t {
         constexpr bool kFuse = decltype(fuse_tag)::value;
         constexpr auto kern = block_fwd_kernel<decltype(ts_tag), decltype(save_tag)::value, decltype(ragged_tag)::value, kFuse, decltype(segments_tag)::value, decltype(stream_tag)::value>;
@@ -530,7 +535,7 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
         return hipGetLastError();
     };
     auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag) -> hipError_t {
-        if constexpr (!decltype(save_tag)::value && !decltype(segments_tag)::value)
+        if constexpr ((!decltype(save_tag)::value || decltype(fuse_tag)::value) && !decltype(segments_tag)::value)
             switch (keep_inputs ? 0 : past_caches(B, T, H)) {
             case 1: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 1>{});
             case 2: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 2>{});
@@ -568,10 +573,10 @@ hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, 
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut, SegmentChain chain)
+                               void *out, void *y, float *stats, void *sT, void *saved_states, RowCut cut, SegmentChain chain, GnSums sums)
 {
     return block_forward_launch(st, state_dtype, B, T, H, r, k, v, w, u, s0, map, y, sT, saved_states, saved_states != nullptr,
-                                gate, gn_scale, gn_offset, gn_eps, out, stats, cut, chain);
+                                gate, gn_scale, gn_offset, gn_eps, out, stats, cut, chain, false, sums);
 }
 
 }  // namespace wkv6

@@ -90,6 +90,7 @@ struct FwdArgs {
     bf16_t *out;
     // training with the fused output stage (then y above is written as well, for the norm's backward):
     float *stats;    // null, or (B, T, H, 2) fp32: mean and 1/sqrt(var + eps) of y over each head's channels
+    GnSums sums;
 };
 
 // ------------------------------------------------------------------------------------------
@@ -135,6 +136,7 @@ __device__ __forceinline__ void fwd_consumer(const FwdArgs &a, const unsigned ch
         typedef typename OutOf<Tin>::type Tout;
         Tout *y_h = reinterpret_cast<Tout *>(a.y) + base;
         if (kSave && GRP == 0 && b == 0 && q == 0 && lane == 0 && a.arrivals) a.arrivals[h] = 0;
+        if (kSave && kFuse && GRP == 0 && b == 0 && q == 0) clear_sums(a.sums, h, lane);
         for (int c = 0; c < nchunk; ++c, ++it) {
             __syncthreads();
             if (kSave && GRP == 0) {
@@ -717,12 +719,13 @@ hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64
 static hipError_t fused_save_from(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                   const void *r, const void *k, const void *v, const void *w, const void *u, const float *s0,
                                   const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                  void *out, void *y, float *stats, void *saved_states, RowCut cut = RowCut())
+                                  void *out, void *y, float *stats, void *saved_states, GnSums sums, RowCut cut = RowCut())
 {
     if (!cut.segments && block_forward_applies(B, T, H))
-        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states);
+        return block_forward_fused(st, kF32, B, T, H, r, k, v, w, u, s0, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved_states,
+                                   RowCut(), SegmentChain(), sums);
     FwdArgs a = {};
-    a.s0 = s0;
+    a.s0 = s0; a.sums = sums;
     a.T = (int)T; a.H = (int)H; a.nitems = (int)(B * H); a.slice = (int)((T + CL - 1) / CL);
     a.r = (const bf16_t *)r; a.k = (const bf16_t *)k; a.v = (const bf16_t *)v; a.w = (const bf16_t *)w; a.u = (const bf16_t *)u;
     a.v_orig = v;
@@ -740,9 +743,9 @@ static hipError_t fused_save_from(hipStream_t st, int64_t B, int64_t T, int64_t 
 hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                     const void *r, const void *k, const void *v, const void *w, const void *u,
                                     const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                    void *out, void *y, float *stats, void *saved_states)
+                                    void *out, void *y, float *stats, void *saved_states, GnSums sums)
 {
-    return fused_save_from(st, B, T, H, r, k, v, w, u, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved_states);
+    return fused_save_from(st, B, T, H, r, k, v, w, u, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved_states, sums);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -980,7 +983,7 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
 hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                              const void *r, const void *k, const void *v, const void *w, const void *u,
                                              const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                             void *out, void *y, float *stats, void *saved, void *extra)
+                                             void *out, void *y, float *stats, void *saved, void *extra, GnSums sums)
 {
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
@@ -988,9 +991,9 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
     hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
-    if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states));
+    if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states), sums);
     if ((e = segment_chain_forward(st, s.P, B, H, s.decay, s.states, nullptr)) != hipSuccess) return e;
-    return fused_save_from(st, rows, L, H, r, k, v, w, u, s.states, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, s.cut);
+    return fused_save_from(st, rows, L, H, r, k, v, w, u, s.states, gate, gn_scale, gn_offset, gn_eps, out, y, stats, saved, sums, s.cut);
 }
 
 }  // namespace wkv6

@@ -13,6 +13,8 @@
 // kernel's input (the gate's own backward, which reads ggate next, takes as long with it in the caches: within 3 % either way from 256 to 16384
 // tokens of H32).  B8 T1024 H32, 168 MB: 31 us = 5.5 TB/s behind the forward that
 // wrote y, 41 us with nothing of it cached (one head per wave, 2 bytes per lane: 49 and 55 us).
+// The sums are added up by one atomic operation per channel and workgroup, onto what the forward cleared (GnSums) or, without it, a kernel
+// ahead of this one (2 to 5 us and a launch: forward and backward B8 T1024 H32 167.4 / 164.1, of host time at small sizes 99 / 95).
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
 
@@ -111,11 +113,11 @@ __global__ void zero2_kernel(int n, float *a, float *b) {
 
 hipError_t gn_gate_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                             const void *gout, const void *y, const float *stats, const void *gate,
-                            const float *scale, const float *offset, void *gy, void *ggate, float *gscale, float *goffset)
+                            const float *scale, const float *offset, void *gy, void *ggate, float *gscale, float *goffset, bool cleared)
 {
     const int C = (int)(H * kN);
     // (a fill kernel rather than a memset node: the call may be captured in a HIP graph)
-    hipLaunchKernelGGL(zero2_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, C, gscale, goffset);
+    if (!cleared) hipLaunchKernelGGL(zero2_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, C, gscale, goffset);
     const int64_t n = B * T;
     const int columns = (C + 511) / 512;
     // as many workgroups as the chip holds at once (four of four waves per compute unit; two or eight: the same time), fewer where tokens run out

@@ -135,13 +135,23 @@ hipError_t block_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, 
                          RowCut cut = RowCut(), SegmentChain chain = SegmentChain(),   // (rows that are segments: cut and chain, s0 = map = sT = null)
                          bool keep_inputs = false);   // a backward will read them again
 
+// The sums over tokens that the norm's backward will add up, (H, 64) each (null: none): the saving fused forward clears them, where the
+// backward would need a launch of its own for it.
+struct GnSums {
+    float *scale = nullptr, *offset = nullptr;
+};
+// by the 64 lanes of one wave per head
+__device__ __forceinline__ void clear_sums(const GnSums &s, int h, int lane) {
+    if (s.scale) { s.scale[h * 64 + lane] = 0.f; s.offset[h * 64 + lane] = 0.f; }
+}
+
 // the block-form forward with the layer's output stage fused in (see chunk_forward_fused / chunk_forward_fused_save):
 // y and stats may be null (inference), saved_states null without a backward to follow
 hipError_t block_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s0, const int64_t *map, const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
                                void *out, void *y, float *stats, void *sT, void *saved_states,
-                               RowCut cut = RowCut(), SegmentChain chain = SegmentChain());
+                               RowCut cut = RowCut(), SegmentChain chain = SegmentChain(), GnSums sums = GnSums());
 bool block_backward_applies(int64_t B, int64_t T, int64_t H);
 // workspace: the chunk-start states as a forward pass leaves them, followed by the per-head counters; gu_sum may be null
 hipError_t block_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
@@ -269,16 +279,16 @@ hipError_t chunk_forward_fused(hipStream_t st, int state_dtype, int64_t B, int64
 hipError_t chunk_forward_fused_save(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                     const void *r, const void *k, const void *v, const void *w, const void *u,
                                     const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                    void *out, void *y, float *stats, void *saved_states);
+                                    void *out, void *y, float *stats, void *saved_states, GnSums sums);
 // ... of a shape whose training pair runs in time segments (saved / extra as in chunk_forward_save_segments)
 hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t T, int64_t H,
                                              const void *r, const void *k, const void *v, const void *w, const void *u,
                                              const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,
-                                             void *out, void *y, float *stats, void *saved, void *extra);
-// backward of the output stage (wkv6_gn.hip): bf16 tensors, gscale / goffset fp32 (C), zeroed inside
+                                             void *out, void *y, float *stats, void *saved, void *extra, GnSums sums);
+// backward of the output stage (wkv6_gn.hip): bf16 tensors, gscale / goffset fp32 (C), zeroed inside unless they are `cleared`
 hipError_t gn_gate_backward(hipStream_t st, int64_t B, int64_t T, int64_t H,
                             const void *gout, const void *y, const float *stats, const void *gate,
-                            const float *scale, const float *offset, void *gy, void *ggate, float *gscale, float *goffset);
+                            const float *scale, const float *offset, void *gy, void *ggate, float *gscale, float *goffset, bool cleared);
 
 // input side of the time-mix layer (wkv6_mix.hip): token shift and the five low-rank mixers, bf16 tensors,
 // rank R in {32, 64}.  h (B,T,5,R), w2t (5,C,R), bias (5,C) and mix_x (C) fp32.

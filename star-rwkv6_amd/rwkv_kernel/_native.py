@@ -33,6 +33,8 @@ SIGNATURES = {
     "wkv6_forward_gn_gate_ex": (_int, [_p, _int, _int] + [_i64] * 4 + [_int, _p] + [_p] * 9 + [ctypes.c_float, _p, _p] + [_p, _sz]),
     "wkv6_forward_gn_gate_save_supported": (_int, [_int] + [_i64] * 4),
     "wkv6_forward_gn_gate_save": (_int, [_p, _int] + [_i64] * 4 + [_p] * 8 + [ctypes.c_float] + [_p] * 4 + [_sz]),
+    "wkv6_forward_gn_gate_save_sums": (_int, [_p, _int] + [_i64] * 4 + [_p] * 8 + [ctypes.c_float] + [_p] * 4 + [_sz] + [_p] * 2),
+    "wkv6_gn_gate_backward_sums": (_int, [_p, _int] + [_i64] * 4 + [_p] * 10),
     "wkv6_gn_gate_backward": (_int, [_p, _int] + [_i64] * 4 + [_p] * 10),
     "wkv6_shift_mix_supported": (_int, [_int, _i64, _i64]),
     "wkv6_shift_mix_x": (_int, [_p, _int] + [_i64] * 3 + [_p] * 3),
