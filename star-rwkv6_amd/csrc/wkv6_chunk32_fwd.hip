@@ -1,16 +1,19 @@
 // Forward of the full-precision chunk form (see wkv6_chunk32.h for the algebra): fp32 and fp16 tensors,
 // every product on v_mfma_f32_16x16x4_f32, relative error that of fp32.
 //
-// One workgroup of twelve waves per (batch, head) pair.  Waves 4..11 load, in two groups of four that take
+// One workgroup of sixteen waves per (batch, head) pair.  Waves 4..11 load, in two groups of four that take
 // the chunks in turn: a group brings its chunk from global memory (16-byte loads issued two chunks ahead,
 // converted to fp32), forms the decay products with row-wide DPP steps and writes the operand tiles to LDS.
 // Waves 0..3 compute: wave q owns value columns 16q..16q+15 of the state (four 16x16 accumulator tiles
 // over the key rows), which never leaves its registers: as a C/D tile it is directly the B operand of
 // R' S.  Two workgroup barriers per chunk:
 //   phase 1  compute: y = R' S ; three of the waves form one tile each of A = R~ K~^T (masked, with the
-//            u diagonal) -> LDS ; y rows of the chunk behind LDS -> global      load: tiles R', K', V, e^{c_32} of the next chunk -> LDS
+//            u diagonal) -> LDS      load: tiles R', K', V, e^{c_32} of the next chunk -> LDS      store: y rows of the chunk behind
 //   phase 2  compute: y += A V -> LDS ;  S = e^{c_32} o S + K'^T V     load: tiles R~, K~ of the next chunk -> LDS;
-//            the operands of the chunk after it formed in registers (decay products over the rows)
+//            the operands of the chunk after it formed in registers (decay products over the rows)      store: the state at the chunk's start
+// Waves 12..15 store: y (whole 256-byte rows) and the chunk-start states reach them through LDS.  A store waits until the memory
+// system takes it, and in the computing waves that held up the matrix instructions: fp32 B8 T1024 H32, the saving forward 135 us with
+// the stores there, 112 so (96 with neither y nor states stored at all); fp16 124 / 106.
 // Saved states (one per chunk, for the backward) are written in fragment order: tile (q, ib) as 64 lanes
 // x 4 consecutive floats, element v of lane (n, g) = S[16 ib + 4g + v][16q + n].
 #include "wkv6_chunk32.h"
@@ -31,6 +34,7 @@ struct C32FwdLds {
     float Rp[2][kC32][kLd], Kp[2][kC32][kLd], V[2][kC32][kLd];   // R', K', v of the chunk in hand and the next
     float Rm[kC32][kLd], Km[kC32][kLd];                          // R~, K~
     float Y[kC32][kLd];                                          // finished y rows on their way out
+    float Sout[kN * kN];                                         // the state at a chunk's start on its way out, in fragment order
     float A[kC32][kLa];
     float e_all[2][kN];                                          // e^{c_32}
     float ruk[4][kC32];                                          // sum_i r u k over each loading wave's channels
@@ -55,7 +59,7 @@ struct C32FwdArgs {
 
 // kOut = false: only the states (chunk states and / or the final one): no y, no R-side operands
 template <typename Tin, typename Tout, typename Ts, int kGroups, bool kOut>
-__global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32FwdArgs a)
+__global__ __launch_bounds__(512 + 256 * kGroups) void chunk32_fwd_kernel(C32FwdArgs a)
 {
     extern __shared__ __align__(16) unsigned char c32_smem[];
     C32FwdLds &L = reinterpret_cast<C32FwdSmem *>(c32_smem)->chunk;
@@ -85,7 +89,34 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
         return any != 0;
     };
 
-    if (wave >= 4) {
+    if (wave >= 4 + 4 * kGroups) {
+        // ---------------- storing waves ----------------
+        // phase 1: y rows of the chunk behind (whole 256-byte rows); phase 2: the state at the chunk's start
+        const int sw = wave - 4 - 4 * kGroups, row = 4 * sw + (lane >> 4), ch = 4 * (lane & 15);
+        auto store_y = [&](int c) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                const f32x4 o = *reinterpret_cast<const f32x4 *>(&L.Y[16 * x + row][ch]);
+                const int t = c * kC32 + 16 * x + row;
+                if (t < T) store4(y + base + (int64_t)t * C + ch, o[0], o[1], o[2], o[3]);
+            }
+        };
+        float *saved = a.saved ? a.saved + (int64_t)pair * a.slice * (kN * kN) + sw * 1024 + lane * 4 : nullptr;
+        __syncthreads();
+        for (int c = 0; c < nchunk; ++c) {
+            if (kOut && c > 0 && y) store_y(c - 1);
+            __syncthreads();
+            if (saved) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    *reinterpret_cast<f32x4 *>(saved + (int64_t)c * (kN * kN) + i * 256) = *reinterpret_cast<const f32x4 *>(&L.Sout[sw * 1024 + i * 256 + lane * 4]);
+            }
+            __syncthreads();
+        }
+        if (kOut && y) store_y(nchunk - 1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a pair that is redone has its rows written again)
+        __syncthreads();
+    } else if (wave >= 4) {
         // ---------------- loading waves ----------------
         const int grp = (wave - 4) >> 2, p = (wave - 4) & 3, t16 = lane & 15, ch = 16 * p + 4 * (lane >> 4);
         float fu[4];
@@ -222,27 +253,13 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
 #pragma unroll
             for (int ib = 0; ib < 4; ++ib) S[ib] = (f32x4){0.f, 0.f, 0.f, 0.f};
         }
-        // the y rows of a finished chunk, LDS -> global as whole 16-byte pieces (the loading waves keep to loads:
-        // loads and stores of one wave complete in no fixed order, and a store in flight would make every
-        // wait for a load a wait for everything)
-        const int t16 = lane & 15, ch = 16 * q + 4 * (lane >> 4);
-        auto store_y = [&](int c) {
-#pragma unroll
-            for (int x = 0; x < 2; ++x) {
-                const int t = c * kC32 + 16 * x + t16;
-                const f32x4 o = *reinterpret_cast<const f32x4 *>(&L.Y[16 * x + t16][ch]);
-                if (t < T) store4(y + base + (int64_t)t * C + ch, o[0], o[1], o[2], o[3]);
-            }
-        };
         if (a.arrivals && b == 0 && tid == 0) a.arrivals[h] = 0;
-        float *saved = a.saved ? a.saved + (int64_t)pair * a.slice * (kN * kN) + (q * 4) * 256 + lane * 4 : nullptr;
         __syncthreads();
         for (int c = 0; c < nchunk; ++c) {
             const int buf = c & 1;
-            if (kOut && c > 0 && y) store_y(c - 1);
-            if (saved) {
+            if (a.saved) {
 #pragma unroll
-                for (int ib = 0; ib < 4; ++ib) *reinterpret_cast<f32x4 *>(saved + (int64_t)c * (kN * kN) + ib * 256) = S[ib];
+                for (int ib = 0; ib < 4; ++ib) *reinterpret_cast<f32x4 *>(&L.Sout[(q * 4 + ib) * 256 + lane * 4]) = S[ib];
             }
             // phase 1: y = R' S, one tile of A
             f32x4 yt[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
@@ -303,7 +320,6 @@ __global__ __launch_bounds__(256 + 256 * kGroups) void chunk32_fwd_kernel(C32Fwd
             }
             __syncthreads();
         }
-        if (kOut && y) store_y(nchunk - 1);
         __syncthreads();   // (the loading waves' flags)
         // the final state (not of a pair that is redone: its initial one, which may lie in the same place, is still needed)
         if (a.sT && !redo()) {
@@ -335,7 +351,7 @@ static hipError_t launch(hipStream_t st, int64_t B, const C32FwdArgs &a) {
     constexpr int kGroups = kC32FwdGroups;
     const hipError_t e = allow_dynamic_lds<chunk32_fwd_kernel<Tin, Tout, Ts, kGroups, kOut>>(lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((chunk32_fwd_kernel<Tin, Tout, Ts, kGroups, kOut>), dim3((unsigned)(B * a.H)), dim3(256 + 256 * kGroups), lds, st, a);
+    hipLaunchKernelGGL((chunk32_fwd_kernel<Tin, Tout, Ts, kGroups, kOut>), dim3((unsigned)(B * a.H)), dim3(256 + 256 * kGroups + (a.y || a.saved ? 256 : 0)), lds, st, a);
     return hipGetLastError();
 }
 
