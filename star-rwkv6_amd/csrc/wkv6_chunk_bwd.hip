@@ -782,7 +782,7 @@ hipError_t chunk_backward_saved_segments(hipStream_t st, int64_t B, int64_t T, i
     // That is the state the FORWARD recurrence builds from zero over the segment read back to front
     // with r in the place of k and gy in the place of v, so the forward kernel's state-only pass does it.
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, r, gy, w, u, s.alone, nullptr, true, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, r, gy, w, u, s.alone, nullptr, true, s.cut, GivenStates(), s.P)
         : chunk_forward(st, kF32, rows, L, H, r, r, gy, w, u, nullptr, nullptr, nullptr, s.gstates, nullptr, nullptr, true, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) {   // (2), (3) and the sums over the segments in one launch

@@ -970,7 +970,7 @@ hipError_t chunk_forward_save_segments(hipStream_t st, int64_t B, int64_t T, int
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut, GivenStates(), s.P)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, y, nullptr, saved, true, s.cut, train_chain(s, s.states));
@@ -988,7 +988,7 @@ hipError_t chunk_forward_fused_save_segments(hipStream_t st, int64_t B, int64_t 
     const TrainSegments s = train_segments_layout(B, T, H, extra);
     const int64_t L = s.L, rows = B * s.P;
     const bool block = segments_in_block_form(rows, H);
-    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut)
+    hipError_t e = block ? segment_states(st, rows, L, H, k, v, w, u, s.alone, s.decay, false, s.cut, GivenStates(), s.P)
         : chunk_forward(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, nullptr, s.states, nullptr, s.decay, false, true, s.cut);
     if (e != hipSuccess) return e;
     if (block) return block_forward_fused(st, kF32, rows, L, H, r, k, v, w, u, nullptr, nullptr, gate, gn_scale, gn_offset, gn_eps, out, y, stats, nullptr, saved, s.cut, train_chain(s, s.states), sums);

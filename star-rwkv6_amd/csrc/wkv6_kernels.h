@@ -112,7 +112,8 @@ struct GivenStates {
 // First pass over the segments (wkv6_state.hip, bf16): the state each row of at most L tokens builds from zero and the decay over it
 // (may be null); reverse: the rows read back to front
 hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, const void *k, const void *v, const void *w, const void *u,
-                          float *states, float *decay, bool reverse, RowCut cut, const GivenStates &given = GivenStates());
+                          float *states, float *decay, bool reverse, RowCut cut, const GivenStates &given = GivenStates(),
+                          int P = 0);   // P: segments of a sequence, of which the last (reverse: the first) is not wanted (its decay is left as zero)
 
 // --- chunk-parallel MFMA form, bf16 tensors only (wkv6_chunk.hip) ---
 hipError_t chunk_forward(hipStream_t st, int state_dtype, int64_t B, int64_t T, int64_t H,
