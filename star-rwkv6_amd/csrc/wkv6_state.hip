@@ -43,6 +43,8 @@ struct StateArgs {
     int P, unused;               // the segments of a sequence, and which of them nobody asks for (P = 0: all are wanted)
 };
 
+// kUnused: a segment of every sequence is not wanted (asked at run time, prompts, of which all are, took 0.1 us longer: 18.26 / 18.35)
+template <bool kUnused>
 __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -57,7 +59,7 @@ __global__ __launch_bounds__(512) void state_kernel(StateArgs a)
     // the other direction's walk, which begins there from zero.  Half of the reading with two segments, an eighth with eight:
     // forward and backward, all passes run / so: B4 T3000 H32 (two) 236.8 / 224.1 us, B10 T1685 H12 (two) 143.3 / 136.7, B1 T3908 H48 (five) 132.3 / 129.0,
     // eight of B1 T8192 H32 165.8 / 164.7.
-    if (a.P && row % a.P == a.unused) {
+    if (kUnused && row % a.P == a.unused) {
         if (a.decay && threadIdx.x < kN) a.decay[(int64_t)pair * kN + threadIdx.x] = 0.f;
         return;
     }
@@ -207,10 +209,13 @@ hipError_t segment_states(hipStream_t st, int64_t rows, int64_t L, int64_t H, co
     a.states = states; a.decay = decay; a.given = given;
     a.P = P; a.unused = reverse ? 0 : P - 1;
     if (P && given.states) return hipErrorInvalidValue;   // (the workgroups of the first segments pass them on)
-    const hipError_t e = allow_dynamic_lds<state_kernel>(StateLds::kBytes);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(state_kernel, dim3((unsigned)(rows * H)), dim3(512), StateLds::kBytes, st, a);
-    return hipGetLastError();
+    auto launch = [&](auto kernel, hipError_t e) -> hipError_t {
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(rows * H)), dim3(512), StateLds::kBytes, st, a);
+        return hipGetLastError();
+    };
+    return P ? launch(state_kernel<true>, allow_dynamic_lds<state_kernel<true>>(StateLds::kBytes))
+             : launch(state_kernel<false>, allow_dynamic_lds<state_kernel<false>>(StateLds::kBytes));
 }
 
 }  // namespace wkv6
