@@ -170,8 +170,10 @@ int wkv6_gn_gate_backward(void *stream, int dtype, int64_t B, int64_t T, int64_t
                           const void *gout, const void *y, const float *stats, const void *gate,
                           const float *gn_scale, const float *gn_offset,
                           void *gy, void *ggate, float *gscale, float *goffset);
-/* The same pair without the launch that zeroes gscale and goffset: the forward does it on the way, and the (first) backward
- * adds to what it left. */
+/* The same pair without the launch that zeroes gscale and goffset: the forward does it on the way, and the backward adds to what
+ * it left.  ONE run of the backward to a run of the forward: a second one would add its sums to the first one's (also as a replay of
+ * a graph that holds the backward alone), and another run of the forward clears what the backward left.  Anything else takes
+ * wkv6_gn_gate_backward, which zeroes them itself and may follow either forward. */
 int wkv6_forward_gn_gate_save_sums(void *stream, int dtype, int64_t B, int64_t T, int64_t C, int64_t H,
                                    const void *r, const void *k, const void *v, const void *w, const void *u,
                                    const void *gate, const float *gn_scale, const float *gn_offset, float gn_eps,

@@ -14,6 +14,7 @@
 //  * kernels go to the current stream of the tensors' device; the interpreter's lock is not held meanwhile.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -63,6 +64,8 @@ void check(int status) {
 }
 
 void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+// whether what goes to the current stream of the current device is recorded into a graph, to run any number of times
+bool is_captured() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 const void *in(const Tensor &t) { return t.defined() ? t.const_data_ptr() : nullptr; }
 void *out(const Tensor &t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
@@ -149,9 +152,10 @@ std::vector<Tensor> wkv6_grads(const Dims &d, int algo, const Tensor &r, const T
   return g;
 }
 
-// The saved chunk states, handed from the forward to the first backward.  A second backward over the same graph
-// (retain_graph) finds none, since their counters are used up, and runs the plain backward.  (torch holds the node's
-// lock while a backward runs.)  The same goes for sums that the forward cleared.
+// The saved chunk states, handed from the forward to the first backward, which gives their memory back.  A second backward over
+// the same graph (retain_graph) finds none and runs the plain backward.  (torch holds the node's lock while a backward runs.  One
+// that is captured leaves the states as they were for its replays: each of them reads them and arms their counters again.)
+// The same goes for sums that the forward cleared, which only one run of a backward can add to: see Wkv6GnGate.
 void keep(AutogradContext *ctx, const Tensor &saved, const char *name = "states") {
   if (saved.defined()) ctx->saved_data[name] = saved;
 }
@@ -221,14 +225,19 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
     // out and what stays for the backward lie in blocks of their own: an output that a caller keeps holds nothing else
     const Tensor res = carve(r, {{{B, T, C}, r.scalar_type(), 5}})[0];
     const auto t = carve(r, {{{B, T, C}, r.scalar_type(), 6}, {{nsave}, at::kByte, 7}, {{B, T, H, 2}, at::kFloat, 0}});
-    // the norm's gradients, which this forward clears for the first backward to add to
-    const Tensor gscale = parameter_gradient(r, sc.sizes(), at::kFloat), goffset = parameter_gradient(r, of.sizes(), at::kFloat);
-    check(wkv6_forward_gn_gate_save_sums(stream_of(r), code, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gate), in_f(sc), in_f(of),
-                                         static_cast<float>(eps), out(res), out(t[0]), out_f(t[2]), out(t[1]), nsave, out_f(gscale),
-                                         out_f(goffset)));
+    if (is_captured()) {   // (each replay would clear the sums again, and with them the gradients a backward gave out)
+      check(wkv6_forward_gn_gate_save(stream_of(r), code, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gate), in_f(sc), in_f(of),
+                                      static_cast<float>(eps), out(res), out(t[0]), out_f(t[2]), out(t[1]), nsave));
+    } else {
+      // the norm's gradients, which this forward clears for the first backward to add to
+      const Tensor gscale = parameter_gradient(r, sc.sizes(), at::kFloat), goffset = parameter_gradient(r, of.sizes(), at::kFloat);
+      check(wkv6_forward_gn_gate_save_sums(stream_of(r), code, B, T, C, H, in(r), in(k), in(v), in(w), in(u), in(gate), in_f(sc), in_f(of),
+                                           static_cast<float>(eps), out(res), out(t[0]), out_f(t[2]), out(t[1]), nsave, out_f(gscale),
+                                           out_f(goffset)));
+      keep(ctx, gscale, "gscale");
+      keep(ctx, goffset, "goffset");
+    }
     keep(ctx, t[1]);
-    keep(ctx, gscale, "gscale");
-    keep(ctx, goffset, "goffset");
     ctx->saved_data["H"] = H;
     ctx->saved_data["scale_type"] = static_cast<int64_t>(scale.scalar_type());
     ctx->saved_data["offset_type"] = static_cast<int64_t>(offset.scalar_type());
@@ -248,9 +257,12 @@ struct Wkv6GnGate : torch::autograd::Function<Wkv6GnGate> {
     const ScalarType t = r.scalar_type();
     const Tensor gy = carve(r, {{{B, T, C}, t, 5}})[0];
     const Tensor ggate = carve(r, {{{B, T, C}, t, 6}})[0];
-    Tensor gscale = take(ctx, "gscale"), goffset = take(ctx, "goffset");
+    // (captured: the forward cleared its sums once, while the replays of this backward, however many follow one forward, each have to
+    // start from zero, in memory of the graph's own)
+    Tensor gscale, goffset;
+    if (!is_captured()) { gscale = take(ctx, "gscale"); goffset = take(ctx, "goffset"); }
     const auto norm_backward = gscale.defined() ? wkv6_gn_gate_backward_sums : wkv6_gn_gate_backward;
-    if (!gscale.defined()) {   // a second backward over the same graph
+    if (!gscale.defined()) {   // (also a second backward over the same graph, and one whose forward was captured)
       gscale = parameter_gradient(r, s[6].sizes(), at::kFloat);
       goffset = parameter_gradient(r, s[7].sizes(), at::kFloat);
     }
