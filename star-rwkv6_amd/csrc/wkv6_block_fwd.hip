@@ -431,7 +431,8 @@ __device__ __forceinline__ void block_output_stage_in_place(const BlockFwdArgs &
 }
 
 // kStream: large tensors, and no backward or one that comes late (past_caches): 1: r, k, v, w and the gate are read without keeping
-// their lines.  What such a call reads it reads once, and lines that stay behind only push out others.  2: y (or out) is written so, too.
+// their lines.  What such a call reads it reads once, and lines that stay behind only push out others.  2: y (or out), larger than the
+// caches, is written so, too.
 // (Two kernels: asked at run time, the two kinds of store became one.)
 // kSegments: rows that are time segments.  Built apart: asked at run time, the other ragged launches, whose
 // pointers then depend on it, took 2 % longer (prompts of B8 T999 H40: 63.1 us, so 61.7).
@@ -494,17 +495,22 @@ bool block_forward_applies(int64_t B, int64_t T, int64_t H) {
     return 2 * pairs > cus && block_grid(B, H) > 0 && T * H * kN < (1LL << 31);
 }
 
-// kStream: from 28 MiB a tensor 1, from 64 MiB 2.  Prompts, kept / 1 / 2, us: B64 T512 H32 with the output
-// stage 186.4 / 179.1 / 152.3 (5.7 TB/s), without 151.8 / 146.6 / 132.3; B16 T1024 (64 MiB) 83.9 / 71.8 / 70.8; B8 T1024 (32 MiB) 43.3 / 38.1,
-// with the output stage 51.3 / 45.8; B8 T900 (28.1 MiB) 40.0 / 37.8.  Below, inputs that other work left in the last-level cache are lost by 1: 23 MiB a
-// tensor (B5 T1184) 38.2 / 38.4, 8 MiB (B6 T350) 16.8 / 17.8; and so is an output by 2: call and a product that reads its y together, B8 T1024
-// 64.1 / 60.4 / 62.2; B16 T1024 109.0 / 99.2 / 101.2 and B64 T512 195.0 / 171.6 / 175.4, where the call by itself gains more.  With a
-// backward that reads the inputs again (keep_inputs) they stay: B8 T1024 through the state 167.3 / 169.1, the training pair 124.5 / 126.9.
-// The saving forward with the output stage reads past them as well: five tensors written and three more read lie between it and the
-// operator's backward (forward and backward B8 T1024 170.7 / 167.4, B16 T512 165.6 / 163.0, B34 T570 H12 171.9 / 167.9).
+// kStream: from 28 MiB a tensor 1, without a backward from 320 MiB 2.  What counts is the call together with what the layer does around
+// it: the projections that have just written r, k, v, w and the gate, and the kernel that reads y (the group norm) or the fused
+// stage's output (a product).  Call and reader behind the projections, kept / 1 / 2, us.  Output stage and product: B8 T1024 H32 (32 MiB) 107.5 /
+// 104.2 / 104.0, B16 T1024 (64) 214 / 191 / 198, B32 T1024 (128) 424 / 375 / 399, B64 T512 (128) 424 / 378 / 388, B48 T1024 (192) 635 / 565 /
+// 591, B56 T1200 (262) 915 / 865 / 870, B96 T1024 (384) 1261 / 1224 / 1192, B128 T1024 (512) 1666 / 1627 / 1604.  Without the stage and an elementwise reader: B8
+// T1024 60.2 / 58.3 / 58.2, B16 118 / 103 / 102, B64 T512 230 / 200 / 203, B48 350 / 298 / 295, B56 T1200 471 / 435 / 413, B96 682 / 678 / 599.  An output that
+// the last-level cache (256 MB) can hold belongs there, also where the call by itself, repeated on inputs that nobody has just
+// written, would be faster without: B64 T512 186 / 175 / 151, without the output stage 155 / 140 / 132.
+// Below 28 MiB, inputs that other work left in the last-level cache are lost by 1: 23 MiB a tensor (B5 T1184) 38.2 / 38.4, 8 MiB (B6 T350)
+// 16.8 / 17.8.  With a backward that reads the inputs again (keep_inputs) they stay: B8 T1024 through the state 150.3 / 152.5, the
+// training pair 124.5 / 126.9.  The saving forward with the output stage reads past the caches as well, since five tensors written
+// and three more read lie between it and the operator's backward (forward and backward B8 T1024 170.7 / 167.4, B16 T512 165.6 / 163.0, B34 T570
+// H12 171.9 / 167.9), and keeps its output: forward, product and backward, 1 / 2: B16 T1024 447.5 / 450.2, B12 T1000 H48 590.6 / 593.6.
 static int past_caches(int64_t B, int64_t T, int64_t H) {
     const int64_t bytes = B * T * H * kN * 2;
-    return bytes >= (64LL << 20) ? 2 : bytes >= (28LL << 20) ? 1 : 0;
+    return bytes >= (320LL << 20) ? 2 : bytes >= (28LL << 20) ? 1 : 0;
 }
 
 // gate != null: the fused output stage (out = (group norm of y) * gate; y and stats only where given)
@@ -535,11 +541,12 @@ static hipError_t block_forward_launch(hipStream_t st, int state_dtype, int64_t 
         return hipGetLastError();
     };
     auto launch = [&](auto ts_tag, auto save_tag, auto ragged_tag, auto fuse_tag, auto segments_tag) -> hipError_t {
-        if constexpr ((!decltype(save_tag)::value || decltype(fuse_tag)::value) && !decltype(segments_tag)::value)
-            switch (keep_inputs ? 0 : past_caches(B, T, H)) {
-            case 1: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 1>{});
-            case 2: return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 2>{});
-            }
+        if constexpr ((!decltype(save_tag)::value || decltype(fuse_tag)::value) && !decltype(segments_tag)::value) {
+            const int stream = keep_inputs ? 0 : past_caches(B, T, H);
+            if constexpr (!decltype(save_tag)::value)
+                if (stream == 2) return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 2>{});
+            if (stream) return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 1>{});
+        }
         return launch_as(ts_tag, save_tag, ragged_tag, fuse_tag, segments_tag, std::integral_constant<int, 0>{});
     };
     auto launch_ts = [&](auto ts_tag, auto save_tag, auto fuse_tag) -> hipError_t {

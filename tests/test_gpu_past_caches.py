@@ -49,3 +49,36 @@ def test_large_calls_give_the_bits_of_small_ones(op, B, few, T, H, sdt, fused):
     y, s = call(B)
     y_few, s_few = call(few)
     assert torch.equal(y[:few], y_few) and torch.equal(s[:few], s_few)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_outputs_larger_than_the_caches(op, fused):
+    # 323 MiB a tensor, a ragged end: y or the fused output is written past the caches, too
+    test_large_calls_give_the_bits_of_small_ones(op, 81, 6, 1023, 32, torch.float32, fused)
+
+
+# (several pairs to a workgroup in both calls: the backward of one pair to a workgroup is another kernel, whose gw rounds differently)
+@pytest.mark.parametrize("B,few,T,H", [(15, 10, 500, 32),     # 29.3 MiB, a ragged end
+                                       (43, 12, 401, 32),     # 67.4 MiB
+                                       (33, 11, 512, 32)])    # 66 MiB, whole chunks
+def test_large_training_calls_with_the_output_stage(op, B, few, T, H):
+    # the saving forward reads past the caches: the output and every row's gradients as in a call below the limit
+    assert few * T * H * N * 2 < 28 * MIB <= B * T * H * N * 2
+    g = torch.Generator(device="cuda").manual_seed(B)
+
+    def normal(*shape, dtype=torch.bfloat16):
+        return torch.randn(*shape, generator=g, device="cuda").to(dtype)
+
+    C = H * N
+    r, k, v, gate, gout = (normal(B, T, C) for _ in range(5))
+    w = (torch.rand(B, T, C, generator=g, device="cuda") * 7 - 6).bfloat16()
+    w[2, T // 2:, :N] = 6.0    # a pair that is redone one timestep at a time
+    u, scale, offset = normal(H, N), normal(H, N, dtype=torch.float32), normal(H, N, dtype=torch.float32)
+
+    def call(n):
+        rows = [x[:n].clone().requires_grad_(True) for x in (r, k, v, w, gate)]
+        out, _ = op.forward_gn_gate(*rows[:4], u, rows[4], scale, offset)
+        return [out, *torch.autograd.grad(out, rows, gout[:n].contiguous())]
+
+    for name, a, b in zip("out gr gk gv gw ggate".split(), call(B), call(few)):
+        assert torch.equal(a[:few], b), name
