@@ -106,15 +106,25 @@ int wkv6_forward_with_state_ex(void *stream, int dtype, int state_dtype, int alg
                                const void *r, const void *k, const void *v, const void *w, const void *u,
                                const void *s, void *y, void *ys,
                                void *workspace, size_t workspace_bytes);
-/* The same call and results, for a caller whose next use of r, k, v and w is the backward: large calls
- * otherwise read them past the caches.  No counterpart in the reference. */
+/* The same call and results (s, state_map and ys may be NULL as there) where no backward follows: r, k, v and w of large calls
+ * (bf16, from 28 MiB a tensor) are read past the caches, which is 8 to 12 % faster, and y from 320 MiB on is written past them.  Every
+ * other forward leaves them in the caches for the backward, which would take longer by more than that (forward and backward
+ * B8 T1024 C2048, pair without saved states, 148.7 / 151.2 us), but for those that have none: wkv6_forward_gn_gate and, like the reference's own
+ * (rwkv_kernel/torch_rwkv_kernel.py:145-168), wkv6_forward_with_state.  No counterpart in the reference. */
+int wkv6_forward_inference(void *stream, int dtype, int state_dtype, int algo,
+                           int64_t B, int64_t T, int64_t C, int64_t H,
+                           int has_init_state, const int64_t *state_map,
+                           const void *r, const void *k, const void *v, const void *w, const void *u,
+                           const void *s, void *y, void *ys,
+                           void *workspace, size_t workspace_bytes);
+/* wkv6_forward_with_state_ex by another name. */
 int wkv6_forward_with_state_for_backward(void *stream, int dtype, int state_dtype, int algo,
                                          int64_t B, int64_t T, int64_t C, int64_t H,
                                          int has_init_state, const int64_t *state_map,
                                          const void *r, const void *k, const void *v, const void *w, const void *u,
                                          const void *s, void *y, void *ys,
                                          void *workspace, size_t workspace_bytes);
-/* Optional workspace of wkv6_forward_ex / wkv6_forward_with_state_ex (0 = none useful).  Where it is
+/* Optional workspace of wkv6_forward_ex / wkv6_forward_with_state_ex / wkv6_forward_inference (0 = none useful).  Where it is
  * non-zero -- a long bf16 sequence with so few (batch, head) pairs that most of the chip would idle --
  * passing that many bytes lets the forward run as time segments side by side (same results to
  * rounding); without it the call works as always.  Batches need T to divide into equal segments

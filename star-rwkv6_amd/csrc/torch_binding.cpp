@@ -190,7 +190,9 @@ struct Wkv6 : torch::autograd::Function<Wkv6> {
       // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
       const size_t n = wkv6_forward_workspace_bytes_any_length(code, algo, B, T, C, H);
       const Tensor ws = bytes(r, n);
-      check(wkv6_forward_ex(stream_of(r), code, algo, B, T, C, H, in(r), in(k), in(v), in(w), in(u), out(y), out(ws), n));
+      // (no gradient is wanted, or the per-timestep kernels run, which read their inputs in one way only)
+      check(wkv6_forward_inference(stream_of(r), code, code_of(out_type(r.scalar_type())), algo, B, T, C, H, 0, nullptr, in(r), in(k), in(v),
+                                   in(w), in(u), nullptr, out(y), nullptr, out(ws), n));
     }
     ctx->saved_data["H"] = H;
     ctx->saved_data["algo"] = algo;
@@ -352,7 +354,7 @@ std::pair<Tensor, Tensor> forward_with_state(int64_t H, const Tensor &map, const
   // optional workspace: a long sequence of few (batch, head) pairs runs as time segments
   const size_t n = wkv6_forward_workspace_bytes_any_length(code, algo, B, T, C, H);
   const Tensor ws = bytes(r, n);
-  const auto forward = backward_follows ? wkv6_forward_with_state_for_backward : wkv6_forward_with_state_ex;
+  const auto forward = backward_follows ? wkv6_forward_with_state_ex : wkv6_forward_inference;
   check(forward(stream_of(r), code, code_of(st), algo, B, T, C, H, s0.defined(), static_cast<const int64_t *>(in(map)), in(r), in(k),
                 in(v), in(w), in(u), in(s0), out(y), out(ys), out(ws), n));
   return {y, ys};

@@ -135,7 +135,7 @@ static int forward_impl(void *stream, int dtype, int state_dtype, int algo,
                         int has_init_state, const int64_t *state_map,
                         const void *r, const void *k, const void *v, const void *w, const void *u,
                         const void *s, void *y, void *ys, void *saved,
-                        void *workspace = nullptr, size_t workspace_bytes = 0, bool keep_inputs = false) {
+                        void *workspace = nullptr, size_t workspace_bytes = 0, bool keep_inputs = true) {
     int rc = check_shape_any(dtype, B, T, C, H);
     if (rc != WKV6_OK && rc != kSmallHead) return rc;
     if (!r || !k || !v || !w || !u || !y) return WKV6_ERR_ARG;
@@ -177,8 +177,17 @@ int wkv6_forward_with_state_for_backward(void *stream, int dtype, int state_dtyp
                                          int has_init_state, const int64_t *state_map,
                                          const void *r, const void *k, const void *v, const void *w, const void *u,
                                          const void *s, void *y, void *ys, void *workspace, size_t workspace_bytes) {
+    return wkv6_forward_with_state_ex(stream, dtype, state_dtype, algo, B, T, C, H, has_init_state, state_map, r, k, v, w, u, s, y, ys,
+                                      workspace, workspace_bytes);
+}
+
+int wkv6_forward_inference(void *stream, int dtype, int state_dtype, int algo,
+                           int64_t B, int64_t T, int64_t C, int64_t H,
+                           int has_init_state, const int64_t *state_map,
+                           const void *r, const void *k, const void *v, const void *w, const void *u,
+                           const void *s, void *y, void *ys, void *workspace, size_t workspace_bytes) {
     return forward_impl(stream, dtype, state_dtype, algo, B, T, C, H, has_init_state, state_map, r, k, v, w, u, s, y, ys,
-                        nullptr, workspace, workspace_bytes, true);
+                        nullptr, workspace, workspace_bytes, false);
 }
 
 int wkv6_forward_gn_gate(void *stream, int dtype, int state_dtype,
@@ -472,8 +481,8 @@ int wkv6_forward_with_state(void *stream, int dtype, int64_t B, int64_t T, int64
                             const void *r, const void *k, const void *v, const void *w, const void *u,
                             const void *s, void *y, void *ys) {
     if (!ys) return WKV6_ERR_ARG;
-    return wkv6_forward_with_state_ex(stream, dtype, out_type(dtype), WKV6_ALGO_AUTO, B, T, C, H, has_init_state,
-                                      state_map, r, k, v, w, u, s, y, ys, nullptr, 0);
+    return wkv6_forward_inference(stream, dtype, out_type(dtype), WKV6_ALGO_AUTO, B, T, C, H, has_init_state,
+                                  state_map, r, k, v, w, u, s, y, ys, nullptr, 0);
 }
 
 int wkv6_forward_ex(void *stream, int dtype, int algo, int64_t B, int64_t T, int64_t C, int64_t H,

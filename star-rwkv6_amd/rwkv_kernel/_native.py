@@ -27,6 +27,7 @@ SIGNATURES = {
     "wkv6_forward_with_state": (_int, [_p, _int] + [_i64] * 4 + [_int, _p] + [_p] * 8),
     "wkv6_forward_with_state_ex": (_int, [_p, _int, _int, _int] + [_i64] * 4 + [_int, _p] + [_p] * 8 + [_p, _sz]),
     "wkv6_forward_with_state_for_backward": (_int, [_p, _int, _int, _int] + [_i64] * 4 + [_int, _p] + [_p] * 8 + [_p, _sz]),
+    "wkv6_forward_inference": (_int, [_p, _int, _int, _int] + [_i64] * 4 + [_int, _p] + [_p] * 8 + [_p, _sz]),
     "wkv6_forward_workspace_bytes": (_sz, [_int, _int] + [_i64] * 4),
     "wkv6_forward_workspace_bytes_any_length": (_sz, [_int, _int] + [_i64] * 4),
     "wkv6_forward_gn_gate": (_int, [_p, _int, _int] + [_i64] * 4 + [_int, _p] + [_p] * 9 + [ctypes.c_float, _p, _p]),

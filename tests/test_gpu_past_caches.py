@@ -82,3 +82,36 @@ def test_large_training_calls_with_the_output_stage(op, B, few, T, H):
 
     for name, a, b in zip("out gr gk gv gw ggate".split(), call(B), call(few)):
         assert torch.equal(a[:few], b), name
+
+
+@pytest.mark.parametrize("B,T,H", [(9, 800, 32), (3, 100, 4)])   # past the caches, and a call of which no form asks
+@pytest.mark.parametrize("sdt", [torch.float32, torch.bfloat16])
+def test_inference_is_the_stateful_call(B, T, H, sdt):
+    from rwkv_kernel import _native
+
+    lib, C = _native.load(), H * N
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r, k, v = (torch.randn(B, T, C, generator=g, device="cuda").bfloat16() for _ in range(3))
+    w = (torch.rand(B, T, C, generator=g, device="cuda") * 7 - 6).bfloat16()
+    u, s = torch.randn(H, N, generator=g, device="cuda").bfloat16(), torch.randn(B, H, N, N, generator=g, device="cuda").to(sdt)
+    code = {torch.float32: _native.F32, torch.bfloat16: _native.BF16}[sdt]
+    P = lambda t: None if t is None else t.data_ptr()
+
+    def call(entry, has, y, ys):
+        return entry(torch.cuda.current_stream().cuda_stream, _native.BF16, code, _native.ALGO_AUTO, B, T, C, H, has, None, P(r), P(k), P(v), P(w),
+                     P(u), P(s) if has else None, P(y), P(ys), None, 0)
+
+    entries = (lib.wkv6_forward_inference, lib.wkv6_forward_with_state_ex, lib.wkv6_forward_with_state_for_backward)
+    for has in (0, 1):
+        got = []
+        for entry in entries:
+            y, ys = torch.full_like(r, float("nan")), torch.full_like(s, float("nan"))
+            _native.check(call(entry, has, y, ys))
+            y2 = torch.full_like(r, float("nan"))
+            _native.check(call(entry, has, y2, None))        # (the final state is not wanted)
+            assert torch.equal(y, y2)
+            got.append((y, ys))
+        for y, ys in got[1:]:
+            assert torch.equal(y, got[0][0]) and torch.equal(ys, got[0][1])
+    for entry in entries:   # refused alike
+        assert call(entry, 1, None, s) == call(entries[1], 1, None, s) != 0
