@@ -188,6 +188,12 @@ __device__ __forceinline__ void unpack4(const s16x4 &a, float (&o)[4]) {
     o[0] = __uint_as_float(t[0] << 16); o[1] = __uint_as_float(t[0] & 0xffff0000u);
     o[2] = __uint_as_float(t[1] << 16); o[3] = __uint_as_float(t[1] & 0xffff0000u);
 }
+// what rounding to bf16 takes off
+__device__ __forceinline__ f32x4 rounded_off(const f32x4 &a) {
+    float hi[4];
+    unpack4(pack4(a), hi);
+    return (f32x4){a[0] - hi[0], a[1] - hi[1], a[2] - hi[2], a[3] - hi[3]};
+}
 __device__ __forceinline__ void unpack8(const bf16x8 &a, float (&o)[8]) {
     const u32x4 t = __builtin_bit_cast(u32x4, a);
 #pragma unroll

@@ -73,3 +73,28 @@ def test_any_length(oracle, B, T, H, segments, fused, sdt):
     assert torch.equal(y, y2) and torch.equal(sT, sT2)
     y3, sT3 = run(s_all, s_all, None, n)
     assert torch.equal(y, y3) and torch.equal(sT, sT3)
+
+
+@pytest.mark.parametrize("B,T,H", [(2, 330, 16), (2, 1000, 8), (3, 705, 16), (7, 577, 12), (1, 1337, 32), (2, 1300, 64)])
+def test_segments_are_no_less_exact_than_one_piece(oracle, B, T, H):
+    # segments run the block form, one piece of so few pairs the tile form.  y of many thousands of values: the 2-norm of its error
+    # differs by 0.2 % from seed to seed, the two forms' on the same inputs by less than that around their own difference
+    from rwkv_kernel import _native
+
+    lib, C = _native.load(), H * N
+    dev, ref = cast_inputs(oracle.make_inputs(B, T, H, N, 60 + B)[:5], torch.bfloat16)
+    n = int(lib.wkv6_forward_workspace_bytes_any_length(_native.BF16, CHUNK, B, T, C, H))
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    P = lambda t: t.data_ptr()
+
+    def run(size):
+        y, sT = torch.empty_like(dev[0]), torch.empty(B, H, N, N, device="cuda")
+        _native.check(lib.wkv6_forward_with_state_ex(torch.cuda.current_stream().cuda_stream, _native.BF16, _native.F32, CHUNK, B, T, C, H, 0, None,
+                                                     *map(P, dev), None, P(y), P(sT), P(ws), size))
+        return to_np(y), to_np(sT)
+
+    y_ref, s_ref = oracle.forward_c(*ref, N)
+    (y, s), (y1, s1) = run(n), run(0)
+    assert n > 0 and not np.array_equal(y, y1)
+    assert rel_l2(y, y_ref) <= rel_l2(y1, y_ref)
+    assert rel_l2(s, s_ref) <= 1.001 * rel_l2(s1, s_ref)   # (the same roundings in another order of additions)
