@@ -842,13 +842,28 @@ RowCut cut_of(int P, int64_t L, int64_t T) {
 // for the chain's rounding, that of a call in one piece.
 bool segments_in_block_form(int64_t rows, int64_t H) { return 4 * rows * H >= compute_units(); }
 
-// Prompts, in one piece / in segments, us.  Four segments and more pay from the first length that has them: B1 H32 T200 11.2 / 10.6, T300
-// 13.0 / 10.9, B2 H16 T330 14.7 / 11.2, T520 19.8 / 13.3, B2 T1000 H8 30.8 / 13.1, B3 T4097 H12 114 / 41.  Three: B3 H28 T330 15.4 / 16.3, T450 18.8 /
-// 19.0, T530 20.5 / 19.4, T700 24.0 / 21.4.  Two: B2 H64 T800 28.7 / 30.8, T1100 37.4 / 37.3, B4 H32 T1500 49.2 / 47.6, T2200 68.8 / 66.0.
-// With the output stage, which the first pass leaves out: four B1 H32 T200 14.6 / 11.7, B2 T2052 H16 102 / 25; three B3 H28 T200 15.3 / 16.0,
-// T260 18.3 / 16.8; two B2 H64 T330 22.5 / 19.3, T500 28.9 / 23.0.
-static bool prompt_takes(int P, int64_t T, bool fused) {
-    return P >= 4 || (P == 3 ? T >= (fused ? 256 : 512) : P == 2 && T >= (fused ? 320 : 1280));
+// From which length a prompt of `pairs` (batch, head) pairs runs in P segments.  Two things move the line besides P and the output stage,
+// which the first pass leaves out.  A prompt of whole chunks runs in one piece on kernels without the checks of a ragged end, and pays later.
+// And the workgroups of a head's segments, H apart in the grid, are on one XCD, where the second pass finds the first one's states in
+// the L2, only if H is a multiple of 8 (else on two, and of four or eight where H is no multiple of 4).  In one piece / in segments, us:
+//   four and more     B1 H32 T200 11.2 / 10.6, B2 H32 T256 12.5 / 11.6, few pairs B2 H8 T256 9.7 / 10.4; B4 H12 T256 11.6 / 12.3, T257 13.6 / 13.1;
+//                     B4 H14 T256 12.1 / 14.4, B4 H10 T384 14.3 / 15.0, T448 16.0 / 15.3, B6 H10 T448 17.3 / 17.7, but B2 H14 T384 13.7 / 13.1
+//   three             B4 H20 T512 18.1 / 19.2, T576 19.8 / 19.5; B6 H14 T640 21.6 / 22.0; B3 H28 T530 20.5 / 19.4, T700 24.0 / 21.4
+//   two               B2 H64 T1344 42.4 / 43.1, T1100 37.4 / 37.3; B6 H20 T1280 39.6 / 40.4, B4 H32 T1500 49.2 / 47.6
+//   with the stage    four B1 H32 T200 14.6 / 11.7, B3 H20 T256 13.8 / 14.8, B4 H14 T256 13.6 / 15.8; three B3 H28 T320 16.5 / 17.5, T260 18.3 / 16.8;
+//                     two B2 H64 T320 17.4 / 19.4, T330 22.5 / 19.3, B4 H30 T448 22.0 / 23.1
+static bool prompt_takes(int P, int64_t T, int64_t pairs, int64_t H, bool fused) {
+    struct Least { int ragged, whole; };
+    static constexpr Least kLeast[3][2][3] = {   // two segments, three, four and more; without and with the output stage; H a multiple of 8, of 4, others
+        {{{1281, 1408}, {1281, 1408}, {1281, 1408}}, {{321, 384}, {321, 512}, {321, 512}}},
+        {{{513, 512}, {513, 576}, {513, 704}}, {{257, 320}, {257, 384}, {257, 384}}},
+        {{{193, 256}, {257, 320}, {385, 512}}, {{193, 256}, {193, 320}, {257, 384}}}};
+    if (P < 2) return false;
+    const int heads = H % 8 == 0 ? 0 : H % 4 == 0 ? 1 : 2;
+    Least l = kLeast[P >= 4 ? 2 : P - 2][fused][heads];
+    if (P >= 4 && !fused && heads == 0 && pairs <= 16) l = {257, 320};
+    if (P >= 4 && !fused && heads == 2 && pairs <= 32) l.whole = 384;
+    return T >= (T % CL == 0 ? l.whole : l.ragged);
 }
 // any_length: a batch's length need not divide into the segments, either.  Without it (wkv6_forward_workspace_bytes, which promises
 // no workspace then) a batch of prompts ran as segments only where 16, 8, 4 or 2 equal ones of whole chunks make its length,
@@ -856,13 +871,13 @@ static bool prompt_takes(int P, int64_t T, bool fused) {
 static int forward_segments_plan(int64_t B, int64_t T, int64_t H, bool fused, bool any_length, int64_t *L) {
     if (B == 1 || any_length) {
         int P = plan_segments(B * H, T, 1, L);
-        if (P > 1 && segments_in_block_form(B * P, H)) return prompt_takes(P, T, fused) ? P : 1;
+        if (P > 1 && segments_in_block_form(B * P, H)) return prompt_takes(P, T, B * H, H, fused) ? P : 1;
         P = T >= 1024 ? plan_segments(B * H, T, 3, L) : 1;
         return P >= 4 ? P : 1;
     }
     for (int P = kMostSegments; P >= 2; P >>= 1)
         if (B * H * P <= compute_units() && T % (P * CL) == 0 &&
-            (segments_in_block_form(B * P, H) ? prompt_takes(P, T, fused) : T >= 1024 && P >= 4 && T / P >= 4 * CL)) {
+            (segments_in_block_form(B * P, H) ? prompt_takes(P, T, B * H, H, fused) : T >= 1024 && P >= 4 && T / P >= 4 * CL)) {
             *L = T / P;
             return P;
         }

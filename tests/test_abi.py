@@ -196,3 +196,21 @@ def test_state_chain_keeps_its_values_in_registers(native, tmp_path):
     a loop that does not unroll puts the values into scratch memory (and takes twice the time)."""
     kernels = {k: v for k, v in _scratch_bytes(native.LIB_PATH, tmp_path).items() if "segment_chain_kernel" in k}
     assert kernels and not any(kernels.values()), kernels
+
+
+@pytest.mark.parametrize("B,T,H,segments", [(4, 320, 32, 0), (4, 321, 32, 2), (4, 384, 32, 2), (4, 384, 30, 0), (4, 385, 30, 2), (3, 320, 28, 0), (3, 319, 28, 3),
+                                            (4, 256, 14, 0), (4, 257, 14, 3), (4, 256, 20, 0), (4, 256, 16, 4), (1, 200, 32, 4), (1, 192, 32, 0)])
+def test_prompts_take_segments_where_they_pay(native, B, T, H, segments):
+    # lengths of whole chunks and heads that are no multiple of 8 are faster in one piece for longer
+    lib = native.load()
+    n = int(lib.wkv6_forward_workspace_bytes_any_length(native.BF16, native.ALGO_CHUNK, B, T, 64 * H, H))
+    assert n == B * segments * H * (2 * 64 * 64 + 64) * 4
+
+
+def test_workspace_of_any_length_is_enough_for_equal_segments(native):
+    lib = native.load()
+    for H in (1, 2, 3, 5, 8, 10, 12, 16, 20, 28, 30, 32, 60, 64):
+        for B in range(1, 128 // H + 1):
+            for T in list(range(64, 2112, 64)) + [333, 1000, 4096]:
+                query = (native.BF16, native.ALGO_CHUNK, B, T, 64 * H, H)
+                assert lib.wkv6_forward_workspace_bytes_any_length(*query) >= lib.wkv6_forward_workspace_bytes(*query), query
