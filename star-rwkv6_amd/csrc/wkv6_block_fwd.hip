@@ -88,7 +88,9 @@ __device__ __forceinline__ float sum_row8(float x) {
 // Prompts in segments (kSegments without kSave): what the rounding to bf16 takes off A01, the products between a block's two groups of 16
 // tokens, is multiplied by v as well.  The same prompts in one piece run the tile form, where those products go through the state;
 // with A01 as one bf16 operand y of a prompt in segments was 0.3 to 0.8 % further from float64 than in one piece (2-norm, B7 T577 H12 3.231e-3 /
-// 3.208e-3).  Larger calls run the block form in one piece, too, and stay as they are.
+// 3.208e-3), with it 0.5 to 0.9 % nearer (3.193e-3).  As a 16x16x32 product on the accumulator of the one before it 0 to 0.8 % of the call's time (B1 T1337 H32
+// 18.25 / 18.34 us, B7 T5063 H12 93.1 / 93.5); as a 16x16x16 product into registers of its own, added up behind, up to 2 %.  Larger calls run the
+// block form in one piece, too, and stay as they are.
 template <typename Ts, bool kSave, bool kFuse, bool kSegments>
 __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsigned char *smem, const int *s_wild, int pair0, int q, int lane)
 {
@@ -181,13 +183,10 @@ __device__ __forceinline__ void block_fwd_consumer(const BlockFwdArgs &a, unsign
                 Y0 = mfma16(vf0, pack4(A00), Y0);
                 Y1 = mfma32(both16(vf0, vf1), acc_as_operand(A01, A11), Y1);
                 if (kSegments && !kSave) {
-                    f32x4 Yrest = mfma16(vf0, pack4(rounded_off(A01)), zero);
-                    settle(Y0, Y1, Yrest);
-#pragma unroll
-                    for (int rr = 0; rr < 4; ++rr) Y1[rr] += Yrest[rr];
-                } else {
-                    settle(Y0, Y1);
+                    // (a 16x16x32 product like the one before it, on the same accumulator)
+                    Y1 = mfma32(both16(vf0, vf0), both16(pack4(rounded_off(A01)), make_s16x4(0, 0)), Y1);
                 }
+                settle(Y0, Y1);
                 *reinterpret_cast<uint2 *>(ys + tile_off(r0, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y0[0], Y0[1]), pack_bf16x2(Y0[2], Y0[3]));
                 *reinterpret_cast<uint2 *>(ys + tile_off(r1, 16 * q + 4 * g)) = make_uint2(pack_bf16x2(Y1[0], Y1[1]), pack_bf16x2(Y1[2], Y1[3]));
             }
