@@ -7,13 +7,35 @@ pytestmark = pytest.mark.gpu
 N = 64
 
 
-@pytest.mark.parametrize("B,T,H", [(1, 70, 3),        # tile form, a pair to a workgroup
-                                   (3, 64, 100),      # tile form, several pairs to a workgroup
-                                   (5, 150, 32),      # block form
-                                   (9, 150, 32),      # block form, two pairs to a workgroup
-                                   (1, 1100, 2),      # segments in tile form
-                                   (2, 1100, 8),      # segments in block form
-                                   (9, 800, 32)])     # inputs read past the caches
+SHAPES = [(1, 70, 3),        # tile form, a pair to a workgroup
+          (3, 64, 100),      # tile form, several pairs to a workgroup
+          (5, 150, 32),      # block form
+          (9, 150, 32),      # block form, two pairs to a workgroup
+          (1, 1100, 2),      # segments in tile form
+          (2, 1100, 8),      # segments in block form
+          (9, 800, 32)]     # inputs read past the caches
+
+
+@pytest.mark.parametrize("B,T,H", SHAPES)
+def test_the_forward_clears_the_sums(B, T, H):
+    from rwkv_kernel import _native
+
+    lib, C = _native.load(), H * N
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r, k, v, gate = (torch.randn(B, T, C, generator=g, device="cuda").bfloat16() for _ in range(4))
+    w = (torch.rand(B, T, C, generator=g, device="cuda") * 7 - 6).bfloat16()
+    u, scale, offset = torch.randn(H, N, device="cuda").bfloat16(), torch.randn(H, N, device="cuda"), torch.randn(H, N, device="cuda")
+    n = int(lib.wkv6_saved_bytes(_native.BF16, _native.ALGO_CHUNK, B, T, C, H))
+    out, y, stats, saved = torch.empty_like(r), torch.empty_like(r), torch.empty(B, T, H, 2, device="cuda"), torch.empty(n, dtype=torch.uint8, device="cuda")
+    sums = torch.full((4, H, N), float("nan"), device="cuda")
+    P = lambda t: t.data_ptr()
+    _native.check(lib.wkv6_forward_gn_gate_save_sums(torch.cuda.current_stream().cuda_stream, _native.BF16, B, T, C, H, P(r), P(k), P(v), P(w), P(u),
+                                                     P(gate), P(scale), P(offset), 64e-5, P(out), P(y), P(stats), P(saved), n, P(sums[1]), P(sums[2])))
+    torch.cuda.synchronize()
+    assert (sums[1:3] == 0).all() and torch.isnan(sums[0]).all() and torch.isnan(sums[3]).all()
+
+
+@pytest.mark.parametrize("B,T,H", SHAPES)
 def test_first_and_second_backward_give_the_same_sums(B, T, H):
     import rwkv_kernel
 
@@ -28,8 +50,9 @@ def test_first_and_second_backward_give_the_same_sums(B, T, H):
     u, scale, offset = normal(H, N), normal(H, N, dtype=torch.float32), normal(H, N, dtype=torch.float32)
     scale.requires_grad_(True)
     offset.requires_grad_(True)
-    torch.full((4 << 20,), float("nan"), device="cuda")   # (what the allocator hands out next is not zero)
     for _ in range(2):
+        poison = [torch.full((H, N), float("nan"), device="cuda") for _ in range(8)]   # (what the allocator hands out next for a sum is not zero)
+        del poison
         out, _ = op.forward_gn_gate(r, k, v, w, u, gate, scale, offset)
         first = torch.autograd.grad(out, [scale, offset], gout, retain_graph=True)
         second = torch.autograd.grad(out, [scale, offset], gout)

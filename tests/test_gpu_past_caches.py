@@ -1,4 +1,4 @@
-"""Large calls without a backward read their inputs and write their output past the caches: the same bits as smaller calls."""
+"""Large calls without a backward read their inputs past the caches, the largest write their output past them: the same bits as smaller calls."""
 import pytest
 import torch
 
@@ -17,11 +17,11 @@ def op():
 
 
 # A pair's result does not depend on the pairs around it, so the first `few` rows by themselves, a call that stays below the limits
-# (28 MiB a tensor for what is read, 64 MiB for what is written), have to be what they are among all rows.
+# (28 MiB a tensor for what is read, 320 MiB for what is written), have to be what they are among all rows.
 @pytest.mark.parametrize("B,few,T,H,sdt", [(9, 8, 800, 32, torch.float32),      # read past the caches, 28.1 MiB; several pairs to a workgroup
                                            (8, 7, 897, 32, torch.bfloat16),     # one pair to a workgroup and a chunk of one token, 28.0 MiB
-                                           (20, 8, 820, 32, torch.float32),     # written past them, too: 64.1 MiB, a ragged end
-                                           (65, 16, 320, 24, torch.float32),    # 60.9 MiB: read only; heads that do not divide the chip
+                                           (20, 8, 820, 32, torch.float32),     # 64.1 MiB, a ragged end
+                                           (65, 16, 320, 24, torch.float32),    # 60.9 MiB, heads that do not divide the chip
                                            (37, 8, 448, 32, None)])             # 64.75 MiB, without a state
 @pytest.mark.parametrize("fused", [False, True])
 def test_large_calls_give_the_bits_of_small_ones(op, B, few, T, H, sdt, fused):
