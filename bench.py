@@ -148,8 +148,8 @@ def bench_stateful(a):
     P = lambda t: t.data_ptr()
 
     def call(x, T, y, si, so):
-        _native.check(lib.wkv6_forward_with_state_ex(st, _native.BF16, _native.F32, _native.ALGO_AUTO, B, T, C, H, 1, None,
-                                                     P(x[0]), P(x[1]), P(x[2]), P(x[3]), P(u), P(si), P(y), P(so), None, 0))
+        _native.check(lib.wkv6_forward_inference(st, _native.BF16, _native.F32, _native.ALGO_AUTO, B, T, C, H, 1, None,
+                                                 P(x[0]), P(x[1]), P(x[2]), P(x[3]), P(u), P(si), P(y), P(so), None, 0))
 
     def timed(fn, reps):
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -183,9 +183,9 @@ def bench_stateful(a):
     ws = torch.empty(max(n_ws, 16), dtype=torch.uint8, device=dev)
 
     def solo_call(use_ws):
-        _native.check(lib.wkv6_forward_with_state_ex(st, _native.BF16, _native.F32, _native.ALGO_AUTO, 1, T1, C, H, 1, None,
-                                                     P(solo[0]), P(solo[1]), P(solo[2]), P(solo[3]), P(u), P(s_solo), P(y_solo),
-                                                     P(s_solo_out), P(ws) if use_ws else None, n_ws if use_ws else 0))
+        _native.check(lib.wkv6_forward_inference(st, _native.BF16, _native.F32, _native.ALGO_AUTO, 1, T1, C, H, 1, None,
+                                                 P(solo[0]), P(solo[1]), P(solo[2]), P(solo[3]), P(u), P(s_solo), P(y_solo),
+                                                 P(s_solo_out), P(ws) if use_ws else None, n_ws if use_ws else 0))
 
     solo_one_ms = timed(lambda: solo_call(False), 20)
     solo_seg_ms = timed(lambda: solo_call(True), 20) if n_ws else None
