@@ -14,8 +14,8 @@
 // workgroup, so the gradients g_s are read twice: mix_reduce_kernel<grad> takes whole rows of a few tokens (gpre
 // complete, nothing to combine between workgroups), mix_grads_kernel takes 64 channels of many tokens (the weight
 // gradients stay in accumulators, one partial per workgroup).
-// B8 T1024 C2048, forward and backward: 182 us of kernels at R32 (x and the gradients read twice more than once: 501 MB in, 232 MB
-// out), 393 us at R64; R32 as four elementwise kernels around six library products (gcoef written and read twice, x_mix
+// B8 T1024 C2048, forward and backward: 178 us of kernels at R32 (x and the gradients read twice more than once: 501 MB in, 232 MB
+// out), 381 us at R64; R32 as four elementwise kernels around six library products (gcoef written and read twice, x_mix
 // written and read) 504 us, of which 235 us the skinny products.
 #include "wkv6_common.h"
 #include "wkv6_kernels.h"
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kReduceWaves * 64) void mix_reduce_kernel(int64_t n
 // traffic alone, 256 MB, would take 50 us; the roles alone take 45, 44 and 32 us: vector instructions and LDS on top.)
 // R = 64: the W and A waves hold accumulators for half of the rank's columns, a second launch without gx waves (kGx false) does the
 // other half.  The gx waves need all of them: a step of the first launch has two parts of 160 columns (32 of each mixer) that go
-// through the same two tiles as at R = 32, and gxx and gxm take each part's share (both are linear in it).  B8 T1024 C2048: 143 + 60 us.
+// through the same two tiles as at R = 32, and gxx and gxm take each part's share (both are linear in it).  B8 T1024 C2048: 136 + 60 us.
 // (Tiles of all 320 columns fit once: filled from memory between two barriers in every step, 181 + 63 us.  Now 15 registers of the first
 // launch are in scratch memory, 3 at R = 32.)
 // ------------------------------------------------------------------------------------------
